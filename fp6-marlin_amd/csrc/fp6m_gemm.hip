@@ -109,7 +109,6 @@ struct DeviceState {
     unsigned char* slot_scratch = nullptr;   // ... and of g_slot_scratch
     unsigned char* pool = nullptr;           // kStaticSlots regions from one hipMalloc (see workspace_region)
     unsigned long long tick = 0;
-    void* pack_temp = nullptr;      // kPackTempBytes for the on-GPU packer's flag and column maxima
     Region regions[kMaxRegions];
 };
 DeviceState g_devices[kMaxDevices];
@@ -318,22 +317,6 @@ int workspace_region(int dev, const void* workspace, bool want_region, bool want
     out->region = (int)(r - d->regions);
     out->partials = r->partials;
     out->gathered = r->gathered;
-    return FP6M_OK;
-}
-
-// Scratch of the on-GPU packer (fp6m_pack.hip): one buffer per device (a pack call waits for its kernels).
-int pack_temp(int dev, void** ptr)
-{
-    std::lock_guard<std::mutex> lock(g_scratch_mutex);
-    DeviceState* d = nullptr;
-    if (int rc = device_state(dev, &d)) return rc;
-    if (!d->pack_temp) {
-        void* mem = nullptr;
-        const hipError_t e = on_device(dev, [&] { return hipMalloc(&mem, kPackTempBytes); });
-        if (e != hipSuccess) return hip_fail(e);
-        d->pack_temp = mem;
-    }
-    *ptr = d->pack_temp;
     return FP6M_OK;
 }
 

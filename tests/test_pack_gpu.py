@@ -41,6 +41,25 @@ def test_device_pack_matches_host_pack(k, n, qc, gs, harness):
     assert same_values(rd, rh)
 
 
+@pytest.mark.parametrize("k,n,qc,gs", [(64, 64, -1, -1), (192, 320, 64, 64), (960, 512, 64, 48), (320, 512, 256, 16), (576, 448, 192, -1),
+                                       (128, 832, 64, 128), (8256, 192, 64, -1), (512, 1088, 320, 512)])
+def test_device_pack_at_the_edges_of_its_workgroups(k, n, qc, gs):
+    """Regions that end inside a workgroup's 256 columns, rows that end inside its 128, every kind of scale group, more row
+    ranges than one for the column maxima; INT4 scales down to zero and through the sub-normal range.  Bit for bit."""
+    import fp6_marlin
+    g = torch.Generator().manual_seed(k + 3 * n)
+    w = torch.randn((k, n), generator=g) * 0.02
+    n4 = n - max(qc, 0)
+    w[:, :n4:5] *= 2.0 ** -torch.randint(0, 16, (1, w[:, :n4:5].shape[1]), generator=g).float()
+    w = w.half()
+    w[:, 9] = 0.0
+    Bh, sh, rh = fp6_marlin.pack_mixed_weight(w, qc, gs, harness_layout=False)
+    Bd, sd, rd = fp6_marlin.pack_mixed_weight(w.to(dev()), qc, gs, harness_layout=False)
+    assert torch.equal(Bd.cpu(), Bh)
+    assert same_bits(sd, sh)
+    assert same_values(rd, rh)
+
+
 def test_every_fp6_code_and_range_errors():
     """A column whose largest magnitude is 28 has scale 1, so its entries are cast as they are: feed every
     binary16 pattern inside [0.0625, 28] (and both zeros) through the GPU cast and compare with the host's."""
