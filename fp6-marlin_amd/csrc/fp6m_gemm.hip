@@ -38,6 +38,7 @@
 #include "gemm_m16.h"
 #include "gemm_sk.h"
 #include "gemm_mb.h"
+#include "gemm_wide.h"
 
 namespace fp6m {
 
@@ -66,7 +67,7 @@ thread_local int g_last_hip_error = 0;
 constexpr int kUnset = INT32_MIN;
 const int g_env_verbose = getenv("FP6M_VERBOSE") ? 1 : 0;
 struct Tuning {
-    int mb = kUnset, ksplit = kUnset, wk16 = kUnset, wk = kUnset, pair = kUnset, wgs = kUnset, share = kUnset, share6 = kUnset, sk = kUnset, cap = kUnset, gather = kUnset, cells = kUnset, xcd = kUnset, gen = kUnset, gen2 = kUnset, gen3 = kUnset, young = kUnset, cls = kUnset, cus = kUnset, cap2 = kUnset;
+    int mb = kUnset, ksplit = kUnset, wk16 = kUnset, wk = kUnset, pair = kUnset, wgs = kUnset, share = kUnset, share6 = kUnset, sk = kUnset, cap = kUnset, gather = kUnset, cells = kUnset, xcd = kUnset, gen = kUnset, gen2 = kUnset, gen3 = kUnset, young = kUnset, cls = kUnset, cus = kUnset, cap2 = kUnset, wide = kUnset;
     int verbose = g_env_verbose;
 };
 Tuning g_tuning;
@@ -439,6 +440,18 @@ void launch_mb_one(const GemmArgs& a, dim3 grid, hipStream_t stream)
     hipLaunchKernelGGL(kernel, grid, dim3(64 * WK), 0, stream, a);
 }
 
+template <int MB, int WN, int WK>
+void launch_wide(const WideArgs& a, bool g128, hipStream_t stream)
+{
+    const dim3 grid((unsigned)(a.n / (64 * WN)), (unsigned)((a.m + 16 * MB - 1) / (16 * MB)));
+    void (*kernel)(const WideArgs) = nullptr;
+    if (a.fused || a.native)
+        kernel = g128 ? gemm_wide_kernel<true, MB, WN, WK, true> : gemm_wide_kernel<false, MB, WN, WK, true>;
+    else
+        kernel = g128 ? gemm_wide_kernel<true, MB, WN, WK, false> : gemm_wide_kernel<false, MB, WN, WK, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * WN * WK), 0, stream, a);
+}
+
 // LEAN: the kernels the dispatcher picks by itself also exist without the extras (those only the tuning hook reaches do not).
 template <int MB, int D4, int D6, bool PAIR, bool LEAN = true>
 void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stream)
@@ -456,6 +469,76 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
     }
 }
 
+// Whether a launch of more than 16 rows goes to gemm_wide_kernel, and with which tile: 1 .. 5, or 0 (gemm_mb_kernel).
+//
+// The wide kernel's tiles (128 or fewer rows x 256 columns, all of k) are large, so what decides is how their number
+// divides into rounds: one workgroup of eight waves per CU (two k slices), or two of four waves (no k split).  Neither
+// kernel nor tile wins everywhere, and the lines follow no simple rule, so each plan's time is estimated and the smallest
+// taken: a start, so much per full round and k, so much for the last, partly filled round (a CU clocks higher while
+// others idle, so that part is not simply a fraction).  The constants are least-squares fits to 1830 random shapes (48 ..
+// 3000 rows, k and n from 2048, both scale modes; 1 us and 4096 rows of k are the units); they reproduce the plans' times
+// to 3-7 %, the plan they choose is 0.3 % off the best on average, and it took 11.8 % off the time of gemm_mb_kernel over
+// all of them, 18 % between 700 and 1200 rows (from 129 to 256 rows 6.9 %, below 65 rows none: not asked).  Two shapes in 1830
+// lost more than 4 %; hence the 3 % that the wide kernel must win by.  Nothing was fitted below k = 2048, where starts and
+// ends are most of the time: not asked either.
+struct WidePlan {
+    int mb, per_cu;               // 16-row blocks per tile; workgroups per CU
+    double start, round, part;    // us: once; per full round; once if the last round is not full
+    double full, full_g;          // us per 4096 rows of k: a full round, what group scales add
+    double low, low_g, low_slope, low_slope_g;   // the last round: up to one workgroup per CU, and per CU filled
+    double high, high_g, high_slope;             // (two per CU:) from one to two workgroups per CU
+};
+constexpr WidePlan kWidePlans[] = {
+    {8, 2, 10.8, 6.9, -6.3, 81.4, 12.1, 50.3, 1.9, 8.0, 0.0, 73.4, 7.6, 24.9},
+    {8, 1, 6.7, 7.7, 0.9, 43.1, 6.6, 36.6, -0.5, 6.5, 4.9, 0, 0, 0},
+    {7, 1, 4.3, 7.5, 3.1, 38.5, 5.2, 33.8, -0.1, 5.7, 4.4, 0, 0, 0},
+    {6, 1, 6.4, 6.6, 0.3, 34.5, 6.4, 31.6, 1.0, 5.0, 3.1, 0, 0, 0},
+    {6, 2, 35.5, 7.2, -30.5, 65.2, 10.0, 44.1, 1.2, 3.3, 0.0, 60.6, 7.3, 19.1},
+};
+inline int wide_plan(int m, int n, int k, bool g128, int mb, int max_par, int cus)
+{
+    if (m <= 64 || k < 2048) return 0;
+    const double kk = k / 4096.0, g = g128 ? 1.0 : 0.0;
+    // gemm_mb_kernel, launch by launch: 128-row tiles come in rounds of one workgroup per CU, 64-row tiles of two (or, if
+    // one per CU is all there is, with the k range split over the idle CUs).
+    double us = 0;
+    const int tile_rows = 16 * mb, tiles_n = n / kTileN;
+    for (int left = (m + tile_rows - 1) / tile_rows; left > 0; left -= max_par) {
+        const long long wgs = (long long)tiles_n * (left < max_par ? left : max_par);
+        us += 7.0;
+        if (mb == 8) {
+            const long long full = wgs / cus, rem = wgs % cus;
+            us += kk * (full * (28.0 + 3.2 * g) + (rem ? 16.4 : 0.0) + 10.6 * rem / cus) + 4.8 * (full + (rem ? 1 : 0));
+        } else if (wgs <= cus) {
+            const double ks = (double)(cus / wgs);
+            us += kk / ks * (11.8 + 5.4 * wgs * ks / cus) + (ks > 1 ? 4.1 : 0.0);
+        } else {
+            const long long full = wgs / (2 * cus), rem = wgs % (2 * cus);
+            us += kk * full * (35.1 + 4.9 * g) + kk * (rem == 0 ? 0.0 : (rem <= cus ? 11.9 : 26.8 + 10.7 * (rem - cus) / cus));
+        }
+    }
+    int best = 0;
+    us *= 0.97;
+    for (int i = 0; i < (int)(sizeof(kWidePlans) / sizeof(kWidePlans[0])); i++) {
+        const WidePlan& p = kWidePlans[i];
+        const long long tiles = (long long)(n / 256) * ((m + 16 * p.mb - 1) / (16 * p.mb));
+        const long long slots = (long long)p.per_cu * cus, full = tiles / slots, rem = tiles % slots;
+        double t = p.start + full * p.round + kk * full * (p.full + p.full_g * g);
+        if (rem) {
+            t += p.part;
+            if (rem <= cus)
+                t += kk * (p.low + p.low_g * g + (p.low_slope + p.low_slope_g * g) * rem / cus);
+            else
+                t += kk * (p.high + p.high_g * g + p.high_slope * (rem - cus) / cus);
+        }
+        if (t < us) {
+            us = t;
+            best = i + 1;
+        }
+    }
+    return best;
+}
+
 }  // namespace fp6m
 
 extern "C" {
@@ -471,7 +554,7 @@ int fp6m_tuning_set(const char* knob, int value)
     }
     const struct { const char* name; int* field; } knobs[] = {
         {"mb", &g_tuning.mb}, {"ksplit", &g_tuning.ksplit},
-        {"wk16", &g_tuning.wk16}, {"wk", &g_tuning.wk}, {"pair", &g_tuning.pair}, {"wgs", &g_tuning.wgs}, {"share", &g_tuning.share}, {"share6", &g_tuning.share6}, {"cap", &g_tuning.cap}, {"sk", &g_tuning.sk}, {"gather", &g_tuning.gather}, {"cells", &g_tuning.cells}, {"xcd", &g_tuning.xcd}, {"gen", &g_tuning.gen}, {"gen2", &g_tuning.gen2}, {"gen3", &g_tuning.gen3}, {"young", &g_tuning.young}, {"cls", &g_tuning.cls}, {"cus", &g_tuning.cus}, {"cap2", &g_tuning.cap2},
+        {"wk16", &g_tuning.wk16}, {"wk", &g_tuning.wk}, {"pair", &g_tuning.pair}, {"wgs", &g_tuning.wgs}, {"share", &g_tuning.share}, {"share6", &g_tuning.share6}, {"cap", &g_tuning.cap}, {"sk", &g_tuning.sk}, {"gather", &g_tuning.gather}, {"cells", &g_tuning.cells}, {"xcd", &g_tuning.xcd}, {"gen", &g_tuning.gen}, {"gen2", &g_tuning.gen2}, {"gen3", &g_tuning.gen3}, {"young", &g_tuning.young}, {"cls", &g_tuning.cls}, {"cus", &g_tuning.cus}, {"cap2", &g_tuning.cap2}, {"wide", &g_tuning.wide},
         {"verbose", &g_tuning.verbose}};
     for (const auto& k : knobs)
         if (!strcmp(knob, k.name)) {
@@ -670,6 +753,48 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             wgs8 * ks8 >= wgs4 && ks8 <= prob_k / (16LL * 128) &&
             (size_t)(tiles_n + qc / kTileN) * ((rows8 + 127) / 128) * ks8 * (8 * 16 * kTileN * sizeof(float)) <= scratch_bytes)
             mb = 8;
+    }
+    // Many rows (gemm_wide.h): one launch over all of them, without a k split across workgroups.
+    if (prob_m > 16 && !row_mix && prob_k % 128 == 0 && prob_n % 256 == 0 && (!fu.a_cols || (size_t)prob_m * prob_k * sizeof(uint16_t) <= kGatherBytes)) {
+        const bool free_plan = tune.mb == kUnset && tune.ksplit == kUnset && tune.wk == kUnset && tune.pair == kUnset && tune.cls == kUnset && sms <= 0;
+        int plan = tune.wide != kUnset ? tune.wide : (free_plan ? wide_plan(prob_m, prob_n, prob_k, g128, mb, max_par, cus) : 0);
+        if (plan > 0) {
+            WideArgs w;
+            w.A = static_cast<const uint16_t*>(A);
+            if (fu.a_cols) {
+                dim3 ggrid((unsigned)((prob_k / 2 + 255) / 256), (unsigned)prob_m);
+                hipLaunchKernelGGL(gather_a_kernel, ggrid, dim3(256), 0, st, w.A, fu.lda, fu.a_cols, sc.gathered, prob_k);
+                w.A = sc.gathered;
+            }
+            w.b_int4 = a.b_int4;
+            w.b_fp6_2 = a.b_fp6_2;
+            w.b_fp6_4 = a.b_fp6_4;
+            w.C = static_cast<uint16_t*>(C);
+            w.s_int4 = a.s_int4;
+            w.s_fp6 = a.s_fp6;
+            w.m = prob_m;
+            w.n = prob_n;
+            w.k = prob_k;
+            w.n4 = n4;
+            w.qc = qc;
+            w.tiles6 = a.tiles6;
+            w.tiles = a.tiles;
+            w.native = a.native;
+            w.c_cols = a.c_cols;
+            w.bias = a.bias;
+            w.residual = fu.residual;
+            w.fused = a.fused;
+            if (tune.verbose) fprintf(stderr, "fp6m_mul m=%d n=%d k=%d: wide, plan %d\n", prob_m, prob_n, prob_k, plan);
+            switch (plan) {
+            case 1: launch_wide<8, 4, 1>(w, g128, st); break;
+            case 2: launch_wide<8, 4, 2>(w, g128, st); break;
+            case 3: launch_wide<7, 4, 2>(w, g128, st); break;
+            case 4: launch_wide<6, 4, 2>(w, g128, st); break;
+            default: launch_wide<6, 4, 1>(w, g128, st); break;
+            }
+            hipError_t e = hipGetLastError();
+            return e != hipSuccess ? hip_fail(e) : FP6M_OK;
+        }
     }
     const int rows_per_tile = 16 * mb;
     const int mtiles_total = (prob_m + rows_per_tile - 1) / rows_per_tile;

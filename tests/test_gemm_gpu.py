@@ -295,6 +295,50 @@ def test_dispatch_picks_128_row_tiles_where_they_fill_the_chip(oracle, capfd):
         assert want in err, (m, n, want, err[-400:])
 
 
+@pytest.mark.parametrize("plan", [1, 2, 3, 4, 5])
+def test_waves_side_by_side_in_n(oracle, plan):
+    """The many-rows kernel (gemm_wide.h) in each of its tiles, forced onto small problems: ragged row tiles, a single
+    trip of its loop (with two k slices: an idle one), an odd number of trips, tiles that lie in both regions, all INT4,
+    all FP6, both scale modes, every row of a small max_par in its one launch, and one-hot rows bit for bit."""
+    e = {"FP6M_WIDE": plan}
+    for m in (17, 96, 128, 129, 300):
+        run(oracle, m, 512, 1024, qc=256, gs=128, env=e)
+        run(oracle, m, 512, 1024, qc=128, env=e)
+    run(oracle, 130, 256, 128, qc=-1, env=e)
+    run(oracle, 130, 768, 384, qc=128, gs=128, env=e)
+    run(oracle, 300, 512, 512, qc=512, max_par=2, env=e)
+    for gs in (-1, 128):
+        one_hot_case(oracle, 200, 768, 1152, 256, gs, {"wide": plan})
+
+
+@pytest.mark.parametrize("plan", [1, 4])
+def test_waves_side_by_side_in_n_with_maps_additions_and_the_gfx950_order(oracle, plan):
+    """The same kernel's build for fp6m_mul_fused: with nothing to add the reordered result is the plain one bit for bit
+    (both word orders), and the additions are rounded once."""
+    import fp6_marlin
+    m, n, k, qc, gs = 150, 768, 512, 256, 128
+    ref, B, s = problem(oracle, n, k, qc, gs)
+    g = torch.Generator().manual_seed(plan)
+    A = torch.randn((m, k), generator=g).half().to(dev())
+    c_cols = torch.randperm(n, generator=g).to(torch.int32).to(dev())
+    bias, residual = torch.randn(n, generator=g).half().to(dev()), torch.randn((m, n), generator=g).half().to(dev())
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    plain, moved, native, added = (torch.full((m, n), float("nan"), dtype=torch.half, device=dev()) for _ in range(4))
+    with fp6_marlin.cabi.tuning(wide=plan):
+        fp6_marlin.mul(A, B, plain, s, ws, qc, group_size=gs)
+        fp6_marlin.mul_fused(A, B, moved, s, ws, qc, gs, c_cols=c_cols)
+        Bn = fp6_marlin.repack_gfx950(B, k, n, qc)
+        fp6_marlin.mul_fused(A, Bn, native, s, ws, qc, gs, c_cols=c_cols, layout="gfx950")
+        fp6_marlin.mul_fused(A, B, added, s, ws, qc, gs, c_cols=c_cols, bias=bias, residual=residual)
+        torch.cuda.synchronize()
+    assert torch.equal(moved[:, c_cols.long()], plain) and torch.equal(native, moved)
+    want = torch.from_numpy(oracle.matmul_ref(A.cpu().numpy(), ref).astype(np.float32)).to(dev())
+    full = torch.empty_like(want)
+    full[:, c_cols.long()] = want
+    full += bias.float() + residual.float()
+    assert ((added.float() - full).abs().mean() / full.abs().mean()).item() <= TOL
+
+
 def test_eight_k_slices_per_workgroup(oracle):
     """The m > 16 kernel with eight waves (k slices) per workgroup, which small grids on long k pick by themselves
     (here: 8192 x 512 at m = 40), forced on and off on ragged shapes."""
