@@ -11,8 +11,8 @@ plus what the reference keeps in its test harness or lacks: ``Layer`` (pack / fo
 quantiser and packer, the scale permutation, the mixed-weight assembler, ``group_size=128`` scales and
 ``mul_fused`` (activation gather, output column scatter, bias and residual inside the GEMM call).
 Everything is computed by ``libfp6m.so`` (C ABI in include/fp6m.h: host packers in C++, GEMM in
-hand-written HIP for gfx950).  The four reference entry points go through ``_fp6m_torch``, a thin
-PyTorch-ROCm C++ extension over that C ABI; ``fp6_marlin.cabi`` binds the same ABI with ctypes.
+hand-written HIP for gfx950).  The four reference entry points, ``mul_fused``, ``mul_rows`` and ``Layer.forward`` go
+through ``_fp6m_torch``, a thin PyTorch-ROCm C++ extension over that C ABI; ``fp6_marlin.cabi`` binds the same ABI with ctypes.
 If either shared object is missing the import fails; there is no fallback.
 """
 from . import cabi
@@ -21,7 +21,7 @@ try:
 except ImportError as e:  # pragma: no cover
     raise ImportError("fp6_marlin/_fp6m_torch.so is missing or does not load: build it with "
                       "`python fp6-marlin_amd/build.py`; there is no fallback implementation") from e
-from .cabi import init, init_workspace, release_workspace, workspace_elems, pack_mixed_weight_device, mul_fused, mul_rows, check_column_map, repack_gfx950, repack_gfx950_host
+from .cabi import init, init_workspace, release_workspace, workspace_elems, pack_mixed_weight_device, check_column_map, repack_gfx950, repack_gfx950_host
 from .layer import Layer, shared_workspace, pack_mixed_weight, pack_row_mix_weight, int4_quantize, int4_pack, permute_scales, unpack_to_fp16
 
 __all__ = ["shared_workspace", "prepacking", "quantize", "dequantize", "mul", "Layer", "pack_mixed_weight", "pack_mixed_weight_device", "int4_quantize",
@@ -62,3 +62,28 @@ def mul(A, B, C, s, workspace, quant_cols=-1, thread_k=-1, thread_n=-1, sms=-1, 
     group_size -1: per-column INT4 scales; 128: INT4 scales [k/128, n-quant_cols] in natural column order
     """
     return _ext.mul(A, B, C, s, workspace, quant_cols, thread_k, thread_n, sms, max_par, group_size)
+
+
+def _extended(name, A, B, C, s, workspace, quant_cols, group_size, quant_rows, a_cols, c_cols, bias, residual, sms, max_par, layout):
+    if layout not in ("reference", "gfx950"):
+        raise ValueError("layout must be 'reference' or 'gfx950'")
+    try:
+        _ext.mul_extended(A, B, C, s, workspace, quant_cols, group_size, quant_rows, a_cols, c_cols, bias, residual, sms, max_par,
+                          layout == "gfx950")
+    except TypeError as e:                                             # (an operand that is no tensor, a size that is no integer)
+        raise RuntimeError(f"{name}: {e}") from None
+
+
+def mul_fused(A, B, C, s, workspace, quant_cols=-1, group_size=-1, a_cols=None, c_cols=None, bias=None, residual=None,
+              sms=-1, max_par=16, layout="reference"):
+    _extended("mul_fused", A, B, C, s, workspace, quant_cols, group_size, 0, a_cols, c_cols, bias, residual, sms, max_par, layout)
+
+
+def mul_rows(A, B, C, s, workspace, quant_rows, a_cols=None, c_cols=None, bias=None, residual=None, sms=-1, max_par=16,
+             layout="reference"):
+    if int(quant_rows) <= 0:
+        raise RuntimeError("quant_rows must be positive and below k")
+    _extended("mul_rows", A, B, C, s, workspace, -1, 128, int(quant_rows), a_cols, c_cols, bias, residual, sms, max_par, layout)
+
+
+mul_fused.__doc__, mul_rows.__doc__ = cabi.mul_fused.__doc__, cabi.mul_rows.__doc__

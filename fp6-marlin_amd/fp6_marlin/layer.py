@@ -6,6 +6,7 @@ harness (test.py:13-152) and has no ``Layer``; here they are library functions b
 import torch
 import torch.nn as nn
 
+from . import _fp6m_torch as _ext
 from . import cabi
 
 int4_quantize = cabi.int4_quantize
@@ -252,19 +253,13 @@ class Layer(nn.Module):
         """y = x @ W (+ bias) (+ residual, float16 of y's shape), as one GEMM call.  ``workspace``: a zeroed int32 CUDA
         tensor of at least outfeatures // 128 * 16 elements that no overlapping call uses (default: the device's
         ``shared_workspace``)."""
-        x2 = x.reshape(-1, x.shape[-1]).to(torch.float16).contiguous()
-        out = torch.empty((x2.shape[0], self.n), dtype=torch.float16, device=x2.device)
-        res = None if residual is None else residual.reshape(-1, self.n).to(torch.float16).contiguous()
+        buffers = self._buffers                                        # (straight from the table: attribute look-ups add up)
         if workspace is None:
-            workspace = shared_workspace(x2.device, self.n // 128 * 16)
-        elif workspace.numel() < self.n // 128 * 16 or workspace.device != x2.device:
+            workspace = _workspaces.get(x.device.index)
+            if workspace is None or workspace.numel() < self.n // 128 * 16:
+                workspace = shared_workspace(x.device, self.n // 128 * 16)
+        elif workspace.numel() < self.n // 128 * 16 or workspace.device != x.device:
             raise ValueError("workspace must be an int32 tensor of at least outfeatures // 128 * 16 elements on x's device")
-        if self.quant_rows:
-            cabi.mul_rows(x2, self.B, out, self.s, workspace, self.quant_rows, a_cols=self.a_cols, bias=self.bias,
-                          residual=res, layout=self.layout)
-        elif self.c_cols is None and self.bias is None and residual is None and self.layout == "reference":
-            cabi.mul(x2, self.B, out, self.s, workspace, self.quant_cols, -1, -1, -1, 16, self.groupsize)
-        else:
-            cabi.mul_fused(x2, self.B, out, self.s, workspace, self.quant_cols, self.groupsize, c_cols=self.c_cols,
-                           bias=self.bias, residual=res, layout=self.layout)
-        return out.reshape(x.shape[:-1] + (self.n,))
+        return _ext.layer_forward(x, residual, buffers["B"], buffers["s"], workspace, self.n, self.quant_cols, self.groupsize, self.quant_rows,
+                                  buffers.get("a_cols", self.__dict__.get("a_cols")), buffers.get("c_cols", self.__dict__.get("c_cols")),
+                                  buffers.get("bias", self.__dict__.get("bias")), self.layout == "gfx950")
