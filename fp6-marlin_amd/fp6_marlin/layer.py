@@ -253,13 +253,15 @@ class Layer(nn.Module):
         """y = x @ W (+ bias) (+ residual, float16 of y's shape), as one GEMM call.  ``workspace``: a zeroed int32 CUDA
         tensor of at least outfeatures // 128 * 16 elements that no overlapping call uses (default: the device's
         ``shared_workspace``)."""
-        buffers = self._buffers                                        # (straight from the table: attribute look-ups add up)
         if workspace is None:
             workspace = _workspaces.get(x.device.index)
             if workspace is None or workspace.numel() < self.n // 128 * 16:
                 workspace = shared_workspace(x.device, self.n // 128 * 16)
         elif workspace.numel() < self.n // 128 * 16 or workspace.device != x.device:
             raise ValueError("workspace must be an int32 tensor of at least outfeatures // 128 * 16 elements on x's device")
-        return _ext.layer_forward(x, residual, buffers["B"], buffers["s"], workspace, self.n, self.quant_cols, self.groupsize, self.quant_rows,
-                                  buffers.get("a_cols", self.__dict__.get("a_cols")), buffers.get("c_cols", self.__dict__.get("c_cols")),
-                                  buffers.get("bias", self.__dict__.get("bias")), self.layout == "gfx950")
+        buffers = self._buffers
+        # (nn.Module finds a registered tensor only after a failed look-up, so what the buffer table holds is taken from
+        # there; what it does not, such as a bias that became a Parameter, is an attribute like any other)
+        held = lambda name: buffers[name] if name in buffers else getattr(self, name)
+        return _ext.layer_forward(x, residual, held("B"), held("s"), workspace, self.n, self.quant_cols, self.groupsize, self.quant_rows,
+                                  held("a_cols"), held("c_cols"), held("bias"), self.layout == "gfx950")

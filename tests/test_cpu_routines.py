@@ -135,3 +135,21 @@ def test_results_do_not_depend_on_thread_count(oracle, monkeypatch):
         q = fp6_marlin.quantize(torch.from_numpy(w))
         outs.append((q.numpy().copy(), fp6_marlin.prepacking(q).numpy().copy()))
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("change", ["buffer", "plain", "parameter", "none"])
+def test_layer_forward_hands_over_the_bias_wherever_it_is_held(monkeypatch, change):
+    """`bias` may be a buffer, an attribute set after construction, or a Parameter that took a buffer's place."""
+    layer_module = __import__("fp6_marlin.layer", fromlist=["layer"])
+    layer = fp6_marlin.Layer(256, 512, groupsize=128, quant_cols=256, bias=change in ("buffer", "parameter"))
+    if change == "plain":
+        layer.bias = torch.ones(512, dtype=torch.float16)
+    if change == "parameter":
+        del layer.bias
+        layer.bias = torch.nn.Parameter(torch.ones(512, dtype=torch.float16), requires_grad=False)
+    seen = []
+    monkeypatch.setattr(layer_module._ext, "layer_forward", lambda *args: seen.append(args))
+    layer(torch.zeros(2, 256, dtype=torch.float16), workspace=torch.zeros(64, dtype=torch.int32))
+    (args,) = seen
+    assert args[2] is layer.B and args[3] is layer.s and args[9] is None and args[10] is None
+    assert args[11] is layer.bias and (args[11] is None) == (change == "none")
