@@ -440,15 +440,20 @@ void launch_mb_one(const GemmArgs& a, dim3 grid, hipStream_t stream)
     hipLaunchKernelGGL(kernel, grid, dim3(64 * WK), 0, stream, a);
 }
 
-template <int MB, int WN, int WK>
+// Workgroups of gemm_wide_kernel per row tile.
+inline int wide_columns(bool narrow6, int wn, int tiles6, int tiles)
+{
+    return narrow6 ? tiles6 + ((tiles - tiles6) & 1) + (tiles - tiles6) / 2 : tiles * 2 / wn;
+}
+template <int MB, int WN, int WK, bool NARROW6 = false>
 void launch_wide(const WideArgs& a, bool g128, hipStream_t stream)
 {
-    const dim3 grid((unsigned)(a.n / (64 * WN)), (unsigned)((a.m + 16 * MB - 1) / (16 * MB)));
+    const dim3 grid((unsigned)wide_columns(NARROW6, WN, a.tiles6, a.tiles), (unsigned)((a.m + 16 * MB - 1) / (16 * MB)));
     void (*kernel)(const WideArgs) = nullptr;
     if (a.fused || a.native)
-        kernel = g128 ? gemm_wide_kernel<true, MB, WN, WK, true> : gemm_wide_kernel<false, MB, WN, WK, true>;
+        kernel = g128 ? gemm_wide_kernel<true, MB, WN, WK, NARROW6, true> : gemm_wide_kernel<false, MB, WN, WK, NARROW6, true>;
     else
-        kernel = g128 ? gemm_wide_kernel<true, MB, WN, WK, false> : gemm_wide_kernel<false, MB, WN, WK, false>;
+        kernel = g128 ? gemm_wide_kernel<true, MB, WN, WK, NARROW6, false> : gemm_wide_kernel<false, MB, WN, WK, NARROW6, false>;
     hipLaunchKernelGGL(kernel, grid, dim3(64 * WN * WK), 0, stream, a);
 }
 
@@ -469,7 +474,7 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
     }
 }
 
-// Whether a launch of more than 16 rows goes to gemm_wide_kernel, and with which tile: 1 .. 5, or 0 (gemm_mb_kernel).
+// Whether a launch of more than 16 rows goes to gemm_wide_kernel, and with which tile: 1 .. 7, or 0 (gemm_mb_kernel).
 //
 // The wide kernel's tiles (128 or fewer rows x 256 columns, all of k) are large, so what decides is how their number
 // divides into rounds: one workgroup of eight waves per CU (two k slices), or two of four waves (no k split).  Neither
@@ -481,6 +486,13 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
 // all of them, 18 % between 700 and 1200 rows (from 129 to 256 rows 6.9 %, below 65 rows none: not asked).  Two shapes in 1830
 // lost more than 4 %; hence the 3 % that the wide kernel must win by.  Nothing was fitted below k = 2048, where starts and
 // ends are most of the time: not asked either.
+//
+// The last two plans (FP6 tiles in workgroups of their own) were fitted to 170 more shapes of 65 to 1600 rows with 256 FP6
+// columns, to 2-3 %; the seven plans' choice is again 0.3 % off the best there.  They are not asked where the extra
+// workgroups would start another round, nor where FP6 is more than a quarter of the columns: an all-FP6 weight has twice
+// the workgroups then (400 x 8192 x 10240: 93 us instead of 78).  Against gemm_mb_kernel they must win by 9 %: where that
+// kernel has exactly a round of 128-row tiles its estimate is too high (512 x 8192 x 8192 with per-column scales: 61 us, not
+// 68; the 80-row tiles 69).
 struct WidePlan {
     int mb, per_cu;               // 16-row blocks per tile; workgroups per CU
     double start, round, part;    // us: once; per full round; once if the last round is not full
@@ -494,8 +506,11 @@ constexpr WidePlan kWidePlans[] = {
     {7, 1, 4.3, 7.5, 3.1, 38.5, 5.2, 33.8, -0.1, 5.7, 4.4, 0, 0, 0},
     {6, 1, 6.4, 6.6, 0.3, 34.5, 6.4, 31.6, 1.0, 5.0, 3.1, 0, 0, 0},
     {6, 2, 35.5, 7.2, -30.5, 65.2, 10.0, 44.1, 1.2, 3.3, 0.0, 60.6, 7.3, 19.1},
+    {6, 1, 6.6, 6.9, 0.6, 33.6, 3.2, 27.4, 1.4, 5.5, 2.9, 0, 0, 0},
+    {5, 1, 6.3, 6.8, 0.3, 28.7, 4.3, 24.4, 3.5, 4.4, 1.7, 0, 0, 0},
 };
-inline int wide_plan(int m, int n, int k, bool g128, int mb, int max_par, int cus)
+constexpr int kWideNarrow = 5;    // from this row on: NARROW6
+inline int wide_plan(int m, int n, int k, int qc, bool g128, int mb, int max_par, int cus)
 {
     if (m <= 64 || k < 2048) return 0;
     const double kk = k / 4096.0, g = g128 ? 1.0 : 0.0;
@@ -521,8 +536,10 @@ inline int wide_plan(int m, int n, int k, bool g128, int mb, int max_par, int cu
     us *= 0.97;
     for (int i = 0; i < (int)(sizeof(kWidePlans) / sizeof(kWidePlans[0])); i++) {
         const WidePlan& p = kWidePlans[i];
-        const long long tiles = (long long)(n / 256) * ((m + 16 * p.mb - 1) / (16 * p.mb));
-        const long long slots = (long long)p.per_cu * cus, full = tiles / slots, rem = tiles % slots;
+        const bool narrow6 = i >= kWideNarrow;
+        const long long tiles_m = (m + 16 * p.mb - 1) / (16 * p.mb), slots = (long long)p.per_cu * cus;
+        const long long tiles = tiles_m * wide_columns(narrow6, 4, qc / kTileN, tiles_n), full = tiles / slots, rem = tiles % slots;
+        if (narrow6 && (4 * qc > n || (tiles + slots - 1) / slots > (tiles_m * (tiles_n / 2) + slots - 1) / slots)) continue;
         double t = p.start + full * p.round + kk * full * (p.full + p.full_g * g);
         if (rem) {
             t += p.part;
@@ -531,7 +548,7 @@ inline int wide_plan(int m, int n, int k, bool g128, int mb, int max_par, int cu
             else
                 t += kk * (p.high + p.high_g * g + p.high_slope * (rem - cus) / cus);
         }
-        if (t < us) {
+        if (t * (narrow6 && !best ? 1.06 : 1.0) < us) {
             us = t;
             best = i + 1;
         }
@@ -757,7 +774,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
     // Many rows (gemm_wide.h): one launch over all of them, without a k split across workgroups.
     if (prob_m > 16 && !row_mix && prob_k % 128 == 0 && prob_n % 256 == 0 && (!fu.a_cols || (size_t)prob_m * prob_k * sizeof(uint16_t) <= kGatherBytes)) {
         const bool free_plan = tune.mb == kUnset && tune.ksplit == kUnset && tune.wk == kUnset && tune.pair == kUnset && tune.cls == kUnset && sms <= 0;
-        int plan = tune.wide != kUnset ? tune.wide : (free_plan ? wide_plan(prob_m, prob_n, prob_k, g128, mb, max_par, cus) : 0);
+        int plan = tune.wide != kUnset ? tune.wide : (free_plan ? wide_plan(prob_m, prob_n, prob_k, qc, g128, mb, max_par, cus) : 0);
         if (plan > 0) {
             WideArgs w;
             w.A = static_cast<const uint16_t*>(A);
@@ -790,7 +807,9 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             case 2: launch_wide<8, 4, 2>(w, g128, st); break;
             case 3: launch_wide<7, 4, 2>(w, g128, st); break;
             case 4: launch_wide<6, 4, 2>(w, g128, st); break;
-            default: launch_wide<6, 4, 1>(w, g128, st); break;
+            case 5: launch_wide<6, 4, 1>(w, g128, st); break;
+            case 6: launch_wide<6, 4, 2, true>(w, g128, st); break;
+            default: launch_wide<5, 4, 2, true>(w, g128, st); break;
             }
             hipError_t e = hipGetLastError();
             return e != hipSuccess ? hip_fail(e) : FP6M_OK;

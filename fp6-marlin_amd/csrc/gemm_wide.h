@@ -278,30 +278,18 @@ struct WideArgs {
     static constexpr int k4 = 0;
 };
 
-// MB: 16-row blocks per tile; WN x WK waves: 64-column groups side by side x k slices; NS: stages of A in LDS.
-// EXTRAS = false: without the fused epilogue and the gfx950 word order.
-template <bool G128, int MB, int WN, int WK, bool EXTRAS>
-__global__ __launch_bounds__(64 * WN * WK, 2) void gemm_wide_kernel(const WideArgs args)
+// One workgroup: 64-column groups `group0` ..  of the tiles in launch order, FP6 first.
+// FP6 / INT4: which regions its waves may lie in.  EXTRAS = false: without the fused epilogue and the gfx950 word order.
+template <bool G128, int MB, int WN, int WK, bool EXTRAS, bool FP6, bool INT4>
+__device__ __forceinline__ void wide_workgroup(const WideArgs& p, unsigned char* smem, int group0)
 {
-    constexpr int kLds = wide_lds_bytes(MB, WN, WK);
-    static_assert(kLds <= 160 * 1024, "LDS of one CU");
-    __shared__ __attribute__((aligned(16))) unsigned char smem[kLds];
-    WideArgs p = args;
-    if constexpr (!EXTRAS) {
-        p.native = 0;
-        p.fused = 0;
-        p.c_cols = nullptr;
-        p.bias = nullptr;
-        p.residual = nullptr;
-    }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int wn = wave % WN, wk = wave / WN;
-    // Workgroups: x walks the columns (64 * WN at a time, the FP6 region first), contiguous ranges per XCD; y the row tiles.
-    const int group = __builtin_amdgcn_readfirstlane(xcd_contiguous_id(blockIdx.x, gridDim.x)) * WN + wn;   // 64-column group
+    const int group = __builtin_amdgcn_readfirstlane(group0) + wn;
     TileInfo ti;
     ti.tile = group >> 1;
     const int sigma = group & 1;
-    ti.fp6 = ti.tile < p.tiles6;
+    ti.fp6 = FP6 && (!INT4 || ti.tile < p.tiles6);
     ti.tcol = ti.fp6 ? ti.tile : ti.tile - p.tiles6;
     ti.region_n = ti.fp6 ? p.qc : p.n4;
     ti.mtile = blockIdx.y;
@@ -318,10 +306,10 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_wide_kernel(const WideAr
 #pragma unroll
         for (int f = 0; f < 4; f++) acc[blk][f] = f4{0.f, 0.f, 0.f, 0.f};
     const uint32_t ring = uniform32(lds_addr(smem)) + wk * (3 * wide_slot_bytes(MB));
-    if (ti.fp6)
-        wide_stream<true, G128, MB, WN>(p, ti, sigma, wn, ring, begin, trips, most, acc);
+    if (FP6 && (!INT4 || ti.fp6))
+        wide_stream<FP6, G128, MB, WN>(p, ti, sigma, wn, ring, begin, trips, most, acc);
     else
-        wide_stream<false, G128, MB, WN>(p, ti, sigma, wn, ring, begin, trips, most, acc);
+        wide_stream<!INT4, G128, MB, WN>(p, ti, sigma, wn, ring, begin, trips, most, acc);
 
     // ---- epilogue: lane 16 q + c holds row c of a block, columns 32 (q >> 1) + 16 jp + 8 half + 4 (q & 1) + 0 .. 3
     const int q = lane >> 4, c = lane & 15;
@@ -410,6 +398,42 @@ __global__ __launch_bounds__(64 * WN * WK, 2) void gemm_wide_kernel(const WideAr
                 store_block(r * WK + wk, sum);
             }
         }
+    }
+}
+
+// MB: 16-row blocks per tile; WN x WK waves: 64-column groups side by side x k slices.
+// NARROW6: FP6 tiles (and the INT4 tile left over where the rest is an odd number of tiles) are workgroups of their own,
+// 128 columns x four k slices instead of 256 x two.  An FP6 step dequantises for twice as long as an INT4 step, and where the
+// whole launch is one round that workgroup is the one it waits for: with 256 FP6 columns 400 x 8192 x 10240 in 80-row tiles
+// took 76.6 us with per-column scales and 76.9 with group scales, without any 60.4 and 70.4; like this 64.7 and 72.7.  (Four
+// slices of tiles above 96 rows do not fit the LDS.)
+template <bool G128, int MB, int WN, int WK, bool NARROW6, bool EXTRAS>
+__global__ __launch_bounds__(64 * WN * WK, 2) void gemm_wide_kernel(const WideArgs args)
+{
+    static_assert(!NARROW6 || (WN == 4 && WK == 2), "eight waves either way");
+    constexpr int kLds = max3(wide_lds_bytes(MB, WN, WK), NARROW6 ? wide_lds_bytes(MB, 2, 4) : 0, 0);
+    static_assert(kLds <= 160 * 1024, "LDS of one CU");
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kLds];
+    WideArgs p = args;
+    if constexpr (!EXTRAS) {
+        p.native = 0;
+        p.fused = 0;
+        p.c_cols = nullptr;
+        p.bias = nullptr;
+        p.residual = nullptr;
+    }
+    // Workgroups: x walks the columns (the FP6 region first), contiguous ranges per XCD; y the row tiles.
+    const int x = __builtin_amdgcn_readfirstlane(xcd_contiguous_id(blockIdx.x, gridDim.x));
+    if constexpr (NARROW6) {
+        const int odd = (p.tiles - p.tiles6) & 1;         // (an INT4 tile that has no other to lie beside)
+        if (x < p.tiles6)
+            wide_workgroup<G128, MB, 2, 4, EXTRAS, true, false>(p, smem, 2 * x);
+        else if (x < p.tiles6 + odd)
+            wide_workgroup<G128, MB, 2, 4, EXTRAS, false, true>(p, smem, 2 * x);
+        else
+            wide_workgroup<G128, MB, WN, WK, EXTRAS, false, true>(p, smem, 2 * (p.tiles6 + odd) + 4 * (x - p.tiles6 - odd));
+    } else {
+        wide_workgroup<G128, MB, WN, WK, EXTRAS, true, true>(p, smem, x * WN);
     }
 }
 

@@ -295,7 +295,7 @@ def test_dispatch_picks_128_row_tiles_where_they_fill_the_chip(oracle, capfd):
         assert want in err, (m, n, want, err[-400:])
 
 
-@pytest.mark.parametrize("plan", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("plan", [1, 2, 3, 4, 5, 6, 7])
 def test_waves_side_by_side_in_n(oracle, plan):
     """The many-rows kernel (gemm_wide.h) in each of its tiles, forced onto small problems: ragged row tiles, a single
     trip of its loop (with two k slices: an idle one), an odd number of trips, tiles that lie in both regions, all INT4,
@@ -311,7 +311,7 @@ def test_waves_side_by_side_in_n(oracle, plan):
         one_hot_case(oracle, 200, 768, 1152, 256, gs, {"wide": plan})
 
 
-@pytest.mark.parametrize("plan", [1, 4])
+@pytest.mark.parametrize("plan", [1, 4, 7])
 def test_waves_side_by_side_in_n_with_maps_additions_and_the_gfx950_order(oracle, plan):
     """The same kernel's build for fp6m_mul_fused: with nothing to add the reordered result is the plain one bit for bit
     (both word orders), and the additions are rounded once."""
