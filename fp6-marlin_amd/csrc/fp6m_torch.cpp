@@ -187,8 +187,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("mul", &mul, "mixed INT4/FP6 x FP16 GEMM (gfx950)", py::arg("A"), py::arg("B"), py::arg("C"), py::arg("s"),
           py::arg("workspace"), py::arg("quant_cols") = -1, py::arg("thread_k") = -1, py::arg("thread_n") = -1,
           py::arg("sms") = -1, py::arg("max_par") = 8, py::arg("group_size") = -1);
-    m.def("mul_extended", &mul_extended, "the GEMM with gather, scatter, bias and residual; column or row mix (gfx950)");
-    m.def("layer_forward", &layer_forward, "one quantised linear layer (gfx950)");
+    // (without the interpreter's lock: a launch may block, and another Python thread may be driving another stream)
+    m.def("mul_extended", &mul_extended, "the GEMM with gather, scatter, bias and residual; column or row mix (gfx950)",
+          py::call_guard<py::gil_scoped_release>());
+    m.def("layer_forward", &layer_forward, "one quantised linear layer (gfx950)", py::call_guard<py::gil_scoped_release>());
     m.def("quantization_cpu", &quantization_cpu, "Weight quantization (CPU)");
     m.def("prepacking_cpu", &prepacking_cpu, "Weight prepacking (CPU)");
     m.def("dequantization_cpu", &dequantization_cpu, "Weight dequantization (CPU)");

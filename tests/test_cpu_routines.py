@@ -153,3 +153,38 @@ def test_layer_forward_hands_over_the_bias_wherever_it_is_held(monkeypatch, chan
     (args,) = seen
     assert args[2] is layer.B and args[3] is layer.s and args[9] is None and args[10] is None
     assert args[11] is layer.bias and (args[11] is None) == (change == "none")
+
+
+@pytest.mark.parametrize("entry", ["layer_forward", "mul_extended"])
+def test_the_native_calls_let_other_python_threads_run(entry):
+    """A launch may block (a full queue, a first call that allocates), and a thread that drives another stream must be able
+    to go on meanwhile.  The interpreter is told never to take the lock from a running thread, so the other thread runs only
+    if the call itself lets go of it.  (The calls end at their first operand check: no GPU is needed.)"""
+    import sys
+    import threading
+
+    x, f = torch.zeros((64, 256), dtype=torch.float16), fp6_marlin._ext
+    words, scales, out = torch.zeros(256, dtype=torch.int32), torch.zeros(256, dtype=torch.float16), torch.zeros((64, 256), dtype=torch.float16)
+    if entry == "layer_forward":
+        call = lambda: f.layer_forward(x, None, words, scales, words, 256, -1, -1, 0, None, None, scales, False)
+    else:
+        call = lambda: f.mul_extended(x, words, out, scales, words, -1, -1, 0, None, None, None, None, -1, 16, False)
+    gate, ran = threading.Event(), []
+    other = threading.Thread(target=lambda: (gate.wait(), ran.append(True)))
+    other.start()
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        gate.set()
+        for _ in range(20000):
+            try:
+                call()
+            except RuntimeError:
+                pass
+            if ran:
+                break
+        in_time = bool(ran)
+    finally:
+        sys.setswitchinterval(interval)
+        other.join()
+    assert in_time
