@@ -25,6 +25,7 @@
 namespace fp6m {
 
 int hip_fail(hipError_t e);            // fp6m_gemm.hip: records the HIP error, returns FP6M_ERR_HIP
+bool capturing(hipStream_t stream);    // fp6m_gemm.hip
 
 namespace {
 
@@ -523,13 +524,15 @@ __global__ void fp6_pack_harness_kernel(const uint16_t* w, int k, int n, int n4,
 
 // The FP6 range flag of a call: a word of pinned host memory that the kernels write (only when something is out of
 // range) and the call reads after its wait, so that no copy back is enqueued.  kFlags words, allocated once and kept; a
-// call holds one of them, so calls on several threads and streams do not meet.
+// call holds one of them, so calls on several threads and streams do not meet.  A word goes back only after a wait that
+// succeeded: until then kernels of this call may still write it, and the next call's check would see that.
 constexpr int kFlags = 64;
 std::mutex g_flag_mutex;
 int* g_flags = nullptr;
-unsigned long long g_flags_taken = 0;
+unsigned long long g_flags_taken = 0, g_flags_lost = 0;                  // (lost: taken for good)
 struct RangeFlag {
     int index = -1;
+    bool idle = true;                                                    // nothing enqueued may still write the word
     hipError_t err = hipSuccess;
     explicit RangeFlag(bool wanted)
     {
@@ -544,6 +547,10 @@ struct RangeFlag {
                     g_flags[index] = 0;
                     return;
                 }
+                if (!~g_flags_lost) {                                    // (64 calls whose wait failed)
+                    err = hipErrorOutOfMemory;
+                    return;
+                }
             }
             std::this_thread::yield();                                   // (64 other threads are inside a pack call)
         }
@@ -552,7 +559,16 @@ struct RangeFlag {
     {
         if (index < 0) return;
         std::lock_guard<std::mutex> lock(g_flag_mutex);
-        g_flags_taken &= ~(1ull << index);
+        if (idle)
+            g_flags_taken &= ~(1ull << index);
+        else
+            g_flags_lost |= 1ull << index;
+    }
+    hipError_t wait(hipStream_t st)
+    {
+        const hipError_t e = hipStreamSynchronize(st);
+        idle = e == hipSuccess;
+        return e;
     }
     int* ptr() const { return index < 0 ? nullptr : g_flags + index; }
 };
@@ -582,6 +598,7 @@ extern "C" int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_col
     uint32_t* plane2 = bp + (size_t)k * n4 / 8;
     uint32_t* plane4 = plane2 + (size_t)k * qc / 16;
     PackArgs a = {wp, k, n, n4, qc, g, (int)per_column, sp, s6, bp, plane2, plane4, rp, nullptr, 0, n4 ? (n4 + 255) / 256 : 1};
+    if (qc > 0 && capturing(st)) return hip_fail(hipErrorStreamCaptureUnsupported);   // (the wait below: refused before anything is recorded)
     RangeFlag flag(qc > 0);
     if (flag.err != hipSuccess) return hip_fail(flag.err);
     a.bad = flag.ptr();
@@ -610,13 +627,13 @@ extern "C" int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_col
         else
             hipLaunchKernelGGL(pack_kernel<false>, dim3(a.wgs6 + wgs4), dim3(512), 0, st, a);
     }
-    if (!qc) {
-        e = hipGetLastError();
-        return e != hipSuccess ? hip_fail(e) : FP6M_OK;
-    }
     e = hipGetLastError();
-    // the range check of the FP6 cast is reported by value, so this call waits for its kernels
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (qc) {
+        // the range check of the FP6 cast is reported by value, so this call waits for its kernels (after a failed launch for
+        // those in front of it: the flag's word is another call's next)
+        const hipError_t waited = flag.wait(st);
+        if (e == hipSuccess) e = waited;
+    }
     if (e != hipSuccess) return hip_fail(e);
-    return *const_cast<volatile int*>(flag.ptr()) ? FP6M_ERR_RANGE : FP6M_OK;
+    return qc && *const_cast<volatile int*>(flag.ptr()) ? FP6M_ERR_RANGE : FP6M_OK;
 }

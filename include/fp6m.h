@@ -290,7 +290,8 @@ int fp6m_unpack_to_fp16(const int32_t* B, const uint16_t* s, uint16_t* w_ref, si
  *            [quant_cols, k] without transposing); 0 = quantise the true transpose (what Layer.pack uses)
  * k % 64 == 0, quant_cols and n - quant_cols multiples of 64, group_size -1 or a divisor of k.
  * Enqueued on `stream`; when quant_cols > 0 the call waits for its kernels, because the FP6 range check
- * (FP6M_ERR_RANGE: a NaN weight or a zero-scale column in the harness layout) is reported by value. */
+ * (FP6M_ERR_RANGE: a NaN or infinite weight, or a zero-scale column in the harness layout) is reported by value, and is
+ * refused (FP6M_ERR_HIP) while `stream` is being captured. */
 int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_cols, int group_size, int harness_layout,
                            void* B, void* s, void* w_ref, int dev, void* stream);
 

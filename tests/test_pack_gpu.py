@@ -84,6 +84,48 @@ def test_every_fp6_code_and_range_errors():
         fp6_marlin.pack_mixed_weight(w.to(dev()), 96, -1)
 
 
+def test_a_pack_that_fails_at_its_launches_still_waits_for_them():
+    """The range flag's word goes to the next call, so nothing that may write it can be left on the stream, also where the
+    call reports a launch error (here one that an earlier HIP call of this thread left behind)."""
+    import ctypes
+    import fp6_marlin
+    lib = fp6_marlin.cabi.lib                                         # (its handle also finds the HIP runtime that it is linked to)
+    w = (torch.randn((4096, 2048), device=dev()) * 0.02).half()
+    want = fp6_marlin.pack_mixed_weight(w, 256, 128, harness_layout=False)
+    a = torch.randn((8192, 8192), device=dev())
+    torch.cuda.synchronize()
+    for _ in range(4):
+        a @ a                                                         # (tens of milliseconds in front of the packer's kernels)
+    assert lib.hipSetDevice(ctypes.c_int(10000)) != 0                 # no such device: the error stays with the thread
+    if lib.hipPeekAtLastError() == 0:
+        pytest.skip("this runtime does not keep the error of an earlier call")
+    with pytest.raises(RuntimeError):
+        fp6_marlin.cabi.pack_mixed_weight_device(w, 256, 128, False)
+    assert torch.cuda.current_stream().query()
+    got = fp6_marlin.pack_mixed_weight(w, 256, 128, harness_layout=False)
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_packing_fp6_columns_is_refused_under_capture():
+    """The call waits for its kernels, which a capture forbids; it says so, keeps no flag, and the capture goes on.  More
+    often than there are flags."""
+    import fp6_marlin
+    w = (torch.randn((256, 512), device=dev()) * 0.02).half()
+    want = fp6_marlin.pack_mixed_weight(w, 256, 128, harness_layout=False)
+    out = torch.zeros(4, device=dev())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(70):
+            with pytest.raises(RuntimeError):
+                fp6_marlin.cabi.pack_mixed_weight_device(w, 256, 128, False)
+        out.add_(1.0)
+    for i in range(3):
+        graph.replay()
+        got = fp6_marlin.pack_mixed_weight(w, 256, 128, harness_layout=False)
+        assert all(torch.equal(x, y) for x, y in zip(got, want)) and out.tolist() == [i + 1.0] * 4
+
+
 def test_fp6_scale_rule_vectors_through_the_gpu_packer():
     """The constructed columns of tests/fp6_scale_vectors.py (exact scales 1, 0.5, 0.0625; values around every e3m2
     grid point; entries below the 0.0625 threshold; a quotient that rounds above 28) through the on-GPU packer: scales
