@@ -509,6 +509,7 @@ constexpr WidePlan kWidePlans[] = {
     {6, 1, 6.6, 6.9, 0.6, 33.6, 3.2, 27.4, 1.4, 5.5, 2.9, 0, 0, 0},
     {5, 1, 6.3, 6.8, 0.3, 28.7, 4.3, 24.4, 3.5, 4.4, 1.7, 0, 0, 0},
 };
+constexpr int kWidePlanCount = sizeof(kWidePlans) / sizeof(kWidePlans[0]);
 constexpr int kWideNarrow = 5;    // from this row on: NARROW6
 inline int wide_plan(int m, int n, int k, int qc, bool g128, int mb, int max_par, int cus)
 {
@@ -534,7 +535,7 @@ inline int wide_plan(int m, int n, int k, int qc, bool g128, int mb, int max_par
     }
     int best = 0;
     us *= 0.97;
-    for (int i = 0; i < (int)(sizeof(kWidePlans) / sizeof(kWidePlans[0])); i++) {
+    for (int i = 0; i < kWidePlanCount; i++) {
         const WidePlan& p = kWidePlans[i];
         const bool narrow6 = i >= kWideNarrow;
         const long long tiles_m = (m + 16 * p.mb - 1) / (16 * p.mb), slots = (long long)p.per_cu * cus;
@@ -569,6 +570,7 @@ int fp6m_tuning_set(const char* knob, int value)
         g_tuning = fp6m::Tuning{};                                    // (`verbose` back to what FP6M_VERBOSE said at load time)
         return FP6M_OK;
     }
+    if (!strcmp(knob, "wide") && (value < 0 || value > fp6m::kWidePlanCount)) return FP6M_ERR_ARG;
     const struct { const char* name; int* field; } knobs[] = {
         {"mb", &g_tuning.mb}, {"ksplit", &g_tuning.ksplit},
         {"wk16", &g_tuning.wk16}, {"wk", &g_tuning.wk}, {"pair", &g_tuning.pair}, {"wgs", &g_tuning.wgs}, {"share", &g_tuning.share}, {"share6", &g_tuning.share6}, {"cap", &g_tuning.cap}, {"sk", &g_tuning.sk}, {"gather", &g_tuning.gather}, {"cells", &g_tuning.cells}, {"xcd", &g_tuning.xcd}, {"gen", &g_tuning.gen}, {"gen2", &g_tuning.gen2}, {"gen3", &g_tuning.gen3}, {"young", &g_tuning.young}, {"cls", &g_tuning.cls}, {"cus", &g_tuning.cus}, {"cap2", &g_tuning.cap2}, {"wide", &g_tuning.wide},

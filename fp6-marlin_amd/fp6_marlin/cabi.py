@@ -69,7 +69,7 @@ class tuning:
         for name, value in self.knobs.items():
             if lib.fp6m_tuning_set(name.encode(), int(value)) != OK:
                 lib.fp6m_tuning_set(None, 0)
-                raise ValueError(f"unknown tuning knob {name!r}")
+                raise ValueError(f"unknown tuning knob {name!r} or value {value!r}")
         return self
 
     def __exit__(self, *exc):

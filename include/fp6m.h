@@ -169,8 +169,9 @@ int fp6m_mul_rows(const void* A, int lda, const void* B, void* C, const void* s,
  * of the second wave of every SIMD in eight-wave workgroups relative to the first one's; 100 = equal slices),
  * "cls" (0: the kernels never put the INT4 tiles in two classes -- whole tiles on the first workgroups, the
  * rest in parts on later ones --, 1: wherever they can), "wide" (the many-rows kernel, whose waves lie side by side in n:
- * 0 never, 1 .. 7 always, with that tile), "cus" (tests: plan for a chip of that many CUs),
- * "verbose" (print every launch's configuration to stderr); knob = NULL clears all overrides.  Unknown knob ->
+ * 0 never, 1 .. 7 with that tile wherever it can: more than 16 rows, k a multiple of 128, n of 256, no row mix, and
+ * gathered activations of at most 64 MiB), "cus" (tests: plan for a chip of that many CUs),
+ * "verbose" (print every launch's configuration to stderr); knob = NULL clears all overrides.  Unknown knob or tile ->
  * FP6M_ERR_ARG.  Not synchronised with GEMM calls running on other threads.  The library reads no environment
  * variables on a call (FP6M_VERBOSE is looked up once at load time).
  */

@@ -34,3 +34,14 @@ def test_argument_validation_needs_no_gpu():
     assert L.fp6m_mul(z, z, z, z, 32, 256, 256, z, 0, z, 128, 128, -1, 16, -1, -1) == 2   # (128,128) needs m <= 16
     assert L.fp6m_mul(z, z, z, z, 0, 256, 256, z, 0, z, -1, -1, -1, 16, -1, -1) == 0      # empty problem
     assert L.fp6m_mul(z, z, z, z, 16, 256, 256, z, 0, z, -1, -1, -1, 16, -1, -1) == 5     # null pointers
+
+
+def test_the_many_rows_tile_is_refused_outside_its_table():
+    """A tile number that does not exist must not silently become another one."""
+    import fp6_marlin
+    L = fp6_marlin.cabi.lib
+    try:
+        assert [L.fp6m_tuning_set(b"wide", v) for v in (0, 1, 7)] == [0, 0, 0]
+        assert [L.fp6m_tuning_set(b"wide", v) for v in (8, 100, -1)] == [fp6_marlin.cabi.ERR_ARG] * 3
+    finally:
+        L.fp6m_tuning_set(None, 0)
