@@ -448,13 +448,24 @@ inline int wide_columns(bool narrow6, int wn, int tiles6, int tiles)
 template <int MB, int WN, int WK, bool NARROW6 = false>
 void launch_wide(const WideArgs& a, bool g128, hipStream_t stream)
 {
-    const dim3 grid((unsigned)wide_columns(NARROW6, WN, a.tiles6, a.tiles), (unsigned)((a.m + 16 * MB - 1) / (16 * MB)));
     void (*kernel)(const WideArgs) = nullptr;
     if (a.fused || a.native)
         kernel = g128 ? gemm_wide_kernel<true, MB, WN, WK, NARROW6, true> : gemm_wide_kernel<false, MB, WN, WK, NARROW6, true>;
     else
         kernel = g128 ? gemm_wide_kernel<true, MB, WN, WK, NARROW6, false> : gemm_wide_kernel<false, MB, WN, WK, NARROW6, false>;
-    hipLaunchKernelGGL(kernel, grid, dim3(64 * WN * WK), 0, stream, a);
+    // (a grid's second dimension ends at 65536: five million rows and more, which fit the memory, take several launches)
+    constexpr int kRows = 65535 * 16 * MB;
+    WideArgs p = a;
+    for (int left = a.m; left > 0; left -= kRows) {
+        p.m = left < kRows ? left : kRows;
+        const dim3 grid((unsigned)wide_columns(NARROW6, WN, a.tiles6, a.tiles), (unsigned)((p.m + 16 * MB - 1) / (16 * MB)));
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * WN * WK), 0, stream, p);
+        if (left > kRows) {
+            p.A += (size_t)kRows * a.k;
+            p.C += (size_t)kRows * a.n;
+            if (p.residual) p.residual += (size_t)kRows * a.n;
+        }
+    }
 }
 
 // LEAN: the kernels the dispatcher picks by itself also exist without the extras (those only the tuning hook reaches do not).

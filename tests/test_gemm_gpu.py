@@ -311,6 +311,26 @@ def test_waves_side_by_side_in_n(oracle, plan):
         one_hot_case(oracle, 200, 768, 1152, 256, gs, {"wide": plan})
 
 
+def test_waves_side_by_side_in_n_with_more_row_tiles_than_a_grid_takes(oracle):
+    """More than 65535 tiles of 80 rows: a second launch, whose rows of A, C and the residual are offset.  Every row of the
+    repeated block must come out as the block's own, bit for bit."""
+    import fp6_marlin
+    block, times, n, k = 1000, 5243, 256, 256                        # 65537.5 tiles
+    _, B, s = problem(oracle, n, k, 128, 128)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    A1 = torch.randn((block, k), generator=g, dtype=torch.half, device=dev())
+    R1 = torch.randn((block, n), generator=g, dtype=torch.half, device=dev())
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    A, R = A1.repeat(times, 1), R1.repeat(times, 1)
+    for residual in (False, True):
+        C1 = torch.full((block, n), float("nan"), dtype=torch.half, device=dev())
+        C = torch.full((block * times, n), float("nan"), dtype=torch.half, device=dev())
+        with fp6_marlin.cabi.tuning(wide=7):
+            fp6_marlin.mul_fused(A1, B, C1, s, ws, 128, 128, residual=R1 if residual else None)
+            fp6_marlin.mul_fused(A, B, C, s, ws, 128, 128, residual=R if residual else None)
+        assert torch.isfinite(C1).all() and bool((C.view(times, block, n) == C1).all())
+
+
 @pytest.mark.parametrize("plan", [1, 4, 7])
 def test_waves_side_by_side_in_n_with_maps_additions_and_the_gfx950_order(oracle, plan):
     """The same kernel's build for fp6m_mul_fused: with nothing to add the reordered result is the plain one bit for bit
