@@ -4,8 +4,9 @@ The GEMM loops never synchronise on data: a direct-to-LDS (or register) load is 
 `s_waitcnt vmcnt(N)` with a constant N allows only the N newest loads to be outstanding, and a ring slot is assumed free
 when its last reader has been waited for.  A count that is one too high, or a fetch one step too early, passes every GPU
 test on most runs, because loads usually land long before they are needed.  Here the issue / wait / read order of the
-loops (gemm_m16.h stream_tile; gemm_mb.h stream_tile_mb and stream_tile_mbp) is restated step by step and run on a
-memory that completes a load only when a wait forces it to (loads complete in issue order, as the counter assumes):
+loops (gemm_m16.h stream_tile; gemm_mb.h stream_tile_mb and stream_tile_mbp; gemm_wide.h wide_stream, whose waves share a
+ring) is restated step by step and run on a memory that completes a load only when a wait forces it to (loads complete in
+issue order, as the counter assumes):
 
 * every read of a step's words, activations or group scales finds the load that brought them complete;
 * no load is issued into a slot, register set or scale slab that still holds data somebody is going to read;
@@ -318,3 +319,196 @@ def test_paired_loop_notices_a_missing_wait(monkeypatch):
     monkeypatch.setattr(Memory, "wait", lenient)
     with pytest.raises(AssertionError, match="before its load completed"):
         run_mb_paired(12, group=False)
+
+
+# ------------------------------------------------------------------------- waves that share a ring (gemm_wide.h wide_stream)
+
+class Wave:
+    """One wave's loads and LDS reads, stamped (barriers passed, position in the wave's own program)."""
+
+    def __init__(self):
+        self.interval = self.position = 0
+        self.ops, self.done = [], 0           # loads in issue order: [place, what, issued, completed]
+        self.reads, self.read_done = [], 0    # LDS reads, likewise
+
+    def now(self):
+        self.position += 1
+        return (self.interval, self.position)
+
+    def load(self, place, what):
+        self.ops.append([place, what, self.now(), None])
+
+    def read_lds(self, places, what):
+        self.reads.append([places, what, self.now(), None])
+
+    def wait(self, vm=None, lds=None):
+        at = self.now()
+        assert vm is None or 0 <= vm <= 63
+        assert lds is None or 0 <= lds <= 15  # counts of read instructions, four to a block
+        if vm is not None:
+            for op in self.ops[self.done:max(self.done, len(self.ops) - vm)]:
+                op[3] = at
+            self.done = max(self.done, len(self.ops) - vm)
+        if lds is not None:
+            keep = lds // 4
+            for op in self.reads[self.read_done:max(self.read_done, len(self.reads) - keep)]:
+                op[3] = at
+            self.read_done = max(self.read_done, len(self.reads) - keep)
+
+    def landed(self, place, what):
+        """A register load: the newest one into `place` brought `what` and has completed."""
+        for op in reversed(self.ops):
+            if op[0] == place:
+                assert op[1] == what, f"{place} holds {op[1]}, not {what}"
+                assert op[3] is not None, f"read of {what} from {place} before its load completed"
+                return
+        raise AssertionError(f"nothing was loaded into {place}")
+
+
+def before(a, wave_a, b, wave_b):
+    """Whether stamp `a` is sure to come before stamp `b`: between two barriers the waves run in any order."""
+    return a is not None and (a < b if wave_a is wave_b else a[0] < b[0])
+
+
+def wide_wave(wn, WN, MB, trips, most, fp6, group, lenient_words=0, lenient_stage=0, skip_barrier=None):
+    """wide_stream: one wave's program.  A `stage` is 64 rows of k of the slice's A, a `step` 32 rows."""
+    w = Wave()
+    group = group and not fp6
+    n_a, n_w, n_s = ((2 * MB + WN - 1) // WN + 1) // 2 * 2, 4 if fp6 else 2, 4 if group else 0
+    ahead = 3 if MB > 3 else MB - 1
+    word_wait = 3 * n_w + 3 * (n_a // 2) + lenient_words
+    stage_wait = 2 * n_w + n_a + lenient_stage
+    assert word_wait - lenient_words + n_s <= 63
+    s = dict(step=0, stage=0, group=0, fill=0)
+    last_step, last_stage, last_group = max(4 * trips - 1, 0), max(2 * trips - 1, 0), max(trips - 1, 0)
+
+    def issue_w(reg_set):
+        for i in range(n_w):
+            w.load(("W", reg_set, i), s["step"])
+        s["step"] = min(s["step"] + 1, last_step)
+
+    def issue_a(x):
+        q = min(wn + WN * x, 2 * MB - 1)
+        w.load(("A", s["fill"], q), s["stage"])
+        if x == n_a - 1:
+            s["fill"] = (s["fill"] + 1) % 3
+            s["stage"] = min(s["stage"] + 1, last_stage)
+
+    def issue_scales():
+        for i in range(n_s):
+            w.load(("S", i), s["group"])
+        s["group"] = min(s["group"] + 1, last_group)
+
+    def words(reg_set, step):
+        for i in range(n_w):
+            w.landed(("W", reg_set, i), min(step, last_step))
+
+    def scales(g):
+        for i in range(n_s):
+            w.landed(("S", i), min(g, last_group))
+
+    def read_block(block, slot, stage):
+        w.read_lds([("A", slot, 2 * block), ("A", slot, 2 * block + 1)], min(stage, last_stage))
+
+    barriers = itertools.count()
+
+    def barrier():
+        if next(barriers) != skip_barrier:
+            w.interval += 1
+
+    if group:
+        issue_scales()
+    for reg_set in range(4):
+        issue_w(reg_set)
+        for x in range(n_a // 2):
+            issue_a((reg_set & 1) * (n_a // 2) + x)
+    w.wait(vm=n_a + 2 * n_w)
+    barrier()
+    for b in range(ahead):
+        read_block(b, 0, 0)
+    if group:
+        scales(0)
+    words(0, 0)
+    slot = 0
+    for trip in range(trips):
+        for u in range(4):
+            step = 4 * trip + u
+            if group and u == 0:
+                issue_scales()
+            issue_w(u)
+            w.wait(vm=word_wait + (0 if u == 3 else n_s))
+            if group and u == 3:
+                scales(trip + 1)
+            words((u + 1) & 3, step + 1)
+            for blk in range(MB):
+                nb = blk + ahead
+                x0, x1 = blk * (n_a // 2) // (MB - ahead + 1), (blk + 1) * (n_a // 2) // (MB - ahead + 1)
+                for x in range(x0, min(x1, n_a // 2)):
+                    issue_a((u & 1) * (n_a // 2) + x)
+                if nb == MB and u & 1:
+                    w.wait(vm=stage_wait + (n_s if u == 1 else 0), lds=0)
+                    barrier()
+                    slot = (slot + 1) % 3
+                # (the reads past the end find the repeated last stage)
+                read_block(nb if nb < MB else nb - MB, slot, step // 2 if nb < MB or not u & 1 else step // 2 + 1)
+                w.wait(lds=4 * ahead)
+            words((u + 1) & 3, step + 1)               # its last use: the set must still hold them
+    for _ in range(trips, most):
+        barrier()
+        barrier()
+    w.wait(vm=0, lds=0)
+    barrier()                                          # (in front of the epilogue, which writes over the ring)
+    w.end = (w.interval, 0)
+    return w
+
+
+def run_wide(WN, WK, MB, trips_all, fp6_waves, group, **planted):
+    """A workgroup: every slice's waves against each other."""
+    ends = set()
+    for wk in range(WK):
+        begin = trips_all * wk // WK
+        trips, most = trips_all * (wk + 1) // WK - begin, (trips_all + WK - 1) // WK
+        assert begin < trips_all                       # (a slice without a trip fetches its first stages all the same)
+        waves = [wide_wave(wn, WN, MB, trips, most, fp6_waves[wn], group, **planted) for wn in range(WN)]
+        loads, reads = {}, {}
+        for w in waves:
+            ends.add(w.interval)
+            assert w.done == len(w.ops) and w.read_done == len(w.reads)
+            for place, what, issued, done in w.ops:
+                if place[0] == "A":
+                    loads.setdefault(place, []).append((what, issued, done, w))
+            for places, what, issued, done in w.reads:
+                for place in places:
+                    reads.setdefault(place, []).append((what, issued, done, w))
+        for place, rs in reads.items():
+            for what, issued, done, w in rs:
+                # The loads of `what` that this read can see (past the end a stage is loaded more than once): all that are
+                # not sure to come after it.  One at least, each complete, and nothing else in the place in between.
+                mine = [l for l in loads[place] if not before(done, w, l[1], l[3])]
+                good = [l for l in mine if l[0] == what]
+                assert any(before(l[2], l[3], issued, w) for l in good), f"read of stage {what} from {place} before its load completed"
+                for l in mine:
+                    if l[0] == what:
+                        assert before(l[2], l[3], issued, w) or what == max(2 * trips - 1, 0), f"late load of stage {what} into {place}"
+                    else:
+                        assert all(before(l[2], l[3], g[1], g[3]) for g in good), f"load of stage {l[0]} into {place} while stage {what} is read from it"
+    assert len(ends) == 1                              # every wave of the workgroup meets the same barriers
+
+
+WIDE_TILES = [(4, 1, 8), (4, 2, 8), (4, 2, 7), (4, 2, 6), (4, 1, 6), (4, 2, 5), (2, 4, 6), (2, 4, 5)]   # launch_wide, NARROW6
+
+
+@pytest.mark.parametrize("WN,WK,MB", WIDE_TILES)
+def test_waves_that_share_a_ring(WN, WK, MB):
+    for trips_all in (1, 2, 3, 5, 8, 9):
+        for group in (True, False):
+            for fp6 in ([False] * WN, [True] * WN, [i < 2 for i in range(WN)]):
+                run_wide(WN, WK, MB, trips_all, fp6, group)
+
+
+@pytest.mark.parametrize("WN,WK,MB", WIDE_TILES)
+@pytest.mark.parametrize("planted", [{"lenient_words": 1}, {"lenient_stage": 1}, {"skip_barrier": 2}])
+def test_waves_that_share_a_ring_notice_a_planted_mistake(WN, WK, MB, planted):
+    """One load more in flight than either wait allows, or one barrier left out."""
+    with pytest.raises(AssertionError, match="before its load completed|late load|while stage"):
+        run_wide(WN, WK, MB, 9, [False] * WN, True, **planted)

@@ -1,13 +1,13 @@
-"""Static checks on the compiler's output for the hand-scheduled m > 16 kernel.
+"""Static checks on the compiler's output for the hand-scheduled m > 16 kernels.
 
-Its MFMAs and direct-to-LDS loads are inline asm, so the compiler's hazard recogniser does not see them; the
+Their MFMAs and direct-to-LDS loads are inline asm, so the compiler's hazard recogniser does not see them; the
 rules it would have enforced are checked here on the generated gfx950 assembly of the shipped source
 (`hipcc -S --cuda-device-only`, about a minute, no GPU):
 
 * no MFMA reads a VGPR/AGPR that a VALU instruction wrote fewer than two wait states earlier;
 * every direct-to-LDS load in scalar-base form got SGPRs for its base and every M0 write an SGPR source
   (an "s" asm operand that the compiler could not prove uniform silently becomes a VGPR);
-* the MFMA loops of the m > 16 kernels move no accumulator (no v_accvgpr_* inside them) and spill nothing.
+* the MFMA loops of the m > 16 kernels (gemm_mb_kernel, gemm_wide_kernel) move no accumulator (no v_accvgpr_* inside them) and spill nothing.
 """
 import os
 import re
@@ -79,11 +79,14 @@ def test_scalar_operands_of_asm_loads(asm):
 
 
 def test_mfma_loops_keep_accumulators_in_place(asm):
-    seen = 0
+    seen = wide = 0
     for name, ins in kernels(asm):
-        if "gemm_mb_kernel" not in name:
+        if "gemm_wide_kernel" in name:
+            wide += 1
+        elif "gemm_mb_kernel" in name:
+            seen += 1
+        else:
             continue
-        seen += 1
         meta = asm[asm.index(".name:           " + name) - 400:asm.index(".name:           " + name) + 800]
         # Between two MFMAs of one loop (fewer than 100 other instructions apart; what separates the FP6 loop from the
         # INT4 loop of the same kernel is longer: with the accumulators in the accumulation registers the deferred
@@ -100,6 +103,8 @@ def test_mfma_loops_keep_accumulators_in_place(asm):
     # MB 8), a second build without the optional paths of those that the dispatcher picks by itself (6 x 2 less
     # one that would spill), and a third, with two classes of INT4 tiles, of two of those (2 x 2 less one that would spill)
     assert seen == 30
+    # (group scales or not) x seven tiles x (with or without the fused epilogue and the gfx950 order)
+    assert wide == 28
     assert not re.findall(r"\.vgpr_spill_count:\s+[1-9]", asm), "a kernel spills VGPRs"
     # nothing may live in private memory either: a pointer that the compiler keeps on the stack costs the decode loop a
     # scratch load and a full `s_waitcnt vmcnt(0)` per step (seen once with pointers advanced under uniform branches)
