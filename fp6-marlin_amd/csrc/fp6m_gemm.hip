@@ -525,12 +525,17 @@ constexpr int kWideNarrow = 5;    // from this row on: NARROW6
 inline int wide_plan(int m, int n, int k, int qc, bool g128, int mb, int max_par, int cus)
 {
     if (m <= 64 || k < 2048) return 0;
+    const int tile_rows = 16 * mb, tiles_n = n / kTileN, row_tiles = (m + tile_rows - 1) / tile_rows;
+    // Without FP6 columns, with per-column scales and at most one workgroup of 128 rows per CU the estimate below is too high
+    // for gemm_mb_kernel, where no workgroup dequantises for longer than the others (77 x 4352 x 23808: 30.9 us, estimated 37.4;
+    // the many-rows kernel 34.6).  Of 93 random shapes that went to the many-rows kernel from here it was 2-16 % slower on 51
+    // and up to 7 % faster on 22, 2.8 % slower on average.
+    if (!qc && !g128 && mb == 8 && row_tiles <= max_par && (long long)tiles_n * row_tiles <= cus) return 0;
     const double kk = k / 4096.0, g = g128 ? 1.0 : 0.0;
     // gemm_mb_kernel, launch by launch: 128-row tiles come in rounds of one workgroup per CU, 64-row tiles of two (or, if
     // one per CU is all there is, with the k range split over the idle CUs).
     double us = 0;
-    const int tile_rows = 16 * mb, tiles_n = n / kTileN;
-    for (int left = (m + tile_rows - 1) / tile_rows; left > 0; left -= max_par) {
+    for (int left = row_tiles; left > 0; left -= max_par) {
         const long long wgs = (long long)tiles_n * (left < max_par ? left : max_par);
         us += 7.0;
         if (mb == 8) {

@@ -295,6 +295,35 @@ def test_dispatch_picks_128_row_tiles_where_they_fill_the_chip(oracle, capfd):
         assert want in err, (m, n, want, err[-400:])
 
 
+def wide_plan_of(capfd, m, k, n, qc, gs, sms=-1):
+    """The tile of the many-rows kernel that a call takes by itself, from its verbose line (0: another kernel)."""
+    import fp6_marlin
+    n4 = n - max(qc, 0)
+    A = torch.zeros((m, k), dtype=torch.half, device=dev())
+    B = torch.zeros(k * n4 // 8 + k * max(qc, 0) * 3 // 16, dtype=torch.int32, device=dev())
+    C = torch.empty((m, n), dtype=torch.half, device=dev())
+    s = torch.ones((n4 if gs == -1 else k // gs * n4) + max(qc, 0), dtype=torch.half, device=dev())
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    capfd.readouterr()
+    with fp6_marlin.cabi.tuning(verbose=1):
+        fp6_marlin.mul(A, B, C, s, ws, qc, -1, -1, sms, 16, gs)
+    torch.cuda.synchronize()
+    err = capfd.readouterr().err
+    assert f"m={m} n={n} k={k}" in err, err[-300:]
+    return int(err.split("wide, plan ")[1].split()[0]) if "wide, plan " in err else 0
+
+
+@pytest.mark.skipif(not torch.cuda.is_available() or torch.cuda.get_device_properties(0).multi_processor_count != 256,
+                    reason="the plans are those of 256 CUs")
+def test_one_round_of_128_row_tiles_without_fp6_columns_keeps_its_kernel(capfd):
+    """All INT4 with per-column scales, at most one workgroup of 128 rows per CU: the many-rows kernel took these and was 4 to
+    12 % slower than gemm_mb_kernel.  With group scales or FP6 columns, or beyond one round, it is the faster one."""
+    for m, k, n in ((388, 3840, 6144), (77, 4352, 23808), (145, 3840, 12800), (176, 8192, 16384), (1050, 2816, 2048)):
+        assert wide_plan_of(capfd, m, k, n, -1, -1) == 0, (m, k, n)
+    assert wide_plan_of(capfd, 300, 4096, 12288, 256, -1) == 7
+    assert wide_plan_of(capfd, 500, 4096, 22016, -1, -1) == 1
+
+
 @pytest.mark.parametrize("plan", [1, 2, 3, 4, 5, 6, 7])
 def test_waves_side_by_side_in_n(oracle, plan):
     """The many-rows kernel (gemm_wide.h) in each of its tiles, forced onto small problems: ragged row tiles, a single
