@@ -115,7 +115,11 @@ __global__ __launch_bounds__(512) void column_scales_kernel(const uint16_t* part
 #pragma unroll
     for (int i = 1; i < 8; i++) m = red[i][threadIdx.x] > m ? red[i][threadIdx.x] : m;
     const int at = first + c;
-    uint16_t sh = f2h(h2f((uint16_t)m) * (at < n4 ? (float)(2.0 / 15.0) : (float)(1.0 / 28.0)));
+    // The product is rounded to binary32 first, as everywhere: a sub-normal scale can then lie half way (a maximum of 70 * 2^-24:
+    // 2.5 units, to even 2), where one rounding of the exact product (v_fma_mixlo_f16, which the compiler takes) gives 3.
+    float product = h2f((uint16_t)m) * (at < n4 ? (float)(2.0 / 15.0) : (float)(1.0 / 28.0));
+    asm("" : "+v"(product));
+    uint16_t sh = f2h(product);
     if (at < n4) {
         s4[scale_pos(at)] = sh;
     } else {

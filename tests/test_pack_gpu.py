@@ -126,6 +126,26 @@ def test_packing_fp6_columns_is_refused_under_capture():
         assert all(torch.equal(x, y) for x, y in zip(got, want)) and out.tolist() == [i + 1.0] * 4
 
 
+def test_fp6_columns_with_sub_normal_scales():
+    """Columns down to the smallest binary16 values: their scales are rounded to few bits, half way cases among them (a maximum
+    of 70 * 2^-24 was scaled by 3 units instead of 2), so that quotients reach beyond 28 (clamped) and fall below 0.0625 (a
+    zero, without its sign), and at last the scale is zero and replaced by one."""
+    import fp6_marlin
+    g = torch.Generator().manual_seed(23)
+    w = torch.randn((576, 320), generator=g) * 0.02
+    w[:, 128:] *= 2.0 ** -(torch.arange(192) % 24).float()
+    w = w.half()
+    for col, units in ((128, 14), (129, 42), (130, 70), (131, 126), (132, 14 * 63)):   # (exactly half way between two scales)
+        w[:, col] = torch.randint(-units, units + 1, (576,), generator=g).float().mul(2.0 ** -24).half()
+        w[0, col] = units * 2.0 ** -24
+    for gs in (-1, 64):
+        Bh, sh, rh = fp6_marlin.pack_mixed_weight(w, 192, gs, harness_layout=False)
+        Bd, sd, rd = fp6_marlin.pack_mixed_weight(w.to(dev()), 192, gs, harness_layout=False)
+        assert torch.equal(Bd.cpu(), Bh)
+        assert same_bits(sd, sh)
+        assert same_values(rd, rh)
+
+
 def test_fp6_scale_rule_vectors_through_the_gpu_packer():
     """The constructed columns of tests/fp6_scale_vectors.py (exact scales 1, 0.5, 0.0625; values around every e3m2
     grid point; entries below the 0.0625 threshold; a quotient that rounds above 28) through the on-GPU packer: scales
