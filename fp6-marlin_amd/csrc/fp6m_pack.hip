@@ -292,8 +292,10 @@ __device__ __forceinline__ void int4_pack(const PackArgs& p, int col_block, int 
                 row = row < p.k ? row : p.k - 1;
                 sh = p.s4[p.per_column ? scale_pos(col0 + tid) : (size_t)(row / p.g) * p.n4 + col0 + tid];
             }
-            // A zero scale (nothing in the group above 2^-23: codes 8) and an infinite one divide as "times zero"; what the
-            // quotient of an infinity or a NaN becomes is settled where it is clamped.
+            // A zero scale (nothing in the group above 3 * 2^-24: codes 8) and an infinite one divide as "times zero"; what the
+            // quotient of an infinity or a NaN becomes is settled where it is clamped.  (With an infinite scale the host path,
+            // which packs the re-quantised check weight, has code 0 for the finite weights too; here they are 8.  Scale and check
+            // weight are the same, and neither is a weight any more.)
             const bool none = (sh & 0x7fffu) == 0 || sh == 0x7c00u;
             sm.s[e][tid] = sh;
             sm.d[e][tid] = none ? 0.f : h2f(sh);

@@ -324,6 +324,18 @@ def test_one_round_of_128_row_tiles_without_fp6_columns_keeps_its_kernel(capfd):
     assert wide_plan_of(capfd, 500, 4096, 22016, -1, -1) == 1
 
 
+@pytest.mark.skipif(not torch.cuda.is_available() or torch.cuda.get_device_properties(0).multi_processor_count != 256,
+                    reason="the plans are those of 256 CUs")
+def test_which_calls_go_to_the_many_rows_kernel(capfd):
+    """The default choice: each tile where the estimates are clearly apart, and the calls that it is never asked for."""
+    for want, m, k, n, qc, gs in ((7, 300, 4096, 12288, 256, 128), (3, 2048, 8192, 10240, 256, 128), (2, 1024, 8192, 8192, 256, 128),
+                                  (1, 700, 2048, 57344, 256, 128), (5, 150, 8192, 40960, 20480, -1), (4, 1509, 6144, 3328, 1024, 128),
+                                  (6, 180, 4096, 24576, 256, 128), (0, 64, 4096, 22016, 256, 128), (0, 128, 8192, 8192, 256, 128),
+                                  (0, 2048, 1920, 8192, 256, 128), (0, 2048, 4160, 8192, 256, -1)):
+        assert wide_plan_of(capfd, m, k, n, qc, gs) == want, (want, m, k, n, qc, gs)
+    assert wide_plan_of(capfd, 2048, 8192, 10240, 256, 128, sms=256) == 0
+
+
 @pytest.mark.parametrize("plan", [1, 2, 3, 4, 5, 6, 7])
 def test_waves_side_by_side_in_n(oracle, plan):
     """The many-rows kernel (gemm_wide.h) in each of its tiles, forced onto small problems: ragged row tiles, a single

@@ -126,6 +126,23 @@ def test_packing_fp6_columns_is_refused_under_capture():
         assert all(torch.equal(x, y) for x, y in zip(got, want)) and out.tolist() == [i + 1.0] * 4
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+def test_range_errors_of_the_true_transpose(value):
+    """Layer.pack's layout has an FP6 kernel of its own: a NaN or infinite weight in that region is a range error there too,
+    wherever it lies, and the call after it is clean."""
+    import fp6_marlin
+    g = torch.Generator().manual_seed(17)
+    w = (torch.randn((1024, 384), generator=g) * 0.02).half().to(dev())
+    want = fp6_marlin.pack_mixed_weight(w, 192, 128, harness_layout=False)
+    for row, col in ((0, 192), (511, 383), (512, 250), (1023, 200)):
+        bad = w.clone()
+        bad[row, col] = value
+        with pytest.raises(ValueError):
+            fp6_marlin.pack_mixed_weight(bad, 192, 128, harness_layout=False)
+        got = fp6_marlin.pack_mixed_weight(w, 192, 128, harness_layout=False)
+        assert all(torch.equal(x, y) for x, y in zip(got, want)), (row, col)
+
+
 def test_fp6_columns_with_sub_normal_scales():
     """Columns down to the smallest binary16 values: their scales are rounded to few bits, half way cases among them (a maximum
     of 70 * 2^-24 was scaled by 3 units instead of 2), so that quotients reach beyond 28 (clamped) and fall below 0.0625 (a
@@ -144,6 +161,33 @@ def test_fp6_columns_with_sub_normal_scales():
         assert torch.equal(Bd.cpu(), Bh)
         assert same_bits(sd, sh)
         assert same_values(rd, rh)
+
+
+@pytest.mark.parametrize("gs", [-1, 128, 64])
+def test_infinite_and_nan_weights_in_the_int4_region(gs):
+    """They are no error there.  Scales and check weight are the host path's, with a NaN where it has one, and so are the words,
+    but for the finite weights of a group with an infinite scale: their code is 8 where the host, which packs the
+    re-quantised check weight (a NaN there), has 0."""
+    import fp6_marlin
+    g = torch.Generator().manual_seed(29)
+    k, n = 256, 512
+    w = (torch.randn((k, n), generator=g) * 0.02).half()
+    for col, values in ((3, ["inf"]), (70, ["-inf"]), (131, ["nan"]), (200, ["inf", "-inf"]), (255, ["nan", "inf"]), (301, ["-inf", "nan"])):
+        for i, v in enumerate(values):
+            w[10 + 100 * i, col] = float(v)
+    w[:, 400] = float("inf")
+    w[:, 401] = float("nan")
+    same = lambda a, b: np.array_equal(a.cpu().numpy().astype(np.float32), b.cpu().numpy().astype(np.float32), equal_nan=True)
+    Bh, sh, rh = fp6_marlin.pack_mixed_weight(w, -1, gs, harness_layout=False)
+    Bd, sd, rd = fp6_marlin.pack_mixed_weight(w.to(dev()), -1, gs, harness_layout=False)
+    assert same(sd, sh)
+    assert same(rd, rh)
+    ones = torch.ones(n, dtype=torch.half)                            # (the words alone: code - 8, with per-column scales of one)
+    got, host = (fp6_marlin.unpack_to_fp16(B.cpu(), ones, k, n, -1, -1) for B in (Bd, Bh))
+    most = w.abs().float().reshape(k // (k if gs == -1 else gs), -1, n).amax(1, keepdim=True)
+    infinite = (most.isinf() & w.isfinite().reshape(most.shape[0], -1, n)).reshape(k, n)
+    assert bool((host[infinite] == -8).all()) and bool((got[infinite] == 0).all()) and int(infinite.sum()) > 300
+    assert torch.equal(got[~infinite], host[~infinite])
 
 
 def test_fp6_scale_rule_vectors_through_the_gpu_packer():
