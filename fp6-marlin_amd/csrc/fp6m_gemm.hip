@@ -496,7 +496,9 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
 // to 3-7 %, the plan they choose is 0.3 % off the best on average, and it took 11.8 % off the time of gemm_mb_kernel over
 // all of them, 18 % between 700 and 1200 rows (from 129 to 256 rows 6.9 %, below 65 rows none: not asked).  Two shapes in 1830
 // lost more than 4 %; hence the 3 % that the wide kernel must win by.  Nothing was fitted below k = 2048, where starts and
-// ends are most of the time: not asked either.
+// ends are most of the time: not asked either.  All shapes of the fit had 256 FP6 columns; against gemm_mb_kernel the choice
+// was then measured on 2689 more, with none (-23 % on average), 256, 512, 1024, a quarter, half and all of the columns in FP6
+// (-23 to -27 % each): 12 of them are more than 2 % slower, the worst 208 x 14080 x 40448 all in FP6, +14 %.
 //
 // The last two plans (FP6 tiles in workgroups of their own) were fitted to 170 more shapes of 65 to 1600 rows with 256 FP6
 // columns, to 2-3 %; the seven plans' choice is again 0.3 % off the best there.  They are not asked where the extra

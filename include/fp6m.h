@@ -63,7 +63,8 @@ int fp6m_abi_version(void);
  *               different kernel here (tile shapes are chosen for 256 CUs / wave64).
  *   sms         -1 = automatic; otherwise an upper bound on the number of workgroups that cooperate
  *               on one column tile's reduction (debug/testing knob, like the reference's).
- *   max_par     as in the reference: bounds how many 64-row blocks of A one launch covers.
+ *   max_par     as in the reference: bounds how many blocks of A (32, 64 or 128 rows) one launch covers, and sizes the
+ *               workspace; the many-rows kernel covers all rows in one launch whatever it says.
  *   quant_cols  -1 (or 0) = all INT4; n = all FP6; otherwise the last quant_cols columns are FP6.
  *               Must be a multiple of 128, as must n - quant_cols.
  *   group_size  -1 = one INT4 scale per column (what the reference kernel supports);

@@ -286,7 +286,8 @@ def test_dispatch_picks_128_row_tiles_where_they_fill_the_chip(oracle, capfd):
     slower per row, finer grain): with 32 column tiles, 8 row tiles of 128 fill one round of 256 CUs exactly (the last
     tile ragged at m = 1000) and 5 of them beat 10 half-size workgroups that no longer fit one per CU; 9 row tiles
     would take two rounds for 1.1 rounds of work, and at m = 300 the 64-row tiles still fit one per CU.  With 256
-    column tiles even a single, ragged row tile of 128 wins (one round instead of 512 half-size workgroups)."""
+    column tiles even a single, ragged row tile of 128 wins (one round instead of 512 half-size workgroups).  (At k = 512
+    gemm_mb_kernel takes them all; from k = 2048 on some go to the many-rows kernel: the next two tests.)"""
     for m, n, want in ((1000, 4096, "MB=8"), (1024, 4096, "MB=8"), (640, 4096, "MB=8"), (1025, 4096, "MB=4"),
                        (300, 4096, "MB=4"), (96, 32768, "MB=8"), (96, 4096, "MB=4"), (64, 32768, "MB=4")):
         capfd.readouterr()
