@@ -97,8 +97,11 @@ __global__ __launch_bounds__(256) void column_maxima_kernel(const uint16_t* w, i
 // Scales from the chunks' maxima, of columns [first, first + cols) of w: INT4 (columns below n4) s = max|w| * 2/15
 // (test.py:88-89), FP6 s = max|w| * 1/28 (test.py:19-23; the real-transpose layout replaces a zero scale by one), in the
 // permuted order.  64 columns per workgroup, eight threads per column: all loads in flight at once.
+// The range check of the true transpose's FP6 cast is settled here (`bad`): the quotients are clamped, so all that can go
+// wrong is a NaN among them, and that takes an infinity or a NaN among the column's weights.  (A finite weight over its own
+// column's scale stays below 43: the scale is the maximum / 28, off by at most a half of the smallest sub-normal, or one.)
 __global__ __launch_bounds__(512) void column_scales_kernel(const uint16_t* part, int chunks, int first, int cols, int n4, int harness,
-                                                            uint16_t* s4, uint16_t* s6)
+                                                            uint16_t* s4, uint16_t* s6, int* bad)
 {
     __shared__ unsigned red[8][64];
     const int c = blockIdx.x * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;   // (cols is a multiple of 64)
@@ -123,6 +126,7 @@ __global__ __launch_bounds__(512) void column_scales_kernel(const uint16_t* part
     if (at < n4) {
         s4[scale_pos(at)] = sh;
     } else {
+        if (bad && m >= 0x7c00u) __hip_atomic_store(bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         if (!harness && (sh & 0x7fffu) == 0) sh = 0x3c00u;
         s6[scale_pos(at - n4)] = sh;
     }
@@ -220,7 +224,7 @@ struct PackArgs {
     uint16_t *s4, *s6;
     uint32_t *words, *plane2, *plane4;
     uint16_t* w_ref;
-    int* bad;
+    int* range_known;                 // host memory, set when the kernel starts: the kernels before it are done (null: not asked for)
     int wgs6, blocks4;                // workgroups of the FP6 region (the first of the grid); INT4 workgroups per 128 rows
 };
 
@@ -402,7 +406,7 @@ __device__ __forceinline__ void fp6_pack(const PackArgs& p, int col_block, int r
         raw[r][1] = *reinterpret_cast<const uint4*>(src + (size_t)k_off(i, r) * p.n + 32);
     }
     if (threadIdx.x < 64) {
-        // (never zero; an infinite or NaN scale comes from such a weight, whose quotient is a NaN: the call fails)
+        // (never zero; an infinite or NaN scale comes from such a weight: the call fails)
         const float d = h2f(p.s6[scale_pos(col_block * 64 + threadIdx.x)]);
         sm.d[threadIdx.x] = d;
         sm.r[threadIdx.x] = 1.0f / d;
@@ -410,7 +414,6 @@ __device__ __forceinline__ void fp6_pack(const PackArgs& p, int col_block, int r
     __syncthreads();
     if (!here) return;
     uint32_t lo[8], hi[8];                                               // [nibble of the word]: nibble t column 2t, 4 + t column 2t + 1
-    us2 most = {0, 0};
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         asm volatile("" : : : "memory");                                 // (reads the scales again: they do not fit the registers)
@@ -425,7 +428,6 @@ __device__ __forceinline__ void fp6_pack(const PackArgs& p, int col_block, int r
                 const float d0 = sm.d[at], d1 = sm.d[at + 1];
                 const h2 wv = as_h2(q[t]);
                 h2 x = {(_Float16)quotient((float)wv[0], d0, sm.r[at]), (_Float16)quotient((float)wv[1], d1, sm.r[at + 1])};
-                most = max2(most, magnitudes(bits(x)));                  // (a NaN stands above everything)
                 x = __builtin_elementwise_min(__builtin_elementwise_max(x, both(-28.0f)), both(28.0f));
                 // Cut to two mantissa bits and scaled by 2^-12, exactly, the value has the code's five magnitude bits in
                 // bits 8 .. 12, sub-normals included: e3m2's are binary16's.  (fp6_code is the same, case by case.)
@@ -465,7 +467,6 @@ __device__ __forceinline__ void fp6_pack(const PackArgs& p, int col_block, int r
 #pragma unroll
     for (int m = 0; m < 4; m++)                                          // (one lane stores columns 0, 2, 4, 6, the other the odd ones)
         p.plane2[(granule + 4 * (2 * m + (upper ? 1 : 0))) * 2 + (j >> 1)] = upper ? o[m + 4] : o[m];
-    if (most[0] > 0x7c00u || most[1] > 0x7c00u) *p.bad = 1;
 }
 
 // One launch packs both regions, the FP6 region's few workgroups first so that they run beside the others.
@@ -481,6 +482,7 @@ __global__ __launch_bounds__(512, 4) void pack_kernel(const PackArgs p)
         Fp6Smem fp6;
     } sm;
     const int b = blockIdx.x;
+    if (b == 0 && threadIdx.x == 0 && p.range_known) __hip_atomic_store(p.range_known, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (b < p.wgs6) {
         const int across = p.qc / 64;
         fp6_pack(p, b % across, b / across, sm.fp6);
@@ -528,29 +530,32 @@ __global__ void fp6_pack_harness_kernel(const uint16_t* w, int k, int n, int n4,
     if (any_bad) *bad = 1;
 }
 
-// The FP6 range flag of a call: a word of pinned host memory that the kernels write (only when something is out of
-// range) and the call reads after its wait, so that no copy back is enqueued.  kFlags words, allocated once and kept; a
-// call holds one of them, so calls on several threads and streams do not meet.  A word goes back only after a wait that
+// The FP6 range flag of a call: a line of pinned host memory that the kernels write (`bad` only when something is out of
+// range) and the call reads after its wait, so that no copy back is enqueued.  kFlags lines, allocated once and kept; a
+// call holds one of them, so calls on several threads and streams do not meet.  A line goes back only after a wait that
 // succeeded: until then kernels of this call may still write it, and the next call's check would see that.
 constexpr int kFlags = 64;
+struct alignas(64) FlagLine {
+    int bad, known;
+};
 std::mutex g_flag_mutex;
-int* g_flags = nullptr;
+FlagLine* g_flags = nullptr;
 unsigned long long g_flags_taken = 0, g_flags_lost = 0;                  // (lost: taken for good)
 struct RangeFlag {
     int index = -1;
-    bool idle = true;                                                    // nothing enqueued may still write the word
+    bool idle = true;                                                    // nothing enqueued may still write the line
     hipError_t err = hipSuccess;
     explicit RangeFlag(bool wanted)
     {
         while (wanted) {
             {
                 std::lock_guard<std::mutex> lock(g_flag_mutex);
-                if (!g_flags && (err = hipHostMalloc(reinterpret_cast<void**>(&g_flags), kFlags * sizeof(int), hipHostMallocPortable | hipHostMallocMapped)) != hipSuccess)
+                if (!g_flags && (err = hipHostMalloc(reinterpret_cast<void**>(&g_flags), kFlags * sizeof(FlagLine), hipHostMallocPortable | hipHostMallocMapped)) != hipSuccess)
                     return;
                 if (~g_flags_taken) {
                     index = __builtin_ctzll(~g_flags_taken);
                     g_flags_taken |= 1ull << index;
-                    g_flags[index] = 0;
+                    g_flags[index] = FlagLine{0, 0};
                     return;
                 }
                 if (!~g_flags_lost) {                                    // (64 calls whose wait failed)
@@ -570,22 +575,38 @@ struct RangeFlag {
         else
             g_flags_lost |= 1ull << index;
     }
+    // All of the call's kernels.
     hipError_t wait(hipStream_t st)
     {
         const hipError_t e = hipStreamSynchronize(st);
         idle = e == hipSuccess;
         return e;
     }
-    int* ptr() const { return index < 0 ? nullptr : g_flags + index; }
+    // Those that decide about the range: true once pack_kernel, which writes nothing here after that, has begun.  Not for
+    // long (the stream may have other work in front): false leaves it to wait().
+    bool known_soon() const
+    {
+        for (int i = 0; i < 20000; i++) {
+            if (__atomic_load_n(&g_flags[index].known, __ATOMIC_ACQUIRE)) return true;
+            __builtin_ia32_pause();
+        }
+        return false;
+    }
+    int* bad() const { return index < 0 ? nullptr : &g_flags[index].bad; }
+    int* known() const { return index < 0 ? nullptr : &g_flags[index].known; }
+    bool out_of_range() const { return index >= 0 && __atomic_load_n(&g_flags[index].bad, __ATOMIC_RELAXED) != 0; }
 };
 
 }  // namespace
 }  // namespace fp6m
 
-extern "C" int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_cols, int group_size, int harness_layout,
-                                      void* B, void* s, void* w_ref, int dev, void* stream)
+namespace fp6m {
+namespace {
+
+// whole: do not return before the call's kernels are done (where the range of the FP6 cast is checked at all).
+int pack_mixed(const void* w, int k, int n, int quant_cols, int group_size, int harness_layout, void* B, void* s, void* w_ref, int dev,
+               void* stream, bool whole)
 {
-    using namespace fp6m;
     if (!w || !B || !s) return FP6M_ERR_ARG;
     const int qc = quant_cols == -1 ? 0 : quant_cols;
     if (k <= 0 || n <= 0 || qc < 0 || qc > n || qc % 64 || (n - qc) % 64 || k % 64 || n % 8) return FP6M_ERR_SHAPE;
@@ -607,7 +628,7 @@ extern "C" int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_col
     if (qc > 0 && capturing(st)) return hip_fail(hipErrorStreamCaptureUnsupported);   // (the wait below: refused before anything is recorded)
     RangeFlag flag(qc > 0);
     if (flag.err != hipSuccess) return hip_fail(flag.err);
-    a.bad = flag.ptr();
+    if (!whole && !harness_layout) a.range_known = flag.known();
     // Scales that span all of k (all columns with per-column scales, else the FP6 region): maxima of at most kMaxChunks row
     // ranges first.  They wait, two bytes each, in B, which is packed afterwards and larger (at least k / 2 bytes a column).
     const int first = per_column ? 0 : n4, cols = n - first;
@@ -615,14 +636,15 @@ extern "C" int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_col
         const int rows = ((k + kMaxChunks - 1) / kMaxChunks + 63) / 64 * 64, chunks = (k + rows - 1) / rows;
         uint16_t* part = reinterpret_cast<uint16_t*>(B);
         hipLaunchKernelGGL(column_maxima_kernel, dim3((cols + 255) / 256, chunks), dim3(256), 0, st, wp + first, k, n, cols, rows, part);
-        hipLaunchKernelGGL(column_scales_kernel, dim3(cols / 64), dim3(512), 0, st, part, chunks, first, cols, n4, harness_layout, sp, s6);
+        hipLaunchKernelGGL(column_scales_kernel, dim3(cols / 64), dim3(512), 0, st, part, chunks, first, cols, n4, harness_layout, sp, s6,
+                           harness_layout ? nullptr : flag.bad());
     }
     if (n4 && !per_column && g != 128)
         hipLaunchKernelGGL(int4_scales_kernel, dim3((n4 / 8 + 255) / 256, k / g), dim3(256), 0, st, wp, k, n, n4, g, sp);
     if (qc && harness_layout) {
         const size_t owners = (size_t)(k / 16) * (qc / 64) * 32;
         hipLaunchKernelGGL(fp6_pack_harness_kernel, dim3((unsigned)((owners + 255) / 256)), dim3(256), 0, st, wp, k, n, n4, qc, s6, plane2,
-                           plane4, rp, a.bad);
+                           plane4, rp, flag.bad());
     } else if (qc) {
         a.wgs6 = qc / 64 * ((k + 511) / 512);
     }
@@ -635,11 +657,31 @@ extern "C" int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_col
     }
     e = hipGetLastError();
     if (qc) {
-        // the range check of the FP6 cast is reported by value, so this call waits for its kernels (after a failed launch for
-        // those in front of it: the flag's word is another call's next)
-        const hipError_t waited = flag.wait(st);
-        if (e == hipSuccess) e = waited;
+        // The range check of the FP6 cast is reported by value, so this call waits: for the kernels in front of pack_kernel,
+        // which find the maxima, or, where the harness layout's kernel checks cast by cast, where something is out of range
+        // or failed to launch (the flag's line is another call's next), and where it is asked for, for all of them.  With
+        // every call waiting for all of them the GPU was idle between one call's last kernel and the next one's first:
+        // 4096 x 22016, group-128 scales, 256 FP6 columns, calls in a row 106.6 -> 85.2 us each.
+        if (!(e == hipSuccess && a.range_known && flag.known_soon() && !flag.out_of_range())) {
+            const hipError_t waited = flag.wait(st);
+            if (e == hipSuccess) e = waited;
+        }
     }
     if (e != hipSuccess) return hip_fail(e);
-    return qc && *const_cast<volatile int*>(flag.ptr()) ? FP6M_ERR_RANGE : FP6M_OK;
+    return flag.out_of_range() ? FP6M_ERR_RANGE : FP6M_OK;
+}
+
+}  // namespace
+}  // namespace fp6m
+
+extern "C" int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_cols, int group_size, int harness_layout,
+                                      void* B, void* s, void* w_ref, int dev, void* stream)
+{
+    return fp6m::pack_mixed(w, k, n, quant_cols, group_size, harness_layout, B, s, w_ref, dev, stream, true);
+}
+
+extern "C" int fp6m_pack_mixed_device_async(const void* w, int k, int n, int quant_cols, int group_size, int harness_layout,
+                                            void* B, void* s, void* w_ref, int dev, void* stream)
+{
+    return fp6m::pack_mixed(w, k, n, quant_cols, group_size, harness_layout, B, s, w_ref, dev, stream, false);
 }

@@ -297,6 +297,13 @@ int fp6m_unpack_to_fp16(const int32_t* B, const uint16_t* s, uint16_t* w_ref, si
 int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_cols, int group_size, int harness_layout,
                            void* B, void* s, void* w_ref, int dev, void* stream);
 
+/* The same without waiting longer than the range check needs: in the true transpose's layout the column maxima settle it,
+ * and the call returns as soon as they are known while the packing itself may still run.  B, s and w_ref are then ready in
+ * stream order, like any kernel's output (as they are from either entry when quant_cols <= 0), and w must stay as it is
+ * until then.  After an error the call's kernels are done. */
+int fp6m_pack_mixed_device_async(const void* w, int k, int n, int quant_cols, int group_size, int harness_layout,
+                                 void* B, void* s, void* w_ref, int dev, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

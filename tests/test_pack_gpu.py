@@ -143,6 +143,45 @@ def test_range_errors_of_the_true_transpose(value):
         assert all(torch.equal(x, y) for x, y in zip(got, want)), (row, col)
 
 
+@pytest.mark.parametrize("k,n,qc", [(64, 128, 64), (1024, 384, 192), (4160, 1088, 1088)])
+def test_the_range_is_known_before_the_packing_is_done(k, n, qc):
+    """The package's calls return once the range is known: on a stream with other work in front (longer than the call polls),
+    on a stream of their own while the caller's tensors go, and for a weight out of range, against the entry that waits."""
+    import ctypes
+    import fp6_marlin
+    cabi = fp6_marlin.cabi
+    g = torch.Generator().manual_seed(31)
+    w = (torch.randn((k, n), generator=g) * 0.02).half().to(dev())
+    out = [torch.empty(size, dtype=dtype, device=dev()) for size, dtype in
+           ((k * (n - qc) // 8 + k * qc * 3 // 16, torch.int32), ((n - qc) + qc, torch.half), ((k, n), torch.half))]
+    torch.cuda.synchronize()
+    assert cabi.lib.fp6m_pack_mixed_device(w.data_ptr(), k, n, qc, -1, 0, *(ctypes.c_void_p(t.data_ptr()) for t in out), 0, None) == 0
+    big = torch.randn((6144, 6144), device=dev()).half()
+    for busy in (0, 30):
+        for _ in range(busy):
+            big @ big
+        got = fp6_marlin.pack_mixed_weight(w, qc, -1, harness_layout=False)
+        assert all(torch.equal(x, y) for x, y in zip(got, out))
+        bad = w.clone()
+        bad[k - 1, n - 1] = float("inf")
+        for _ in range(busy):
+            big @ big
+        with pytest.raises(ValueError):
+            fp6_marlin.pack_mixed_weight(bad, qc, -1, harness_layout=False)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    results = []
+    for i in range(4):
+        mine = w.clone()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            results.append(fp6_marlin.pack_mixed_weight(mine, qc, -1, harness_layout=False))
+        del mine
+        torch.full((k, n), float("nan"), dtype=torch.half, device=dev())
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for got in results for x, y in zip(got, out))
+
+
 def test_fp6_columns_with_sub_normal_scales():
     """Columns down to the smallest binary16 values: their scales are rounded to few bits, half way cases among them (a maximum
     of 70 * 2^-24 was scaled by 3 units instead of 2), so that quotients reach beyond 28 (clamped) and fall below 0.0625 (a
