@@ -746,15 +746,18 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
     if (const char* e = getenv("FP6M_TIMELINE_PTR")) a.timeline = reinterpret_cast<unsigned long long*>(strtoull(e, nullptr, 0));
 #endif
 
-    // Row blocks per workgroup pass: 32 rows up to m = 32, 64 rows (accumulators in 128 VGPRs, two
-    // workgroups per CU) beyond; 128 rows for large launches whose grid allows it (below).
-    int mb = prob_m <= 16 ? 1 : (prob_m <= 32 ? 2 : 4);
     const Tuning tune = g_tuning;              // tuning/testing overrides (all unset in production)
+    // Row blocks per workgroup pass: 32 rows up to m = 32, 48 up to m = 48, 64 rows (accumulators in 128 VGPRs, two
+    // workgroups per CU) beyond; 128 rows for large launches whose grid allows it (below).
+    // (48-row tiles against 64-row tiles, which multiply, reduce and exchange a quarter more for these rows, 33 to 48 rows on
+    // sixteen shapes, us: 13824 x 5120 20.4 -> 17.0, 8192 x 8192 19.4 -> 17.7, 4096 x 12288 16.7 -> 15.2, 4096 x 22016
+    // 20.4 -> 17.5, 28672 x 8192 42.6 -> 39.8, 8192 x 57344 76.1 -> 67.0.  They have the paired loop only.)
+    int mb = prob_m <= 16 ? 1 : (prob_m <= 32 ? 2 : (prob_m <= 48 && !(tune.pair != kUnset && tune.pair == 0) ? 3 : 4));
     // share of a SIMD that the second of two waves of a workgroup gets, in per cent of the first one's (make_wave_rule).
     // Measured (alternating, us, equal slices -> 72 %): 8192 x 8192 at 8 / 16 / 128 / 256 rows 12.65 -> 12.03 / 13.2 -> 12.65 /
     // 27.95 -> 27.4 / 42.3 -> 41.2, 8192 x 10240 at 16 rows 14.3 -> 13.7; 60 % and 85 % within 1 % of it.
     const int young_pct = tune.young != kUnset ? tune.young : 72;
-    if (tune.mb != kUnset && prob_m > 16 && (tune.mb == 2 || tune.mb == 4 || tune.mb == 8)) mb = tune.mb;
+    if (tune.mb != kUnset && prob_m > 16 && (tune.mb == 2 || tune.mb == 3 || tune.mb == 4 || tune.mb == 8)) mb = tune.mb;
     // Row mix: the kWaves * ks slices of a tile are dealt to the two segments in proportion to their cost (an FP6
     // step costs about two INT4 steps), at least one each.
     auto deal_slices = [&](int total) {
@@ -1470,9 +1473,14 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             // Re-measured with every tile on the paired loop (ten shapes x 32 .. 256 rows, alternating): still 5-13 % on
             // wide weights up to two row tiles (4096 x 11008 at 128 rows 25.3 -> 22.2 us, 8192 x 28672 at 32 rows
             // 38.2 -> 34.5), but 3-8 % slower from three row tiles on (5120 x 5120 at 256 rows 27.4 -> 29.7): up to two.
-            if (env_ks < 1 && !row_mix && a.tiles6 > 0 && units >= 4 * ks * wk && mb != 8 && mtiles <= 2 &&
-                (base + (long long)a.tiles6 * mtiles) * ks <= resident)
-                a.ks6 = 2 * (int)ks;
+            // Where twice does not fit, as finely as does (13824 x 5120 with 512 FP6 columns, per-column scales, 64 rows: 6 parts for
+            // all tiles 22.1 us, 10 for the FP6 tiles 21.4).
+            if (env_ks < 1 && !row_mix && a.tiles6 > 0 && mb != 8 && mtiles <= 2) {
+                long long c6 = units / (2 * wk) < 2 * ks ? units / (2 * wk) : 2 * ks;
+                const long long room = (resident - (base - (long long)a.tiles6 * mtiles) * ks) / ((long long)a.tiles6 * mtiles);
+                if (c6 > room) c6 = room;
+                if (c6 > ks) a.ks6 = (int)c6;
+            }
             // One row tile and somewhat more tiles than CUs: workgroups of four waves, two to a CU, run both at little more
             // than half speed, so the CUs that get two set the launch's length at 1.76 x that of a grid that fits
             // (8192 x 36864 at 32 rows: 288 tiles 60.9 us, 256 tiles 34.6).  Two classes of INT4 tiles instead (as in the
@@ -1501,7 +1509,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                     // 264 .. 360 tiles, both scale modes): what these bars take gained 0-33 %, what they leave out
                     // was within -4 .. +8 % when forced.
                     const double gain = prob_k / 128.0 * (0.76 - 1.0 / (double)cb);
-                    const double bar = mb == 4 ? 16.0 : 7.5 + 0.37 * (32 - a.m);
+                    const double bar = mb >= 3 ? 16.0 : 7.5 + 0.37 * (32 - a.m);
                     if ((cb >= 2 && gain >= bar) || (tune.cls == 1 && cb >= 1)) {
                         wk = wk_c;
                         a.ks4 = 1;
@@ -1557,6 +1565,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                     launch_mb<2, 4, 3, false>(a, g128, wk, grid, st);
                 }
             }
+            else if (mb == 3) launch_mb<3, 3, 3, true>(a, g128, wk, grid, st);
             else if (pair) launch_mb<4, 3, 3, true>(a, g128, wk, grid, st);
             else launch_mb<4, 3, 3, false, false>(a, g128, wk, grid, st);
         }

@@ -7,7 +7,7 @@ namespace fp6m {
 // ------------------------------------------------------------------------------------------------ 16 < m: ring kernel with MB row blocks
 //
 // Same lane routing and k-sliced workgroup as the m <= 16 kernel, but a wave multiplies MB blocks of 16 rows of A and
-// every dequantised weight fragment feeds 2*MB MFMAs, so the packed words are read once per 16*MB rows.  MB = 2 or
+// every dequantised weight fragment feeds 2*MB MFMAs, so the packed words are read once per 16*MB rows.  MB = 2, 3 or
 // 4 (accumulators in ordinary registers, two waves per SIMD) or 8 (accumulators in the accumulation registers, one
 // wave per SIMD; launches whose 128-row tiles fill the chip).  Two loops: stream_tile_mb keeps the words and one step of
 // A (MB x 1 KiB) per slot of a ring; stream_tile_mbp (launches with more than 32 rows, and 32-row tiles in eight-wave
@@ -213,6 +213,9 @@ __device__ __forceinline__ void mfma_blocks_row(f4 (&acc)[MB][8], const h8 (&fra
     }
 }
 
+// Register buffers of A that a loop's blocks walk: four, or as many as blocks where three serve (every step then starts
+// with the first one; a buffer is read into when the MFMAs of the block it held have all been issued).
+constexpr int a_buffers(int mb) { return mb == 3 ? 3 : 4; }
 struct MbCtx {
     uint32_t abuf[4][4];
     uint32_t addr_cur[4], addr_next[4];
@@ -237,7 +240,7 @@ struct MbBlocks {
     {
         if constexpr (BLK < MB) {
             constexpr int nb = BLK + 2;
-            uint32_t (&dst)[4] = cx.abuf[(phase + nb) & 3];
+            uint32_t (&dst)[4] = cx.abuf[(phase + nb) % a_buffers(MB)];
             if constexpr (PAIRH < 0) {
                 if constexpr (nb < MB)
                     lds_read_a4<nb * 1024>(dst, cx.addr_cur);
@@ -255,7 +258,7 @@ struct MbBlocks {
             // extra reads must be complete as well
             constexpr int allow = BLK == 0 ? (8 + kExtra < 15 ? 8 + kExtra : 15) : 8;
             __builtin_amdgcn_s_waitcnt(lgkmcnt_only(allow));
-            uint32_t (&src)[4] = cx.abuf[(phase + BLK) & 3];
+            uint32_t (&src)[4] = cx.abuf[(phase + BLK) % a_buffers(MB)];
             asm volatile("" : "+v"(src[0]), "+v"(src[1]), "+v"(src[2]), "+v"(src[3]));
             const h8 av = __builtin_bit_cast(h8, u4{src[0], src[1], src[2], src[3]});
             mfma_blocks_row<MB, BLK>(acc, frag, av, hook);
@@ -517,7 +520,7 @@ template <bool FP6, bool G128, int MB>
 __device__ __forceinline__ void stream_tile_mbp(const GemmArgs& p, const TileInfo& ti, unsigned char* ring,
                                                 int step_begin, int step_end, f4 (&acc)[MB][8])
 {
-    static_assert(MB == 2 || MB == 4 || MB == 8, "the A register ring");
+    static_assert(MB == 2 || MB == 3 || MB == 4 || MB == 8, "the A register ring");
     constexpr int kOddPhase = MB == 2 ? 2 : 0;            // (two blocks per step walk the four register buffers in two steps)
     constexpr bool kGroup = G128 && !FP6;
     constexpr int kPair = MB * kPairBlock;                // one pair slot
@@ -728,7 +731,6 @@ __device__ __forceinline__ void wg_finish_mb(const GemmArgs& p, const TileInfo& 
     // BPR: 16-row blocks per round of the reduction through LDS (a wave's region holds BPR * 16 rows of kRedStride
     // floats).  The rounds are bound by LDS bandwidth (every wave writes and reads its whole accumulator once) plus two
     // barriers each, so fewer rounds help; the gather below keeps the loads of up to 32 rows in flight per lane.
-    static_assert(MB % BPR == 0, "whole rounds");
     constexpr int RMAX = 16 / WK;                                    // rows of a block one wave finishes
     // The gather keeps up to 32 8-byte loads per lane in flight.
     constexpr int kInFlight = 32;
@@ -779,7 +781,7 @@ __device__ __forceinline__ void wg_finish_mb(const GemmArgs& p, const TileInfo& 
         if (mb0 == 0) FP6M_MARK(p, 1);                               // every wave of the group has left its loop
         float* mine = reinterpret_cast<float*>(smem + wk * wave_lds) + c * kRedStride + 64 * (q >> 1) + 4 * (q & 1);
 #pragma unroll
-        for (int b = 0; b < BPR; b++)
+        for (int b = 0; b < BPR && mb0 + b < MB; b++)
 #pragma unroll
             for (int t = 0; t < 8; t++)
                 *reinterpret_cast<f4*>(mine + b * 16 * kRedStride + 16 * (t >> 1) + 8 * (t & 1)) = acc[mb0 + b][t];
@@ -787,7 +789,7 @@ __device__ __forceinline__ void wg_finish_mb(const GemmArgs& p, const TileInfo& 
         // all LDS reads of the round first (rows beyond m are read too: the slab is there), one wait, then the sums
         f2 tv[BPR][RMAX][WK];
 #pragma unroll
-        for (int b = 0; b < BPR; b++)
+        for (int b = 0; b < BPR && mb0 + b < MB; b++)
 #pragma unroll
             for (int r = 0; r < RMAX; r++)
 #pragma unroll
@@ -795,7 +797,7 @@ __device__ __forceinline__ void wg_finish_mb(const GemmArgs& p, const TileInfo& 
                     tv[b][r][j] = *reinterpret_cast<const f2*>(reinterpret_cast<const float*>(smem + j * wave_lds) +
                                                                (b * 16 + wk + r * WK) * kRedStride + 2 * lane);
 #pragma unroll
-        for (int b = 0; b < BPR; b++)
+        for (int b = 0; b < BPR && mb0 + b < MB; b++)
 #pragma unroll
             for (int r = 0; r < RMAX; r++) {
                 const int row = 16 * (mb0 + b) + wk + r * WK;

@@ -305,6 +305,21 @@ def test_paired_loop_of_the_row_block_kernel():
         run_mb_paired(steps, group=False)
 
 
+@pytest.mark.parametrize("mb", [3, 8])
+def test_paired_loop_with_other_numbers_of_row_blocks(mb):
+    """Three blocks walk three register buffers (a_buffers): a block's rows must still be there when its MFMAs are issued."""
+    for steps in (4, 8, 36):
+        run_mb_paired(steps, True, mb)
+    for steps in (2, 4, 6, 30):
+        run_mb_paired(steps, False, mb)
+    buffers, held = 3 if mb == 3 else 4, {0: (0, 0), 1: (0, 1)}       # register buffer -> (step, block), read ahead
+    for step in range(12):
+        for blk in range(mb):
+            ahead = (step, blk + 2) if blk + 2 < mb else (step + 1, blk + 2 - mb)
+            held[(blk + 2) % buffers] = ahead                          # issued in front of this block's MFMAs
+            assert held[blk % buffers] == (step, blk)
+
+
 def test_paired_loop_notices_a_missing_wait(monkeypatch):
     """Without the wait in the middle of a pair's second step the next pair is read while it may still be in flight."""
     real_wait = Memory.wait

@@ -261,6 +261,27 @@ def test_two_classes_of_int4_tiles_beyond_sixteen_rows(oracle, capfd):
             one_hot_case(oracle, m, n, k, qc, gs, {"cls": 1, "cus": cus})
 
 
+def test_three_row_blocks_per_wave(oracle, capfd):
+    """48-row tiles: what 33 to 48 rows take, at both edges, ragged, several row tiles (forced), all FP6 and all INT4, both scale
+    modes, four and eight slices, k splits with the FP6 tiles cut as finely and finer; one-hot rows bit for bit."""
+    for m in (33, 40, 47, 48):
+        for wk in (4, 8):
+            e = {"FP6M_WK": wk}
+            run(oracle, m, 512, 1024, qc=256, env=e)
+            run(oracle, m, 768, 1024, qc=128, gs=128, env=e)
+            run(oracle, m, 512, 2048, qc=256, gs=128, ksplit=2, env=e)
+    for m, n, k, qc, gs in ((33, 256, 512, -1, 128), (48, 256, 512, 256, -1), (41, 512, 64, 256, -1), (34, 512, 128, 128, 128)):
+        run(oracle, m, n, k, qc=qc, gs=gs)
+    for gs in (-1, 128):
+        for m in (33, 48, 100):
+            one_hot_case(oracle, m, 768, 1024, 256, gs, {"mb": 3})
+            one_hot_case(oracle, m, 768, 1024, 256, gs, {"mb": 3, "ksplit": 3})
+    capfd.readouterr()
+    run(oracle, 33, 5120, 13824, qc=512, env={"FP6M_VERBOSE": 1})         # (the dispatcher's own finer cut of the FP6 tiles)
+    out = capfd.readouterr().err
+    assert "MB=3 row tiles 1 ks4=6" in out and "ks6=6 " not in out, out
+
+
 def test_eight_row_blocks_per_wave(oracle):
     """The m > 16 kernel with eight 16-row blocks per wave (128-row tiles, accumulators in the accumulation
     registers), forced onto small problems: ragged row tiles, both regions, both scale modes, k splits through the

@@ -99,10 +99,10 @@ def test_mfma_loops_keep_accumulators_in_place(asm):
             assert len(moved) <= 300, f"{name}: {len(moved)} accumulator copies between MFMAs"
             continue
         assert not moved, f"{name}: accumulator copies between MFMAs: {moved[:4]}"
-    # (group scales or not) x ((MB 2, MB 4, MB 4 with paired A fetches) x (4, 8 k slices) + MB 2 paired with 8 slices +
-    # MB 8), a second build without the optional paths of those that the dispatcher picks by itself (6 x 2 less
-    # one that would spill), and a third, with two classes of INT4 tiles, of two of those (2 x 2 less one that would spill)
-    assert seen == 30
+    # (group scales or not) x ((MB 2, MB 3, MB 4, MB 4 with paired A fetches) x (4, 8 k slices) + MB 2 paired with 8 slices +
+    # MB 8), a second build without the optional paths of those that the dispatcher picks by itself (8 x 2 less
+    # one that would spill), and a third, with two classes of INT4 tiles, of three of those (3 x 2 less one that would spill)
+    assert seen == 40
     # (group scales or not) x seven tiles x (with or without the fused epilogue and the gfx950 order)
     assert wide == 28
     assert not re.findall(r"\.vgpr_spill_count:\s+[1-9]", asm), "a kernel spills VGPRs"
@@ -131,4 +131,4 @@ def test_kernel_arguments_are_loaded_in_one_batch(asm):
         # the code of the epilogue may be laid out ahead of the loops: its loads (fused-epilogue pointers) do not count
         late = [(n, l) for n, l in late if not re.search(r"0x(c8|d0|d8)$", l)]
         assert not late, f"{name}: kernel-argument loads after the prologue: {late[:4]}"
-    assert seen == 72            # (the m <= 16 kernel's builds with the partial tiles exchanged inside one XCD are 8 of them)
+    assert seen == 82            # (the m <= 16 kernel's builds with the partial tiles exchanged inside one XCD are 8 of them)
