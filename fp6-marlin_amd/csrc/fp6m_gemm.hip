@@ -485,6 +485,72 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
     }
 }
 
+// How a launch of gemm_mb_kernel cuts the k range: parts per INT4 and FP6 tile, k slices (waves) per workgroup.
+struct MbSplit {
+    long long ks, ks6;
+    int wk;
+    bool too_large;           // more partial tiles than a scratch of fixed size holds
+};
+
+// The time of one launch of gemm_mb_kernel, us, for the choice among its tiles of 32, 48 and 64 rows.
+//
+// None of them wins everywhere: a taller tile dequantises less often and reads fewer words, a shorter one fills its rows and
+// the CUs better and reduces less per workgroup.  Which of them does follows from how many workgroups there are and how long
+// their slices get, so the launch is estimated from its split (least squares without negative terms, over 882 points: 28
+// shapes and 130 random ones of k = 2048 .. 20480 by n = 2048 .. 40960 at 33 to 400 rows, both scale modes, none to 1024 FP6
+// columns; they reproduce the times to 3-6 %).  Against the one tile height that the rows suggested (64 from 49 on, or 128, or
+// the many-rows kernel where those were estimated faster) the choice takes 6.4 % off over all those points and is within
+// 0.7 % of the best of all of them on average, where that rule was 7.6 % off; fitted to one half of the points it does the
+// same on the other.  A challenger must be 5 % faster by the estimate; of 403 points where the choice changes ten lose more
+// than 1.5 % (the worst 17 %, 121 x 15360 x 2304).  Together with the 48-row
+// tile itself 287 other random points of 33 to 1200 rows: -7.7 % (33-96 rows -13 to -14 %, 129-192 -8 %, 301-500 -2 %), the
+// worst +4.9 % (166 x 19968 x 3072), from 500 rows on nothing changes.
+// 32-row tiles: 64 x 4096 x 4096 14.4 -> 10.9 us, 96 x 5120 x 5120 18.5 -> 14.7, 80 x 8192 x 10240 36.4 -> 28.7; 48-row
+// tiles: 96 x 8192 x 8192 26.7 -> 24.1, 96 x 13824 x 5120 29.9 -> 26.7, 144 x 4096 x 12288 33.1 -> 29.3.
+struct MbTime {
+    // At most one workgroup per CU: us once; per k step (32 rows) of the mean and of the longest slice, and what group scales
+    // and full occupation add per step; per step by which an FP6 slice exceeds 0.7 of an INT4 slice; with a split: us once,
+    // per part, and for full occupation.
+    double start, mean, longest, group, busy, fp6, split, part, split_busy;
+};
+struct MbTimeMany {
+    // More: per CU two workgroups of four waves at a time.  us once; per step of a full round, and with group scales; the last
+    // round up to one workgroup per CU, by occupation and once, and beyond one, once and by occupation; us per round; group
+    // scales in the last round.
+    double start, full, full_group, low_busy, low, high, high_busy, round, last_group;
+};
+constexpr MbTime kMbTimeEight[] = {{5.479, 0.322, 0.224, 0.046, 0.125, 0.181, 1.422, 0.099, 0.427},    // 32, 48, 64 rows, eight waves
+                                   {6.556, 0.302, 0.268, 0.043, 0.237, 0.249, 0.924, 0.311, 0.588},
+                                   {7.479, 0.488, 0.107, 0.054, 0.358, 0.284, 0.0, 0.509, 1.348}};
+constexpr MbTime kMbTimeFour[] = {{0.0, 0.0, 1.241, 0.0, 0.0, 0.298, 0.0, 0.0, 0.702},                 // ... four waves
+                                  {6.091, 0.0, 0.429, 0.025, 0.0, 0.143, 0.312, 0.618, 0.841},
+                                  {7.553, 0.032, 0.375, 0.0, 0.079, 0.102, 0.372, 0.676, 1.243}};
+constexpr MbTime kMbTimeTall = {9.971, 0.0, 0.533, 0.01, 0.191, 0.224, 2.606, 0.959, 0.0};             // 128 rows
+constexpr MbTimeMany kMbTimeMany[] = {{1.919, 0.91, 0.034, 0.24, 0.207, 0.749, 0.179, 1.99, 0.018},
+                                      {3.003, 0.932, 0.037, 0.241, 0.172, 0.679, 0.24, 2.954, 0.066},
+                                      {4.016, 1.055, 0.06, 0.289, 0.208, 0.804, 0.246, 3.459, 0.052}};
+// tiles: all, tiles6 of them FP6.  No estimate for 128-row tiles beyond one workgroup per CU (0).
+inline double mb_time(int mb, const MbSplit& sp, long long tiles, long long tiles6, long long mtiles, int k, int units, bool g128, int cus)
+{
+    const double per_unit = k / (32.0 * units), g = g128 ? 1.0 : 0.0;
+    auto longest = [&](long long slices) { return (double)((units + slices - 1) / slices) * per_unit; };
+    const double s = longest(sp.ks * sp.wk), mean = k / (32.0 * sp.ks * sp.wk);
+    const long long base = tiles * mtiles;
+    if (base * sp.ks <= cus) {
+        const MbTime& c = mb == 8 ? kMbTimeTall : (sp.wk == 8 ? kMbTimeEight : kMbTimeFour)[mb - 2];
+        const double busy = (double)((tiles - tiles6) * sp.ks + tiles6 * sp.ks6) * mtiles / cus;
+        const double mean6 = tiles6 ? k / (32.0 * sp.ks6 * sp.wk) : 0.0, over6 = mean6 - 0.7 * mean;
+        return c.start + c.mean * mean + c.longest * s + c.group * mean * g + c.busy * mean * busy + (over6 > 0 ? c.fp6 * over6 : 0.0) +
+               (sp.ks > 1 ? c.split + c.part * sp.ks + c.split_busy * busy : 0.0);
+    }
+    if (mb == 8) return 0.0;
+    const MbTimeMany& c = kMbTimeMany[mb - 2];
+    const long long wgs = base * sp.ks, full = wgs / (2 * cus), rem = wgs % (2 * cus);
+    double t = c.start + full * s * (c.full + c.full_group * g) + c.round * (full + (rem ? 1 : 0));
+    if (rem) t += s * (c.last_group * g + (rem <= cus ? c.low + c.low_busy * rem / cus : c.high + c.high_busy * (rem - cus) / cus));
+    return t;
+}
+
 // Whether a launch of more than 16 rows goes to gemm_wide_kernel, and with which tile: 1 .. 7, or 0 (gemm_mb_kernel).
 //
 // The wide kernel's tiles (128 or fewer rows x 256 columns, all of k) are large, so what decides is how their number
@@ -524,8 +590,10 @@ constexpr WidePlan kWidePlans[] = {
 };
 constexpr int kWidePlanCount = sizeof(kWidePlans) / sizeof(kWidePlans[0]);
 constexpr int kWideNarrow = 5;    // from this row on: NARROW6
-inline int wide_plan(int m, int n, int k, int qc, bool g128, int mb, int max_par, int cus)
+// `est`: the estimate of what is chosen, gemm_mb_kernel with `mb` included (0: none).
+inline int wide_plan(int m, int n, int k, int qc, bool g128, int mb, int max_par, int cus, double* est)
 {
+    *est = 0.0;
     if (m <= 64 || k < 2048) return 0;
     const int tile_rows = 16 * mb, tiles_n = n / kTileN, row_tiles = (m + tile_rows - 1) / tile_rows;
     // Without FP6 columns, with per-column scales and at most one workgroup of 128 rows per CU the estimate below is too high
@@ -552,6 +620,7 @@ inline int wide_plan(int m, int n, int k, int qc, bool g128, int mb, int max_par
         }
     }
     int best = 0;
+    *est = us;
     us *= 0.97;
     for (int i = 0; i < kWidePlanCount; i++) {
         const WidePlan& p = kWidePlans[i];
@@ -570,6 +639,7 @@ inline int wide_plan(int m, int n, int k, int qc, bool g128, int mb, int max_par
         if (t * (narrow6 && !best ? 1.06 : 1.0) < us) {
             us = t;
             best = i + 1;
+            *est = us;
         }
     }
     return best;
@@ -794,10 +864,115 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             (size_t)(tiles_n + qc / kTileN) * ((rows8 + 127) / 128) * ks8 * (8 * 16 * kTileN * sizeof(float)) <= scratch_bytes)
             mb = 8;
     }
+    const int units = g128 ? prob_k / 128 : prob_k / 64;
+    const long long env_ks = tune.ksplit != kUnset ? tune.ksplit : 0;
+    // The split of one launch of gemm_mb_kernel (16 rows and more) with tiles of 16 * mb rows.
+    auto split_mb = [&](int mb, int mtiles) {
+        const int rows_per_tile = 16 * mb;
+        // m > 16: a task is one workgroup (one tile x four k slices) on one row tile and k part.
+        // Split k only as far as needed to give every CU a workgroup; partial tiles are 16*MB rows
+        // of fp32, so the split is also capped by their traffic relative to the weight stream.
+        const long long base = (long long)a.tiles * mtiles;
+        const size_t tile_bytes = (size_t)rows_per_tile * kTileN * sizeof(float);
+        MbSplit sp;
+        sp.too_large = false;
+        long long ks = cus / base;
+        // (two k units per wave at least, one on a short k up to four parts; a grid that leaves half of the CUs idle even
+        // so may split twice as far as the partial tiles' traffic would otherwise allow: 2048 x 2560 .. 7680 at 32 and
+        // 64 rows 10.4 -> 9.2-9.8 us and 13.8 -> 12.7-13.0; eight parts instead of four on k = 4096 cost 6-12 %)
+        long long ks_k = units / (kWaves * 2);
+        if (ks_k < 4) ks_k = units / kWaves < 4 ? units / kWaves : 4;
+        if (ks_k < 1) ks_k = 1;
+        long long cap = (long long)prob_k / (16LL * rows_per_tile) > 0 ? (long long)prob_k / (16LL * rows_per_tile) : 1;
+        if (base * 2 * cap <= cus) cap *= 2;
+        if (ks > ks_k) ks = ks_k;
+        if (ks > cap) ks = cap;
+        if (sms > 0 && ks > sms) ks = sms;
+        if (env_ks >= 1) ks = env_ks;
+        if (ks < 1) ks = 1;
+        sp.too_large = fixed_scratch && ks > 1 && (size_t)(a.tiles + a.tiles6) * mtiles * ks * tile_bytes > scratch_bytes;
+        while (ks > 1 && (size_t)(a.tiles + a.tiles6) * mtiles * ks * tile_bytes > scratch_bytes) ks--;   // (FP6 tiles: 2 ks)
+        // A grid of at most one workgroup per CU would leave every SIMD a single wave: give the workgroup eight
+        // k slices instead of four (same partial-sum traffic, two waves per SIMD) when k is long enough.
+        // (Two waves on a SIMD take turns at its one VALU/MFMA port: eight half-length slices last as long as four
+        // whole ones, so eight (which hide latency better: 13824 x 5120 at 256 rows 60.6 vs 67.8 us) only pay while
+        // their longest slice, in whole k units, is no more than 0.58 of the longest of four: 5120 x 13824 at 64
+        // rows, 40 units over 16 slices of up to 3: 24.1 us, over 8 slices of 5: 21.7.)
+        // From forced tables (4 or 8 slices x 1 .. 8 parts, 32 / 64 / 128 rows): a split is no finer than its longest
+        // slice needs (8192 x 6144 at 32 rows: 64 units in 5 parts = 20 slices of up to 4, 16.7 us; in 4 parts = 16
+        // slices of 4, 16.0; as eight-wave workgroups 14.3); one unit per wave is enough for eight (8192 x 2048 at
+        // 32 rows 12.8 -> 12.0); 0.58 rather than 0.55 (14336 x 8192 at 32 rows, 4 against 7 units, 23.0 -> 20.5);
+        // and beyond eight parts the partners' partial tiles cost more than shorter slices gain (14336 x 2048 at
+        // 32 rows: 14 parts of four slices 16.7 us, 8 parts of eight 14.8; at 64 rows 24.0 -> 21.0).
+        auto longest = [&](long long slices) { return (units + slices - 1) / slices; };
+        const bool free_split = env_ks < 1 && sms <= 0 && !row_mix && mb != 8;
+        if (free_split)
+            while (ks > 1 && longest(4 * (ks - 1)) == longest(4 * ks)) ks--;
+        // (32-row tiles are not issue-bound: two waves per SIMD pay up to two thirds, 11008 x 2560 at 32 rows 14.9 -> 13.2)
+        const bool eight_pays = mb == 2 ? 3 * longest(8 * ks) <= 2 * longest(4 * ks) : 50 * longest(8 * ks) <= 29 * longest(4 * ks);
+        int wk = base * ks <= cus && units / 8 >= ks && eight_pays ? 8 : kWaves;
+        if (free_split && tune.wk == kUnset && ks > 8 && base * 8 <= cus && units / 8 >= 8) {
+            wk = 8;
+            ks = 8;
+        }
+        if (tune.wk != kUnset) wk = tune.wk == 8 ? 8 : kWaves;
+        if (mb == 8) wk = kWaves;                                  // (512 registers per wave: one wave per SIMD)
+        // An FP6 step costs more issue slots than an INT4 one, and in a grid that is resident all at once the few
+        // FP6 tiles' workgroups set the length of the launch (8192 x 8192 at m = 128: 33 us against 29 us with INT4
+        // only).  Their k range is cut twice as finely where every slice still gets two units and the grid still
+        // fits the CUs in one go (5120 x 13824 at m = 128: 40 -> 31 us; a grid whose last workgroups must wait for
+        // a free CU loses far more than that).  A forced split applies to both kinds.
+        sp.ks = sp.ks6 = ks;
+        sp.wk = wk;
+        // (a grid that fits one workgroup per CU must still do so afterwards: a CU with two runs both at little
+        // more than half speed, 11008 x 4096 at 256 rows 34 -> 52 us with 272 workgroups)
+        const long long resident = (long long)cus * (wk == 8 || mb == 8 || base * ks <= cus ? 1 : 2);
+        // (Not for 128-row tiles, whose FP6 workgroups are only a few per cent behind: there the second partner's
+        // partial tiles cost more than the shorter loop gains, 8192 x 8192 at m = 384 61.8 vs 58.4 us.)
+        // Re-measured with every tile on the paired loop (ten shapes x 32 .. 256 rows, alternating): still 5-13 % on
+        // wide weights up to two row tiles (4096 x 11008 at 128 rows 25.3 -> 22.2 us, 8192 x 28672 at 32 rows
+        // 38.2 -> 34.5), but 3-8 % slower from three row tiles on (5120 x 5120 at 256 rows 27.4 -> 29.7): up to two.
+        // Where twice does not fit, as finely as does (13824 x 5120 with 512 FP6 columns, per-column scales, 64 rows: 6 parts for
+        // all tiles 22.1 us, 10 for the FP6 tiles 21.4).
+        if (env_ks < 1 && !row_mix && a.tiles6 > 0 && mb != 8 && mtiles <= 2) {
+            long long c6 = units / (2 * wk) < 2 * ks ? units / (2 * wk) : 2 * ks;
+            const long long room = (resident - (base - (long long)a.tiles6 * mtiles) * ks) / ((long long)a.tiles6 * mtiles);
+            if (c6 > room) c6 = room;
+            if (c6 > ks) sp.ks6 = c6;
+        }
+        return sp;
+    };
     // Many rows (gemm_wide.h): one launch over all of them, without a k split across workgroups.
-    if (prob_m > 16 && !row_mix && prob_k % 128 == 0 && prob_n % 256 == 0 && (!fu.a_cols || (size_t)prob_m * prob_k * sizeof(uint16_t) <= kGatherBytes)) {
-        const bool free_plan = tune.mb == kUnset && tune.ksplit == kUnset && tune.wk == kUnset && tune.pair == kUnset && tune.cls == kUnset && sms <= 0;
-        int plan = tune.wide != kUnset ? tune.wide : (free_plan ? wide_plan(prob_m, prob_n, prob_k, qc, g128, mb, max_par, cus) : 0);
+    const bool free_plan = tune.mb == kUnset && tune.ksplit == kUnset && tune.wk == kUnset && tune.pair == kUnset && tune.cls == kUnset && sms <= 0;
+    const bool wide_fits = prob_m > 16 && !row_mix && prob_k % 128 == 0 && prob_n % 256 == 0 &&
+                           (!fu.a_cols || (size_t)prob_m * prob_k * sizeof(uint16_t) <= kGatherBytes);
+    double est = 0.0;
+    int plan = !wide_fits ? 0 : (tune.wide != kUnset ? tune.wide : (free_plan ? wide_plan(prob_m, prob_n, prob_k, qc, g128, mb, max_par, cus, &est) : 0));
+    // Tiles of 32, 48 or 64 rows instead (MbTime).  Not asked below k = 2048, where nothing was fitted, for what one launch
+    // does not cover, nor where one row tile meets more column tiles than CUs (two classes of tiles, below; not in the fit).
+    if (prob_m > 32 && !row_mix && free_plan && tune.wide == kUnset && prob_k >= 2048) {
+        auto time_of = [&](int mb_try) {
+            const int mtiles = (prob_m + 16 * mb_try - 1) / (16 * mb_try);
+            if (mtiles > max_par || (mtiles == 1 && a.tiles > cus)) return 0.0;
+            const MbSplit sp = split_mb(mb_try, mtiles);
+            return sp.too_large ? 0.0 : mb_time(mb_try, sp, a.tiles, a.tiles6, mtiles, prob_k, units, g128, cus);
+        };
+        const bool low = plan == 0 && mb < 8;              // what stands is one of the three itself
+        if (plan == 0) {
+            const double t = time_of(mb);
+            if (t > 0.0 || low) est = t;
+        }
+        est *= 0.95;
+        for (int mb_try = 2; mb_try <= 4; mb_try++) {
+            const double t = time_of(mb_try);
+            if (t > 0.0 && t < est) {
+                est = t;
+                mb = mb_try;
+                plan = 0;
+            }
+        }
+    }
+    if (wide_fits) {
         if (plan > 0) {
             WideArgs w;
             w.A = static_cast<const uint16_t*>(A);
@@ -840,7 +1015,6 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
     }
     const int rows_per_tile = 16 * mb;
     const int mtiles_total = (prob_m + rows_per_tile - 1) / rows_per_tile;
-    const int units = g128 ? prob_k / 128 : prob_k / 64;
 
     if (fu.a_cols) {
         const long long launch_rows = prob_m < (long long)rows_per_tile * max_par ? prob_m : (long long)rows_per_tile * max_par;
@@ -863,9 +1037,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             a.A = sc.gathered;
         };
 
-        const size_t tile_bytes = (size_t)mb * 16 * kTileN * sizeof(float);
         const long long traffic_cap = (long long)prob_k / (64LL * a.m) > 0 ? (long long)prob_k / (64LL * a.m) : 1;
-        const long long env_ks = tune.ksplit != kUnset ? tune.ksplit : 0;
         if (mb == 1 && !row_mix && (tune.sk != kUnset ? tune.sk != 0 && a.m <= 4 : a.m == 1) && prob_k / 64 < 65536 && (long long)a.tiles * (prob_k / 64) < (1 << 24) &&
                    (long long)prob_k * prob_n / 2 < (1LL << 32) && (long long)(prob_n / 128) * max_par >= 2 &&
                    (g128 || n4 == 0 || units >= 2)) {
@@ -1411,76 +1583,12 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             launch_m16_any(cfg, a, g128, grid, st);
         } else {
             gather_pass();
-            // m > 16: a task is one workgroup (one tile x four k slices) on one row tile and k part.
-            // Split k only as far as needed to give every CU a workgroup; partial tiles are 16*MB rows
-            // of fp32, so the split is also capped by their traffic relative to the weight stream.
-            const long long base = (long long)a.tiles * mtiles;
-            long long ks = cus / base;
-            // (two k units per wave at least, one on a short k up to four parts; a grid that leaves half of the CUs idle even
-            // so may split twice as far as the partial tiles' traffic would otherwise allow: 2048 x 2560 .. 7680 at 32 and
-            // 64 rows 10.4 -> 9.2-9.8 us and 13.8 -> 12.7-13.0; eight parts instead of four on k = 4096 cost 6-12 %)
-            long long ks_k = units / (kWaves * 2);
-            if (ks_k < 4) ks_k = units / kWaves < 4 ? units / kWaves : 4;
-            if (ks_k < 1) ks_k = 1;
-            long long cap = (long long)prob_k / (16LL * rows_per_tile) > 0 ? (long long)prob_k / (16LL * rows_per_tile) : 1;
-            if (base * 2 * cap <= cus) cap *= 2;
-            if (ks > ks_k) ks = ks_k;
-            if (ks > cap) ks = cap;
-            if (sms > 0 && ks > sms) ks = sms;
-            if (env_ks >= 1) ks = env_ks;
-            if (ks < 1) ks = 1;
-            if (fixed_scratch && ks > 1 && (size_t)(a.tiles + a.tiles6) * mtiles * ks * tile_bytes > scratch_bytes) return FP6M_ERR_SCRATCH;
-            while (ks > 1 && (size_t)(a.tiles + a.tiles6) * mtiles * ks * tile_bytes > scratch_bytes) ks--;   // (FP6 tiles: 2 ks)
-            a.ksplit = (int)ks;
-            // A grid of at most one workgroup per CU would leave every SIMD a single wave: give the workgroup eight
-            // k slices instead of four (same partial-sum traffic, two waves per SIMD) when k is long enough.
-            // (Two waves on a SIMD take turns at its one VALU/MFMA port: eight half-length slices last as long as four
-            // whole ones, so eight (which hide latency better: 13824 x 5120 at 256 rows 60.6 vs 67.8 us) only pay while
-            // their longest slice, in whole k units, is no more than 0.58 of the longest of four: 5120 x 13824 at 64
-            // rows, 40 units over 16 slices of up to 3: 24.1 us, over 8 slices of 5: 21.7.)
-            // From forced tables (4 or 8 slices x 1 .. 8 parts, 32 / 64 / 128 rows): a split is no finer than its longest
-            // slice needs (8192 x 6144 at 32 rows: 64 units in 5 parts = 20 slices of up to 4, 16.7 us; in 4 parts = 16
-            // slices of 4, 16.0; as eight-wave workgroups 14.3); one unit per wave is enough for eight (8192 x 2048 at
-            // 32 rows 12.8 -> 12.0); 0.58 rather than 0.55 (14336 x 8192 at 32 rows, 4 against 7 units, 23.0 -> 20.5);
-            // and beyond eight parts the partners' partial tiles cost more than shorter slices gain (14336 x 2048 at
-            // 32 rows: 14 parts of four slices 16.7 us, 8 parts of eight 14.8; at 64 rows 24.0 -> 21.0).
-            auto longest = [&](long long slices) { return (units + slices - 1) / slices; };
-            const bool free_split = env_ks < 1 && sms <= 0 && !row_mix && mb != 8;
-            if (free_split)
-                while (ks > 1 && longest(4 * (ks - 1)) == longest(4 * ks)) ks--;
-            // (32-row tiles are not issue-bound: two waves per SIMD pay up to two thirds, 11008 x 2560 at 32 rows 14.9 -> 13.2)
-            const bool eight_pays = mb == 2 ? 3 * longest(8 * ks) <= 2 * longest(4 * ks) : 50 * longest(8 * ks) <= 29 * longest(4 * ks);
-            int wk = base * ks <= cus && units / 8 >= ks && eight_pays ? 8 : kWaves;
-            if (free_split && tune.wk == kUnset && ks > 8 && base * 8 <= cus && units / 8 >= 8) {
-                wk = 8;
-                ks = 8;
-            }
-            if (tune.wk != kUnset) wk = tune.wk == 8 ? 8 : kWaves;
-            if (mb == 8) wk = kWaves;                                  // (512 registers per wave: one wave per SIMD)
-            a.ksplit = (int)ks;
-            // An FP6 step costs more issue slots than an INT4 one, and in a grid that is resident all at once the few
-            // FP6 tiles' workgroups set the length of the launch (8192 x 8192 at m = 128: 33 us against 29 us with INT4
-            // only).  Their k range is cut twice as finely where every slice still gets two units and the grid still
-            // fits the CUs in one go (5120 x 13824 at m = 128: 40 -> 31 us; a grid whose last workgroups must wait for
-            // a free CU loses far more than that).  A forced split applies to both kinds.
-            a.ks4 = (int)ks;
-            a.ks6 = (int)ks;
-            // (a grid that fits one workgroup per CU must still do so afterwards: a CU with two runs both at little
-            // more than half speed, 11008 x 4096 at 256 rows 34 -> 52 us with 272 workgroups)
-            const long long resident = (long long)cus * (wk == 8 || mb == 8 || base * ks <= cus ? 1 : 2);
-            // (Not for 128-row tiles, whose FP6 workgroups are only a few per cent behind: there the second partner's
-            // partial tiles cost more than the shorter loop gains, 8192 x 8192 at m = 384 61.8 vs 58.4 us.)
-            // Re-measured with every tile on the paired loop (ten shapes x 32 .. 256 rows, alternating): still 5-13 % on
-            // wide weights up to two row tiles (4096 x 11008 at 128 rows 25.3 -> 22.2 us, 8192 x 28672 at 32 rows
-            // 38.2 -> 34.5), but 3-8 % slower from three row tiles on (5120 x 5120 at 256 rows 27.4 -> 29.7): up to two.
-            // Where twice does not fit, as finely as does (13824 x 5120 with 512 FP6 columns, per-column scales, 64 rows: 6 parts for
-            // all tiles 22.1 us, 10 for the FP6 tiles 21.4).
-            if (env_ks < 1 && !row_mix && a.tiles6 > 0 && mb != 8 && mtiles <= 2) {
-                long long c6 = units / (2 * wk) < 2 * ks ? units / (2 * wk) : 2 * ks;
-                const long long room = (resident - (base - (long long)a.tiles6 * mtiles) * ks) / ((long long)a.tiles6 * mtiles);
-                if (c6 > room) c6 = room;
-                if (c6 > ks) a.ks6 = (int)c6;
-            }
+            const MbSplit sp = split_mb(mb, mtiles);
+            const long long base = (long long)a.tiles * mtiles, ks = sp.ks;
+            int wk = sp.wk;
+            if (sp.too_large) return FP6M_ERR_SCRATCH;
+            a.ksplit = a.ks4 = (int)sp.ks;
+            a.ks6 = (int)sp.ks6;
             // One row tile and somewhat more tiles than CUs: workgroups of four waves, two to a CU, run both at little more
             // than half speed, so the CUs that get two set the launch's length at 1.76 x that of a grid that fits
             // (8192 x 36864 at 32 rows: 288 tiles 60.9 us, 256 tiles 34.6).  Two classes of INT4 tiles instead (as in the
@@ -1499,6 +1607,8 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                     long long cb = cus / nb;
                     const long long cb_k = prob_k / 1024 > 0 ? prob_k / 1024 : 1;               // 128 rows of k per wave at least
                     if (cb > cb_k) cb = cb_k;
+                    const long long cap = (long long)prob_k / (16LL * rows_per_tile) > 0 ? (long long)prob_k / (16LL * rows_per_tile) : 1;
+                    const size_t tile_bytes = (size_t)rows_per_tile * kTileN * sizeof(float);
                     if (cb > cap) cb = cap;
                     // (partial-tile slots are numbered over all tiles, the whole ones of the first class included)
                     while (cb > 1 && (size_t)(a.tiles6 * c6 + na + nb * cb) * tile_bytes > scratch_bytes) cb--;

@@ -282,6 +282,22 @@ def test_three_row_blocks_per_wave(oracle, capfd):
     assert "MB=3 row tiles 1 ks4=6" in out and "ks6=6 " not in out, out
 
 
+def test_row_tiles_by_estimate(oracle, capfd):
+    """From k = 2048 on the height of the row tiles (32, 48 or 64 rows) follows from estimated times: row counts at both sides
+    of every tile's edges, both scale modes, with FP6 columns and without; below, from the rows alone."""
+    import re
+    capfd.readouterr()
+    for gs in (128, -1):
+        for m in (33, 48, 49, 64, 65, 96, 97, 129, 144, 145, 200, 257):
+            run(oracle, m, 768, 2048, qc=256, gs=gs, env={"FP6M_VERBOSE": 1})
+        run(oracle, 64, 768, 4096, qc=-1, gs=gs, env={"FP6M_VERBOSE": 1})
+        run(oracle, 96, 1280, 2048, qc=1280, gs=gs, env={"FP6M_VERBOSE": 1})
+    # (so few columns: 32-row tiles throughout; 48-row tiles by the estimate are in the test of the long k below)
+    assert set(re.findall(r"MB=(\d)", capfd.readouterr().err)) == {"2"}
+    run(oracle, 65, 768, 1920, qc=256, env={"FP6M_VERBOSE": 1})
+    assert "MB=4" in capfd.readouterr().err
+
+
 def test_eight_row_blocks_per_wave(oracle):
     """The m > 16 kernel with eight 16-row blocks per wave (128-row tiles, accumulators in the accumulation
     registers), forced onto small problems: ragged row tiles, both regions, both scale modes, k splits through the
@@ -908,10 +924,10 @@ def test_random_shapes_rows_and_limits_against_unpacked_words(oracle):
 def test_long_k_with_a_poorly_filled_grid_takes_128_row_tiles_with_a_k_split(capfd):
     """13824 x 5120 at 256 rows: 160 workgroups of 64 rows would occupy 160 of 256 CUs with nothing left to split; the
     dispatcher takes 128-row tiles with three k parts instead (read back from its verbose output) and the result is
-    checked per region against the pinned unpacker; on k = 8192 the rule does not apply."""
+    checked per region against the pinned unpacker; on k = 8192 the rule does not apply (240 workgroups of 48 rows)."""
     import fp6_marlin
     g = torch.Generator().manual_seed(9)
-    for k, n, want in ((13824, 5120, "MB=8 row tiles 2 ks4=3"), (8192, 5120, "MB=4")):
+    for k, n, want in ((13824, 5120, "MB=8 row tiles 2 ks4=3"), (8192, 5120, "MB=3 row tiles 6")):
         qc, gs, m = 256, 128, 256
         n4 = n - qc
         B = torch.randint(-2 ** 31, 2 ** 31 - 1, (k * n4 // 8 + k * qc * 3 // 16,), generator=g, dtype=torch.int64).to(torch.int32)
