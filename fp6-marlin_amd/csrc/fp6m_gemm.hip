@@ -566,12 +566,17 @@ inline double mb_time(int mb, const MbSplit& sp, long long tiles, long long tile
 // was then measured on 2689 more, with none (-23 % on average), 256, 512, 1024, a quarter, half and all of the columns in FP6
 // (-23 to -27 % each): 12 of them are more than 2 % slower, the worst 208 x 14080 x 40448 all in FP6, +14 %.
 //
-// The last two plans (FP6 tiles in workgroups of their own) were fitted to 170 more shapes of 65 to 1600 rows with 256 FP6
+// Plans 6 and 7 (FP6 tiles in workgroups of their own) were fitted to 170 more shapes of 65 to 1600 rows with 256 FP6
 // columns, to 2-3 %; the seven plans' choice is again 0.3 % off the best there.  They are not asked where the extra
 // workgroups would start another round, nor where FP6 is more than a quarter of the columns: an all-FP6 weight has twice
 // the workgroups then (400 x 8192 x 10240: 93 us instead of 78).  Against gemm_mb_kernel they must win by 9 %: where that
 // kernel has exactly a round of 128-row tiles its estimate is too high (512 x 8192 x 8192 with per-column scales: 61 us, not
 // 68; the 80-row tiles 69).
+// Plans 8 and 9 are the same with 64 and 48 rows, for launches that taller tiles leave CUs idle in (300 x 4096 x 12288: 196
+// workgroups of 80 rows, 245 of 64), fitted to 206 shapes of 65 to 900 rows with none to 1024 FP6 columns (1.9 %, the worst
+// 8 %).  Over 420 shapes of those rows, half of them not in the fit, they are taken on 42: -11 % on average there, none slower;
+// us: 300 x 4096 x 12288 40.7 -> 39.4, 181 x 3072 x 14592 with per-column scales 28.7 -> 23.3, 229 x 3584 x 10496 32.1 -> 25.5,
+// 178 x 8960 x 17920 86.4 -> 75.4, 525 x 2816 x 5376 29.8 -> 24.1.
 struct WidePlan {
     int mb, per_cu;               // 16-row blocks per tile; workgroups per CU
     double start, round, part;    // us: once; per full round; once if the last round is not full
@@ -587,6 +592,8 @@ constexpr WidePlan kWidePlans[] = {
     {6, 2, 35.5, 7.2, -30.5, 65.2, 10.0, 44.1, 1.2, 3.3, 0.0, 60.6, 7.3, 19.1},
     {6, 1, 6.6, 6.9, 0.6, 33.6, 3.2, 27.4, 1.4, 5.5, 2.9, 0, 0, 0},
     {5, 1, 6.3, 6.8, 0.3, 28.7, 4.3, 24.4, 3.5, 4.4, 1.7, 0, 0, 0},
+    {4, 1, 0.0, 3.9, 5.8, 28.2, 4.2, 22.5, 3.8, 3.6, 0.6, 0, 0, 0},
+    {3, 1, 3.2, 3.7, 2.4, 23.8, 3.9, 20.7, 2.9, 2.7, 0.4, 0, 0, 0},
 };
 constexpr int kWidePlanCount = sizeof(kWidePlans) / sizeof(kWidePlans[0]);
 constexpr int kWideNarrow = 5;    // from this row on: NARROW6
@@ -1007,7 +1014,9 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             case 4: launch_wide<6, 4, 2>(w, g128, st); break;
             case 5: launch_wide<6, 4, 1>(w, g128, st); break;
             case 6: launch_wide<6, 4, 2, true>(w, g128, st); break;
-            default: launch_wide<5, 4, 2, true>(w, g128, st); break;
+            case 7: launch_wide<5, 4, 2, true>(w, g128, st); break;
+            case 8: launch_wide<4, 4, 2, true>(w, g128, st); break;
+            default: launch_wide<3, 4, 2, true>(w, g128, st); break;
             }
             hipError_t e = hipGetLastError();
             return e != hipSuccess ? hip_fail(e) : FP6M_OK;

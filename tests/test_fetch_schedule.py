@@ -510,7 +510,7 @@ def run_wide(WN, WK, MB, trips_all, fp6_waves, group, **planted):
     assert len(ends) == 1                              # every wave of the workgroup meets the same barriers
 
 
-WIDE_TILES = [(4, 1, 8), (4, 2, 8), (4, 2, 7), (4, 2, 6), (4, 1, 6), (4, 2, 5), (2, 4, 6), (2, 4, 5)]   # launch_wide, NARROW6
+WIDE_TILES = [(4, 1, 8), (4, 2, 8), (4, 2, 7), (4, 2, 6), (4, 1, 6), (4, 2, 5), (2, 4, 6), (2, 4, 5), (4, 2, 4), (2, 4, 4), (4, 2, 3), (2, 4, 3)]   # launch_wide, NARROW6
 
 
 @pytest.mark.parametrize("WN,WK,MB", WIDE_TILES)

@@ -358,7 +358,7 @@ def test_one_round_of_128_row_tiles_without_fp6_columns_keeps_its_kernel(capfd):
     12 % slower than gemm_mb_kernel.  With group scales or FP6 columns, or beyond one round, it is the faster one."""
     for m, k, n in ((388, 3840, 6144), (77, 4352, 23808), (145, 3840, 12800), (176, 8192, 16384), (1050, 2816, 2048)):
         assert wide_plan_of(capfd, m, k, n, -1, -1) == 0, (m, k, n)
-    assert wide_plan_of(capfd, 300, 4096, 12288, 256, -1) == 7
+    assert wide_plan_of(capfd, 300, 4096, 12288, 256, -1) == 8
     assert wide_plan_of(capfd, 500, 4096, 22016, -1, -1) == 1
 
 
@@ -366,7 +366,8 @@ def test_one_round_of_128_row_tiles_without_fp6_columns_keeps_its_kernel(capfd):
                     reason="the plans are those of 256 CUs")
 def test_which_calls_go_to_the_many_rows_kernel(capfd):
     """The default choice: each tile where the estimates are clearly apart, and the calls that it is never asked for."""
-    for want, m, k, n, qc, gs in ((7, 300, 4096, 12288, 256, 128), (3, 2048, 8192, 10240, 256, 128), (2, 1024, 8192, 8192, 256, 128),
+    for want, m, k, n, qc, gs in ((8, 300, 4096, 12288, 256, 128), (7, 400, 4096, 12288, 256, 128), (9, 144, 4096, 20480, 256, 128),
+                                  (3, 2048, 8192, 10240, 256, 128), (2, 1024, 8192, 8192, 256, 128),
                                   (1, 700, 2048, 57344, 256, 128), (5, 150, 8192, 40960, 20480, -1), (4, 1509, 6144, 3328, 1024, 128),
                                   (6, 180, 4096, 24576, 256, 128), (0, 64, 4096, 22016, 256, 128), (0, 128, 8192, 8192, 256, 128),
                                   (0, 2048, 1920, 8192, 256, 128), (0, 2048, 4160, 8192, 256, -1)):
@@ -374,7 +375,7 @@ def test_which_calls_go_to_the_many_rows_kernel(capfd):
     assert wide_plan_of(capfd, 2048, 8192, 10240, 256, 128, sms=256) == 0
 
 
-@pytest.mark.parametrize("plan", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("plan", [1, 2, 3, 4, 5, 6, 7, 8, 9])
 def test_waves_side_by_side_in_n(oracle, plan):
     """The many-rows kernel (gemm_wide.h) in each of its tiles, forced onto small problems: ragged row tiles, a single
     trip of its loop (with two k slices: an idle one), an odd number of trips, tiles that lie in both regions, all INT4,
@@ -410,7 +411,7 @@ def test_waves_side_by_side_in_n_with_more_row_tiles_than_a_grid_takes(oracle):
         assert torch.isfinite(C1).all() and bool((C.view(times, block, n) == C1).all())
 
 
-@pytest.mark.parametrize("plan", [1, 4, 7])
+@pytest.mark.parametrize("plan", [1, 4, 7, 8, 9])
 def test_waves_side_by_side_in_n_with_maps_additions_and_the_gfx950_order(oracle, plan):
     """The same kernel's build for fp6m_mul_fused: with nothing to add the reordered result is the plain one bit for bit
     (both word orders), and the additions are rounded once."""

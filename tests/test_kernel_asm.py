@@ -103,8 +103,8 @@ def test_mfma_loops_keep_accumulators_in_place(asm):
     # MB 8), a second build without the optional paths of those that the dispatcher picks by itself (8 x 2 less
     # one that would spill), and a third, with two classes of INT4 tiles, of three of those (3 x 2 less one that would spill)
     assert seen == 40
-    # (group scales or not) x seven tiles x (with or without the fused epilogue and the gfx950 order)
-    assert wide == 28
+    # (group scales or not) x nine tiles x (with or without the fused epilogue and the gfx950 order)
+    assert wide == 36
     assert not re.findall(r"\.vgpr_spill_count:\s+[1-9]", asm), "a kernel spills VGPRs"
     # nothing may live in private memory either: a pointer that the compiler keeps on the stack costs the decode loop a
     # scratch load and a full `s_waitcnt vmcnt(0)` per step (seen once with pointers advanced under uniform branches)
