@@ -170,6 +170,11 @@ def test_the_range_is_known_before_the_packing_is_done(k, n, qc):
             fp6_marlin.pack_mixed_weight(bad, qc, -1, harness_layout=False)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):                      # a stream of the caller's own: done when the call returns
+        for _ in range(30):
+            big @ big
+        fp6_marlin.pack_mixed_weight(w, qc, -1, harness_layout=False)
+        assert side.query()
     results = []
     for i in range(4):
         mine = w.clone()
