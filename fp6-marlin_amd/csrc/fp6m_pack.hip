@@ -659,9 +659,10 @@ int pack_mixed(const void* w, int k, int n, int quant_cols, int group_size, int 
     if (qc) {
         // The range check of the FP6 cast is reported by value, so this call waits: for the kernels in front of pack_kernel,
         // which find the maxima, or, where the harness layout's kernel checks cast by cast, where something is out of range
-        // or failed to launch (the flag's line is another call's next), and where it is asked for, for all of them.  With
-        // every call waiting for all of them the GPU was idle between one call's last kernel and the next one's first:
-        // 4096 x 22016, group-128 scales, 256 FP6 columns, calls in a row 106.6 -> 85.2 us each.
+        // or failed to launch (the flag's line is another call's next), and from the entry that waits, for all of them.  With
+        // every call waiting for all of them the GPU is idle between one call's last kernel and the next one's first:
+        // 4096 x 22016, group-128 scales, 256 FP6 columns, calls in a row 106.6 us each, 85.2 from the other entry (a call
+        // that is waited for takes as long from either).
         if (!(e == hipSuccess && a.range_known && flag.known_soon() && !flag.out_of_range())) {
             const hipError_t waited = flag.wait(st);
             if (e == hipSuccess) e = waited;

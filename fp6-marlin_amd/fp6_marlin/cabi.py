@@ -184,8 +184,9 @@ def unpack_to_fp16(B, s, k, n, quant_cols=-1, group_size=-1):
 def pack_mixed_weight_device(w, quant_cols=-1, group_size=-1, harness_layout=True, want_ref=True):
     """Quantise and pack a CUDA float16 weight [k, n] on the GPU; same outputs, bit for bit, as the host path
     (`layer.pack_mixed_weight`).  Returns (B int32 1-D, s float16 1-D, w_ref float16 [k, n] or None), all on
-    w's device.  On the default stream they are ready in its order, like the results of any operation on the GPU; on a
-    stream of the caller's own, with FP6 columns, when the call returns, so that one may hand them to other streams."""
+    w's device.  With FP6 columns they are ready when the call returns, on whatever stream it was made: they may go to other
+    streams (torch's are not ordered against the default one) and w may be overwritten.  Without, the call does not
+    wait: they are ready in stream order."""
     if not isinstance(w, torch.Tensor) or not w.is_cuda or w.dtype != torch.float16 or w.dim() != 2:
         raise ValueError("w must be a 2-D CUDA float16 tensor")
     w = w.contiguous()
@@ -199,10 +200,10 @@ def pack_mixed_weight_device(w, quant_cols=-1, group_size=-1, harness_layout=Tru
     ref = torch.empty((k, n), dtype=torch.float16, device=w.device) if want_ref else None
     with torch.cuda.device(w.device):
         stream = torch.cuda.current_stream()
-        w.record_stream(stream)                       # (the packing may still read it when the call returns)
-        pack = lib.fp6m_pack_mixed_device_async if stream == torch.cuda.default_stream() else lib.fp6m_pack_mixed_device
-        code = pack(w.data_ptr(), k, n, qc, int(group_size), int(bool(harness_layout)), B.data_ptr(), s.data_ptr(),
-                    ref.data_ptr() if want_ref else None, w.device.index, stream.cuda_stream)
+        w.record_stream(stream)                       # (without FP6 columns the packing may still read it when the call returns)
+        code = lib.fp6m_pack_mixed_device(w.data_ptr(), k, n, qc, int(group_size), int(bool(harness_layout)), B.data_ptr(),
+                                          s.data_ptr(), ref.data_ptr() if want_ref else None, w.device.index,
+                                          stream.cuda_stream)
     if code == ERR_HIP:
         raise RuntimeError(f"fp6m_pack_mixed_device: {strerror(code)} (hip error {lib.fp6m_last_hip_error()})")
     _raise_cpu(code)

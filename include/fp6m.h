@@ -300,7 +300,9 @@ int fp6m_pack_mixed_device(const void* w, int k, int n, int quant_cols, int grou
 /* The same without waiting longer than the range check needs: in the true transpose's layout the column maxima settle it,
  * and the call returns as soon as they are known while the packing itself may still run.  B, s and w_ref are then ready in
  * stream order, like any kernel's output (as they are from either entry when quant_cols <= 0), and w must stay as it is
- * until then.  After an error the call's kernels are done. */
+ * until then: a caller that hands the results to another stream, or refills w from one, records an event on `stream` first
+ * (streams made with hipStreamNonBlocking, as PyTorch's are, do not wait for the default stream either).  After an error the
+ * call's kernels are done.  For loaders that keep one stream; the Python package uses the entry above. */
 int fp6m_pack_mixed_device_async(const void* w, int k, int n, int quant_cols, int group_size, int harness_layout,
                                  void* B, void* s, void* w_ref, int dev, void* stream);
 

@@ -143,48 +143,110 @@ def test_range_errors_of_the_true_transpose(value):
         assert all(torch.equal(x, y) for x, y in zip(got, want)), (row, col)
 
 
-@pytest.mark.parametrize("k,n,qc", [(64, 128, 64), (1024, 384, 192), (4160, 1088, 1088)])
-def test_the_range_is_known_before_the_packing_is_done(k, n, qc):
-    """The package's calls return once the range is known: on a stream with other work in front (longer than the call polls),
-    on a stream of their own while the caller's tensors go, and for a weight out of range, against the entry that waits."""
+def entry_outputs(k, n, qc):
+    """B, s, w_ref for the C entries, per-column scales."""
+    return [torch.empty(size, dtype=dtype, device=dev()) for size, dtype in
+            ((k * (n - qc) // 8 + k * qc * 3 // 16, torch.int32), (n, torch.half), ((k, n), torch.half))]
+
+
+def entry(name, w, qc, out, stream):
     import ctypes
     import fp6_marlin
-    cabi = fp6_marlin.cabi
+    return getattr(fp6_marlin.cabi.lib, name)(w.data_ptr(), w.shape[0], w.shape[1], qc, -1, 0, *(ctypes.c_void_p(t.data_ptr()) for t in out),
+                                              0, ctypes.c_void_p(stream.cuda_stream))
+
+
+@pytest.mark.parametrize("harness", [True, False])
+@pytest.mark.parametrize("own", [False, True])
+def test_packed_weights_are_ready_for_every_stream_when_the_call_returns(own, harness):
+    """On the default stream as on one of the caller's own: torch's streams are not ordered against the default one, so a
+    `mul` on another stream and a copy that refills the source may follow without an event."""
+    import fp6_marlin
+    k, n, qc, gs = 4096, 8192, 256, 128
+    g = torch.Generator().manual_seed(37)
+    staged = (torch.randn((k, n), generator=g) * 0.02).half()
+    A = torch.randn((16, k), generator=g).half().to(dev())
+    big = torch.randn((4096, 4096), device=dev()).half()
+    want = fp6_marlin.pack_mixed_weight(staged.to(dev()), qc, gs, harness_layout=harness)
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    C = torch.empty((16, n), dtype=torch.half, device=dev())
+    fp6_marlin.mul(A, want[0], C, want[1], ws, qc, group_size=gs)
+    torch.cuda.synchronize()
+    other = torch.cuda.Stream()
+    for busy in (0, 30):                               # (alone, and with more work in front than a short poll outlasts)
+        w = staged.to(dev())
+        nan = torch.full_like(w, float("nan"))
+        C1 = torch.full_like(C, float("nan"))
+        torch.cuda.synchronize()
+        stream = torch.cuda.Stream() if own else torch.cuda.default_stream()
+        with torch.cuda.stream(stream):
+            for _ in range(busy):
+                big @ big
+            got = fp6_marlin.pack_mixed_weight(w, qc, gs, harness_layout=harness)
+            assert stream.query()
+        with torch.cuda.stream(other):
+            w.copy_(nan)
+            fp6_marlin.mul(A, got[0], C1, got[1], ws, qc, group_size=gs)
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, want)) and torch.equal(C, C1)
+
+
+@pytest.mark.parametrize("k,n,qc", [(64, 128, 64), (1024, 384, 192), (4160, 1088, 1088)])
+@pytest.mark.parametrize("own", [False, True])
+def test_the_entry_that_leaves_the_packing_to_the_stream(own, k, n, qc):
+    """fp6m_pack_mixed_device_async on either kind of stream, alone and with other work in front (longer than it polls): its
+    results in stream order, and for another stream after an event, with the source's memory used again in stream order in
+    between; a weight out of range is still an error by value, with nothing left on the stream."""
+    import fp6_marlin
     g = torch.Generator().manual_seed(31)
     w = (torch.randn((k, n), generator=g) * 0.02).half().to(dev())
-    out = [torch.empty(size, dtype=dtype, device=dev()) for size, dtype in
-           ((k * (n - qc) // 8 + k * qc * 3 // 16, torch.int32), ((n - qc) + qc, torch.half), ((k, n), torch.half))]
+    bad = w.clone()
+    bad[k - 1, n - 1] = float("inf")
+    want = entry_outputs(k, n, qc)
+    assert entry("fp6m_pack_mixed_device", w, qc, want, torch.cuda.default_stream()) == 0
+    big = torch.randn((4096, 4096), device=dev()).half()
     torch.cuda.synchronize()
-    assert cabi.lib.fp6m_pack_mixed_device(w.data_ptr(), k, n, qc, -1, 0, *(ctypes.c_void_p(t.data_ptr()) for t in out), 0, None) == 0
-    big = torch.randn((6144, 6144), device=dev()).half()
+    stream, other = torch.cuda.Stream() if own else torch.cuda.default_stream(), torch.cuda.Stream()
     for busy in (0, 30):
-        for _ in range(busy):
-            big @ big
-        got = fp6_marlin.pack_mixed_weight(w, qc, -1, harness_layout=False)
-        assert all(torch.equal(x, y) for x, y in zip(got, out))
-        bad = w.clone()
-        bad[k - 1, n - 1] = float("inf")
-        for _ in range(busy):
-            big @ big
-        with pytest.raises(ValueError):
-            fp6_marlin.pack_mixed_weight(bad, qc, -1, harness_layout=False)
-    side = torch.cuda.Stream()
-    side.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(side):                      # a stream of the caller's own: done when the call returns
-        for _ in range(30):
-            big @ big
-        fp6_marlin.pack_mixed_weight(w, qc, -1, harness_layout=False)
-        assert side.query()
-    results = []
-    for i in range(4):
-        mine = w.clone()
-        side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
-            results.append(fp6_marlin.pack_mixed_weight(mine, qc, -1, harness_layout=False))
-        del mine
-        torch.full((k, n), float("nan"), dtype=torch.half, device=dev())
-    torch.cuda.synchronize()
-    assert all(torch.equal(x, y) for got in results for x, y in zip(got, out))
+        out = entry_outputs(k, n, qc)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            mine = w.clone()
+            for _ in range(busy):
+                big @ big
+            assert entry("fp6m_pack_mixed_device_async", mine, qc, out, stream) == 0
+            del mine
+            torch.full((k, n), float("nan"), dtype=torch.half, device=dev())
+            copies = [t.clone() for t in out]
+            ready = stream.record_event()
+        with torch.cuda.stream(other):
+            other.wait_event(ready)
+            late = [t.clone() for t in out]
+        torch.cuda.synchronize()
+        for got in (out, copies, late):
+            assert all(torch.equal(x, y) for x, y in zip(got, want))
+        with torch.cuda.stream(stream):
+            for _ in range(busy):
+                big @ big
+            assert entry("fp6m_pack_mixed_device_async", bad, qc, out, stream) == fp6_marlin.cabi.ERR_RANGE
+            assert stream.query()
+
+
+def test_the_entry_that_leaves_the_packing_to_the_stream_returns_before_it_is_done():
+    """Half a millisecond of packing is still running when the call returns."""
+    k, n, qc = 8192, 28672, 256
+    w = torch.randn((k, n), dtype=torch.half, device=dev()).mul_(0.02)
+    out, want = entry_outputs(k, n, qc), entry_outputs(k, n, qc)
+    stream = torch.cuda.default_stream()
+    assert entry("fp6m_pack_mixed_device", w, qc, want, stream) == 0
+    assert stream.query()
+    early = 0
+    for _ in range(5):                                 # (a host thread that is descheduled in between would see it done)
+        assert entry("fp6m_pack_mixed_device_async", w, qc, out, stream) == 0
+        early += not stream.query()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(out, want))
+    assert early >= 1
 
 
 def test_fp6_columns_with_sub_normal_scales():
