@@ -218,13 +218,18 @@ __device__ __forceinline__ void exchange(uint4& a, uint4& b, bool odd)
     }
 }
 
+// What pack_kernel tells a host that polls (0: nothing yet).
+constexpr int kInRange = 1, kOutOfRange = 2;
 struct PackArgs {
     const uint16_t* w;
     int k, n, n4, qc, g, per_column;
     uint16_t *s4, *s6;
     uint32_t *words, *plane2, *plane4;
     uint16_t* w_ref;
-    int* range_known;                 // host memory, set when the kernel starts: the kernels before it are done (null: not asked for)
+    // Host memory, for a caller that does not wait (null: not asked for): when the kernel starts, and the kernels before it are
+    // done, it tells the host what they found about the range.
+    const int* bad;
+    int* verdict;
     int wgs6, blocks4;                // workgroups of the FP6 region (the first of the grid); INT4 workgroups per 128 rows
 };
 
@@ -482,7 +487,12 @@ __global__ __launch_bounds__(512, 4) void pack_kernel(const PackArgs p)
         Fp6Smem fp6;
     } sm;
     const int b = blockIdx.x;
-    if (b == 0 && threadIdx.x == 0 && p.range_known) __hip_atomic_store(p.range_known, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (b == 0 && threadIdx.x == 0 && p.verdict) {
+        // One word says both that the range is known and what it is: the host relies on no order between this store and the
+        // earlier kernel's store to `bad`, which has arrived when the load has returned its value.
+        const int bad = __hip_atomic_load(p.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(p.verdict, bad ? kOutOfRange : kInRange, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     if (b < p.wgs6) {
         const int across = p.qc / 64;
         fp6_pack(p, b % across, b / across, sm.fp6);
@@ -536,7 +546,7 @@ __global__ void fp6_pack_harness_kernel(const uint16_t* w, int k, int n, int n4,
 // succeeded: until then kernels of this call may still write it, and the next call's check would see that.
 constexpr int kFlags = 64;
 struct alignas(64) FlagLine {
-    int bad, known;
+    int bad, verdict;
 };
 std::mutex g_flag_mutex;
 FlagLine* g_flags = nullptr;
@@ -582,18 +592,18 @@ struct RangeFlag {
         idle = e == hipSuccess;
         return e;
     }
-    // Those that decide about the range: true once pack_kernel, which writes nothing here after that, has begun.  Not for
-    // long (the stream may have other work in front): false leaves it to wait().
-    bool known_soon() const
+    // Those that decide about the range: true once pack_kernel, which writes nothing here after that, has said that nothing is
+    // out of it.  Not for long (the stream may have other work in front): false leaves it to wait().
+    bool in_range_soon() const
     {
         for (int i = 0; i < 20000; i++) {
-            if (__atomic_load_n(&g_flags[index].known, __ATOMIC_ACQUIRE)) return true;
+            if (const int v = __atomic_load_n(&g_flags[index].verdict, __ATOMIC_ACQUIRE)) return v == kInRange;
             __builtin_ia32_pause();
         }
         return false;
     }
     int* bad() const { return index < 0 ? nullptr : &g_flags[index].bad; }
-    int* known() const { return index < 0 ? nullptr : &g_flags[index].known; }
+    int* verdict() const { return index < 0 ? nullptr : &g_flags[index].verdict; }
     bool out_of_range() const { return index >= 0 && __atomic_load_n(&g_flags[index].bad, __ATOMIC_RELAXED) != 0; }
 };
 
@@ -624,11 +634,14 @@ int pack_mixed(const void* w, int k, int n, int quant_cols, int group_size, int 
     uint16_t* s6 = sp + (per_column ? (size_t)n4 : (size_t)(k / g) * n4);
     uint32_t* plane2 = bp + (size_t)k * n4 / 8;
     uint32_t* plane4 = plane2 + (size_t)k * qc / 16;
-    PackArgs a = {wp, k, n, n4, qc, g, (int)per_column, sp, s6, bp, plane2, plane4, rp, nullptr, 0, n4 ? (n4 + 255) / 256 : 1};
+    PackArgs a = {wp, k, n, n4, qc, g, (int)per_column, sp, s6, bp, plane2, plane4, rp, nullptr, nullptr, 0, n4 ? (n4 + 255) / 256 : 1};
     if (qc > 0 && capturing(st)) return hip_fail(hipErrorStreamCaptureUnsupported);   // (the wait below: refused before anything is recorded)
     RangeFlag flag(qc > 0);
     if (flag.err != hipSuccess) return hip_fail(flag.err);
-    if (!whole && !harness_layout) a.range_known = flag.known();
+    if (!whole && !harness_layout) {
+        a.bad = flag.bad();
+        a.verdict = flag.verdict();
+    }
     // Scales that span all of k (all columns with per-column scales, else the FP6 region): maxima of at most kMaxChunks row
     // ranges first.  They wait, two bytes each, in B, which is packed afterwards and larger (at least k / 2 bytes a column).
     const int first = per_column ? 0 : n4, cols = n - first;
@@ -663,10 +676,9 @@ int pack_mixed(const void* w, int k, int n, int quant_cols, int group_size, int 
         // every call waiting for all of them the GPU is idle between one call's last kernel and the next one's first:
         // 4096 x 22016, group-128 scales, 256 FP6 columns, calls in a row 106.6 us each, 85.2 from the other entry (a call
         // that is waited for takes as long from either).
-        if (!(e == hipSuccess && a.range_known && flag.known_soon() && !flag.out_of_range())) {
-            const hipError_t waited = flag.wait(st);
-            if (e == hipSuccess) e = waited;
-        }
+        if (e == hipSuccess && a.verdict && flag.in_range_soon()) return FP6M_OK;
+        const hipError_t waited = flag.wait(st);
+        if (e == hipSuccess) e = waited;
     }
     if (e != hipSuccess) return hip_fail(e);
     return flag.out_of_range() ? FP6M_ERR_RANGE : FP6M_OK;

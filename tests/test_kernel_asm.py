@@ -20,15 +20,19 @@ SRC = os.path.join(ROOT, "fp6-marlin_amd", "csrc", "fp6m_gemm.hip")
 HIPCC = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
 
 
-@pytest.fixture(scope="module")
-def asm(tmp_path_factory):
+def assembly(tmp_path_factory, src):
     if not os.path.exists(HIPCC):
         pytest.skip("hipcc not available")
-    out = tmp_path_factory.mktemp("asm") / "fp6m_gemm.s"
+    out = tmp_path_factory.mktemp("asm") / "out.s"
     subprocess.check_call([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
                            "-packed-fp32-ops", f"-I{ROOT}/include", f"-I{ROOT}/fp6-marlin_amd/csrc", "-S",
-                           "--cuda-device-only", "-o", str(out), SRC], stderr=subprocess.DEVNULL)
+                           "--cuda-device-only", "-o", str(out), src], stderr=subprocess.DEVNULL)
     return out.read_text()
+
+
+@pytest.fixture(scope="module")
+def asm(tmp_path_factory):
+    return assembly(tmp_path_factory, SRC)
 
 
 def kernels(asm):
@@ -132,3 +136,24 @@ def test_kernel_arguments_are_loaded_in_one_batch(asm):
         late = [(n, l) for n, l in late if not re.search(r"0x(c8|d0|d8)$", l)]
         assert not late, f"{name}: kernel-argument loads after the prologue: {late[:4]}"
     assert seen == 82            # (the m <= 16 kernel's builds with the partial tiles exchanged inside one XCD are 8 of them)
+
+
+def test_the_packer_tells_the_host_one_word_and_releases_it(tmp_path_factory):
+    """A host that does not wait for the stream learns from pack_kernel that the range of the FP6 cast is known and what it is.
+    That has to be one store: a system-scope load of the earlier kernel's flag, a wait for it, then the verdict, released
+    (write-back and wait in front of it)."""
+    seen = 0
+    for name, ins in kernels(assembly(tmp_path_factory, SRC.replace("fp6m_gemm", "fp6m_pack"))):
+        if "pack_kernelILb" not in name:
+            continue
+        seen += 1
+        system = [n for n, l in enumerate(ins) if "sc0 sc1" in l and l.startswith(("global_", "flat_"))]
+        assert len(system) == 2, f"{name}: {[ins[n] for n in system]}"
+        load, store = system
+        assert "_load_dword " in ins[load] and "_store_dword " in ins[store], f"{name}: {ins[load]}; {ins[store]}"
+        between = ins[load + 1:store]
+        assert any(l.startswith("buffer_wbl2 sc0 sc1") for l in between), f"{name}: {between}"
+        assert re.search(r"vmcnt\(0\)", "\n".join(between)), f"{name}: {between}"
+        flag = ins[load].split()[1].rstrip(",")
+        assert any(re.search(rf"\b{flag}\b", l) for l in between), f"{name}: the verdict does not follow from the flag: {between}"
+    assert seen == 2
