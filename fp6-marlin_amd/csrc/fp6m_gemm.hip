@@ -485,13 +485,6 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
     }
 }
 
-// How a launch of gemm_mb_kernel cuts the k range: parts per INT4 and FP6 tile, k slices (waves) per workgroup.
-struct MbSplit {
-    long long ks, ks6;
-    int wk;
-    bool too_large;           // more partial tiles than a scratch of fixed size holds
-};
-
 // The time of one launch of gemm_mb_kernel, us, for the choice among its tiles of 32, 48 and 64 rows.
 //
 // None of them wins everywhere: a taller tile dequantises less often and reads fewer words, a shorter one fills its rows and
@@ -875,79 +868,8 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
     const long long env_ks = tune.ksplit != kUnset ? tune.ksplit : 0;
     // The split of one launch of gemm_mb_kernel (16 rows and more) with tiles of 16 * mb rows.
     auto split_mb = [&](int mb, int mtiles) {
-        const int rows_per_tile = 16 * mb;
-        // m > 16: a task is one workgroup (one tile x four k slices) on one row tile and k part.
-        // Split k only as far as needed to give every CU a workgroup; partial tiles are 16*MB rows
-        // of fp32, so the split is also capped by their traffic relative to the weight stream.
-        const long long base = (long long)a.tiles * mtiles;
-        const size_t tile_bytes = (size_t)rows_per_tile * kTileN * sizeof(float);
-        MbSplit sp;
-        sp.too_large = false;
-        long long ks = cus / base;
-        // (two k units per wave at least, one on a short k up to four parts; a grid that leaves half of the CUs idle even
-        // so may split twice as far as the partial tiles' traffic would otherwise allow: 2048 x 2560 .. 7680 at 32 and
-        // 64 rows 10.4 -> 9.2-9.8 us and 13.8 -> 12.7-13.0; eight parts instead of four on k = 4096 cost 6-12 %)
-        long long ks_k = units / (kWaves * 2);
-        if (ks_k < 4) ks_k = units / kWaves < 4 ? units / kWaves : 4;
-        if (ks_k < 1) ks_k = 1;
-        long long cap = (long long)prob_k / (16LL * rows_per_tile) > 0 ? (long long)prob_k / (16LL * rows_per_tile) : 1;
-        if (base * 2 * cap <= cus) cap *= 2;
-        if (ks > ks_k) ks = ks_k;
-        if (ks > cap) ks = cap;
-        if (sms > 0 && ks > sms) ks = sms;
-        if (env_ks >= 1) ks = env_ks;
-        if (ks < 1) ks = 1;
-        sp.too_large = fixed_scratch && ks > 1 && (size_t)(a.tiles + a.tiles6) * mtiles * ks * tile_bytes > scratch_bytes;
-        while (ks > 1 && (size_t)(a.tiles + a.tiles6) * mtiles * ks * tile_bytes > scratch_bytes) ks--;   // (FP6 tiles: 2 ks)
-        // A grid of at most one workgroup per CU would leave every SIMD a single wave: give the workgroup eight
-        // k slices instead of four (same partial-sum traffic, two waves per SIMD) when k is long enough.
-        // (Two waves on a SIMD take turns at its one VALU/MFMA port: eight half-length slices last as long as four
-        // whole ones, so eight (which hide latency better: 13824 x 5120 at 256 rows 60.6 vs 67.8 us) only pay while
-        // their longest slice, in whole k units, is no more than 0.58 of the longest of four: 5120 x 13824 at 64
-        // rows, 40 units over 16 slices of up to 3: 24.1 us, over 8 slices of 5: 21.7.)
-        // From forced tables (4 or 8 slices x 1 .. 8 parts, 32 / 64 / 128 rows): a split is no finer than its longest
-        // slice needs (8192 x 6144 at 32 rows: 64 units in 5 parts = 20 slices of up to 4, 16.7 us; in 4 parts = 16
-        // slices of 4, 16.0; as eight-wave workgroups 14.3); one unit per wave is enough for eight (8192 x 2048 at
-        // 32 rows 12.8 -> 12.0); 0.58 rather than 0.55 (14336 x 8192 at 32 rows, 4 against 7 units, 23.0 -> 20.5);
-        // and beyond eight parts the partners' partial tiles cost more than shorter slices gain (14336 x 2048 at
-        // 32 rows: 14 parts of four slices 16.7 us, 8 parts of eight 14.8; at 64 rows 24.0 -> 21.0).
-        auto longest = [&](long long slices) { return (units + slices - 1) / slices; };
-        const bool free_split = env_ks < 1 && sms <= 0 && !row_mix && mb != 8;
-        if (free_split)
-            while (ks > 1 && longest(4 * (ks - 1)) == longest(4 * ks)) ks--;
-        // (32-row tiles are not issue-bound: two waves per SIMD pay up to two thirds, 11008 x 2560 at 32 rows 14.9 -> 13.2)
-        const bool eight_pays = mb == 2 ? 3 * longest(8 * ks) <= 2 * longest(4 * ks) : 50 * longest(8 * ks) <= 29 * longest(4 * ks);
-        int wk = base * ks <= cus && units / 8 >= ks && eight_pays ? 8 : kWaves;
-        if (free_split && tune.wk == kUnset && ks > 8 && base * 8 <= cus && units / 8 >= 8) {
-            wk = 8;
-            ks = 8;
-        }
-        if (tune.wk != kUnset) wk = tune.wk == 8 ? 8 : kWaves;
-        if (mb == 8) wk = kWaves;                                  // (512 registers per wave: one wave per SIMD)
-        // An FP6 step costs more issue slots than an INT4 one, and in a grid that is resident all at once the few
-        // FP6 tiles' workgroups set the length of the launch (8192 x 8192 at m = 128: 33 us against 29 us with INT4
-        // only).  Their k range is cut twice as finely where every slice still gets two units and the grid still
-        // fits the CUs in one go (5120 x 13824 at m = 128: 40 -> 31 us; a grid whose last workgroups must wait for
-        // a free CU loses far more than that).  A forced split applies to both kinds.
-        sp.ks = sp.ks6 = ks;
-        sp.wk = wk;
-        // (a grid that fits one workgroup per CU must still do so afterwards: a CU with two runs both at little
-        // more than half speed, 11008 x 4096 at 256 rows 34 -> 52 us with 272 workgroups)
-        const long long resident = (long long)cus * (wk == 8 || mb == 8 || base * ks <= cus ? 1 : 2);
-        // (Not for 128-row tiles, whose FP6 workgroups are only a few per cent behind: there the second partner's
-        // partial tiles cost more than the shorter loop gains, 8192 x 8192 at m = 384 61.8 vs 58.4 us.)
-        // Re-measured with every tile on the paired loop (ten shapes x 32 .. 256 rows, alternating): still 5-13 % on
-        // wide weights up to two row tiles (4096 x 11008 at 128 rows 25.3 -> 22.2 us, 8192 x 28672 at 32 rows
-        // 38.2 -> 34.5), but 3-8 % slower from three row tiles on (5120 x 5120 at 256 rows 27.4 -> 29.7): up to two.
-        // Where twice does not fit, as finely as does (13824 x 5120 with 512 FP6 columns, per-column scales, 64 rows: 6 parts for
-        // all tiles 22.1 us, 10 for the FP6 tiles 21.4).
-        if (env_ks < 1 && !row_mix && a.tiles6 > 0 && mb != 8 && mtiles <= 2) {
-            long long c6 = units / (2 * wk) < 2 * ks ? units / (2 * wk) : 2 * ks;
-            const long long room = (resident - (base - (long long)a.tiles6 * mtiles) * ks) / ((long long)a.tiles6 * mtiles);
-            if (c6 > room) c6 = room;
-            if (c6 > ks) sp.ks6 = c6;
-        }
-        return sp;
+        return mb_split(mb, MbLaunch{a.tiles, a.tiles6, mtiles, prob_k, units, cus, sms, env_ks, tune.wk == kUnset ? 0 : tune.wk == 8 ? 8 : kWaves,
+                                     row_mix, fixed_scratch, scratch_bytes});
     };
     // Many rows (gemm_wide.h): one launch over all of them, without a k split across workgroups.
     const bool free_plan = tune.mb == kUnset && tune.ksplit == kUnset && tune.wk == kUnset && tune.pair == kUnset && tune.cls == kUnset && sms <= 0;
@@ -1514,6 +1436,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             a.ks4 = (int)ks;
             a.ks6 = (int)ks6_of(ks, cfg.wk);
             if (sms > 0 && a.ks6 > sms) a.ks6 = sms;
+            while (a.ks6 > ks && slots_used(ks, a.ks6, a.groups4, a.groups6, 1) * slot_bytes > scratch_bytes) a.ks6--;   // (ks == 1: not looked at above)
             if (cls_na > 0) {
                 const long long c6 = a.groups6 ? ks6_of(1, 4) : 0, nb = a.groups4 - cls_na;
                 const size_t slots = (size_t)(a.groups6 * c6 + cls_na + nb * cls_cb);
@@ -1629,7 +1552,8 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                     // was within -4 .. +8 % when forced.
                     const double gain = prob_k / 128.0 * (0.76 - 1.0 / (double)cb);
                     const double bar = mb >= 3 ? 16.0 : 7.5 + 0.37 * (32 - a.m);
-                    if ((cb >= 2 && gain >= bar) || (tune.cls == 1 && cb >= 1)) {
+                    const bool fits = (size_t)(a.tiles6 * c6 + na + nb * cb) * tile_bytes <= scratch_bytes;
+                    if (fits && ((cb >= 2 && gain >= bar) || (tune.cls == 1 && cb >= 1))) {
                         wk = wk_c;
                         a.ks4 = 1;
                         a.ks6 = (int)c6;

@@ -7,6 +7,7 @@
 
 #include "fp6m.h"
 #include "fp6m_layout.h"
+#include "mb_plan.h"
 
 namespace fp6m {
 
@@ -16,8 +17,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
-constexpr int kWaves = 4;
-constexpr int kTileN = 128;          // columns per tile
 constexpr int kRedStride = kTileN + 4;                       // floats per row of the reduction slab
 constexpr size_t kScratchBytes = size_t(16) << 20;           // partial-sum scratch of one workspace
 

@@ -1,0 +1,113 @@
+// How a launch of more than 16 rows is cut: plain host arithmetic of the dispatcher (fp6m_gemm.hip).
+#pragma once
+#include <cstddef>
+
+namespace fp6m {
+
+constexpr int kWaves = 4;
+constexpr int kTileN = 128;          // columns per tile
+
+// Partial tiles that a launch may write to: the highest slot in use, plus one.  Slots are numbered row tile by row tile, FP6 tiles
+// first, over all (tile, part), those of tiles in one part included, which are stored directly.
+inline size_t slots_used(long long parts4, long long parts6, long long tiles4, long long tiles6, long long mtiles)
+{
+    const long long slots4 = tiles4 * parts4, slots6 = tiles6 * parts6;
+    const long long last = parts4 > 1 && tiles4 ? slots6 + slots4 : (parts6 > 1 ? slots6 : 0);
+    return last ? (size_t)((mtiles - 1) * (slots6 + slots4) + last) : 0;
+}
+
+// How a launch of gemm_mb_kernel cuts the k range: parts per INT4 and FP6 tile, k slices (waves) per workgroup.
+struct MbSplit {
+    long long ks, ks6;
+    int wk;
+    bool too_large;           // more partial tiles than a scratch of fixed size holds
+};
+struct MbLaunch {
+    long long tiles, tiles6;  // column tiles, and FP6 ones among them
+    int mtiles, k, units;     // row tiles; rows of the weight, and in units that slices are made of (128 rows with group scales, else 64)
+    int cus, sms;             // compute units; the caller's limit on parts per tile (<= 0: none)
+    long long forced_parts;   // tuning hook: parts per tile (< 1: not forced), waves per workgroup (0: not forced)
+    int forced_waves;
+    bool row_mix, fixed_scratch;
+    size_t scratch_bytes;
+};
+
+// The split of one launch of gemm_mb_kernel with tiles of 16 * mb rows (16 rows and more).
+inline MbSplit mb_split(int mb, const MbLaunch& l)
+{
+    // m > 16: a task is one workgroup (one tile x four k slices) on one row tile and k part.
+    // Split k only as far as needed to give every CU a workgroup; partial tiles are 16*MB rows
+    // of fp32, so the split is also capped by their traffic relative to the weight stream.
+    const int rows_per_tile = 16 * mb, units = l.units;
+    const long long base = l.tiles * l.mtiles;
+    const size_t tile_bytes = (size_t)rows_per_tile * kTileN * sizeof(float);
+    MbSplit sp;
+    long long ks = l.cus / base;
+    // (two k units per wave at least, one on a short k up to four parts; a grid that leaves half of the CUs idle even
+    // so may split twice as far as the partial tiles' traffic would otherwise allow: 2048 x 2560 .. 7680 at 32 and
+    // 64 rows 10.4 -> 9.2-9.8 us and 13.8 -> 12.7-13.0; eight parts instead of four on k = 4096 cost 6-12 %)
+    long long ks_k = units / (kWaves * 2);
+    if (ks_k < 4) ks_k = units / kWaves < 4 ? units / kWaves : 4;
+    if (ks_k < 1) ks_k = 1;
+    long long cap = (long long)l.k / (16LL * rows_per_tile) > 0 ? (long long)l.k / (16LL * rows_per_tile) : 1;
+    if (base * 2 * cap <= l.cus) cap *= 2;
+    if (ks > ks_k) ks = ks_k;
+    if (ks > cap) ks = cap;
+    if (l.sms > 0 && ks > l.sms) ks = l.sms;
+    if (l.forced_parts >= 1) ks = l.forced_parts;
+    if (ks < 1) ks = 1;
+    sp.too_large = l.fixed_scratch && ks > 1 && (size_t)(l.tiles + l.tiles6) * l.mtiles * ks * tile_bytes > l.scratch_bytes;
+    while (ks > 1 && (size_t)(l.tiles + l.tiles6) * l.mtiles * ks * tile_bytes > l.scratch_bytes) ks--;   // (FP6 tiles: 2 ks)
+    // A grid of at most one workgroup per CU would leave every SIMD a single wave: give the workgroup eight
+    // k slices instead of four (same partial-sum traffic, two waves per SIMD) when k is long enough.
+    // (Two waves on a SIMD take turns at its one VALU/MFMA port: eight half-length slices last as long as four
+    // whole ones, so eight (which hide latency better: 13824 x 5120 at 256 rows 60.6 vs 67.8 us) only pay while
+    // their longest slice, in whole k units, is no more than 0.58 of the longest of four: 5120 x 13824 at 64
+    // rows, 40 units over 16 slices of up to 3: 24.1 us, over 8 slices of 5: 21.7.)
+    // From forced tables (4 or 8 slices x 1 .. 8 parts, 32 / 64 / 128 rows): a split is no finer than its longest
+    // slice needs (8192 x 6144 at 32 rows: 64 units in 5 parts = 20 slices of up to 4, 16.7 us; in 4 parts = 16
+    // slices of 4, 16.0; as eight-wave workgroups 14.3); one unit per wave is enough for eight (8192 x 2048 at
+    // 32 rows 12.8 -> 12.0); 0.58 rather than 0.55 (14336 x 8192 at 32 rows, 4 against 7 units, 23.0 -> 20.5);
+    // and beyond eight parts the partners' partial tiles cost more than shorter slices gain (14336 x 2048 at
+    // 32 rows: 14 parts of four slices 16.7 us, 8 parts of eight 14.8; at 64 rows 24.0 -> 21.0).
+    auto longest = [&](long long slices) { return (units + slices - 1) / slices; };
+    const bool free_split = l.forced_parts < 1 && l.sms <= 0 && !l.row_mix && mb != 8;
+    if (free_split)
+        while (ks > 1 && longest(4 * (ks - 1)) == longest(4 * ks)) ks--;
+    // (32-row tiles are not issue-bound: two waves per SIMD pay up to two thirds, 11008 x 2560 at 32 rows 14.9 -> 13.2)
+    const bool eight_pays = mb == 2 ? 3 * longest(8 * ks) <= 2 * longest(4 * ks) : 50 * longest(8 * ks) <= 29 * longest(4 * ks);
+    int wk = base * ks <= l.cus && units / 8 >= ks && eight_pays ? 8 : kWaves;
+    if (free_split && !l.forced_waves && ks > 8 && base * 8 <= l.cus && units / 8 >= 8) {
+        wk = 8;
+        ks = 8;
+    }
+    if (l.forced_waves) wk = l.forced_waves;
+    if (mb == 8) wk = kWaves;                                  // (512 registers per wave: one wave per SIMD)
+    // An FP6 step costs more issue slots than an INT4 one, and in a grid that is resident all at once the few
+    // FP6 tiles' workgroups set the length of the launch (8192 x 8192 at m = 128: 33 us against 29 us with INT4
+    // only).  Their k range is cut twice as finely where every slice still gets two units and the grid still
+    // fits the CUs in one go (5120 x 13824 at m = 128: 40 -> 31 us; a grid whose last workgroups must wait for
+    // a free CU loses far more than that).  A forced split applies to both kinds.
+    sp.ks = sp.ks6 = ks;
+    sp.wk = wk;
+    // (a grid that fits one workgroup per CU must still do so afterwards: a CU with two runs both at little
+    // more than half speed, 11008 x 4096 at 256 rows 34 -> 52 us with 272 workgroups)
+    const long long resident = (long long)l.cus * (wk == 8 || mb == 8 || base * ks <= l.cus ? 1 : 2);
+    // (Not for 128-row tiles, whose FP6 workgroups are only a few per cent behind: there the second partner's
+    // partial tiles cost more than the shorter loop gains, 8192 x 8192 at m = 384 61.8 vs 58.4 us.)
+    // Re-measured with every tile on the paired loop (ten shapes x 32 .. 256 rows, alternating): still 5-13 % on
+    // wide weights up to two row tiles (4096 x 11008 at 128 rows 25.3 -> 22.2 us, 8192 x 28672 at 32 rows
+    // 38.2 -> 34.5), but 3-8 % slower from three row tiles on (5120 x 5120 at 256 rows 27.4 -> 29.7): up to two.
+    // Where twice does not fit, as finely as does (13824 x 5120 with 512 FP6 columns, per-column scales, 64 rows: 6 parts for
+    // all tiles 22.1 us, 10 for the FP6 tiles 21.4).
+    if (l.forced_parts < 1 && !l.row_mix && l.tiles6 > 0 && mb != 8 && l.mtiles <= 2) {
+        long long c6 = units / (2 * wk) < 2 * ks ? units / (2 * wk) : 2 * ks;
+        const long long room = (resident - (base - l.tiles6 * l.mtiles) * ks) / (l.tiles6 * l.mtiles);
+        if (c6 > room) c6 = room;
+        while (c6 > ks && slots_used(ks, c6, l.tiles - l.tiles6, l.tiles6, l.mtiles) * tile_bytes > l.scratch_bytes) c6--;
+        if (c6 > ks) sp.ks6 = c6;
+    }
+    return sp;
+}
+
+}  // namespace fp6m

@@ -86,9 +86,9 @@ int fp6m_mul(const void* A, const void* B, void* C, const void* s, int prob_m, i
  *     array's address out of the first call;
  *   - a launch of more than 16 rows whose k split needs more than the 12 MiB the array has for partial tiles returns
  *     FP6M_ERR_SCRATCH (fp6m_mul would shrink the split instead).  The need is (workgroups that share column tiles) x
- *     (32, 64 or 128 rows) x 128 columns x 4 bytes; the dispatcher sizes its own splits to the 12 MiB (it keeps 64-row
- *     tiles where a split of 128-row tiles would not fit), so this only triggers for splits forced with
- *     fp6m_tuning_set or on devices with more compute units.  Launches of up to 4 rows never fail this way (without
+ *     (32, 48, 64 or 128 rows) x 128 columns x 4 bytes; the dispatcher sizes its own splits to the 12 MiB (it keeps 64-row
+ *     tiles where a split of 128-row tiles would not fit, and cuts the FP6 tiles no finer than fits), so this only triggers
+ *     for splits forced with fp6m_tuning_set, on weights that are mostly FP6, or on devices with more compute units.  Launches of up to 4 rows never fail this way (without
  *     room for their cells, n * m * 8 bytes > 8 MiB, no tile is shared); those of 5 to 16 rows only with a forced split;
  *   - every call on a GPU shares that GPU's array: calls that overlap on one GPU race, whatever their workspaces
  *     and streams.  `workspace` keeps its role (tile counters, zero on entry and on exit).

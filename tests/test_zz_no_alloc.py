@@ -77,3 +77,36 @@ def test_static_scratch_entry_refuses_what_does_not_fit():
     assert call(L.fp6m_mul_static, A, B, C, s, ws, m, n, k, qc, gs) == cabi.OK    # the dispatcher's own split fits
     torch.cuda.synchronize()
     assert int(ws.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("m,k,n,qc", [(64, 1024, 38400, 25600), (16, 512, 131200, 131072)])
+def test_static_scratch_holds_the_fp6_tiles_own_split(m, k, n, qc):
+    """Few parts of very many FP6 tiles: in two parts each they would not fit the array, and the cells behind it, which the decode
+    kernel counts in, would be overwritten.  The result, and a decode call through those cells afterwards, are right."""
+    import fp6_marlin
+    from fp6_marlin import cabi
+    L = cabi.lib
+    assert L.fp6m_init(0) == cabi.OK
+    n4 = n - qc
+    g = torch.Generator().manual_seed(70 + m)
+    B = torch.randint(-2 ** 31, 2 ** 31 - 1, (k * n4 // 8 + k * qc * 3 // 16,), generator=g, dtype=torch.int64).to(torch.int32)
+    s = (torch.rand(n, generator=g) * 0.01 + 0.001).half()
+    A = torch.randn((m, k), generator=g).half()
+    ref = A.float() @ fp6_marlin.unpack_to_fp16(B, s, k, n, qc, -1).float()
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device="cuda")
+    C = torch.full((m, n), float("nan"), dtype=torch.half, device="cuda")
+    Ad, Bd, sd = A.cuda(), B.cuda(), s.cuda()
+    assert call(L.fp6m_mul_static, Ad, Bd, C, sd, ws, m, n, k, qc, -1) == cabi.OK
+    torch.cuda.synchronize()
+    got = C.float().cpu()
+    for part in (slice(0, n4), slice(n4, n)):
+        assert float((got - ref)[:, part].abs().mean() / ref[:, part].abs().mean()) <= 1e-3
+    assert int(ws.abs().sum()) == 0
+    for rows in (1, 4):
+        A, B, s = operands(rows, 8192, 4096, 256, 128, 71)
+        want, late = (torch.full((rows, 4096), float("nan"), dtype=torch.half, device="cuda") for _ in range(2))
+        assert call(L.fp6m_mul, A, B, want, s, ws, rows, 4096, 8192, 256, 128) == cabi.OK
+        assert call(L.fp6m_mul_static, A, B, late, s, ws, rows, 4096, 8192, 256, 128) == cabi.OK
+        torch.cuda.synchronize()
+        assert torch.equal(want, late)
+    cabi.release_workspace(ws)
