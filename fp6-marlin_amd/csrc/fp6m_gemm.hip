@@ -329,29 +329,6 @@ inline SliceRule make_rule(int units, int nslices)
     return r;
 }
 
-// k slices of the `ks` parts x `wk` waves of a tile (WaveRule, gemm_common.h).  With eight waves per workgroup and at
-// least two units for every wave, the second wave of every SIMD (waves 4-7) gets `young_pct` per cent of what the
-// first gets; otherwise all waves get the same.  What does not divide goes to the older waves first.
-inline WaveRule make_wave_rule(long long units, long long ks, int wk, int young_pct)
-{
-    WaveRule r;
-    if (ks < 1) ks = 1;
-    const long long per_part = units / ks;
-    long long lo = per_part / wk, ly = lo;
-    if (wk == 8 && per_part >= 16 && young_pct > 0 && young_pct < 100) {
-        lo = (per_part * 100 + 2 * (100 + young_pct)) / (4 * (100 + young_pct));     // per_part / (4 (1 + share)), rounded
-        if (4 * lo > per_part) lo = per_part / 4;
-        ly = (per_part - 4 * lo) / 4;
-        if (ly > lo) ly = lo;
-    }
-    const long long rem = units - ks * (4 * lo + (wk - 4) * ly);
-    r.lo = (int)lo;
-    r.ly = (int)ly;
-    r.eo = (int)(rem < 4 * ks ? rem : 4 * ks);
-    r.ey = (int)(rem - r.eo);
-    return r;
-}
-
 inline FastDiv make_div(long long d, long long max_n)
 {
     FastDiv f;
@@ -869,7 +846,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
     // The split of one launch of gemm_mb_kernel (16 rows and more) with tiles of 16 * mb rows.
     auto split_mb = [&](int mb, int mtiles) {
         return mb_split(mb, MbLaunch{a.tiles, a.tiles6, mtiles, prob_k, units, cus, sms, env_ks, tune.wk == kUnset ? 0 : tune.wk == 8 ? 8 : kWaves,
-                                     row_mix, fixed_scratch, scratch_bytes});
+                                     row_mix, fixed_scratch, scratch_bytes, young_pct});
     };
     // Many rows (gemm_wide.h): one launch over all of them, without a k split across workgroups.
     const bool free_plan = tune.mb == kUnset && tune.ksplit == kUnset && tune.wk == kUnset && tune.pair == kUnset && tune.cls == kUnset && sms <= 0;

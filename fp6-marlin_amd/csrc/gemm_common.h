@@ -32,16 +32,7 @@ __host__ __device__ inline int slice_begin(const SliceRule& r, int i)
     return i * r.q + (extra > 0 ? extra : 0);
 }
 
-// The k slices of a tile by wave, in units.  A workgroup of eight waves puts two on every SIMD, and the SIMD serves
-// the one that arrived first (waves 0-3) ahead of the other (waves 4-7): with equal slices the second wave of every
-// SIMD leaves its loop a third later than the first (8192 x 8192 at 128 rows: 14.3 against 19.6 us), and the
-// workgroup's reduction waits for it.  So a part (workgroup) of a tile gives its first four waves `lo` units each and
-// the others `ly` <= lo; what does not divide goes, a unit each, to the first `eo` older waves in (part, wave) order,
-// then to the first `ey` younger ones.  Four-wave workgroups have older waves only.  Slices follow each other along
-// k in (part, wave) order.
-struct WaveRule {
-    int lo, ly, eo, ey;
-};
+// Where the slice of `wave` of part `part` begins (WaveRule).
 __host__ __device__ inline int wave_rule_begin(const WaveRule& r, int wk, int part, int wave)
 {
     const int no = 4, ny = wk - 4;

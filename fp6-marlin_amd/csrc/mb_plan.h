@@ -16,6 +16,42 @@ inline size_t slots_used(long long parts4, long long parts6, long long tiles4, l
     return last ? (size_t)((mtiles - 1) * (slots6 + slots4) + last) : 0;
 }
 
+// The k slices of a tile by wave, in units.  A workgroup of eight waves puts two on every SIMD, and the SIMD serves
+// the one that arrived first (waves 0-3) ahead of the other (waves 4-7): with equal slices the second wave of every
+// SIMD leaves its loop a third later than the first (8192 x 8192 at 128 rows: 14.3 against 19.6 us), and the
+// workgroup's reduction waits for it.  So a part (workgroup) of a tile gives its first four waves `lo` units each and
+// the others `ly` <= lo; what does not divide goes, a unit each, to the first `eo` older waves in (part, wave) order,
+// then to the first `ey` younger ones.  Four-wave workgroups have older waves only.  Slices follow each other along
+// k in (part, wave) order.
+struct WaveRule {
+    int lo, ly, eo, ey;
+};
+// k slices of the `ks` parts x `wk` waves of a tile.  With eight waves per workgroup and at least two units for every
+// wave, the second wave of every SIMD (waves 4-7) gets `young_pct` per cent of what the first gets; otherwise all waves
+// get the same.  What does not divide goes to the older waves first.
+inline WaveRule make_wave_rule(long long units, long long ks, int wk, int young_pct)
+{
+    WaveRule r;
+    if (ks < 1) ks = 1;
+    const long long per_part = units / ks;
+    long long lo = per_part / wk, ly = lo;
+    if (wk == 8 && per_part >= 16 && young_pct > 0 && young_pct < 100) {
+        lo = (per_part * 100 + 2 * (100 + young_pct)) / (4 * (100 + young_pct));     // per_part / (4 (1 + share)), rounded
+        if (4 * lo > per_part) lo = per_part / 4;
+        ly = (per_part - 4 * lo) / 4;
+        if (ly > lo) ly = lo;
+    }
+    const long long rem = units - ks * (4 * lo + (wk - 4) * ly);
+    r.lo = (int)lo;
+    r.ly = (int)ly;
+    r.eo = (int)(rem < 4 * ks ? rem : 4 * ks);
+    r.ey = (int)(rem - r.eo);
+    return r;
+}
+// Units of the longest slice among the older and among the younger waves.
+inline int longest_older(const WaveRule& r) { return r.lo + (r.eo > 0); }
+inline int longest_younger(const WaveRule& r, int wk) { return wk > 4 ? r.ly + (r.ey > 0) : 0; }
+
 // How a launch of gemm_mb_kernel cuts the k range: parts per INT4 and FP6 tile, k slices (waves) per workgroup.
 struct MbSplit {
     long long ks, ks6;
@@ -30,6 +66,7 @@ struct MbLaunch {
     int forced_waves;
     bool row_mix, fixed_scratch;
     size_t scratch_bytes;
+    int young_pct = 72;       // make_wave_rule
 };
 
 // The split of one launch of gemm_mb_kernel with tiles of 16 * mb rows (16 rows and more).
@@ -99,12 +136,30 @@ inline MbSplit mb_split(int mb, const MbLaunch& l)
     // wide weights up to two row tiles (4096 x 11008 at 128 rows 25.3 -> 22.2 us, 8192 x 28672 at 32 rows
     // 38.2 -> 34.5), but 3-8 % slower from three row tiles on (5120 x 5120 at 256 rows 27.4 -> 29.7): up to two.
     // Where twice does not fit, as finely as does (13824 x 5120 with 512 FP6 columns, per-column scales, 64 rows: 6 parts for
-    // all tiles 22.1 us, 10 for the FP6 tiles 21.4).
+    // all tiles 22.1 us, 10 for the FP6 tiles 21.4).  In four-wave workgroups and beyond eight parts only if that shortens the
+    // loop by 128 rows of k at least, for a wave served first or for a SIMD: with less, the additional partial tiles cost more
+    // than the loop gains (3840 x 2048 at 86 rows 15.4 -> 17.4 us).
+    // Two row tiles whose workgroups are a multiple of eight apart must stay so: the same part of both is then on one XCD,
+    // whose L2 reads the words once (16384 x 2560 at 110 rows: 120 workgroups per row tile 23.6 us, 122 25.5).  A cut that
+    // makes it a multiple is taken.
+    // Random shapes from k = 2048 against no finer cut: what is cut takes 4.9 % less on 84 of 17 to 32 rows and on 35 of 49 to
+    // 128 (the worst 8 % more); what is not would take 3.9 % more on 6 and 5.8 % on 21 for want of 128 rows, and 6.2 % on the 14
+    // whose row tiles would come apart.
     if (l.forced_parts < 1 && !l.row_mix && l.tiles6 > 0 && mb != 8 && l.mtiles <= 2) {
         long long c6 = units / (2 * wk) < 2 * ks ? units / (2 * wk) : 2 * ks;
         const long long room = (resident - (base - l.tiles6 * l.mtiles) * ks) / (l.tiles6 * l.mtiles);
         if (c6 > room) c6 = room;
         while (c6 > ks && slots_used(ks, c6, l.tiles - l.tiles6, l.tiles6, l.mtiles) * tile_bytes > l.scratch_bytes) c6--;
+        auto shared_l2 = [&](long long parts6) { return l.mtiles == 1 || ((l.tiles - l.tiles6) * ks + l.tiles6 * parts6) % 8 == 0; };
+        auto pays = [&](long long parts6) {
+            if (parts6 == 2 * ks) return true;
+            if (shared_l2(ks) != shared_l2(parts6)) return shared_l2(parts6);
+            if (wk == 8 && parts6 <= 8) return true;
+            const WaveRule now = make_wave_rule(units, ks, wk, l.young_pct), cut = make_wave_rule(units, parts6, wk, l.young_pct);
+            const int older = longest_older(now) - longest_older(cut), both = older + longest_younger(now, wk) - longest_younger(cut, wk);
+            return (older > both ? older : both) * (long long)(l.k / units) >= 128;
+        };
+        while (c6 > ks && !pays(c6)) c6--;
         if (c6 > ks) sp.ks6 = c6;
     }
     return sp;

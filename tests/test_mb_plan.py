@@ -100,3 +100,46 @@ def test_no_split_leaves_its_scratch(plan):
         shared += top >= 0
         assert (top + 1) * 16 * mb * 128 * 4 <= scratch, (mb, tiles, tiles6, mtiles, k, group, fixed, ks, ks6)
     assert shared > 10000
+
+
+def longest(units, parts, wk):
+    """Units of the longest slice of a wave that is served first, and of the two waves of a SIMD (make_wave_rule)."""
+    per_part = units // parts
+    lo = ly = per_part // wk
+    if wk == 8 and per_part >= 16:
+        lo = min((per_part * 100 + 344) // 688, per_part // 4)
+        ly = min((per_part - 4 * lo) // 4, lo)
+    rem = units - parts * (4 * lo + (wk - 4) * ly)
+    older = lo + (rem > 0)
+    return older, older + ((ly + (rem > 4 * parts)) if wk == 8 else 0)
+
+
+def test_a_finer_cut_of_the_fp6_tiles_shortens_the_loop_and_keeps_row_tiles_together(plan):
+    """Short of twice as finely as the INT4 tiles: with four waves or beyond eight parts only for 128 rows of k less at least, and
+    not where two row tiles, a multiple of eight workgroups apart, would no longer read their words through one XCD's L2."""
+    def of(mb, m, k, n, qc, group):
+        return plan(mb, n // 128, qc // 128, -(-m // (16 * mb)), k, group)[:3]
+
+    assert of(4, 86, 3840, 2048, 256, False) == (5, 5, 4)             # slices of 3 units in 5 parts and in 7
+    assert of(2, 22, 9472, 2048, 1024, False) == (8, 8, 8)
+    assert of(4, 110, 16384, 2560, 128, True)[:2] == (6, 6)         # 120 workgroups per row tile; 122 in 8 parts
+    assert of(4, 114, 16128, 3584, 512, True)[:2] == (4, 6)           # 112; 120 in 6 parts, 124 in the 7 that fit
+    assert of(3, 33, 13824, 5120, 512, False) == (6, 10, 8)
+    assert of(2, 20, 4352, 9472, 1024, False) == (3, 4, 8)            # (a unit less, four parts)
+    rng = random.Random(9)
+    finer = 0
+    for _ in range(40000):
+        mb, group, mtiles = rng.choice([2, 3, 4]), rng.random() < 0.5, rng.choice([1, 1, 2])
+        tiles, k = rng.randint(8, 160), 128 * rng.randint(8, 224)
+        tiles6 = min(tiles, rng.choice([1, 2, 4, 8, tiles // 2]))
+        group = group and tiles6 < tiles
+        ks, ks6, wk, _ = plan(mb, tiles, tiles6, mtiles, k, group)
+        if not ks < ks6 < 2 * ks:
+            continue
+        finer += 1
+        unit = 128 if group else 64
+        before, after = longest(k // unit, ks, wk), longest(k // unit, ks6, wk)
+        apart = [mtiles > 1 and grid % 8 != 0 for grid in (tiles * ks, (tiles - tiles6) * ks + tiles6 * ks6)]
+        less = max(b - a for a, b in zip(after, before)) * unit
+        assert (apart[0] and not apart[1]) or (apart[0] == apart[1] and (less >= 128 or (wk == 8 and ks6 <= 8))), (mb, tiles, tiles6, mtiles, k, group)
+    assert finer > 1000
