@@ -730,7 +730,8 @@ __device__ __forceinline__ void wg_finish_mb(const GemmArgs& p, const TileInfo& 
 {
     // BPR: 16-row blocks per round of the reduction through LDS (a wave's region holds BPR * 16 rows of kRedStride
     // floats).  The rounds are bound by LDS bandwidth (every wave writes and reads its whole accumulator once) plus two
-    // barriers each, so fewer rounds help; the gather below keeps the loads of up to 32 rows in flight per lane.
+    // barriers each, so fewer rounds help; the gather below keeps the loads of up to 32 rows in flight per lane.  (Three
+    // blocks: the last round has one of them.  Its bound is in the loops of that build alone: in the others it alters the code.)
     constexpr int RMAX = 16 / WK;                                    // rows of a block one wave finishes
     // The gather keeps up to 32 8-byte loads per lane in flight.
     constexpr int kInFlight = 32;
@@ -781,7 +782,7 @@ __device__ __forceinline__ void wg_finish_mb(const GemmArgs& p, const TileInfo& 
         if (mb0 == 0) FP6M_MARK(p, 1);                               // every wave of the group has left its loop
         float* mine = reinterpret_cast<float*>(smem + wk * wave_lds) + c * kRedStride + 64 * (q >> 1) + 4 * (q & 1);
 #pragma unroll
-        for (int b = 0; b < BPR && mb0 + b < MB; b++)
+        for (int b = 0; b < BPR && (MB % BPR == 0 || mb0 + b < MB); b++)
 #pragma unroll
             for (int t = 0; t < 8; t++)
                 *reinterpret_cast<f4*>(mine + b * 16 * kRedStride + 16 * (t >> 1) + 8 * (t & 1)) = acc[mb0 + b][t];
@@ -789,7 +790,7 @@ __device__ __forceinline__ void wg_finish_mb(const GemmArgs& p, const TileInfo& 
         // all LDS reads of the round first (rows beyond m are read too: the slab is there), one wait, then the sums
         f2 tv[BPR][RMAX][WK];
 #pragma unroll
-        for (int b = 0; b < BPR && mb0 + b < MB; b++)
+        for (int b = 0; b < BPR && (MB % BPR == 0 || mb0 + b < MB); b++)
 #pragma unroll
             for (int r = 0; r < RMAX; r++)
 #pragma unroll
@@ -797,7 +798,7 @@ __device__ __forceinline__ void wg_finish_mb(const GemmArgs& p, const TileInfo& 
                     tv[b][r][j] = *reinterpret_cast<const f2*>(reinterpret_cast<const float*>(smem + j * wave_lds) +
                                                                (b * 16 + wk + r * WK) * kRedStride + 2 * lane);
 #pragma unroll
-        for (int b = 0; b < BPR && mb0 + b < MB; b++)
+        for (int b = 0; b < BPR && (MB % BPR == 0 || mb0 + b < MB); b++)
 #pragma unroll
             for (int r = 0; r < RMAX; r++) {
                 const int row = 16 * (mb0 + b) + wk + r * WK;
