@@ -462,65 +462,6 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
     }
 }
 
-// The time of one launch of gemm_mb_kernel, us, for the choice among its tiles of 32, 48 and 64 rows.
-//
-// None of them wins everywhere: a taller tile dequantises less often and reads fewer words, a shorter one fills its rows and
-// the CUs better and reduces less per workgroup.  Which of them does follows from how many workgroups there are and how long
-// their slices get, so the launch is estimated from its split (least squares without negative terms, over 882 points: 28
-// shapes and 130 random ones of k = 2048 .. 20480 by n = 2048 .. 40960 at 33 to 400 rows, both scale modes, none to 1024 FP6
-// columns; they reproduce the times to 3-6 %).  Against the one tile height that the rows suggested (64 from 49 on, or 128, or
-// the many-rows kernel where those were estimated faster) the choice takes 6.4 % off over all those points and is within
-// 0.7 % of the best of all of them on average, where that rule was 7.6 % off; fitted to one half of the points it does the
-// same on the other.  A challenger must be 5 % faster by the estimate; of 403 points where the choice changes ten lose more
-// than 1.5 % (the worst 17 %, 121 x 15360 x 2304).  Together with the 48-row
-// tile itself 287 other random points of 33 to 1200 rows: -7.7 % (33-96 rows -13 to -14 %, 129-192 -8 %, 301-500 -2 %), the
-// worst +4.9 % (166 x 19968 x 3072), from 500 rows on nothing changes.
-// 32-row tiles: 64 x 4096 x 4096 14.4 -> 10.9 us, 96 x 5120 x 5120 18.5 -> 14.7, 80 x 8192 x 10240 36.4 -> 28.7; 48-row
-// tiles: 96 x 8192 x 8192 26.7 -> 24.1, 96 x 13824 x 5120 29.9 -> 26.7, 144 x 4096 x 12288 33.1 -> 29.3.
-struct MbTime {
-    // At most one workgroup per CU: us once; per k step (32 rows) of the mean and of the longest slice, and what group scales
-    // and full occupation add per step; per step by which an FP6 slice exceeds 0.7 of an INT4 slice; with a split: us once,
-    // per part, and for full occupation.
-    double start, mean, longest, group, busy, fp6, split, part, split_busy;
-};
-struct MbTimeMany {
-    // More: per CU two workgroups of four waves at a time.  us once; per step of a full round, and with group scales; the last
-    // round up to one workgroup per CU, by occupation and once, and beyond one, once and by occupation; us per round; group
-    // scales in the last round.
-    double start, full, full_group, low_busy, low, high, high_busy, round, last_group;
-};
-constexpr MbTime kMbTimeEight[] = {{5.479, 0.322, 0.224, 0.046, 0.125, 0.181, 1.422, 0.099, 0.427},    // 32, 48, 64 rows, eight waves
-                                   {6.556, 0.302, 0.268, 0.043, 0.237, 0.249, 0.924, 0.311, 0.588},
-                                   {7.479, 0.488, 0.107, 0.054, 0.358, 0.284, 0.0, 0.509, 1.348}};
-constexpr MbTime kMbTimeFour[] = {{0.0, 0.0, 1.241, 0.0, 0.0, 0.298, 0.0, 0.0, 0.702},                 // ... four waves
-                                  {6.091, 0.0, 0.429, 0.025, 0.0, 0.143, 0.312, 0.618, 0.841},
-                                  {7.553, 0.032, 0.375, 0.0, 0.079, 0.102, 0.372, 0.676, 1.243}};
-constexpr MbTime kMbTimeTall = {9.971, 0.0, 0.533, 0.01, 0.191, 0.224, 2.606, 0.959, 0.0};             // 128 rows
-constexpr MbTimeMany kMbTimeMany[] = {{1.919, 0.91, 0.034, 0.24, 0.207, 0.749, 0.179, 1.99, 0.018},
-                                      {3.003, 0.932, 0.037, 0.241, 0.172, 0.679, 0.24, 2.954, 0.066},
-                                      {4.016, 1.055, 0.06, 0.289, 0.208, 0.804, 0.246, 3.459, 0.052}};
-// tiles: all, tiles6 of them FP6.  No estimate for 128-row tiles beyond one workgroup per CU (0).
-inline double mb_time(int mb, const MbSplit& sp, long long tiles, long long tiles6, long long mtiles, int k, int units, bool g128, int cus)
-{
-    const double per_unit = k / (32.0 * units), g = g128 ? 1.0 : 0.0;
-    auto longest = [&](long long slices) { return (double)((units + slices - 1) / slices) * per_unit; };
-    const double s = longest(sp.ks * sp.wk), mean = k / (32.0 * sp.ks * sp.wk);
-    const long long base = tiles * mtiles;
-    if (base * sp.ks <= cus) {
-        const MbTime& c = mb == 8 ? kMbTimeTall : (sp.wk == 8 ? kMbTimeEight : kMbTimeFour)[mb - 2];
-        const double busy = (double)((tiles - tiles6) * sp.ks + tiles6 * sp.ks6) * mtiles / cus;
-        const double mean6 = tiles6 ? k / (32.0 * sp.ks6 * sp.wk) : 0.0, over6 = mean6 - 0.7 * mean;
-        return c.start + c.mean * mean + c.longest * s + c.group * mean * g + c.busy * mean * busy + (over6 > 0 ? c.fp6 * over6 : 0.0) +
-               (sp.ks > 1 ? c.split + c.part * sp.ks + c.split_busy * busy : 0.0);
-    }
-    if (mb == 8) return 0.0;
-    const MbTimeMany& c = kMbTimeMany[mb - 2];
-    const long long wgs = base * sp.ks, full = wgs / (2 * cus), rem = wgs % (2 * cus);
-    double t = c.start + full * s * (c.full + c.full_group * g) + c.round * (full + (rem ? 1 : 0));
-    if (rem) t += s * (c.last_group * g + (rem <= cus ? c.low + c.low_busy * rem / cus : c.high + c.high_busy * (rem - cus) / cus));
-    return t;
-}
-
 // Whether a launch of more than 16 rows goes to gemm_wide_kernel, and with which tile: 1 .. 7, or 0 (gemm_mb_kernel).
 //
 // The wide kernel's tiles (128 or fewer rows x 256 columns, all of k) are large, so what decides is how their number
