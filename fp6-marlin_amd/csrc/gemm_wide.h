@@ -315,10 +315,12 @@ __device__ __forceinline__ void wide_workgroup(const WideArgs& p, unsigned char*
     const int q = lane >> 4, c = lane & 15;
     const int col_lane = 32 * (q >> 1) + 4 * (q & 1);
     const int row0 = ti.mtile * 16 * MB;
+    constexpr bool kThroughSlab = EXTRAS && WK > 1;
+    const bool fused = kThroughSlab && p.fused;
     f4 scale[4];
 #pragma unroll
     for (int f = 0; f < 4; f++) scale[f] = f4{1.f, 1.f, 1.f, 1.f};
-    if (ti.fp6 || !G128) {
+    if ((ti.fp6 || !G128) && !fused) {
         const uint16_t* sp = (ti.fp6 ? p.s_fp6 : p.s_int4) + ti.tcol * kTileN + 64 * sigma;
         const float re_bias = ti.fp6 ? 4096.0f : 1.0f;    // the deferred e3m2 exponent re-bias
 #pragma unroll
@@ -332,8 +334,69 @@ __device__ __forceinline__ void wide_workgroup(const WideArgs& p, unsigned char*
             }
     }
     unsigned char* slab = smem + wide_round_bytes(WN, WK) + wave * 16 * kWideSlabRow;
-    FusedCols fc[EXTRAS ? 4 : 1][2];
-    if constexpr (EXTRAS) {
+    // The fused epilogue (column map, bias, residual): a lane takes one column, and a block's rows, as fp32, change hands through
+    // the wave's slab, eight at a time.  A row is then one load and one store of whole lines (of the mapped columns' lines, which
+    // are mostly neighbours), and a block's residual is on its way while the slices are summed.  (Each lane adding to its own
+    // fragments, two bytes of 64 lines at a time and in turn with the stores, as the residual may be C, cost a round of 48-row
+    // tiles 10 us, more than these tiles gain over gemm_mb_kernel's: with bias and residual, us, 107 x 3328 x 19712 with that
+    // kernel 36.2, here 40.0 -> 33.5; 300 x 4096 x 12288 52.0 -> 40.9, without additions 39.3; 2048 x 8192 x 10240 358 -> 308, 300.
+    // 200 and 300 random calls: 18-28 % for every tile, none slower.)
+    // Without slices there is no sum to wait for, and the accumulators of 128 rows leave no registers: there it is as it was.
+    unsigned fcol = 0;                                    // bytes
+    float fscale = 1.f, fbias = 0.f;
+    uint16_t res[kThroughSlab ? 16 : 1] = {};
+    if constexpr (kThroughSlab) {
+        if (fused) {
+            int col = ti.col0 + lane;
+            if (p.c_cols) {
+                col = p.c_cols[col];
+                col = col < 0 ? 0 : (col >= p.n ? p.n - 1 : col);         // (a bad map cannot write outside C)
+            }
+            fcol = 2u * (unsigned)col;
+            if (p.bias) fbias = (float)__builtin_bit_cast(_Float16, p.bias[col]);
+            if (ti.fp6 || !G128)
+                fscale = (float)reinterpret_cast<const _Float16*>(ti.fp6 ? p.s_fp6 : p.s_int4)[ti.tcol * kTileN + 64 * sigma + (lane & 32) + scale_slot(lane & 31)] *
+                         (ti.fp6 ? 4096.0f : 1.0f);
+        }
+    }
+    auto load_residual = [&](int blk) {
+        if constexpr (kThroughSlab) {
+            const int first = row0 + 16 * blk;
+            if (!p.residual || first >= p.m) return;      // (uniform)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int row = first + r < p.m ? first + r : p.m - 1;
+                res[r] = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const unsigned char*>(p.residual + (size_t)row * p.n) + fcol);
+            }
+        }
+    };
+    auto store_fused_block = [&](int blk, const f4 (&v)[4]) {
+        if constexpr (kThroughSlab) {
+            const int first = row0 + 16 * blk;
+            if (first >= p.m) return;                     // (uniform)
+            constexpr int kRow = 64 + 4;                  // floats
+            static_assert(8 * kRow * 4 <= 16 * kWideSlabRow, "eight rows of a block");
+            float* rows = reinterpret_cast<float*>(slab);
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                __builtin_amdgcn_wave_barrier();
+                if ((c >> 3) == half) {
+#pragma unroll
+                    for (int f = 0; f < 4; f++) *reinterpret_cast<f4*>(rows + (c & 7) * kRow + col_lane + 16 * (f >> 1) + 8 * (f & 1)) = v[f];
+                }
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int r = 0; r < 8; r++) {
+                    const int row = first + 8 * half + r;
+                    float o = rows[r * kRow + lane] * fscale + fbias;
+                    if (p.residual) o += (float)__builtin_bit_cast(_Float16, res[8 * half + r]);
+                    if (row < p.m) *reinterpret_cast<uint16_t*>(reinterpret_cast<unsigned char*>(p.C + (size_t)row * p.n) + fcol) = __builtin_bit_cast(uint16_t, (_Float16)o);
+                }
+            }
+        }
+    };
+    FusedCols fc[EXTRAS && !kThroughSlab ? 4 : 1][2];
+    if constexpr (EXTRAS && !kThroughSlab) {
 #pragma unroll
         for (int f = 0; f < 4; f++)
 #pragma unroll
@@ -342,7 +405,7 @@ __device__ __forceinline__ void wide_workgroup(const WideArgs& p, unsigned char*
     auto store_block = [&](int blk, const f4 (&v)[4]) {
         const int first = row0 + 16 * blk;
         if (first >= p.m) return;                         // (uniform)
-        if constexpr (EXTRAS) {
+        if constexpr (EXTRAS && !kThroughSlab) {
             if (p.fused) {
                 if (first + c >= p.m) return;
 #pragma unroll
@@ -378,6 +441,7 @@ __device__ __forceinline__ void wide_workgroup(const WideArgs& p, unsigned char*
     } else {
 #pragma unroll
         for (int r = 0; r < (MB + WK - 1) / WK; r++) {
+            if (fused && r * WK + wk < MB) load_residual(r * WK + wk);
             __syncthreads();
             f4* out = reinterpret_cast<f4*>(smem) + (size_t)(wn * WK * WK) * 256 + lane;   // [wn][owner][slice][fragment] 1 KiB each
 #pragma unroll
@@ -395,7 +459,10 @@ __device__ __forceinline__ void wide_workgroup(const WideArgs& p, unsigned char*
 #pragma unroll
                     for (int s = 1; s < WK; s++) sum[f] += out[(wk * WK + s) * 256 + 64 * f];
                 }
-                store_block(r * WK + wk, sum);
+                if (fused)
+                    store_fused_block(r * WK + wk, sum);
+                else
+                    store_block(r * WK + wk, sum);
             }
         }
     }

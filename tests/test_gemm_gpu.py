@@ -439,6 +439,35 @@ def test_waves_side_by_side_in_n_with_maps_additions_and_the_gfx950_order(oracle
     assert ((added.float() - full).abs().mean() / full.abs().mean()).item() <= TOL
 
 
+@pytest.mark.parametrize("plan", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("m,n,k,qc,gs", [(65, 512, 256, 256, 128), (131, 1280, 512, 1280, -1), (241, 768, 384, 128, -1), (48, 512, 256, 0, 128)])
+def test_waves_side_by_side_in_n_with_each_addition(oracle, plan, m, n, k, qc, gs):
+    """Map, bias and residual one by one and together, in every tile: rows that end inside a block, tiles of both regions and of
+    one, the residual in place of C (bit for bit what it gives beside it)."""
+    import fp6_marlin
+    ref, B, s = problem(oracle, n, k, qc if qc else -1, gs)
+    g = torch.Generator().manual_seed(10 * plan + m)
+    A = torch.randn((m, k), generator=g).half().to(dev())
+    c_cols = torch.randperm(n, generator=g).to(torch.int32).to(dev())
+    bias, residual = torch.randn(n, generator=g).half().to(dev()), torch.randn((m, n), generator=g).half().to(dev())
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    want = torch.from_numpy(oracle.matmul_ref(A.cpu().numpy(), ref).astype(np.float32)).to(dev())
+    with fp6_marlin.cabi.tuning(wide=plan):
+        for mapped in (False, True):
+            for b, r in ((bias, None), (None, residual), (bias, residual)) + (((None, None),) if mapped else ()):
+                C = torch.full((m, n), float("nan"), dtype=torch.half, device=dev())
+                fp6_marlin.mul_fused(A, B, C, s, ws, qc if qc else -1, gs, c_cols=c_cols if mapped else None, bias=b, residual=r)
+                full = want.clone()
+                if mapped:
+                    full[:, c_cols.long()] = want
+                full += (0 if b is None else b.float()) + (0 if r is None else r.float())
+                assert ((C.float() - full).abs().mean() / full.abs().mean()).item() <= TOL, (mapped, b is None, r is None)
+                if r is not None:
+                    over = r.clone()
+                    fp6_marlin.mul_fused(A, B, over, s, ws, qc if qc else -1, gs, c_cols=c_cols if mapped else None, bias=b, residual=over)
+                    assert torch.equal(over, C)
+
+
 def test_eight_k_slices_per_workgroup(oracle):
     """The m > 16 kernel with eight waves (k slices) per workgroup, which small grids on long k pick by themselves
     (here: 8192 x 512 at m = 40), forced on and off on ragged shapes."""
