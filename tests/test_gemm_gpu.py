@@ -261,6 +261,21 @@ def test_two_classes_of_int4_tiles_beyond_sixteen_rows(oracle, capfd):
             one_hot_case(oracle, m, n, k, qc, gs, {"cls": 1, "cus": cus})
 
 
+def test_two_classes_with_three_row_blocks(oracle, capfd):
+    """48-row tiles have the two classes with per-column scales as well (64-row tiles do not): both edges of their rows, the second
+    class in one and in two parts, with and without FP6 columns; one-hot rows bit for bit."""
+    import re
+    for cus, n, k, qc in ((8, 1536, 2048, 256), (8, 1536, 4096, 256), (16, 3072, 2048, -1)):
+        for gs in (-1, 128):
+            capfd.readouterr()
+            for m in (33, 40, 48):
+                run(oracle, m, n, k, qc=qc, gs=gs, env={"FP6M_CLS": 1, "FP6M_CUS": cus, "FP6M_VERBOSE": 1})
+            out = capfd.readouterr().err
+            second = [int(x) for x in re.findall(r"MB=3 row tiles 1 .*\(\+ (\d+) tiles in \d+ parts\)", out)]
+            assert len(second) == 6 and all(x > 0 for x in second), out[-3000:]
+            one_hot_case(oracle, 48, n, k, qc, gs, {"cls": 1, "cus": cus})
+
+
 def test_three_row_blocks_per_wave(oracle, capfd):
     """48-row tiles: what 33 to 48 rows take, at both edges, ragged, several row tiles (forced), all FP6 and all INT4, both scale
     modes, four and eight slices, k splits with the FP6 tiles cut as finely and finer; one-hot rows bit for bit."""
@@ -296,6 +311,39 @@ def test_row_tiles_by_estimate(oracle, capfd):
     assert set(re.findall(r"MB=(\d)", capfd.readouterr().err)) == {"2"}
     run(oracle, 65, 768, 1920, qc=256, env={"FP6M_VERBOSE": 1})
     assert "MB=4" in capfd.readouterr().err
+
+
+@pytest.mark.skipif(not torch.cuda.is_available() or torch.cuda.get_device_properties(0).multi_processor_count != 256,
+                    reason="the choices are those of 256 CUs")
+def test_heights_by_estimate_in_place_of_taller_tiles(capfd):
+    """Each height where its estimate is clearly the smallest: instead of 64-row tiles, and of 128-row tiles (what the rows and
+    columns alone would take); sms, a limit on parts, leaves those alone.  Results against the unpacked words, per region."""
+    import fp6_marlin
+    g = torch.Generator().manual_seed(12)
+    for m, k, n, qc, gs, want in ((64, 4096, 4096, 256, 128, "MB=2"), (96, 8192, 8192, 256, 128, "MB=3"), (143, 12544, 6144, 256, -1, "MB=2"),
+                                  (139, 23808, 6656, 1024, -1, "MB=3"), (364, 18176, 9984, 0, 128, "MB=8")):
+        n4 = n - qc
+        B = torch.randint(-2 ** 31, 2 ** 31 - 1, (k * n4 // 8 + k * qc * 3 // 16,), generator=g, dtype=torch.int64).to(torch.int32)
+        s = (torch.rand((n4 if gs == -1 else k // gs * n4) + qc, generator=g) * 0.01 + 0.001).half()
+        A = torch.randn((m, k), generator=g).half().to(dev())
+        C = torch.full((m, n), float("nan"), dtype=torch.half, device=dev())
+        ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+        ref = A.float() @ fp6_marlin.unpack_to_fp16(B, s, k, n, qc or -1, gs).to(dev()).float()
+        capfd.readouterr()
+        with fp6_marlin.cabi.tuning(verbose=1):
+            fp6_marlin.mul(A, B.to(dev()), C, s.to(dev()), ws, qc or -1, -1, -1, -1, 16, gs)
+            torch.cuda.synchronize()
+            err = capfd.readouterr().err
+            assert want in err, (m, k, n, want, err[-400:])
+            for part in (slice(0, n4), slice(n4, n)):
+                if part.start < part.stop:
+                    assert float((C.float() - ref)[:, part].abs().mean() / ref[:, part].abs().mean()) <= TOL
+        if want != "MB=8":
+            with fp6_marlin.cabi.tuning(verbose=1):
+                fp6_marlin.mul(A, B.to(dev()), C, s.to(dev()), ws, qc or -1, -1, -1, 256, 16, gs)
+            torch.cuda.synchronize()
+            err = capfd.readouterr().err
+            assert ("MB=8" if m > 100 else "MB=4") in err, (m, k, n, err[-400:])
 
 
 def test_eight_row_blocks_per_wave(oracle):
