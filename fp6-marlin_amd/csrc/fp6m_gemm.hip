@@ -462,7 +462,7 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
     }
 }
 
-// Whether a launch of more than 16 rows goes to gemm_wide_kernel, and with which tile: 1 .. 7, or 0 (gemm_mb_kernel).
+// Whether a launch of more than 16 rows goes to gemm_wide_kernel, and with which tile: 1 .. 9, or 0 (gemm_mb_kernel).
 //
 // The wide kernel's tiles (128 or fewer rows x 256 columns, all of k) are large, so what decides is how their number
 // divides into rounds: one workgroup of eight waves per CU (two k slices), or two of four waves (no k split).  Neither
@@ -486,7 +486,7 @@ void launch_mb(const GemmArgs& a, bool g128, int wk, dim3 grid, hipStream_t stre
 // Plans 8 and 9 are the same with 64 and 48 rows, for launches that taller tiles leave CUs idle in (300 x 4096 x 12288: 196
 // workgroups of 80 rows, 245 of 64), fitted to 206 shapes of 65 to 900 rows with none to 1024 FP6 columns (1.9 %, the worst
 // 8 %).  Over 420 shapes of those rows, half of them not in the fit, they are taken on 42: -11 % on average there, none slower;
-// us: 300 x 4096 x 12288 40.7 -> 39.4, 181 x 3072 x 14592 with per-column scales 28.7 -> 23.3, 229 x 3584 x 10496 32.1 -> 25.5,
+// us: 300 x 4096 x 12288 39.9 -> 39.5 (new inputs each pass), 181 x 3072 x 14592 with per-column scales 28.7 -> 23.3, 229 x 3584 x 10496 32.1 -> 25.5,
 // 178 x 8960 x 17920 86.4 -> 75.4, 525 x 2816 x 5376 29.8 -> 24.1.
 struct WidePlan {
     int mb, per_cu;               // 16-row blocks per tile; workgroups per CU

@@ -222,7 +222,7 @@ struct MbCtx {
 };
 
 // One step of the MB loop, fully static in BLK: block by block the 16 rows of A are multiplied into
-// the step's eight weight fragments.  Activations travel through a ring of four register buffers,
+// the step's eight weight fragments.  Activations travel through a ring of a_buffers(MB) register buffers,
 // fetched from LDS two blocks ahead of their use (the latency hides behind 16 MFMAs); the s_waitcnt
 // immediates follow from the fixed issue order: [A(0), A(1)] from the previous step, the next step's
 // weight words (kExtra reads), then A(2), A(3), ...  After every MFMA `hook(block, t)` runs: the caller
@@ -488,7 +488,7 @@ __device__ __forceinline__ void stream_tile_mb(const GemmArgs& p, const TileInfo
     }
 }
 
-// The MB = 4 variant of stream_tile_mb: activations fetched a pair of k steps at a time, packed words through
+// The paired variant of stream_tile_mb (MB = 2, 3, 4 and 8): activations fetched a pair of k steps at a time, packed words through
 // registers.
 //
 // What bounds a workgroup's rate is its requests in flight, and A dominated them: 64 half-lines per step and

@@ -63,7 +63,7 @@ int fp6m_abi_version(void);
  *               different kernel here (tile shapes are chosen for 256 CUs / wave64).
  *   sms         -1 = automatic; otherwise an upper bound on the number of workgroups that cooperate
  *               on one column tile's reduction (debug/testing knob, like the reference's).
- *   max_par     as in the reference: bounds how many blocks of A (32, 64 or 128 rows) one launch covers, and sizes the
+ *   max_par     as in the reference: bounds how many blocks of A (32, 48, 64 or 128 rows) one launch covers, and sizes the
  *               workspace; the many-rows kernel covers all rows in one launch whatever it says.
  *   quant_cols  -1 (or 0) = all INT4; n = all FP6; otherwise the last quant_cols columns are FP6.
  *               Must be a multiple of 128, as must n - quant_cols.
@@ -157,7 +157,7 @@ int fp6m_mul_rows(const void* A, int lda, const void* B, void* C, const void* s,
 /*
  * Testing / tuning hook: overrides one of the dispatcher's per-shape choices for all later calls in this process.
  * No counterpart in the reference (whose only such knob is the `sms` argument).  knob = "ksplit" (k parts per tile),
- * "wk16" / "wk" (waves per workgroup of the m <= 16 / m > 16 kernel: 4 or 8), "mb" (16-row blocks per wave: 2, 4 or 8),
+ * "wk16" / "wk" (waves per workgroup of the m <= 16 / m > 16 kernel: 4 or 8), "mb" (16-row blocks per wave: 2, 3, 4 or 8),
  * "pair" (paired activation fetch on/off),
  * "sk" (the one-wave decode kernel on for m <= 4 / off), "share" / "share6" (k units per chunk of its work list: both
  * regions / the FP6 region only), "cap" (the waves it aims at), "wgs" (exactly that many waves, one-unit chunks drawn
@@ -170,7 +170,7 @@ int fp6m_mul_rows(const void* A, int lda, const void* B, void* C, const void* s,
  * of the second wave of every SIMD in eight-wave workgroups relative to the first one's; 100 = equal slices),
  * "cls" (0: the kernels never put the INT4 tiles in two classes -- whole tiles on the first workgroups, the
  * rest in parts on later ones --, 1: wherever they can), "wide" (the many-rows kernel, whose waves lie side by side in n:
- * 0 never, 1 .. 7 with that tile wherever it can: more than 16 rows, k a multiple of 128, n of 256, no row mix, and
+ * 0 never, 1 .. 9 with that tile wherever it can: more than 16 rows, k a multiple of 128, n of 256, no row mix, and
  * gathered activations of at most 64 MiB), "cus" (tests: plan for a chip of that many CUs),
  * "verbose" (print every launch's configuration to stderr); knob = NULL clears all overrides.  Unknown knob or tile ->
  * FP6M_ERR_ARG.  Not synchronised with GEMM calls running on other threads.  The library reads no environment
