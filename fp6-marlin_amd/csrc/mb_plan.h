@@ -174,7 +174,8 @@ inline MbSplit mb_split(int mb, const MbLaunch& l)
 // columns; they reproduce the times to 3-6 %).  The entry of 32-row tiles in four-wave workgroups, which only short k takes, is
 // from 110 shapes of its own up to k = 3840 (3.6 %, the worst 11 %): the 882 held too few, and gave it no start (64 x 2048 x 2560
 // without FP6 columns 5.4 us, measured 9.2; now 8.9).  No choice in 30000 random shapes depends on that.
-// Fitted to plain calls, and used as it is for fused ones and the gfx950 word order.
+// Fitted to plain calls; against the rule before, 500 random calls with bias and residual and 200 in the gfx950 word order are
+// 14 % and 8 % faster on average, none more than 1.5 % slower.
 // Against the one tile height that the rows suggested (64 from 49 on, or 128, or the many-rows kernel where those were
 // estimated faster) the choice takes 6.4 % off over all 882 and is within 0.7 % of the best of all of them on average, where that rule
 // was 7.6 % off; fitted to one half of the points it does the same on the other.  A challenger must be 5 % faster by the
