@@ -24,6 +24,7 @@
 // gemm_common.h  argument block, tile bookkeeping, load / wait / dequantisation helpers
 // gemm_sk.h      gemm_sk_kernel (one row: the decode kernel)
 // gemm_m16.h     gemm_m16_kernel (m <= 16)
+// gemm_m16h.h    gemm_m16h_kernel (m <= 16, tiles of 64 columns; the choice between the two: m16_plan.h)
 // gemm_mb.h      gemm_mb_kernel (16 < m)
 // this file      activation gather, per-device scratch, dispatch and the extern "C" entry points
 #include <hip/hip_runtime.h>
@@ -36,9 +37,11 @@
 #include "fp6m.h"
 #include "gemm_common.h"
 #include "gemm_m16.h"
+#include "gemm_m16h.h"
 #include "gemm_sk.h"
 #include "gemm_mb.h"
 #include "gemm_wide.h"
+#include "m16_plan.h"
 
 namespace fp6m {
 
@@ -67,7 +70,7 @@ thread_local int g_last_hip_error = 0;
 constexpr int kUnset = INT32_MIN;
 const int g_env_verbose = getenv("FP6M_VERBOSE") ? 1 : 0;
 struct Tuning {
-    int mb = kUnset, ksplit = kUnset, wk16 = kUnset, wk = kUnset, pair = kUnset, wgs = kUnset, share = kUnset, share6 = kUnset, sk = kUnset, cap = kUnset, gather = kUnset, cells = kUnset, xcd = kUnset, gen = kUnset, gen2 = kUnset, gen3 = kUnset, young = kUnset, cls = kUnset, cus = kUnset, cap2 = kUnset, wide = kUnset;
+    int mb = kUnset, ksplit = kUnset, wk16 = kUnset, wk = kUnset, pair = kUnset, wgs = kUnset, share = kUnset, share6 = kUnset, sk = kUnset, cap = kUnset, gather = kUnset, cells = kUnset, xcd = kUnset, gen = kUnset, gen2 = kUnset, gen3 = kUnset, young = kUnset, cls = kUnset, cus = kUnset, cap2 = kUnset, wide = kUnset, half = kUnset;
     int verbose = g_env_verbose;
 };
 Tuning g_tuning;
@@ -400,6 +403,25 @@ inline void launch_m16_any(const M16Config& cfg, const GemmArgs& a, bool g128, d
         launch_m16<16, 1, 4, 4, 3>(a, g128, grid, stream);
 }
 
+// The same on 64-column tiles, with rings of 4, 8 or 16 rows of A (up to four rows always with the cells).
+template <bool G128, int AROWS, int WK, bool EXTRAS>
+void launch_m16h_one(const GemmArgs& a, dim3 grid, hipStream_t stream)
+{
+    void (*kernel)(const GemmArgs) = gemm_m16h_kernel<G128, AROWS, WK, 4, 3, AROWS == 4, EXTRAS>;
+    if constexpr (AROWS > 4 && WK == 4) {
+        if (a.xcd_local) kernel = gemm_m16h_kernel<G128, AROWS, WK, 4, 3, false, EXTRAS, true>;
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * WK), 0, stream, a);
+}
+template <int AROWS, int WK>
+void launch_m16h(const GemmArgs& a, bool g128, dim3 grid, hipStream_t stream)
+{
+    if (needs_extras(a))
+        g128 ? launch_m16h_one<true, AROWS, WK, true>(a, grid, stream) : launch_m16h_one<false, AROWS, WK, true>(a, grid, stream);
+    else
+        g128 ? launch_m16h_one<true, AROWS, WK, false>(a, grid, stream) : launch_m16h_one<false, AROWS, WK, false>(a, grid, stream);
+}
+
 template <bool G128, int MB, int D4, int D6, int WK, bool PAIR, bool LEAN>
 void launch_mb_one(const GemmArgs& a, dim3 grid, hipStream_t stream)
 {
@@ -579,7 +601,7 @@ int fp6m_tuning_set(const char* knob, int value)
     if (!strcmp(knob, "wide") && (value < 0 || value > fp6m::kWidePlanCount)) return FP6M_ERR_ARG;
     const struct { const char* name; int* field; } knobs[] = {
         {"mb", &g_tuning.mb}, {"ksplit", &g_tuning.ksplit},
-        {"wk16", &g_tuning.wk16}, {"wk", &g_tuning.wk}, {"pair", &g_tuning.pair}, {"wgs", &g_tuning.wgs}, {"share", &g_tuning.share}, {"share6", &g_tuning.share6}, {"cap", &g_tuning.cap}, {"sk", &g_tuning.sk}, {"gather", &g_tuning.gather}, {"cells", &g_tuning.cells}, {"xcd", &g_tuning.xcd}, {"gen", &g_tuning.gen}, {"gen2", &g_tuning.gen2}, {"gen3", &g_tuning.gen3}, {"young", &g_tuning.young}, {"cls", &g_tuning.cls}, {"cus", &g_tuning.cus}, {"cap2", &g_tuning.cap2}, {"wide", &g_tuning.wide},
+        {"wk16", &g_tuning.wk16}, {"half", &g_tuning.half}, {"wk", &g_tuning.wk}, {"pair", &g_tuning.pair}, {"wgs", &g_tuning.wgs}, {"share", &g_tuning.share}, {"share6", &g_tuning.share6}, {"cap", &g_tuning.cap}, {"sk", &g_tuning.sk}, {"gather", &g_tuning.gather}, {"cells", &g_tuning.cells}, {"xcd", &g_tuning.xcd}, {"gen", &g_tuning.gen}, {"gen2", &g_tuning.gen2}, {"gen3", &g_tuning.gen3}, {"young", &g_tuning.young}, {"cls", &g_tuning.cls}, {"cus", &g_tuning.cus}, {"cap2", &g_tuning.cap2}, {"wide", &g_tuning.wide},
         {"verbose", &g_tuning.verbose}};
     for (const auto& k : knobs)
         if (!strcmp(knob, k.name)) {
@@ -748,10 +770,10 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
     if (tune.mb != kUnset && prob_m > 16 && (tune.mb == 2 || tune.mb == 3 || tune.mb == 4 || tune.mb == 8)) mb = tune.mb;
     // Row mix: the kWaves * ks slices of a tile are dealt to the two segments in proportion to their cost (an FP6
     // step costs about two INT4 steps), at least one each.
-    auto deal_slices = [&](int total) {
+    auto deal_slices = [&](int total, int unit6) {                      // (unit6: rows that FP6 slices are made of)
         const long long c4 = k4 / 32, c6 = 2LL * (fu.quant_rows / 32);
         long long n6 = (total * c6 + (c4 + c6) / 2) / (c4 + c6);
-        if (n6 > fu.quant_rows / 64) n6 = fu.quant_rows / 64;
+        if (n6 > fu.quant_rows / unit6) n6 = fu.quant_rows / unit6;
         if (n6 > total - 1) n6 = total - 1;
         if (n6 < 1) n6 = 1;
         return (int)(total - n6);
@@ -1178,13 +1200,23 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             // split is bounded so that every wave keeps at least one k unit, partial-sum traffic stays
             // well below the weight stream and the partial tiles fit the scratch.
             M16Config cfg = m16_config(a.m);
+            // 64-column tiles (gemm_m16h.h): k and the segments of a row mix in whole 128 rows, words in reference order, and for up
+            // to four rows the cells, beyond twice the counters in `workspace`.
+            const bool half_fits = prob_k % 128 == 0 && fu.quant_rows % 128 == 0 && !a.native &&
+                                   (a.m <= 4 ? tune.cells == kUnset && (size_t)prob_n * 16 * sizeof(unsigned long long) <= kCellBytes : max_par >= 2);
+            bool half = tune.half == 1 && half_fits;
+            int units16 = half ? prob_k / 128 : units;                  // rows of the weight in units that slices are made of
             a.groups6 = (a.tiles6 + cfg.wn - 1) / cfg.wn;
             a.groups4 = (a.tiles - a.tiles6 + cfg.wn - 1) / cfg.wn;
+            if (half) {
+                a.groups6 *= 2;
+                a.groups4 *= 2;
+            }
             const long long groups = a.groups6 + a.groups4;
             const int unit_steps = g128 ? 4 : 2;
             // Bounds of the split for a workgroup of wk waves: at least one k unit and four k steps per wave, and the
             // partial-sum traffic well below the weight stream.
-            auto ks_units = [&](int wk) { return units / wk > 0 ? (long long)(units / wk) : 1LL; };
+            auto ks_units = [&](int wk) { return units16 / wk > 0 ? (long long)(units16 / wk) : 1LL; };
             auto ks_limit = [&](int wk) {
                 long long c = prob_k / 32 / (4 * wk) > 0 ? prob_k / 32 / (4 * wk) : 1;
                 if (c > ks_units(wk)) c = ks_units(wk);
@@ -1232,7 +1264,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                         if (c > 1 && prob_k < 160 * 8 * c) return 1e9;
                         t = 0.56;
                     }
-                    auto longest = [&](long long slices) { return (double)((units + slices - 1) / slices) * unit_steps; };
+                    auto longest = [&](long long slices) { return (double)((units16 + slices - 1) / slices) * unit_steps; };
                     auto tail = [](long long partners) { return partners > 1 ? 2.5 + 0.15 * partners : 0.0; };
                     const double int4_us = a.groups4 ? longest(c * wk) * t + tail(c) : 0.0;
                     const double fp6_us = a.groups6 ? 1.5 * longest(c6 * wk) * t + tail(c6) : 0.0;   // an FP6 step moves 1.5x the bytes
@@ -1322,7 +1354,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                 // ways over 56 shapes (k = 2048 .. 14336, 312 .. 424 tiles, 8 and 16 rows) that is where it won (k = 2048
                 // in four parts -7 .. -12 %, k >= 4096 in two or more -5 .. -19 %) and the rest was within -1 .. +4 %.
                 // With the first class split as well (fewer tiles than CUs) every forced plan lost 5-30 %: not tried.
-                if (!row_mix && cfg.wn == 1 && sms <= 0 && env_ks < 1 && tune.wk16 == kUnset && a.groups4 > 0 &&
+                if (!half && !row_mix && cfg.wn == 1 && sms <= 0 && env_ks < 1 && tune.wk16 == kUnset && a.groups4 > 0 &&
                     !(tune.cls != kUnset && tune.cls == 0)) {
                     const long long c6 = a.groups6 ? ks6_of(1, 4) : 0;
                     const long long first = cus - a.groups6 * c6;                      // workgroups the first round has left
@@ -1342,13 +1374,62 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                     }
                 }
             }
+            // 64-column tiles instead, by estimated time (M16Time); not below k = 1024, where nothing was measured.
+            if (half_fits && tune.half == kUnset && tune.wk16 == kUnset && tune.cells == kUnset && tune.xcd == kUnset &&
+                !(tune.cls != kUnset && tune.cls == 1) && env_ks < 1 && sms <= 0 && prob_k >= 1024 && cls_na == 0) {
+                const double mbytes = (prob_k * (double)(prob_n - qc) * 0.5 + prob_k * (double)qc * 0.75) * 1e-6;
+                auto cut_of = [&](bool h, int wk, long long c) {
+                    const int u = h ? prob_k / 128 : units, per_unit = h ? 2 : unit_steps;
+                    const long long t6 = (long long)a.tiles6 * (h ? 2 : 1), t4 = (long long)a.tiles * (h ? 2 : 1) - t6;
+                    const long long limit = u / wk > 0 ? u / wk : 1;
+                    M16Cut cut{wk, c, t4 * c, 0.0, 0.0, 0.0, (double)u * per_unit / (double)(c * wk)};
+                    if (row_mix) {
+                        const int n4 = deal_slices((int)(c * wk), h ? 128 : 64), n6 = (int)(c * wk) - n4;
+                        const int u6 = fu.quant_rows / (h ? 128 : 64);
+                        cut.longest = cut.younger = (double)((k4 / 128 + n4 - 1) / n4) * (h ? 2 : 4);
+                        cut.longest6 = (double)((u6 + n6 - 1) / n6) * 2;
+                        return cut;
+                    }
+                    const WaveRule r = make_wave_rule(u, c, wk, young_pct);
+                    cut.longest = longest_older(r) * per_unit;
+                    cut.younger = longest_younger(r, wk) * per_unit;
+                    if (t6 > 0) {
+                        const long long c6 = t4 == 0 ? (c < limit ? c : limit) : (2 * c <= limit ? 2 * c : (c > limit ? c : limit));
+                        cut.wgs += t6 * c6;
+                        cut.longest6 = longest_older(make_wave_rule(u, c6, wk, young_pct)) * per_unit;
+                    }
+                    return cut;
+                };
+                double best = 0.98 * m16_time(false, cut_of(false, cfg.wk, ks), a.m, g128, mbytes, cus);
+                int best_wk = 0;
+                long long best_ks = 0;
+                for (int wk = 4; wk <= 8; wk += 4)
+                    for (long long c = 1; c <= 12 && c <= prob_k / 128 / wk; c++) {
+                        // (what is not refused or cut back for want of scratch with 128 columns must not be with 64)
+                        if (c > 1 && (size_t)(2 * a.tiles + 2 * a.tiles6) * c * (16 * 64 * sizeof(float)) > scratch_bytes) break;
+                        const double us = m16_time(true, cut_of(true, wk, c), a.m, g128, mbytes, cus);
+                        if (us > 0.0 && us < best) {
+                            best = us;
+                            best_wk = wk;
+                            best_ks = c;
+                        }
+                    }
+                if (best_wk) {
+                    half = true;
+                    units16 = prob_k / 128;
+                    a.groups6 *= 2;
+                    a.groups4 *= 2;
+                    cfg.wk = best_wk;
+                    ks = best_ks;
+                }
+            }
             if (tune.wk16 != kUnset) cfg.wk = tune.wk16 == 8 ? 8 : 4;
             const long long ks_k = ks_units(cfg.wk);
             if (ks > ks_k) ks = ks_k;
             if (sms > 0 && ks > sms) ks = sms;
             if (env_ks >= 1) ks = env_ks;
             if (ks < 1) ks = 1;
-            const size_t slot_bytes = (size_t)cfg.wn * 16 * kTileN * sizeof(float);
+            const size_t slot_bytes = (size_t)cfg.wn * 16 * (half ? kTileN / 2 : kTileN) * sizeof(float);
             if (fixed_scratch && ks > 1 && (size_t)(a.groups4 + 2 * a.groups6) * ks * slot_bytes > scratch_bytes) return FP6M_ERR_SCRATCH;
             while (ks > 1 && (size_t)(a.groups4 + 2 * a.groups6) * ks * slot_bytes > scratch_bytes) ks--;
             a.ks4 = (int)ks;
@@ -1378,15 +1459,15 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                 a.cells = reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(a.scratch) + scratch_bytes);
             if (row_mix) {
                 a.ks6 = 0;                                            // no FP6 column region: groups6 is 0
-                a.slices4 = deal_slices(a.ks4 * cfg.wk);
+                a.slices4 = deal_slices(a.ks4 * cfg.wk, half ? 128 : 64);
                 a.rule[0] = make_rule(k4 / 128, a.slices4);
-                a.rule[1] = make_rule(fu.quant_rows / 64, a.ks4 * cfg.wk - a.slices4);
+                a.rule[1] = make_rule(fu.quant_rows / (half ? 128 : 64), a.ks4 * cfg.wk - a.slices4);
             } else {
-                a.rule[0] = make_rule(units, a.ks4 * cfg.wk);
-                a.rule[1] = make_rule(units, (a.ks6 > 0 ? a.ks6 : 1) * cfg.wk);
-                a.wrule[0] = make_wave_rule(units, a.ks4, cfg.wk, young_pct);
-                a.wrule[1] = make_wave_rule(units, a.ks6 > 0 ? a.ks6 : 1, cfg.wk, young_pct);
-                a.wrule_b = make_wave_rule(units, a.ks4b, cfg.wk, young_pct);
+                a.rule[0] = make_rule(units16, a.ks4 * cfg.wk);
+                a.rule[1] = make_rule(units16, (a.ks6 > 0 ? a.ks6 : 1) * cfg.wk);
+                a.wrule[0] = make_wave_rule(units16, a.ks4, cfg.wk, young_pct);
+                a.wrule[1] = make_wave_rule(units16, a.ks6 > 0 ? a.ks6 : 1, cfg.wk, young_pct);
+                a.wrule_b = make_wave_rule(units16, a.ks4b, cfg.wk, young_pct);
             }
             long long wgs = (long long)a.groups6 * a.ks6 + (long long)a.groups4 * a.ks4 + (long long)a.groups4b * a.ks4b;
             a.div[0] = make_div(a.groups4, wgs);
@@ -1428,9 +1509,17 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             }
             dim3 grid((unsigned)wgs, 1);
             if (tune.verbose)
-                fprintf(stderr, "fp6m_mul m=%d n=%d k=%d: cfg %d (%dx%d waves) groups %d+%d ks4=%d ks6=%d (+ %d tiles in %d parts) gain %.1f grid=%u%s\n", a.m, prob_n,
-                        prob_k, cfg.id, cfg.wn, cfg.wk, a.groups6, a.groups4, a.ks4, a.ks6, a.groups4b, a.ks4b, cls_gain, grid.x, a.xcd_local ? " (tiles placed per XCD)" : "");
-            launch_m16_any(cfg, a, g128, grid, st);
+                fprintf(stderr, "fp6m_mul m=%d n=%d k=%d: cfg %d%s (%dx%d waves) groups %d+%d ks4=%d ks6=%d (+ %d tiles in %d parts) gain %.1f grid=%u%s\n", a.m, prob_n,
+                        prob_k, cfg.id, half ? " half" : "", cfg.wn, cfg.wk, a.groups6, a.groups4, a.ks4, a.ks6, a.groups4b, a.ks4b, cls_gain, grid.x, a.xcd_local ? " (tiles placed per XCD)" : "");
+            if (half) {
+                const bool a8 = a.m <= 8;
+                if (cfg.wk == 8)
+                    cfg.id == 0 ? launch_m16h<4, 8>(a, g128, grid, st) : a8 ? launch_m16h<8, 8>(a, g128, grid, st) : launch_m16h<16, 8>(a, g128, grid, st);
+                else
+                    cfg.id == 0 ? launch_m16h<4, 4>(a, g128, grid, st) : a8 ? launch_m16h<8, 4>(a, g128, grid, st) : launch_m16h<16, 4>(a, g128, grid, st);
+            } else {
+                launch_m16_any(cfg, a, g128, grid, st);
+            }
         } else {
             gather_pass();
             const MbSplit sp = split_mb(mb, mtiles);
@@ -1481,7 +1570,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                 }
             }
             if (row_mix) {
-                a.slices4 = deal_slices(a.ksplit * wk);
+                a.slices4 = deal_slices(a.ksplit * wk, 64);
                 a.rule[0] = make_rule(k4 / 128, a.slices4);
                 a.rule[1] = make_rule(fu.quant_rows / 64, a.ksplit * wk - a.slices4);
             } else {

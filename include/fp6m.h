@@ -168,6 +168,7 @@ int fp6m_mul_rows(const void* A, int lda, const void* B, void* C, const void* s,
  * assumes for the waves of the second / third generation, which sets their chunk lengths), "cap2" (the most chunks per
  * tile that it gives those generations), "young" (per cent: the k slice
  * of the second wave of every SIMD in eight-wave workgroups relative to the first one's; 100 = equal slices),
+ * "half" (the m <= 16 kernel on tiles of 64 columns: 0 never, 1 wherever it can),
  * "cls" (0: the kernels never put the INT4 tiles in two classes -- whole tiles on the first workgroups, the
  * rest in parts on later ones --, 1: wherever they can), "wide" (the many-rows kernel, whose waves lie side by side in n:
  * 0 never, 1 .. 9 with that tile wherever it can: more than 16 rows, k a multiple of 128, n of 256, no row mix, and

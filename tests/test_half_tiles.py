@@ -1,0 +1,156 @@
+"""The m <= 16 kernel on tiles of 64 columns (gemm_m16h.h): its fetch schedule replayed on the CPU, and on the GPU every ring width,
+wave count and protocol forced on the smallest and on ragged problems, against the oracle and, where only the split of the
+columns differs, bit for bit against tiles of 128."""
+import pytest
+import torch
+
+from test_fetch_schedule import Memory
+from test_gemm_gpu import dev, one_hot_case, run
+from test_rows_gpu import run as run_rows
+
+
+def replay(steps, depth, arows, fp6, group, lenient=0):
+    """stream_half: `steps` steps of 64 rows of k (even)."""
+    group = group and not fp6
+    ops = (2 if arows == 16 else 1) + (3 if fp6 else 2)
+    wait = (depth - 2) * ops + (1 if group else 0) + lenient
+    mem, issued, last = Memory(), 0, steps - 1
+
+    def issue(slot, even):
+        nonlocal issued
+        for o in range(ops):
+            mem.load(("step", slot, o), issued)
+        mem.expect(("step", slot, 0), issued)
+        if group and even:
+            place = ("S", (issued >> 1) % 4)
+            if mem.content.get(place, (None,))[0] == issued >> 1:
+                place = ("again", 0)                            # (past the end: the same bytes to where they are already)
+            mem.load(place, issued >> 1)
+            if place[0] == "S":
+                mem.expect(place, issued >> 1)
+        issued = min(issued + 1, last)
+
+    def fetch(step, slot):
+        for o in range(ops):
+            mem.read(("step", slot, o), step)
+
+    slot_in, slot_rd = 0, 1
+    for d in range(depth - 1):
+        issue(slot_in, d % 2 == 0)
+        slot_in = (slot_in + 1) % depth
+    mem.wait(wait)
+    fetch(0, 0)
+    for s in range(0, steps, 2):
+        for u in range(2):
+            issue(slot_in, (u + depth - 1) % 2 == 0)
+            slot_in = (slot_in + 1) % depth
+            mem.wait(wait)
+            if s + u + 1 <= last:
+                fetch(s + u + 1, slot_rd)
+            else:                                               # the look-ahead past the end reads a refetched last step
+                mem.pending_reads.clear()
+            slot_rd = (slot_rd + 1) % depth
+        if group:
+            mem.read(("S", (s >> 1) % 4), s >> 1)
+    mem.wait(0)
+
+
+@pytest.mark.parametrize("arows", [4, 8, 16])
+def test_fetch_schedule(arows):
+    for steps in (2, 4, 6, 8, 14, 32):
+        replay(steps, 4, arows, fp6=False, group=True)
+        replay(steps, 4, arows, fp6=False, group=False)
+        replay(steps, 3, arows, fp6=True, group=False)
+
+
+def test_fetch_schedule_notices_a_lenient_wait():
+    with pytest.raises(AssertionError, match="before its load completed"):
+        replay(16, 4, 16, fp6=False, group=True, lenient=1)
+
+
+# (n, k, quant_cols): one tile of one unit, all FP6, all INT4, ragged numbers of units and tiles
+SHAPES = [(128, 128, -1), (256, 128, 256), (384, 640, 128), (512, 1152, 256), (640, 2048, -1), (256, 1408, 256)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wk", [4, 8])
+@pytest.mark.parametrize("m", [2, 4, 5, 8, 9, 16])
+def test_against_oracle(oracle, m, wk):
+    for n, k, qc in SHAPES:
+        for gs in (-1, 128):
+            for ks in (1, 2, 5):
+                run(oracle, m, n, k, 128, 128, qc=qc, gs=gs, ksplit=ks, env={"FP6M_HALF": 1, "FP6M_WK16": wk})
+    run(oracle, m, 512, 1152, qc=256, gs=128, ksplit=3, env={"FP6M_HALF": 1, "FP6M_XCD": 1})
+    for gs in (-1, 128):
+        one_hot_case(oracle, m, 512, 1152, 256, gs, {"half": 1, "wk16": wk, "ksplit": 2})
+        one_hot_case(oracle, m, 384, 640, 128, gs, {"half": 1, "wk16": wk, "ksplit": 1})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 4, 7, 16])
+def test_row_mix(oracle, m):
+    import fp6_marlin
+    for k, qr in ((512, 256), (1024, 128), (1024 + 896, 896), (256, 128)):
+        for ks in (None, 3):
+            real = fp6_marlin.cabi.tuning
+            try:
+                fp6_marlin.cabi.tuning = lambda **kw: real(half=1, **kw)
+                run_rows(oracle, m, k, 384, qr, ksplit=ks)
+            finally:
+                fp6_marlin.cabi.tuning = real
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 6, 16])
+def test_additions_are_an_exact_reorder_of_the_plain_call(oracle, m):
+    """Column map, bias and residual (in place too) with everything a power of two, so that any order of the sums is exact."""
+    import fp6_marlin
+    n, k, qc = 640, 1152, 128
+    g = torch.Generator().manual_seed(m)
+    from test_gemm_gpu import problem
+    _, B, s = problem(oracle, n, k, qc, 128)
+    A = torch.randn((m, k), generator=g).half().to(dev())
+    c_cols = torch.randperm(n, generator=g).to(torch.int32).to(dev())
+    bias = torch.randn(n, generator=g).half().to(dev())
+    res = torch.randn((m, n), generator=g).half().to(dev())
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    for ks in (1, 3):
+        with fp6_marlin.cabi.tuning(half=1, ksplit=ks):
+            plain = torch.empty((m, n), dtype=torch.half, device=dev())
+            fp6_marlin.mul(A, B, plain, s, ws, qc, group_size=128)
+            mapped = torch.empty_like(plain)
+            fp6_marlin.mul_fused(A, B, mapped, s, ws, qc, 128, c_cols=c_cols)
+            full = torch.empty_like(plain)
+            fp6_marlin.mul_fused(A, B, full, s, ws, qc, 128, c_cols=c_cols, bias=bias, residual=res)
+            inplace = res.clone()
+            fp6_marlin.mul_fused(A, B, inplace, s, ws, qc, 128, c_cols=c_cols, bias=bias, residual=inplace)
+            torch.cuda.synchronize()
+        assert torch.equal(mapped[:, c_cols.long()], plain)
+        assert torch.equal(full, inplace)
+        want = mapped.float() + bias.float() + res.float()       # (mapped is rounded once more: half an ulp of the product)
+        assert ((full.float() - want).abs() <= 2 ** -10 * want.abs() + 2 ** -10 * mapped.float().abs() + 1e-6).all()
+        assert int(ws.abs().sum()) == 0
+
+
+@pytest.mark.gpu
+def test_where_the_narrow_tiles_are_taken(oracle, capfd):
+    """Both sides of the choice, and what keeps calls on 128 columns: k or quant_rows not in whole 128 rows, one counter per tile."""
+    import fp6_marlin
+
+    def takes(m, n, k, qc=256, gs=128, max_par=16, **kw):
+        _, B, s = None, torch.zeros(k * n // 8 + k * max(qc, 0) // 16, dtype=torch.int32, device=dev()), \
+            torch.zeros((k // 128 if gs == 128 else 1) * (n - max(qc, 0)) + max(qc, 0), dtype=torch.half, device=dev())
+        A = torch.zeros((m, k), dtype=torch.half, device=dev())
+        C = torch.full((m, n), float("nan"), dtype=torch.half, device=dev())
+        ws = torch.zeros(n // 128 * max_par, dtype=torch.int32, device=dev())
+        capfd.readouterr()
+        with fp6_marlin.cabi.tuning(verbose=1):
+            fp6_marlin.mul(A, B, C, s, ws, qc, max_par=max_par, group_size=gs, **kw)
+            torch.cuda.synchronize()
+        assert int(C.count_nonzero()) == 0 and int(ws.abs().sum()) == 0
+        return " half " in capfd.readouterr().err
+
+    assert takes(16, 4096, 4096) and takes(5, 15360, 5120) and takes(8, 4096, 11008) and takes(2, 4096, 4096)
+    assert not takes(16, 8192, 8192, gs=-1) and not takes(8, 28672, 6144)
+    assert not takes(16, 4096, 4096, max_par=1) and takes(2, 4096, 4096, max_par=1)
+    assert not takes(16, 4096, 4096 + 64, gs=-1, thread_k=64, thread_n=256) and not takes(16, 4096, 4096, sms=2)
