@@ -1200,9 +1200,9 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             // split is bounded so that every wave keeps at least one k unit, partial-sum traffic stays
             // well below the weight stream and the partial tiles fit the scratch.
             M16Config cfg = m16_config(a.m);
-            // 64-column tiles (gemm_m16h.h): k and the segments of a row mix in whole 128 rows, words in reference order, and for up
-            // to four rows the cells, beyond twice the counters in `workspace`.
-            const bool half_fits = prob_k % 128 == 0 && fu.quant_rows % 128 == 0 && !a.native &&
+            // 64-column tiles (gemm_m16h.h): k and the segments of a row mix in whole 128 rows, and for up to four rows the cells,
+            // beyond twice the counters in `workspace`.
+            const bool half_fits = prob_k % 128 == 0 && fu.quant_rows % 128 == 0 &&
                                    (a.m <= 4 ? tune.cells == kUnset && (size_t)prob_n * 16 * sizeof(unsigned long long) <= kCellBytes : max_par >= 2);
             bool half = tune.half == 1 && half_fits;
             int units16 = half ? prob_k / 128 : units;                  // rows of the weight in units that slices are made of

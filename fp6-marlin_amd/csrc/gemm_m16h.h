@@ -53,11 +53,14 @@ __device__ __forceinline__ void stream_half(const Args& p, const TileInfo& ti, i
     const PlaneGeometry geo = plane_geometry(p, ti);
     const size_t row4 = geo.row4, row2 = geo.row2;
     const int lg = lane & 31;
-    const uint32_t v4 = (uint32_t)((lane >> 5) * row4) + (lg ^ ((lg >> 3) & 3)) * 16;
+    // (gfx950 order: owner 4 l + i lies at granule 16 i + 8 sigma + l of the 128-column tile, so this half is four whole lines
+    // of every k-block; granules of the 2-bit plane are loaded in pairs, and so stay in that order in the ring)
+    const int o4 = lg ^ ((lg >> 3) & 3);
+    const uint32_t v4 = (uint32_t)((lane >> 5) * row4) + (p.native ? 16 * (o4 & 3) + (o4 >> 2) : o4) * 16;
     const unsigned char* base4 = reinterpret_cast<const unsigned char*>(FP6 ? p.b_fp6_4 : p.b_int4) + geo.tile4 +
-                                 512 * sigma + (size_t)(4 * step_begin) * row4;
-    const uint32_t v2 = (uint32_t)((lane >> 4) * row2) + (lane & 15) * 16;
-    const unsigned char* base2 = reinterpret_cast<const unsigned char*>(p.b_fp6_2) + geo.tile2 + 256 * sigma +
+                                 (p.native ? 128 : 512) * sigma + (size_t)(4 * step_begin) * row4;
+    const uint32_t v2 = (uint32_t)((lane >> 4) * row2) + (p.native ? 128 * ((lane >> 2) & 3) + 16 * (lane & 3) : 16 * (lane & 15));
+    const unsigned char* base2 = reinterpret_cast<const unsigned char*>(p.b_fp6_2) + geo.tile2 + (p.native ? 64 : 256) * sigma +
                                  (size_t)(4 * step_begin) * row2;
     // A: as in stream_tile, a slot per step
     const bool a_lane = AROWS >= 8 || lane < 32;
@@ -99,7 +102,7 @@ __device__ __forceinline__ void stream_half(const Args& p, const TileInfo& ti, i
     const int owner = 4 * l + i;
     const uint32_t ring_lds = lds_addr(ring);
     const uint32_t rd4 = ring_lds + (owner ^ ((owner >> 3) & 3)) * 16 + 8 * b;
-    const uint32_t rd2 = ring_lds + 2048 + owner * 8 + 4 * b;
+    const uint32_t rd2 = ring_lds + 2048 + (p.native ? 8 * i + l : owner) * 8 + 4 * b;
     const int ar = c & (AROWS - 1);                       // rows beyond AROWS re-read a valid row; their sums are never stored
     uint32_t rda[4];
 #pragma unroll
@@ -406,8 +409,7 @@ __device__ __forceinline__ void wg_finish_half(const GemmArgs& p, const TileInfo
     if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Workgroups and their k slices as in gemm_m16_kernel; a group is a 64-column tile (groups6 / groups4 count those).  Reference-order
-// words only.
+// Workgroups and their k slices as in gemm_m16_kernel; a group is a 64-column tile (groups6 / groups4 count those).
 template <bool G128, int AROWS, int WK, int D4, int D6, bool CELLS, bool EXTRAS, bool LOCAL = false>
 __global__ __launch_bounds__(64 * WK, WK == 8 || AROWS > 4 ? 2 : 3) void gemm_m16h_kernel(const GemmArgs args)
 {
@@ -417,10 +419,10 @@ __global__ __launch_bounds__(64 * WK, WK == 8 || AROWS > 4 ? 2 : 3) void gemm_m1
     __shared__ __attribute__((aligned(16))) unsigned char smem[WK * kWaveLds + 16];
 
     GemmArgs p = args;
-    p.native = 0;
     if constexpr (!EXTRAS) {
         p.k4 = 0;
         p.slices4 = 0;
+        p.native = 0;
         p.fused = 0;
         p.c_cols = nullptr;
         p.bias = nullptr;

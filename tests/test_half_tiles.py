@@ -154,3 +154,30 @@ def test_where_the_narrow_tiles_are_taken(oracle, capfd):
     assert not takes(16, 8192, 8192, gs=-1) and not takes(8, 28672, 6144)
     assert not takes(16, 4096, 4096, max_par=1) and takes(2, 4096, 4096, max_par=1)
     assert not takes(16, 4096, 4096 + 64, gs=-1, thread_k=64, thread_n=256) and not takes(16, 4096, 4096, sms=2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [2, 7, 16])
+def test_gfx950_order_gives_the_same_bits(oracle, m):
+    """Words in either order through tiles of 64 columns: the smallest tile, ragged units, all FP6, FP6 rows."""
+    import fp6_marlin
+    from test_repack_layout import gpu_case
+    for wk in (4, 8):
+        for ks in (1, 3):
+            env = {"FP6M_HALF": 1, "FP6M_WK16": wk, "FP6M_KSPLIT": ks}
+            gpu_case(oracle, m, 128, 256, 128, 128, env)
+            gpu_case(oracle, m, 1152, 640, 256, -1, env)
+            gpu_case(oracle, m, 640, 256, 256, -1, env)
+    import numpy as np
+    k, n, qr = 1024 + 384, 384, 384
+    ref, b, s = oracle.gen_row_mix_weight(np.random.default_rng(m).normal(0, 0.02, (k, n)).astype(np.float16), qr)
+    B, sd = torch.from_numpy(b).to(dev()), torch.from_numpy(s).to(dev())
+    Bn = fp6_marlin.repack_gfx950(B, k, n, quant_rows=qr)
+    A = torch.randn((m, k), generator=torch.Generator().manual_seed(m)).half().to(dev())
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    out = [torch.empty((m, n), dtype=torch.half, device=dev()) for _ in range(2)]
+    with fp6_marlin.cabi.tuning(half=1, ksplit=2):
+        fp6_marlin.mul_rows(A, B, out[0], sd, ws, qr)
+        fp6_marlin.mul_rows(A, Bn, out[1], sd, ws, qr, layout="gfx950")
+        torch.cuda.synchronize()
+    assert torch.equal(*out) and oracle.rel_err(out[0].cpu().numpy(), oracle.matmul_ref(A.cpu().numpy(), ref)) <= 1e-3
