@@ -23,6 +23,7 @@
 //
 // gemm_common.h  argument block, tile bookkeeping, load / wait / dequantisation helpers
 // gemm_sk.h      gemm_sk_kernel (one row: the decode kernel)
+// gemm_m1.h      gemm_m1_kernel (one row, tiles of 64 columns; the choice between the two: m1_plan.h)
 // gemm_m16.h     gemm_m16_kernel (m <= 16)
 // gemm_m16h.h    gemm_m16h_kernel (m <= 16, tiles of 64 columns; the choice between the two: m16_plan.h)
 // gemm_mb.h      gemm_mb_kernel (16 < m)
@@ -38,10 +39,12 @@
 #include "gemm_common.h"
 #include "gemm_m16.h"
 #include "gemm_m16h.h"
+#include "gemm_m1.h"
 #include "gemm_sk.h"
 #include "gemm_mb.h"
 #include "gemm_wide.h"
 #include "m16_plan.h"
+#include "m1_plan.h"
 
 namespace fp6m {
 
@@ -70,7 +73,7 @@ thread_local int g_last_hip_error = 0;
 constexpr int kUnset = INT32_MIN;
 const int g_env_verbose = getenv("FP6M_VERBOSE") ? 1 : 0;
 struct Tuning {
-    int mb = kUnset, ksplit = kUnset, wk16 = kUnset, wk = kUnset, pair = kUnset, wgs = kUnset, share = kUnset, share6 = kUnset, sk = kUnset, cap = kUnset, gather = kUnset, cells = kUnset, xcd = kUnset, gen = kUnset, gen2 = kUnset, gen3 = kUnset, young = kUnset, cls = kUnset, cus = kUnset, cap2 = kUnset, wide = kUnset, half = kUnset;
+    int mb = kUnset, ksplit = kUnset, wk16 = kUnset, wk = kUnset, pair = kUnset, wgs = kUnset, share = kUnset, share6 = kUnset, sk = kUnset, cap = kUnset, gather = kUnset, cells = kUnset, xcd = kUnset, gen = kUnset, gen2 = kUnset, gen3 = kUnset, young = kUnset, cls = kUnset, cus = kUnset, cap2 = kUnset, wide = kUnset, half = kUnset, m1 = kUnset;
     int verbose = g_env_verbose;
 };
 Tuning g_tuning;
@@ -422,6 +425,17 @@ void launch_m16h(const GemmArgs& a, bool g128, dim3 grid, hipStream_t stream)
         g128 ? launch_m16h_one<true, AROWS, WK, false>(a, grid, stream) : launch_m16h_one<false, AROWS, WK, false>(a, grid, stream);
 }
 
+template <int WK, int D4>
+void launch_m1(const M1Args& a, bool g128, bool staged, dim3 grid, hipStream_t stream)
+{
+    const bool extras = a.a_cols || a.c_cols || a.bias || a.residual || a.native;
+    void (*kernel)(const M1Args) =
+        staged ? (g128 ? gemm_m1_kernel<true, WK, D4, 3, true, true> : gemm_m1_kernel<false, WK, D4, 3, true, true>)
+        : extras ? (g128 ? gemm_m1_kernel<true, WK, D4, 3, true, false> : gemm_m1_kernel<false, WK, D4, 3, true, false>)
+                 : (g128 ? gemm_m1_kernel<true, WK, D4, 3, false, false> : gemm_m1_kernel<false, WK, D4, 3, false, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * WK), 0, stream, a);
+}
+
 template <bool G128, int MB, int D4, int D6, int WK, bool PAIR, bool LEAN>
 void launch_mb_one(const GemmArgs& a, dim3 grid, hipStream_t stream)
 {
@@ -601,7 +615,7 @@ int fp6m_tuning_set(const char* knob, int value)
     if (!strcmp(knob, "wide") && (value < 0 || value > fp6m::kWidePlanCount)) return FP6M_ERR_ARG;
     const struct { const char* name; int* field; } knobs[] = {
         {"mb", &g_tuning.mb}, {"ksplit", &g_tuning.ksplit},
-        {"wk16", &g_tuning.wk16}, {"half", &g_tuning.half}, {"wk", &g_tuning.wk}, {"pair", &g_tuning.pair}, {"wgs", &g_tuning.wgs}, {"share", &g_tuning.share}, {"share6", &g_tuning.share6}, {"cap", &g_tuning.cap}, {"sk", &g_tuning.sk}, {"gather", &g_tuning.gather}, {"cells", &g_tuning.cells}, {"xcd", &g_tuning.xcd}, {"gen", &g_tuning.gen}, {"gen2", &g_tuning.gen2}, {"gen3", &g_tuning.gen3}, {"young", &g_tuning.young}, {"cls", &g_tuning.cls}, {"cus", &g_tuning.cus}, {"cap2", &g_tuning.cap2}, {"wide", &g_tuning.wide},
+        {"wk16", &g_tuning.wk16}, {"half", &g_tuning.half}, {"m1", &g_tuning.m1}, {"wk", &g_tuning.wk}, {"pair", &g_tuning.pair}, {"wgs", &g_tuning.wgs}, {"share", &g_tuning.share}, {"share6", &g_tuning.share6}, {"cap", &g_tuning.cap}, {"sk", &g_tuning.sk}, {"gather", &g_tuning.gather}, {"cells", &g_tuning.cells}, {"xcd", &g_tuning.xcd}, {"gen", &g_tuning.gen}, {"gen2", &g_tuning.gen2}, {"gen3", &g_tuning.gen3}, {"young", &g_tuning.young}, {"cls", &g_tuning.cls}, {"cus", &g_tuning.cus}, {"cap2", &g_tuning.cap2}, {"wide", &g_tuning.wide},
         {"verbose", &g_tuning.verbose}};
     for (const auto& k : knobs)
         if (!strcmp(knob, k.name)) {
@@ -907,6 +921,72 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             hipLaunchKernelGGL(gather_a_kernel, ggrid, dim3(256), 0, st, a.A, fu.lda, fu.a_cols, sc.gathered, prob_k);
             a.A = sc.gathered;
         };
+
+        // One row on tiles of 64 columns (gemm_m1.h), by estimated time: whole units of 128 rows, addresses that 16-byte loads to
+        // LDS take (of the scales too, which the other kernels load four bytes at a time), and cells for every column.  (Against `sk_time` with 3 % to its favour 13 of
+        // the 789 shapes are slower than before, one of them by 8 %, eleven by 1-4 %; the rest 12 % faster on average.)
+        if (prob_m == 1 && !row_mix && prob_k % 128 == 0 && tune.m1 != 0 && (size_t)prob_n * sizeof(unsigned long long) <= kCellBytes &&
+            ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(s)) & 15) == 0) {
+            const int u = prob_k / 128;
+            M1Plan plan{0, 0, 0, 0, 0, 0.0};
+            if (tune.m1 == 3 || tune.m1 == 4) {                        // (forced: ring, waves, parts)
+                plan.depth = tune.m1;
+                plan.wk = tune.wk16 == 4 ? 4 : 8;
+                plan.ks4 = env_ks >= 1 ? env_ks : 1;
+                plan.ks6 = tune.share6 != kUnset && tune.share6 > 0 ? tune.share6 : plan.ks4;
+                if (plan.ks4 <= kMaxParts && plan.ks6 <= kMaxParts && m1_slices(u, plan.wk, plan.ks4, plan.ks6, n4 > 0, qc > 0, young_pct).fit)
+                    plan.us = 1.0;
+            } else if (tune.sk == kUnset && tune.half == kUnset && tune.wk16 == kUnset && tune.cells == kUnset && tune.xcd == kUnset && tune.cls == kUnset &&
+                       tune.wgs == kUnset && tune.cap == kUnset && tune.share == kUnset && tune.share6 == kUnset && tune.gen == kUnset &&
+                       tune.gen2 == kUnset && tune.gen3 == kUnset && tune.cap2 == kUnset && env_ks < 1 && sms <= 0 && u >= 8) {
+                plan = m1_plan(u, n4, qc, g128, cus, young_pct);
+                if (plan.us > 0.97 * sk_time(u, n4, qc, g128)) plan.us = 0.0;
+            }
+            if (plan.us > 0.0) {
+                const bool gather_inside = fu.a_cols && tune.gather != 0;
+                if (!gather_inside) gather_pass();
+                M1Args d;
+                d.A = a.A;
+                d.b_int4 = a.b_int4;
+                d.b_fp6_2 = a.b_fp6_2;
+                d.b_fp6_4 = a.b_fp6_4;
+                d.s_int4 = a.s_int4;
+                d.s_fp6 = a.s_fp6;
+                d.C = a.C;
+                d.cells = reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(a.scratch) + scratch_bytes);
+                d.n4 = n4;
+                d.qc = qc;
+                d.groups6 = qc / 64;
+                d.groups4 = n4 / 64;
+                d.ks6 = (int)plan.ks6;
+                d.ks4 = (int)plan.ks4;
+                d.rule6 = make_wave_rule(u, plan.ks6, plan.wk, young_pct);
+                d.rule4 = make_wave_rule(u, plan.ks4, plan.wk, young_pct);
+                const long long wgs = d.groups6 * plan.ks6 + d.groups4 * plan.ks4;
+                d.div6 = make_div(d.groups6 > 0 ? d.groups6 : 1, wgs);
+                d.div4 = make_div(d.groups4 > 0 ? d.groups4 : 1, wgs);
+                d.c_cols = a.c_cols;
+                d.bias = a.bias;
+                d.residual = a.residual;
+                d.n = prob_n;
+                d.native = a.native;
+                d.a_cols = gather_inside ? fu.a_cols : nullptr;
+                d.lda = fu.lda;
+                d.tile4 = (size_t)(prob_k / 16) * 1024;
+                d.tile2 = (size_t)(prob_k / 16) * 512;
+                if (tune.verbose)
+                    fprintf(stderr, "fp6m_mul m=1 n=%d k=%d: 64-column tiles, %d waves, ring of %d, ks4=%d ks6=%d grid=%lld (%.1f us, else %.1f)\n", prob_n, prob_k,
+                            plan.wk, plan.depth, d.ks4, d.ks6, wgs, plan.us, sk_time(u, n4, qc, g128));
+                // (the gather from a staged row: where the row fits, in whole 16 bytes, and no third workgroup shares a CU)
+                const bool staged = d.a_cols && 2LL * fu.lda <= kM1RowBytes && fu.lda % 8 == 0 && wgs <= (plan.wk == 8 ? 1LL : 2LL) * cus;
+                const dim3 grid((unsigned)wgs);
+                if (plan.wk == 8)
+                    plan.depth == 3 ? launch_m1<8, 3>(d, g128, staged, grid, st) : launch_m1<8, 4>(d, g128, staged, grid, st);
+                else
+                    plan.depth == 3 ? launch_m1<4, 3>(d, g128, staged, grid, st) : launch_m1<4, 4>(d, g128, staged, grid, st);
+                continue;
+            }
+        }
 
         const long long traffic_cap = (long long)prob_k / (64LL * a.m) > 0 ? (long long)prob_k / (64LL * a.m) : 1;
         if (mb == 1 && !row_mix && (tune.sk != kUnset ? tune.sk != 0 && a.m <= 4 : a.m == 1) && prob_k / 64 < 65536 && (long long)a.tiles * (prob_k / 64) < (1 << 24) &&

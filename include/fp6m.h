@@ -119,7 +119,7 @@ int fp6m_repack_gfx950(const int32_t* in, int32_t* out, size_t k, size_t n, int 
  * any bias / residual addition to separate kernels of the caller.
  *   A, lda    device fp16 [m, lda] row-major.  Without a_cols, lda must equal prob_k.
  *   a_cols    device int32 [prob_k] or NULL: row kk of the packed weight multiplies column a_cols[kk] of A
- *             (0 <= a_cols[kk] < lda).  With one row the decode kernel fetches A through the map itself; otherwise a
+ *             (0 <= a_cols[kk] < lda).  With one row the decode kernels fetch A through the map themselves; otherwise a
  *             pass of its own gathers the rows into a 64 MiB buffer of the call's workspace, which the first call with a_cols
  *             allocates; min(prob_m, 64 * max_par) * prob_k * 2 bytes must fit (else FP6M_ERR_ARG).
  *   c_cols    device int32 [prob_n] or NULL: packed column j (INT4 columns first, then the FP6 columns) is written
@@ -169,6 +169,7 @@ int fp6m_mul_rows(const void* A, int lda, const void* B, void* C, const void* s,
  * tile that it gives those generations), "young" (per cent: the k slice
  * of the second wave of every SIMD in eight-wave workgroups relative to the first one's; 100 = equal slices),
  * "half" (the m <= 16 kernel on tiles of 64 columns: 0 never, 1 wherever it can),
+ * "m1" (one row on tiles of 64 columns: 0 never, 3 / 4 with a ring of that many steps in "ksplit" and "share6" parts),
  * "cls" (0: the kernels never put the INT4 tiles in two classes -- whole tiles on the first workgroups, the
  * rest in parts on later ones --, 1: wherever they can), "wide" (the many-rows kernel, whose waves lie side by side in n:
  * 0 never, 1 .. 9 with that tile wherever it can: more than 16 rows, k a multiple of 128, n of 256, no row mix, and

@@ -1,0 +1,107 @@
+"""One row on tiles of 64 columns (gemm_m1.h): every ring, wave count and number of k parts forced on the smallest and on ragged problems,
+against the oracle; both word orders, the additions, and which calls take it."""
+import pytest
+import torch
+
+from test_gemm_gpu import dev, one_hot_case, problem, run
+from test_repack_layout import gpu_case
+
+# (n, k, quant_cols): one tile of one unit of 128 rows, all FP6, all INT4, waves without a slice, ragged slices, the longest slice
+SHAPES = [(128, 128, -1), (256, 128, 256), (384, 640, 128), (512, 1152, 256), (640, 2048, -1), (256, 1408, 256), (256, 4096, 128)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wk", [4, 8])
+@pytest.mark.parametrize("depth", [3, 4])
+def test_against_oracle(oracle, depth, wk):
+    for n, k, qc in SHAPES:
+        for gs in (-1, 128):
+            for ks, ks6 in ((1, 1), (1, 3), (2, 2), (5, 8)):
+                run(oracle, 1, n, k, 128, 128, qc=qc, gs=gs, ksplit=ks, env={"FP6M_M1": depth, "FP6M_WK16": wk, "FP6M_SHARE6": ks6})
+    for gs in (-1, 128):
+        for ks in (1, 3):
+            one_hot_case(oracle, 1, 512, 1152, 256, gs, {"m1": depth, "wk16": wk, "ksplit": ks})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gs", [-1, 128])
+def test_gfx950_order_gives_the_same_bits(oracle, gs):
+    for ks in (1, 3):
+        env = {"FP6M_M1": 3, "FP6M_WK16": 4, "FP6M_KSPLIT": ks}
+        for k, n, qc in ((128, 256, 128), (1152, 640, 256), (640, 256, 256)):
+            gpu_case(oracle, 1, k, n, qc, gs, env)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ks", [1, 3])
+def test_additions(oracle, ks):
+    """Column map, bias and residual (in place too) are added in float32 and rounded once."""
+    import fp6_marlin
+    n, k, qc = 640, 1152, 128
+    g = torch.Generator().manual_seed(ks)
+    _, B, s = problem(oracle, n, k, qc, 128)
+    A = torch.randn((1, k), generator=g).half().to(dev())
+    c_cols = torch.randperm(n, generator=g).to(torch.int32).to(dev())
+    bias, res = torch.randn(n, generator=g).half().to(dev()), torch.randn((1, n), generator=g).half().to(dev())
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    plain, mapped, full = (torch.empty((1, n), dtype=torch.half, device=dev()) for _ in range(3))
+    with fp6_marlin.cabi.tuning(m1=4, ksplit=ks):
+        fp6_marlin.mul(A, B, plain, s, ws, qc, group_size=128)
+        fp6_marlin.mul_fused(A, B, mapped, s, ws, qc, 128, c_cols=c_cols)
+        fp6_marlin.mul_fused(A, B, full, s, ws, qc, 128, c_cols=c_cols, bias=bias, residual=res)
+        inplace = res.clone()
+        fp6_marlin.mul_fused(A, B, inplace, s, ws, qc, 128, c_cols=c_cols, bias=bias, residual=inplace)
+        torch.cuda.synchronize()
+    assert torch.equal(mapped[:, c_cols.long()], plain) and torch.equal(full, inplace)
+    want = mapped.float() + bias.float() + res.float()           # (mapped is rounded once more: half an ulp of the product)
+    assert ((full.float() - want).abs() <= 2 ** -10 * want.abs() + 2 ** -10 * mapped.float().abs() + 1e-6).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("more", [40, 41, 11000])
+@pytest.mark.parametrize("k", [128, 640, 2048, 4096])
+def test_gather_is_an_exact_reorder(oracle, k, more):
+    """Slices of two steps to the longest, among them ones that end inside a group of four; entries out of range are clamped.
+    Rows that are staged in LDS, and rows that are too long or not in whole 16 bytes."""
+    import fp6_marlin
+    n, qc, lda = 512, 256, k + more
+    _, B, s = problem(oracle, n, k, qc, 128)
+    g = torch.Generator().manual_seed(k)
+    A = torch.randn((1, lda), generator=g).half().to(dev())
+    cols = torch.randperm(lda, generator=g)[:k].to(torch.int32)
+    cols[0], cols[k - 1] = -5, lda + 3
+    cols = cols.to(dev())
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    for wk in (4, 8):
+        for ks in (1, 3):
+            out = [torch.full((1, n), float("nan"), dtype=torch.half, device=dev()) for _ in range(2)]
+            with fp6_marlin.cabi.tuning(m1=3, wk16=wk, ksplit=ks):
+                fp6_marlin.mul(A[:, cols.long().clamp(0, lda - 1)].contiguous(), B, out[0], s, ws, qc, group_size=128)
+                fp6_marlin.mul_fused(A, B, out[1], s, ws, qc, 128, a_cols=cols)
+                torch.cuda.synchronize()
+            assert torch.equal(*out)
+
+
+@pytest.mark.gpu
+def test_which_calls_take_it(oracle, capfd):
+    """Both sides of the estimate; k not in whole 128 rows, scales off their 16 bytes, and `sms` stay with the other kernel."""
+    import fp6_marlin
+
+    def takes(n, k, qc=256, gs=128, shift=0, **kw):
+        n6 = max(qc, 0)
+        B = torch.zeros(k * (n - n6) // 8 + k * n6 * 3 // 16, dtype=torch.int32, device=dev())
+        s = torch.zeros((k // 128 if gs == 128 else 1) * (n - n6) + n6 + shift, dtype=torch.half, device=dev())[shift:]
+        A = torch.zeros((1, k), dtype=torch.half, device=dev())
+        C = torch.full((1, n), float("nan"), dtype=torch.half, device=dev())
+        ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+        capfd.readouterr()
+        with fp6_marlin.cabi.tuning(verbose=1):
+            fp6_marlin.mul(A, B, C, s, ws, qc, group_size=gs, **kw)
+            torch.cuda.synchronize()
+        assert int(C.count_nonzero()) == 0
+        return "64-column tiles" in capfd.readouterr().err
+
+    assert takes(4096, 4096) and takes(12288, 4096) and takes(8192, 8192) and takes(4096, 11008, gs=-1)
+    assert not takes(57344, 8192) and not takes(4096, 512)
+    assert not takes(4096, 4096 + 64, gs=-1, thread_k=64, thread_n=256) and not takes(4096, 4096, sms=2)
+    assert not takes(4096, 4096, shift=2)
