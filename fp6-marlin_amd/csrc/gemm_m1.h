@@ -50,20 +50,6 @@ constexpr int kM1ABytes = kM1Steps * 128;
 constexpr int kM1ScaleBytes = kM1Steps / 2 * 128;         // group scales of a slice; or the tile's column scales
 constexpr int m1_wave_lds(int d4, int d6) { return max3(d4 * 2048, d6 * 3072, 0) + kM1ABytes + kM1ScaleBytes; }
 
-// At most `newer` steps of OPS loads each outstanding.
-template <int OPS, int MOST>
-__device__ __forceinline__ void wait_steps(int newer)
-{
-    if constexpr (MOST == 0) {
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-    } else {
-        if (newer >= MOST)
-            __builtin_amdgcn_s_waitcnt(vmcnt_only(OPS * MOST));
-        else
-            wait_steps<OPS, MOST - 1>(newer);
-    }
-}
-
 // One wave's slice: `steps` (even, 2 .. kM1Steps) steps of 64 rows of a 64-column tile.  base4 / base2: the slice's first k-block
 // of the planes, row4 / row2: bytes between k-blocks; base_gs: the slice's first group's scales, gs_row bytes apart.  `native`:
 // gfx950 order (see stream_half).
@@ -140,7 +126,7 @@ __device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t r
     for (int d = 0; d < DEPTH - 1; d++)
         if (d < steps) issue();
     if (gather.map) {
-        wait_steps<kOps, DEPTH - 1>(issued);              // (and this wave's piece of the staged row)
+        wait_steps<kOps, false, false, DEPTH - 1>(issued);              // (and this wave's piece of the staged row)
         if (STAGED) __builtin_amdgcn_s_barrier();         // (every wave of the workgroup passes one: see the kernel)
         some([&](int t) {
             asm volatile("" : "+v"(entry[t]));
@@ -221,7 +207,7 @@ __device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t r
     };
 
     Regs regs[2];
-    wait_steps<kOps, DEPTH - 2>(issued - 1);
+    wait_steps<kOps, false, false, DEPTH - 2>(issued - 1);
     fetch(regs[0]);
     f4 grp[4];
 #pragma unroll 1
@@ -229,7 +215,7 @@ __device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t r
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             if (issued < steps) issue();                          // step s+u+DEPTH-1, to the slot that step s+u-1 was read from
-            wait_steps<kOps, DEPTH - 2>(issued - (s + u + 2));    // step s+u+1 has landed (past the end: all has)
+            wait_steps<kOps, false, false, DEPTH - 2>(issued - (s + u + 2));    // step s+u+1 has landed (past the end: all has)
             fetch(regs[(u + 1) & 1]);                             // (past the end: bytes that nobody uses)
             __builtin_amdgcn_s_waitcnt(lgkmcnt_only(kReads));     // reads of step s+u (older) are done
             settle(regs[u & 1]);

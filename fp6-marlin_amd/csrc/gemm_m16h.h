@@ -16,8 +16,10 @@ namespace fp6m {
 // A step is 64 rows of k: four k-blocks of 512 bytes (FP6: + 4 x 256), as many bytes as 32 rows of 128 columns, and one whole
 // 128-byte line of every row of A; slices are whole pairs of steps.  Lane 16 i + 8 b + l reads words 2b and 2b + 1 of fragment
 // owner 4 l + i from the ring, so that fragment (jp, half) is columns 32 b + 16 jp + 8 half + l of the tile.  Order of a step's
-// loads: A, words, group scales (every other step); past a slice's end the last ones are repeated, so the counts of the waits
-// never change.
+// loads: A, words, group scales (every other step).  Nothing is fetched past a slice's end, the waits go by the steps that are
+// still to land: repeating the last step instead, so that their counts never change, was three steps more on slices of four to
+// eight (5 x 5120 x 15360 9.9 -> 9.1 us, 8 x 11008 x 4096 10.1 -> 9.7).  A ring of three steps, better for one row (gemm_m1.h), is
+// up to 15 % slower here (16 x 4096 x 12288 9.5 -> 11.1).
 struct HalfRegs {
     u2 q[4];            // words of the four k-blocks
     uint32_t t[4];      // FP6 2-bit plane
@@ -26,18 +28,31 @@ struct HalfRegs {
 constexpr int kHalfStride = 64 + 4;                          // floats per row of the reduction slab
 constexpr int kHalfScaleSlabs = 4;                           // groups of two steps, fetched up to three steps ahead
 
+// At most `newer` steps of OPS loads each outstanding, with one load more (group scales) in the first, third, .. (EVEN) or the
+// second, fourth, .. of them; MOST: the most there can be.
+template <int OPS, bool GROUP, bool EVEN, int MOST>
+__device__ __forceinline__ void wait_steps(int newer)
+{
+    if constexpr (MOST == 0) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+    } else {
+        if (newer >= MOST)
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(OPS * MOST + (GROUP ? (MOST + (EVEN ? 1 : 0)) / 2 : 0)));
+        else
+            wait_steps<OPS, GROUP, EVEN, MOST - 1>(newer);
+    }
+}
+
 template <bool FP6, bool G128, int DEPTH, int AROWS, typename Args>
 __device__ __forceinline__ void stream_half(const Args& p, const TileInfo& ti, int sigma, unsigned char* ring,
                                             int step_begin, int step_end, f4 (&acc)[4])
 {
     static_assert(DEPTH >= 3, "needs two steps of look-ahead");
     constexpr bool kGroup = G128 && !FP6;                 // group scales apply to INT4 tiles only
-    static_assert(!kGroup || DEPTH == 4, "one load of group scales among the two newer steps of every wait");
     constexpr int kPair = pair_bytes(AROWS);
     constexpr int kSlot = FP6 ? 3072 : 2048;              // a step's packed words
     constexpr int kAOps = AROWS == 16 ? 2 : 1;
     constexpr int kOps = kAOps + (FP6 ? 3 : 2);           // direct-to-LDS loads per step
-    constexpr int kWait = (DEPTH - 2) * kOps + (kGroup ? 1 : 0);
     constexpr int kReads = FP6 ? 16 : 12;                 // LDS reads per step
     const int lane = threadIdx.x & 63;
     const int i = lane >> 4, c = lane & 15, b = c >> 3, l = c & 7;
@@ -78,8 +93,7 @@ __device__ __forceinline__ void stream_half(const Args& p, const TileInfo& ti, i
     const uint32_t vgs = 4 * lg;                          // (128 bytes, twice: a tile's scales end where the region may end)
     unsigned char* gs_ring = a_ring + DEPTH * kPair;
 
-    int issued = step_begin;                              // next step to fetch (clamped at the last one)
-    const int last = step_end - 1;
+    int issued = step_begin;                              // next step to fetch
     auto issue = [&](int slot, bool even) {
         unsigned char* dst = ring + slot * kSlot;
         unsigned char* adst = a_ring + slot * kPair;
@@ -90,12 +104,10 @@ __device__ __forceinline__ void stream_half(const Args& p, const TileInfo& ti, i
         if (FP6) dma16_stream(base2 + v2, dst + 2048);
         if (kGroup && even)
             dma4(base_gs + (size_t)(issued >> 1) * p.n4 * 2 + vgs, gs_ring + ((issued >> 1) & (kHalfScaleSlabs - 1)) * 256);
-        if (issued < last) {                              // uniform: pointers move on the scalar unit
-            issued++;
-            base4 += 4 * row4;
-            base2 += 4 * row2;
-            base_a += 128;
-        }
+        issued++;                                         // uniform: pointers move on the scalar unit
+        base4 += 4 * row4;
+        base2 += 4 * row2;
+        base_a += 128;
     };
 
     // ---- read side (lane = MFMA identity)
@@ -160,13 +172,13 @@ __device__ __forceinline__ void stream_half(const Args& p, const TileInfo& ti, i
 
     int slot_in = 0;
 #pragma unroll
-    for (int d = 0; d < DEPTH - 1; d++) {
-        issue(slot_in, (d & 1) == 0);
-        slot_in = slot_in + 1 == DEPTH ? 0 : slot_in + 1;
-    }
+    for (int d = 0; d < DEPTH - 1; d++)
+        if (issued < step_end) {                          // (two steps at least)
+            issue(slot_in, (d & 1) == 0);
+            slot_in = slot_in + 1 == DEPTH ? 0 : slot_in + 1;
+        }
     HalfRegs regs[2];
-    // (the same count for the first step: of the two newer steps of the prologue one is even as well)
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(kWait));
+    wait_steps<kOps, kGroup, false, DEPTH - 2>(issued - step_begin - 1);
     FP6M_MARK(p, 1);
     fetch(regs[0], 0);
     int slot_rd = 1;                                      // slot of the step whose LDS reads come next
@@ -175,9 +187,14 @@ __device__ __forceinline__ void stream_half(const Args& p, const TileInfo& ti, i
     for (int s = step_begin; s < step_end; s += 2) {
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            issue(slot_in, ((u + DEPTH - 1) & 1) == 0);
-            slot_in = slot_in + 1 == DEPTH ? 0 : slot_in + 1;
-            __builtin_amdgcn_s_waitcnt(vmcnt_only(kWait));                // step s+u+1 has landed
+            if (issued < step_end) {
+                issue(slot_in, ((u + DEPTH - 1) & 1) == 0);
+                slot_in = slot_in + 1 == DEPTH ? 0 : slot_in + 1;
+            }
+            if (u == 0)                                                   // step s+u+1 has landed (past the end: all has)
+                wait_steps<kOps, kGroup, true, DEPTH - 2>(issued - (s + 2));
+            else
+                wait_steps<kOps, kGroup, false, DEPTH - 2>(issued - (s + 3));
             fetch(regs[(u + 1) & 1], slot_rd);
             slot_rd = slot_rd + 1 == DEPTH ? 0 : slot_rd + 1;
             __builtin_amdgcn_s_waitcnt(lgkmcnt_only(kReads < 15 ? kReads : 15));   // reads of step s+u (older) are done
@@ -206,7 +223,7 @@ __device__ __forceinline__ void stream_half(const Args& p, const TileInfo& ti, i
             }
         }
     }
-    // Redundant tail prefetches and look-ahead reads may still be in flight; the epilogue reuses the ring.
+    // The look-ahead past the end reads bytes that nobody uses, and may still be in flight; the epilogue reuses the ring.
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0) & lgkmcnt_only(0));
     settle(regs[0]);
     if (FP6) {

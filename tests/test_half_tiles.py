@@ -13,22 +13,22 @@ def replay(steps, depth, arows, fp6, group, lenient=0):
     """stream_half: `steps` steps of 64 rows of k (even)."""
     group = group and not fp6
     ops = (2 if arows == 16 else 1) + (3 if fp6 else 2)
-    wait = (depth - 2) * ops + (1 if group else 0) + lenient
-    mem, issued, last = Memory(), 0, steps - 1
+    mem, issued = Memory(), 0
 
     def issue(slot, even):
         nonlocal issued
+        assert even == (issued % 2 == 0)
         for o in range(ops):
             mem.load(("step", slot, o), issued)
         mem.expect(("step", slot, 0), issued)
         if group and even:
-            place = ("S", (issued >> 1) % 4)
-            if mem.content.get(place, (None,))[0] == issued >> 1:
-                place = ("again", 0)                            # (past the end: the same bytes to where they are already)
-            mem.load(place, issued >> 1)
-            if place[0] == "S":
-                mem.expect(place, issued >> 1)
-        issued = min(issued + 1, last)
+            mem.load(("S", (issued >> 1) % 4), issued >> 1)
+            mem.expect(("S", (issued >> 1) % 4), issued >> 1)
+        issued += 1
+
+    def wait(newer, even):                                      # wait_steps
+        newer = max(0, min(newer, depth - 2))
+        mem.wait(ops * newer + ((newer + even) // 2 if group else 0) + (lenient if newer else 0))
 
     def fetch(step, slot):
         for o in range(ops):
@@ -36,18 +36,20 @@ def replay(steps, depth, arows, fp6, group, lenient=0):
 
     slot_in, slot_rd = 0, 1
     for d in range(depth - 1):
-        issue(slot_in, d % 2 == 0)
-        slot_in = (slot_in + 1) % depth
-    mem.wait(wait)
+        if issued < steps:
+            issue(slot_in, d % 2 == 0)
+            slot_in = (slot_in + 1) % depth
+    wait(issued - 1, 0)
     fetch(0, 0)
     for s in range(0, steps, 2):
         for u in range(2):
-            issue(slot_in, (u + depth - 1) % 2 == 0)
-            slot_in = (slot_in + 1) % depth
-            mem.wait(wait)
-            if s + u + 1 <= last:
+            if issued < steps:
+                issue(slot_in, (u + depth - 1) % 2 == 0)
+                slot_in = (slot_in + 1) % depth
+            wait(issued - (s + u + 2), 1 - u)
+            if s + u + 1 < steps:
                 fetch(s + u + 1, slot_rd)
-            else:                                               # the look-ahead past the end reads a refetched last step
+            else:                                               # the look-ahead past the end reads what nobody uses
                 mem.pending_reads.clear()
             slot_rd = (slot_rd + 1) % depth
         if group:
