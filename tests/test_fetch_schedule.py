@@ -13,8 +13,8 @@ issue order, as the counter assumes):
 * a wait never names more loads than can be in flight (a 6-bit counter).
 
 Restated from the kernels: the order of loads inside a step's batch, where the load of group scales goes, the counts of
-newer_step_ops / kWaitOdd / kWaitEven / the +1 for group scales, the slot rotation, the clamped redundant fetches past
-the end.  The GPU tests run the compiled loops themselves.
+newer_step_ops / kWaitOdd / kWaitEven / the +1 for group scales, the slot rotation, and what happens past the end: fetches
+of the last step again, or none and waits that know it.  The GPU tests run the compiled loops themselves.
 """
 import itertools
 
@@ -66,7 +66,7 @@ def run_m16(steps, depth, arows, fp6, group):
     wait_even = newer_step_ops(word_ops, a_ops, 0, depth - 2)
     mem = Memory()
     state = dict(issued=0, pairs_issued=0, pair_in=0)
-    last, last_pair = steps - 1, steps // 2 - 1
+    last = steps - 1
 
     def issue(slot, even):
         step = state["issued"]
@@ -76,8 +76,7 @@ def run_m16(steps, depth, arows, fp6, group):
                 mem.load(("A", state["pair_in"], o), ("A", pair))
             mem.expect(("A", state["pair_in"], 0), ("A", pair))
             state["pair_in"] = (state["pair_in"] + 1) % pair_slots
-            if state["pairs_issued"] < last_pair:
-                state["pairs_issued"] += 1
+            state["pairs_issued"] += 1
         for w in range(word_ops):
             mem.load(("W", slot, w), ("W", step))
         mem.expect(("W", slot, 0), ("W", step))
@@ -85,8 +84,7 @@ def run_m16(steps, depth, arows, fp6, group):
         if scales:
             mem.load(("S", (step // 4) % 2), ("S", step // 4))
             mem.expect(("S", (step // 4) % 2), ("S", step // 4))
-        if state["issued"] < last:
-            state["issued"] += 1
+        state["issued"] += 1
         return scales
 
     def fetch(step, slot, pair_slot):
@@ -99,24 +97,30 @@ def run_m16(steps, depth, arows, fp6, group):
 
     slot_in = 0
     for d in range(depth - 1):
-        issue(slot_in, d % 2 == 0)
-        slot_in = (slot_in + 1) % depth
-    mem.wait(wait_odd)
+        if d < 2 or state["issued"] < steps:
+            issue(slot_in, d % 2 == 0)
+            slot_in = (slot_in + 1) % depth
+    mem.wait(word_ops if depth == 4 and steps == 2 else wait_odd)
     fetch(0, 0, 0)
     slot_rd, pair_rd, scales_in_flight = 1, 0, False
     for s in range(0, steps, unroll):
         for u in range(unroll):
-            scales = issue(slot_in, (u + depth - 1) % 2 == 0)
-            slot_in = (slot_in + 1) % depth
+            more, scales = state["issued"] < steps, False
+            if more:
+                scales = issue(slot_in, (u + depth - 1) % 2 == 0)
+                slot_in = (slot_in + 1) % depth
             if group and u == 1:
                 scales_in_flight = scales
             one_more = group and u in (1, 2) and scales_in_flight
-            mem.wait((wait_odd if u % 2 else wait_even) + (1 if one_more else 0))
+            if more:
+                mem.wait((wait_odd if u % 2 else wait_even) + (1 if one_more else 0))
+            else:
+                mem.wait(word_ops if depth == 4 and steps - (s + u) == 3 else 0)
             if u % 2:
                 pair_rd = (pair_rd + 1) % pair_slots
             if s + u + 1 <= last:
                 fetch(s + u + 1, slot_rd, pair_rd)
-            else:                                                # the look-ahead past the end reads a refetched last step
+            else:                                                # the look-ahead past the end reads what nobody uses
                 mem.pending_reads.clear()
             slot_rd = (slot_rd + 1) % depth
         if group:
@@ -232,6 +236,7 @@ def run_mb_paired(steps, group, mb=4):
     mem = Memory()
     state = dict(issued=0, pairs_issued=0, a_slot=0)
     last, last_pair = steps - 1, steps // 2 - 1
+    repeat = mb == 8                                              # the last pair again past the end; otherwise nothing
 
     def issue_a():
         pair = state["pairs_issued"]
@@ -239,7 +244,7 @@ def run_mb_paired(steps, group, mb=4):
             mem.load(("A", state["a_slot"], q), ("A", pair))
         mem.expect(("A", state["a_slot"], 0), ("A", pair))
         state["a_slot"] ^= 1
-        if state["pairs_issued"] < last_pair:
+        if not repeat or state["pairs_issued"] < last_pair:
             state["pairs_issued"] += 1
 
     def issue_w(reg_set):
@@ -251,7 +256,7 @@ def run_mb_paired(steps, group, mb=4):
         for w in range(w_ops):
             mem.load(("W", reg_set, w), ("W", step))
         mem.expect(("W", reg_set, 0), ("W", step))
-        if state["issued"] < last:
+        if not repeat or state["issued"] < last:
             state["issued"] += 1
         return scales
 
@@ -276,10 +281,13 @@ def run_mb_paired(steps, group, mb=4):
     for s in range(0, steps, unroll):
         for u in range(unroll):
             step = s + u
-            scales = issue_w(u & 1)
-            if u % 2 == 0:
-                issue_a()
-            mem.wait(a_ops + w_ops + (1 if (u % 2 == 0 and scales) else 0))
+            if repeat or u + 2 < unroll or s + unroll < steps:
+                scales = issue_w(u & 1)
+                if u % 2 == 0:
+                    issue_a()
+                mem.wait(a_ops + w_ops + (1 if (u % 2 == 0 and scales) else 0))
+            else:
+                mem.wait(0)
             nxt = step + 1
             if group and u == unroll - 1 and nxt <= last:
                 mem.read(("S", (nxt // 4) % 2), ("S", nxt // 4))
