@@ -23,6 +23,8 @@ struct M16Cut {
 // 64-column tiles are taken on 55 % of those shapes; the choice is 1 % behind the best of all measured splits, 9.5 % faster than 128-column
 // tiles alone, and three of 650 lost (the worst 3 %).  us: 16 x 4096 x 4096 8.5 -> 7.1, 5 x 5120 x 15360 12.7 -> 10.6,
 // 8 x 11008 x 4096 11.2 -> 9.9, 16 x 2816 x 2304 9.3 -> 6.4; 16 x 8192 x 8192 keeps 128 columns (12.3, 13.1 with 64).
+// Fitted before either kernel stopped fetching past the end of a slice, which took 1 to 9 % off both; on fourteen shapes the choice is
+// still within 1.5 % of the best forced split.
 struct M16Time {
     // us once; once with a split, per part, and per part and row; per step of the longest slice, of the mean one, of the mean one
     // at full occupation, per row that A is fetched in, and with group scales; per step by which 1.7 FP6 steps exceed an INT4
