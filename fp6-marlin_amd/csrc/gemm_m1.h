@@ -11,7 +11,7 @@ namespace fp6m {
 // tile has several k parts these meet in its cells, one atomic per column and workgroup.  gemm_sk_kernel cuts a tile of 128
 // columns into one-wave workgroups and pays a returning atomic per column and wave, eight to thirty times as many, and a
 // thousand workgroups to dispatch; it keeps the problems that are not resident here at once (m1_plan.h).
-// us in a graph, one-wave workgroups -> this: 4096 x 4096 5.8 -> 5.2, 4096 x 12288 8.7 -> 7.4, 4096 x 22016 12.2 -> 11.5,
+// us in a graph, one-wave workgroups -> this: 4096 x 4096 5.8 -> 5.2, 4096 x 12288 8.7 -> 7.4,
 // 11008 x 4096 8.3 -> 7.8, 8192 x 8192 10.5 -> 9.5, 24192 x 2048 12.6 -> 7.5; 789 random shapes 12 % on average.
 //
 // What bounds it is the launch (3 us), then requests in flight -- where more is worse: a CU with eight waves wants two or three
