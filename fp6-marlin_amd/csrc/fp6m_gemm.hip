@@ -411,7 +411,7 @@ template <bool G128, int AROWS, int WK, bool EXTRAS>
 void launch_m16h_one(const GemmArgs& a, dim3 grid, hipStream_t stream)
 {
     void (*kernel)(const GemmArgs) = gemm_m16h_kernel<G128, AROWS, WK, 4, 3, AROWS == 4, EXTRAS>;
-    if constexpr (AROWS > 4 && WK == 4) {
+    if constexpr (m16h_has_local(AROWS, WK)) {
         if (a.xcd_local) kernel = gemm_m16h_kernel<G128, AROWS, WK, 4, 3, false, EXTRAS, true>;
     }
     hipLaunchKernelGGL(kernel, grid, dim3(64 * WK), 0, stream, a);
@@ -1567,6 +1567,9 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             bool want_local = cfg.wk == 4 && a.ks4 > 1;
             if (tune.xcd != kUnset) want_local = tune.xcd != 0;
             if (a.groups4b > 0) want_local = false;
+            // (64-column tiles in eight-wave workgroups have no such build: the surplus workgroups of a padded grid would be parts
+            // beyond the last one)
+            if (half && !m16h_has_local(16, cfg.wk)) want_local = false;
             if (want_local && cfg.id == 1 && cfg.wn == 1 && !a.cells && xcd_placement == 1 && (a.ks4 > 1 || a.ks6 > 1) &&
                 a.ks4 <= kMaxLocalParts && a.ks6 <= kMaxLocalParts) {
                 long long most = 0;

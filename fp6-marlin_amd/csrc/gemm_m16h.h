@@ -426,11 +426,15 @@ __device__ __forceinline__ void wg_finish_half(const GemmArgs& p, const TileInfo
     if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Which builds there are with tiles placed per XCD (LOCAL): only they may be given the padded grid of such a launch.
+constexpr bool m16h_has_local(int arows, int wk) { return arows > 4 && wk == 4; }
+
 // Workgroups and their k slices as in gemm_m16_kernel; a group is a 64-column tile (groups6 / groups4 count those).
 template <bool G128, int AROWS, int WK, int D4, int D6, bool CELLS, bool EXTRAS, bool LOCAL = false>
 __global__ __launch_bounds__(64 * WK, WK == 8 || AROWS > 4 ? 2 : 3) void gemm_m16h_kernel(const GemmArgs args)
 {
     static_assert(!LOCAL || !CELLS, "the cells are atomics, which have no XCD-local form");
+    static_assert(!LOCAL || m16h_has_local(AROWS, WK), "a build that the dispatcher does not know of");
     constexpr int kWaveLds = half_wave_lds_bytes(D4, D6, AROWS);
     static_assert(WK * kWaveLds + 16 <= 160 * 1024, "LDS of one CU");
     __shared__ __attribute__((aligned(16))) unsigned char smem[WK * kWaveLds + 16];

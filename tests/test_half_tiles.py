@@ -89,6 +89,19 @@ def test_against_oracle(oracle, m, wk):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [5, 8, 16])
+def test_placement_per_xcd_only_where_it_is_built(oracle, capfd, m):
+    """Ten tiles of 64 columns in two parts are 20 workgroups; placed per XCD the grid is padded to 32.  Workgroups of eight waves
+    have no build that knows the twelve surplus ones, whatever is asked for."""
+    for wk, placed in ((8, False), (4, True)):
+        capfd.readouterr()
+        run(oracle, m, 640, 2048, qc=-1, gs=128, ksplit=2, thread_k=128, thread_n=128,
+            env={"FP6M_HALF": 1, "FP6M_XCD": 1, "FP6M_WK16": wk, "FP6M_VERBOSE": 1})
+        err = capfd.readouterr().err
+        assert f" half (1x{wk} waves)" in err and ("placed per XCD" in err) == placed and ("grid=20" in err) == (not placed), err
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 4, 7, 16])
 def test_row_mix(oracle, m):
     import fp6_marlin
