@@ -1510,12 +1510,16 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             if (sms > 0 && ks > sms) ks = sms;
             if (env_ks >= 1) ks = env_ks;
             if (ks < 1) ks = 1;
+            // (up to four rows 64-column tiles meet in cells alone, which count to kMaxParts)
+            const bool cells_only = half && a.m <= 4;
+            if (cells_only && ks > kMaxParts) ks = kMaxParts;
             const size_t slot_bytes = (size_t)cfg.wn * 16 * (half ? kTileN / 2 : kTileN) * sizeof(float);
             if (fixed_scratch && ks > 1 && (size_t)(a.groups4 + 2 * a.groups6) * ks * slot_bytes > scratch_bytes) return FP6M_ERR_SCRATCH;
             while (ks > 1 && (size_t)(a.groups4 + 2 * a.groups6) * ks * slot_bytes > scratch_bytes) ks--;
             a.ks4 = (int)ks;
             a.ks6 = (int)ks6_of(ks, cfg.wk);
             if (sms > 0 && a.ks6 > sms) a.ks6 = sms;
+            if (cells_only && a.ks6 > kMaxParts) a.ks6 = kMaxParts;
             while (a.ks6 > ks && slots_used(ks, a.ks6, a.groups4, a.groups6, 1) * slot_bytes > scratch_bytes) a.ks6--;   // (ks == 1: not looked at above)
             if (cls_na > 0) {
                 const long long c6 = a.groups6 ? ks6_of(1, 4) : 0, nb = a.groups4 - cls_na;

@@ -102,6 +102,17 @@ def test_placement_per_xcd_only_where_it_is_built(oracle, capfd, m):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [2, 4])
+def test_no_more_parts_than_the_cells_count(oracle, capfd, m):
+    """Up to four rows these tiles have no way to meet but the cells, whose count of arrivals ends at 255."""
+    for ks, want in ((300, "ks4=255 ks6=255"), (255, "ks4=255 ks6=255"), (254, "ks4=254 ks6=254")):
+        capfd.readouterr()
+        run(oracle, m, 256, 640, 128, 128, qc=128, gs=128, ksplit=ks, env={"FP6M_HALF": 1, "FP6M_VERBOSE": 1})
+        err = capfd.readouterr().err
+        assert " half " in err and want in err, err
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [1, 4, 7, 16])
 def test_row_mix(oracle, m):
     import fp6_marlin
