@@ -428,7 +428,7 @@ void launch_m16h(const GemmArgs& a, bool g128, dim3 grid, hipStream_t stream)
 template <int WK, int D4>
 void launch_m1(const M1Args& a, bool g128, bool staged, dim3 grid, hipStream_t stream)
 {
-    const bool extras = a.a_cols || a.c_cols || a.bias || a.residual || a.native;
+    const bool extras = a.c_cols || a.bias || a.residual || a.native;
     void (*kernel)(const M1Args) =
         staged ? (g128 ? gemm_m1_kernel<true, WK, D4, 3, true, true> : gemm_m1_kernel<false, WK, D4, 3, true, true>)
         : extras ? (g128 ? gemm_m1_kernel<true, WK, D4, 3, true, false> : gemm_m1_kernel<false, WK, D4, 3, true, false>)
@@ -943,9 +943,15 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                 plan = m1_plan(u, n4, qc, g128, cus, young_pct);
                 if (plan.us > 0.95 * sk_time(u, n4, qc, g128)) plan.us = 0.0;
             }
+            // The gather: from a staged row, where the row fits, in whole 16 bytes, and no third workgroup shares a CU.  Any other
+            // stays with the one-wave kernel, which gathers from memory once per 128 columns: gathered here, once per 64, 11008 of
+            // 27392 x 4096 took 12.4 us against 9.3 there, 28672 x 4096 20.8 against 17.4, 2048 of 18432 x 24192 11.5 against 9.4.
+            const long long wgs = qc / 64 * plan.ks6 + n4 / 64 * plan.ks4;
+            const bool staged = fu.a_cols && tune.gather != 0 && 2LL * fu.lda <= kM1RowBytes && fu.lda % 8 == 0 &&
+                                wgs <= (plan.wk == 8 ? 1LL : 2LL) * cus;
+            if (fu.a_cols && !staged && tune.gather != 0 && tune.m1 == kUnset) plan.us = 0.0;
             if (plan.us > 0.0) {
-                const bool gather_inside = fu.a_cols && tune.gather != 0;
-                if (!gather_inside) gather_pass();
+                if (!staged) gather_pass();
                 M1Args d;
                 d.A = a.A;
                 d.b_int4 = a.b_int4;
@@ -963,7 +969,6 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                 d.ks4 = (int)plan.ks4;
                 d.rule6 = make_wave_rule(u, plan.ks6, plan.wk, young_pct);
                 d.rule4 = make_wave_rule(u, plan.ks4, plan.wk, young_pct);
-                const long long wgs = d.groups6 * plan.ks6 + d.groups4 * plan.ks4;
                 d.div6 = make_div(d.groups6 > 0 ? d.groups6 : 1, wgs);
                 d.div4 = make_div(d.groups4 > 0 ? d.groups4 : 1, wgs);
                 d.c_cols = a.c_cols;
@@ -971,15 +976,13 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                 d.residual = a.residual;
                 d.n = prob_n;
                 d.native = a.native;
-                d.a_cols = gather_inside ? fu.a_cols : nullptr;
+                d.a_cols = staged ? fu.a_cols : nullptr;
                 d.lda = fu.lda;
                 d.tile4 = (size_t)(prob_k / 16) * 1024;
                 d.tile2 = (size_t)(prob_k / 16) * 512;
                 if (tune.verbose)
                     fprintf(stderr, "fp6m_mul m=1 n=%d k=%d: 64-column tiles, %d waves, ring of %d, ks4=%d ks6=%d grid=%lld (%.1f us, else %.1f)\n", prob_n, prob_k,
                             plan.wk, plan.depth, d.ks4, d.ks6, wgs, plan.us, sk_time(u, n4, qc, g128));
-                // (the gather from a staged row: where the row fits, in whole 16 bytes, and no third workgroup shares a CU)
-                const bool staged = d.a_cols && 2LL * fu.lda <= kM1RowBytes && fu.lda % 8 == 0 && wgs <= (plan.wk == 8 ? 1LL : 2LL) * cus;
                 const dim3 grid((unsigned)wgs);
                 if (plan.wk == 8)
                     plan.depth == 3 ? launch_m1<8, 3>(d, g128, staged, grid, st) : launch_m1<8, 4>(d, g128, staged, grid, st);

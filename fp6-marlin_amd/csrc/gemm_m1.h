@@ -53,14 +53,13 @@ constexpr int m1_wave_lds(int d4, int d6) { return max3(d4 * 2048, d6 * 3072, 0)
 // One wave's slice: `steps` (even, 2 .. kM1Steps) steps of 64 rows of a 64-column tile.  base4 / base2: the slice's first k-block
 // of the planes, row4 / row2: bytes between k-blocks; base_gs: the slice's first group's scales, gs_row bytes apart.  `native`:
 // gfx950 order (see stream_half).
-// The gather costs a cycle of the CU's address unit per element where the values come from memory (11008 x 4096: 2.6 us on
-// 7.7); from LDS, which the workgroup has its CU's waves fetch the whole row to with a few wide loads, next to nothing.
+// STAGED: with the gather, from a row that the workgroup has fetched to LDS whole with a few wide loads.  (From memory it costs a
+// cycle of the CU's address unit per element, 11008 x 4096 2.6 us on 7.7; from LDS next to nothing.)
 constexpr int kM1RowBytes = 28 * 1024;                    // two workgroups of four waves still share a CU
 struct M1Gather {
-    const int32_t* map;       // of the slice's rows of k; null: A is in order already
-    const uint16_t* A;
+    const int32_t* map;       // of the slice's rows of k
     int lda;
-    uint32_t row_lds;         // the staged row, where there is one
+    uint32_t row_lds;         // the staged row
 };
 template <bool FP6, bool GROUP, int DEPTH, bool STAGED>
 __device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t row4, const unsigned char* base2, uint32_t row2,
@@ -107,7 +106,7 @@ __device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t r
                 for (int t = t0; t < t0 + 4; t++) f(t);
             }
     };
-    if (gather.map) {
+    if constexpr (STAGED) {
         const uint32_t last = 64u * steps - 1;            // (past the slice's end: its last row again)
         some([&](int t) {
             const uint32_t row = 64u * t + lane;
@@ -125,22 +124,16 @@ __device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t r
 #pragma unroll
     for (int d = 0; d < DEPTH - 1; d++)
         if (d < steps) issue();
-    if (gather.map) {
+    if constexpr (STAGED) {
         wait_steps<kOps, false, false, DEPTH - 1>(issued);              // (and this wave's piece of the staged row)
-        if (STAGED) __builtin_amdgcn_s_barrier();         // (every wave of the workgroup passes one: see the kernel)
+        __builtin_amdgcn_s_barrier();                     // (every wave of the workgroup passes one: see the kernel)
         some([&](int t) {
             asm volatile("" : "+v"(entry[t]));
             int col = (int)entry[t];
             col = col < 0 ? 0 : (col >= gather.lda ? gather.lda - 1 : col);
-            if (STAGED)
-                asm volatile("ds_read_u16 %0, %1" : "=&v"(entry[t]) : "v"(gather.row_lds + 2u * (uint32_t)col) : "memory");
-            else
-                asm volatile("global_load_ushort %0, %1, %2" : "=&v"(entry[t]) : "v"(2u * (uint32_t)col), "s"(gather.A) : "memory");
+            asm volatile("ds_read_u16 %0, %1" : "=&v"(entry[t]) : "v"(gather.row_lds + 2u * (uint32_t)col) : "memory");
         });
-        if (STAGED)
-            __builtin_amdgcn_s_waitcnt(lgkmcnt_only(0));
-        else
-            __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+        __builtin_amdgcn_s_waitcnt(lgkmcnt_only(0));
         some([&](int t) {
             asm volatile("" : "+v"(entry[t]));
             asm volatile("ds_write_b16 %0, %1" : : "v"(lds_addr(a_lds) + 128 * t + 2 * lane), "v"(entry[t]) : "memory");
@@ -250,7 +243,7 @@ __device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t r
     }
 }
 
-// EXTRAS: the build with map, bias, residual, gather and gfx950 order.  STAGED: with the gather from a staged row.
+// EXTRAS: the build with map, bias, residual and gfx950 order.  STAGED: with the gather as well.
 template <bool G128, int WK, int D4, int D6, bool EXTRAS, bool STAGED>
 __global__ __launch_bounds__(64 * WK, 2) void gemm_m1_kernel(const M1Args p)
 {
@@ -297,8 +290,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_m1_kernel(const M1Args p)
     if (steps > 0) {
         const unsigned char* base_a = reinterpret_cast<const unsigned char*>(p.A) + 256 * (size_t)unit;
         const bool native = EXTRAS && p.native != 0;
-        const M1Gather gather = {EXTRAS && p.a_cols ? p.a_cols + 128 * (size_t)unit : nullptr, p.A, EXTRAS ? p.lda : 0,
-                                 lds_addr(smem + WK * kWaveLds)};
+        const M1Gather gather = {STAGED ? p.a_cols + 128 * (size_t)unit : nullptr, STAGED ? p.lda : 0, lds_addr(smem + WK * kWaveLds)};
         const size_t at4 = native ? (group >> 1) * p.tile4 + 128 * (group & 1) : 512 * (size_t)group;
         const size_t at2 = native ? (group >> 1) * p.tile2 + 64 * (group & 1) : 256 * (size_t)group;
         if (fp6) {

@@ -105,3 +105,28 @@ def test_which_calls_take_it(oracle, capfd):
     assert not takes(57344, 8192) and not takes(4096, 512)
     assert not takes(4096, 4096 + 64, gs=-1, thread_k=64, thread_n=256) and not takes(4096, 4096, sms=2)
     assert not takes(4096, 4096, shift=2)
+
+
+@pytest.mark.gpu
+def test_a_gather_that_no_staged_row_serves_stays_with_the_one_wave_kernel(oracle, capfd):
+    """Gathered from memory, 64-column tiles were up to a third slower than one-wave workgroups: rows longer than the slab, rows
+    not in whole 16 bytes, and launches whose workgroups share a CU by threes."""
+    import fp6_marlin
+
+    def takes(n, k, lda, qc=256, gs=128):
+        B = torch.zeros(k * (n - qc) // 8 + k * qc * 3 // 16, dtype=torch.int32, device=dev())
+        s = torch.zeros((k // 128 if gs == 128 else 1) * (n - qc) + qc, dtype=torch.half, device=dev())
+        A = torch.zeros((1, lda), dtype=torch.half, device=dev())
+        C = torch.full((1, n), float("nan"), dtype=torch.half, device=dev())
+        ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+        cols = torch.arange(k - 1, -1, -1, dtype=torch.int32, device=dev())
+        capfd.readouterr()
+        with fp6_marlin.cabi.tuning(verbose=1):
+            fp6_marlin.mul_fused(A, B, C, s, ws, qc, gs, a_cols=cols)
+            torch.cuda.synchronize()
+        assert int(C.count_nonzero()) == 0
+        return "64-column tiles" in capfd.readouterr().err
+
+    assert takes(4096, 11008, 11008) and takes(12288, 4096, 4104) and takes(8192, 8192, 14336)
+    assert not takes(4096, 11008, 11009) and not takes(8192, 8192, 14344) and not takes(24192, 2048, 18432)
+    assert not takes(4096, 28672, 28672) and not takes(40960, 2048, 2048)
