@@ -940,8 +940,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             } else if (tune.sk == kUnset && tune.half == kUnset && tune.wk16 == kUnset && tune.cells == kUnset && tune.xcd == kUnset && tune.cls == kUnset &&
                        tune.wgs == kUnset && tune.cap == kUnset && tune.share == kUnset && tune.share6 == kUnset && tune.gen == kUnset &&
                        tune.gen2 == kUnset && tune.gen3 == kUnset && tune.cap2 == kUnset && env_ks < 1 && sms <= 0 && u >= 8) {
-                plan = m1_plan(u, n4, qc, g128, cus, young_pct);
-                if (plan.us > 0.95 * sk_time(u, n4, qc, g128)) plan.us = 0.0;
+                plan = m1_choice(u, n4, qc, g128, cus, young_pct);
             }
             // The gather: from a staged row, where the row fits, in whole 16 bytes, and no third workgroup shares a CU.  Any other
             // stays with the one-wave kernel, which gathers from memory once per 128 columns: gathered here, once per 64, 11008 of

@@ -50,6 +50,19 @@ constexpr M1Time kM1Time[2][4] = {
      {3.074, 0.738, 0.0032, 0.275, 0.0, 0.168, 0.233, 0.1046, 0.0640, 0.341},
      {2.819, 0.868, 0.0210, 0.341, 0.0, 0.547, 0.298, 0.0968, 0.0917, 0.0},
      {3.103, 0.489, 0.0182, 0.041, 0.188, 0.472, 0.368, 0.0595, 0.0487, 5.588}}};
+// The same for FP6 columns alone, which have one ring (7900 launches, every cut of 1016 shapes, k = 1024 .. 28672, n = 1024 ..
+// 48000: 2-4 %).  By the entries above, which charge parts and slices of INT4 tiles, 116 of those shapes were more than 2 % slower
+// than with the one-wave kernel (3712 x 9216 10.5 us against 9.2); by these none is, nor any of 1208 calls at other random shapes.
+constexpr M1Time kM1TimeFp6[4] = {{2.808, 0.528, 0.0105, 0.667, 0.0, 0.161, 0.0, 0.0469, 0.0, 0.0},
+                                  {3.344, 0.742, 0.0, 0.650, 0.0, 0.172, 0.0, 0.0852, 0.0, 3.719},
+                                  {2.980, 1.126, 0.0072, 0.739, 0.0, 1.114, 0.0, 0.0606, 0.0, 0.286},
+                                  {3.248, 0.518, 0.0146, 0.349, 0.304, 0.392, 0.0, 0.0559, 0.0, 9.641}};
+
+inline double m1_time(const M1Time& t, long long ks, int longest, int younger, double mean, double over6, double mbytes, bool g128, double edge)
+{
+    return t.start + (ks > 1 ? t.split : 0.0) + t.part * ks + t.longest * longest + t.younger * younger + t.mean * mean +
+           t.fp6 * (over6 > 0.0 ? over6 : 0.0) + t.mbytes * mbytes + (g128 ? t.group * longest : 0.0) + t.edge * (edge > 0.0 ? edge : 0.0);
+}
 
 // The best cut of one row over k = 128 * units, n4 INT4 and qc FP6 columns that is resident at once: one workgroup of eight waves
 // or three of four per CU.
@@ -58,32 +71,37 @@ inline M1Plan m1_plan(int units, long long n4, long long qc, bool g128, int cus,
     M1Plan best{0, 0, 0, 0, 0, 0.0};
     const double mbytes = 128.0 * units * (n4 * 0.5 + qc * 0.75) * 1e-6;
     for (int wk = 4; wk <= 8; wk += 4)
-        for (long long ks4 = 1; ks4 <= 16 && ks4 * wk <= units; ks4++)
-            for (int fine = 1; fine <= (qc ? 2 : 1); fine++) {
-                const long long ks6 = fine * ks4, wgs = n4 / 64 * ks4 + qc / 64 * ks6;
+        for (long long ks = 1; ks <= (n4 ? 16 : 24) && ks * wk <= units; ks++)
+            for (int fine = 1; fine <= (n4 && qc ? 2 : 1); fine++) {
+                const long long ks6 = fine * ks, wgs = n4 / 64 * ks + qc / 64 * ks6;
                 if (ks6 * wk > units || wgs > (wk == 8 ? 1LL : 3LL) * cus) continue;
-                const M1Slices s = m1_slices(units, wk, ks4, ks6, n4 > 0, qc > 0, young_pct);
+                const M1Slices s = m1_slices(units, wk, ks, ks6, n4 > 0, qc > 0, young_pct);
                 if (!s.fit) continue;
-                const long long edge = (wk == 8 ? cus : 2LL * cus) - cus / 16;
-                for (int four = 0; four < 2; four++) {
-                    const M1Time& t = kM1Time[four][wk == 8 ? 3 : (int)((wgs - 1) / cus)];
-                    double us = t.start + t.part * ks4 + t.longest * s.longest4 + t.younger * s.younger4 +
-                                t.mean * units / (double)(ks4 * wk) + t.mbytes * mbytes;
-                    if (ks4 > 1) us += t.split;
-                    if (g128) us += t.group * s.longest4;
-                    if (1.7 * s.longest6 > s.longest4) us += t.fp6 * (1.7 * s.longest6 - s.longest4);
-                    if (wgs > edge) us += t.edge * (wgs - edge) / (double)cus;
-                    if (best.us == 0.0 || us < best.us) best = M1Plan{3 + four, wk, ks4, ks6, wgs, us};
+                const double edge = (wgs - ((wk == 8 ? cus : 2LL * cus) - cus / 16)) / (double)cus, mean = units / (double)(ks * wk);
+                const int where = wk == 8 ? 3 : (int)((wgs - 1) / cus);
+                for (int four = 0; four < (n4 ? 2 : 1); four++) {
+                    const double us = n4 ? m1_time(kM1Time[four][where], ks, s.longest4, s.younger4, mean, 1.7 * s.longest6 - s.longest4, mbytes, g128, edge)
+                                         : m1_time(kM1TimeFp6[where], ks, s.longest6, s.younger6, mean, 0.0, mbytes, false, edge);
+                    if (best.us == 0.0 || us < best.us) best = M1Plan{3 + four, wk, ks, ks6, wgs, us};
                 }
             }
     return best;
 }
 
-// The same of gemm_sk_kernel's launch (the same shapes, to 4 %).
+// The same of gemm_sk_kernel's launch (the same shapes, to 4-5 %).
 inline double sk_time(int units, long long n4, long long qc, bool g128)
 {
     const double mbytes = 128.0 * units * (n4 * 0.5 + qc * 0.75) * 1e-6, tiles = (n4 + qc) / 128.0;
+    if (n4 == 0) return 4.352 + 0.1634 * mbytes + 0.0051 * units + 0.00224 * tiles + 0.1331 * units / tiles;
     return 4.137 + (g128 ? 0.1656 : 0.1511) * mbytes + 0.0061 * units + 0.00116 * tiles + 0.1546 * units / tiles + 0.0261 * qc / 256.0;
+}
+
+// The plan that is taken in place of gemm_sk_kernel; us = 0: none.
+inline M1Plan m1_choice(int units, long long n4, long long qc, bool g128, int cus, int young_pct)
+{
+    M1Plan plan = m1_plan(units, n4, qc, g128, cus, young_pct);
+    if (plan.us > 0.95 * sk_time(units, n4, qc, g128)) plan.us = 0.0;
+    return plan;
 }
 
 }  // namespace fp6m

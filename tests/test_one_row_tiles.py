@@ -1,5 +1,9 @@
 """One row on tiles of 64 columns (gemm_m1.h): every ring, wave count and number of k parts forced on the smallest and on ragged problems,
-against the oracle; both word orders, the additions, and which calls take it."""
+against the oracle; both word orders, the additions, and which calls take it (the estimate, m1_plan.h, also by itself on the CPU)."""
+import ctypes
+import os
+import subprocess
+
 import pytest
 import torch
 
@@ -8,6 +12,33 @@ from test_repack_layout import gpu_case
 
 # (n, k, quant_cols): one tile of one unit of 128 rows, all FP6, all INT4, waves without a slice, ragged slices, the longest slice
 SHAPES = [(128, 128, -1), (256, 128, 256), (384, 640, 128), (512, 1152, 256), (640, 2048, -1), (256, 1408, 256), (256, 4096, 128)]
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+WRAPPER = """
+#include "m1_plan.h"
+extern "C" int takes(int units, long long n4, long long qc, int group) { return fp6m::m1_choice(units, n4, qc, group != 0, 256, 72).us > 0.0; }
+"""
+
+
+@pytest.fixture(scope="module")
+def choice(tmp_path_factory):
+    d = tmp_path_factory.mktemp("m1_plan")
+    (d / "plan.cpp").write_text(WRAPPER)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{ROOT}/fp6-marlin_amd/csrc",
+                           "-o", str(d / "plan.so"), str(d / "plan.cpp")])
+    takes = ctypes.CDLL(str(d / "plan.so")).takes
+    takes.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong, ctypes.c_int]
+    return lambda k, n, qc, gs: bool(takes(k // 128, n - qc, qc, gs == 128))
+
+
+def test_fp6_columns_alone_are_estimated_by_their_own_cuts(choice):
+    """us of one-wave workgroups and of the best cut of 64-column tiles, where one of them is 3 % to 40 % behind."""
+    for k, n, one_wave, tiles64 in ((2816, 17664, 10.67, 11.79), (3328, 19328, 12.06, 13.40), (3200, 33152, 17.97, 19.69),
+                                    (2688, 33152, 15.45, 16.98), (4608, 18304, 15.55, 16.95), (2688, 37120, 16.39, 17.86)):
+        assert not choice(k, n, n, -1), (k, n, one_wave, tiles64)
+    for k, n, one_wave, tiles64 in ((4224, 5760, 7.39, 7.19), (12928, 1024, 8.50, 5.68), (16512, 1024, 9.45, 6.10), (8832, 1792, 9.07, 5.77),
+                                    (11136, 1408, 9.08, 5.71), (8064, 1280, 8.74, 5.49)):
+        assert choice(k, n, n, -1), (k, n, one_wave, tiles64)
 
 
 @pytest.mark.gpu
