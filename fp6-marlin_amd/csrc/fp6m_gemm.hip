@@ -923,9 +923,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
         };
 
         // One row on tiles of 64 columns (gemm_m1.h), by estimated time: whole units of 128 rows, addresses that 16-byte loads to
-        // LDS take (of the scales too, which the other kernels load four bytes at a time), and cells for every column.  (Against `sk_time` with 3 % to its favour 13 of
-        // the 789 shapes were slower than before, one of them by 8 %, eleven by 1-4 %, the rest 12 % faster on average; that
-        // kernel is 2 % faster since, 22784 x 5632 14.6 us against 15.1 here: 5 %.)
+        // LDS take (of the scales too, which the other kernels load four bytes at a time), and cells for every column.
         if (prob_m == 1 && !row_mix && prob_k % 128 == 0 && tune.m1 != 0 && (size_t)prob_n * sizeof(unsigned long long) <= kCellBytes &&
             ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(s)) & 15) == 0) {
             const int u = prob_k / 128;

@@ -37,20 +37,18 @@ inline M1Slices m1_slices(int units, int wk, long long ks4, long long ks6, bool 
 // random shapes (k = 1024 .. 28672, n = 1024 .. 51200, no to 1024 FP6 columns, both scale modes), which they reproduce to 2-4 %.
 // Terms: once; with a split; per part; per unit of 128 rows of the longest older and younger slices and of the mean one; per
 // unit by which 1.7 FP6 units exceed the longest slice; per MB of weights; per unit with group scales; per CU beyond `edge`
-// workgroups (shares of all CUs).  [ring of four steps][workgroups beyond one, two per CU, or eight waves].
+// workgroups (shares of all CUs).  [ring of four steps][up to one, up to two workgroups per CU, eight waves].
 struct M1Time {
     double start, split, part, longest, younger, mean, fp6, mbytes, group, edge;
 };
-constexpr M1Time kM1Time[2][4] = {
+constexpr M1Time kM1Time[2][3] = {
     {{2.591, 0.534, 0.0131, 0.490, 0.0, 0.221, 0.125, 0.0457, 0.0380, 0.0},
      {2.850, 0.765, 0.0049, 0.398, 0.0, 0.174, 0.220, 0.0892, 0.0601, 1.137},
-     {2.770, 0.889, 0.0256, 0.372, 0.0, 0.238, 0.343, 0.1144, 0.0929, 0.0},
      {2.975, 0.522, 0.0219, 0.178, 0.067, 0.542, 0.253, 0.0523, 0.0441, 4.187}},
     {{2.730, 0.484, 0.0148, 0.309, 0.0, 0.233, 0.331, 0.0438, 0.0424, 0.0},
      {3.074, 0.738, 0.0032, 0.275, 0.0, 0.168, 0.233, 0.1046, 0.0640, 0.341},
-     {2.819, 0.868, 0.0210, 0.341, 0.0, 0.547, 0.298, 0.0968, 0.0917, 0.0},
      {3.103, 0.489, 0.0182, 0.041, 0.188, 0.472, 0.368, 0.0595, 0.0487, 5.588}}};
-// The same for FP6 columns alone, which have one ring (7900 launches, every cut of 1016 shapes, k = 1024 .. 28672, n = 1024 ..
+// The same for FP6 columns alone, which have one ring; [.. up to three workgroups per CU, eight waves] (7900 launches, every cut of 1016 shapes, k = 1024 .. 28672, n = 1024 ..
 // 48000: 2-4 %).  By the entries above, which charge parts and slices of INT4 tiles, 116 of those shapes were more than 2 % slower
 // than with the one-wave kernel (3712 x 9216 10.5 us against 9.2); by these none is, nor any of 1208 calls at other random shapes.
 constexpr M1Time kM1TimeFp6[4] = {{2.808, 0.528, 0.0105, 0.667, 0.0, 0.161, 0.0, 0.0469, 0.0, 0.0},
@@ -65,7 +63,8 @@ inline double m1_time(const M1Time& t, long long ks, int longest, int younger, d
 }
 
 // The best cut of one row over k = 128 * units, n4 INT4 and qc FP6 columns that is resident at once: one workgroup of eight waves
-// or three of four per CU.
+// or two of four per CU.  (A third fits, but with INT4 tiles 24 of the 104 shapes that took it were more than 2 % slower than one-wave
+// workgroups, 21632 x 5888 15.6 us against 14.4, and the others no more than 2 % faster on average.)
 inline M1Plan m1_plan(int units, long long n4, long long qc, bool g128, int cus, int young_pct)
 {
     M1Plan best{0, 0, 0, 0, 0, 0.0};
@@ -74,11 +73,11 @@ inline M1Plan m1_plan(int units, long long n4, long long qc, bool g128, int cus,
         for (long long ks = 1; ks <= (n4 ? 16 : 24) && ks * wk <= units; ks++)
             for (int fine = 1; fine <= (n4 && qc ? 2 : 1); fine++) {
                 const long long ks6 = fine * ks, wgs = n4 / 64 * ks + qc / 64 * ks6;
-                if (ks6 * wk > units || wgs > (wk == 8 ? 1LL : 3LL) * cus) continue;
+                if (ks6 * wk > units || wgs > (wk == 8 ? 1LL : (n4 ? 2LL : 3LL)) * cus) continue;
                 const M1Slices s = m1_slices(units, wk, ks, ks6, n4 > 0, qc > 0, young_pct);
                 if (!s.fit) continue;
                 const double edge = (wgs - ((wk == 8 ? cus : 2LL * cus) - cus / 16)) / (double)cus, mean = units / (double)(ks * wk);
-                const int where = wk == 8 ? 3 : (int)((wgs - 1) / cus);
+                const int where = wk == 8 ? (n4 ? 2 : 3) : (int)((wgs - 1) / cus);
                 for (int four = 0; four < (n4 ? 2 : 1); four++) {
                     const double us = n4 ? m1_time(kM1Time[four][where], ks, s.longest4, s.younger4, mean, 1.7 * s.longest6 - s.longest4, mbytes, g128, edge)
                                          : m1_time(kM1TimeFp6[where], ks, s.longest6, s.younger6, mean, 0.0, mbytes, false, edge);
@@ -88,7 +87,7 @@ inline M1Plan m1_plan(int units, long long n4, long long qc, bool g128, int cus,
     return best;
 }
 
-// The same of gemm_sk_kernel's launch (the same shapes, to 4-5 %).
+// The same of gemm_sk_kernel's launch, to 4-5 %.  With INT4 tiles it is the fit over the 789 shapes; that kernel has become 3 % faster since.
 inline double sk_time(int units, long long n4, long long qc, bool g128)
 {
     const double mbytes = 128.0 * units * (n4 * 0.5 + qc * 0.75) * 1e-6, tiles = (n4 + qc) / 128.0;
@@ -96,11 +95,15 @@ inline double sk_time(int units, long long n4, long long qc, bool g128)
     return 4.137 + (g128 ? 0.1656 : 0.1511) * mbytes + 0.0061 * units + 0.00116 * tiles + 0.1546 * units / tiles + 0.0261 * qc / 256.0;
 }
 
-// The plan that is taken in place of gemm_sk_kernel; us = 0: none.
+// The plan that is taken in place of gemm_sk_kernel; us = 0: none.  The margin covers what that kernel gained since its fit and 2 % of
+// what the estimates miss: of 5250 calls at other random shapes (no to 1024 FP6 columns, both scale modes) 3400 take 64-column tiles
+// by it, 14 % faster on average; 25 of those are more than 2 % slower, the worst 8 %.  With 6 % instead of 5 it would be fewer, but square
+// shapes in whole parts, 8192 x 8192 9.4 us against 10.3, would go back.  Fewer than twelve units with a fifth or more of the columns in FP6,
+// whose few waves then end last, were 2 % slower on average (1280 x 3968, 1024 of them FP6, 4.9 us against 4.5).
 inline M1Plan m1_choice(int units, long long n4, long long qc, bool g128, int cus, int young_pct)
 {
     M1Plan plan = m1_plan(units, n4, qc, g128, cus, young_pct);
-    if (plan.us > 0.95 * sk_time(units, n4, qc, g128)) plan.us = 0.0;
+    if (plan.us > 0.95 * sk_time(units, n4, qc, g128) || (n4 > 0 && units < 12 && 5 * qc >= n4 + qc)) plan.us = 0.0;
     return plan;
 }
 

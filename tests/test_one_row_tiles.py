@@ -41,6 +41,16 @@ def test_fp6_columns_alone_are_estimated_by_their_own_cuts(choice):
         assert choice(k, n, n, -1), (k, n, one_wave, tiles64)
 
 
+def test_no_third_workgroup_on_a_cu(choice):
+    """us of one-wave workgroups and of 64-column tiles, three workgroups to a CU; and launches that fit by twos."""
+    for k, n, qc, one_wave, tiles64 in ((21632, 5888, 256, 14.36, 15.55), (17536, 7808, 0, 14.53, 15.68), (22400, 5376, 256, 14.25, 15.27),
+                                        (1920, 33664, 256, 9.08, 9.71), (2560, 37888, 256, 11.56, 12.16), (16896, 6144, 512, 12.88, 13.53)):
+        assert not choice(k, n, qc, 128), (k, n, one_wave, tiles64)
+    for k, n, qc, one_wave, tiles64 in ((1152, 2432, 1024, 4.46, 4.86), (1280, 3968, 1024, 4.54, 4.90), (1280, 4608, 1024, 4.68, 4.93)):
+        assert not choice(k, n, qc, -1) and not choice(k, n, qc, 128), (k, n, one_wave, tiles64)    # (short k, much of it FP6)
+    assert choice(8192, 8192, 256, 128) and choice(4096, 4096, 256, 128) and choice(4096, 12288, 256, 128) and choice(11008, 4096, 256, -1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("wk", [4, 8])
 @pytest.mark.parametrize("depth", [3, 4])
