@@ -1455,6 +1455,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                     }
                 }
             }
+            double us_wide = 0.0, us_half = 0.0;                        // (for the verbose line)
             // 64-column tiles instead, by estimated time (M16Time); not below k = 1024, where nothing was measured.
             if (half_fits && tune.half == kUnset && tune.wk16 == kUnset && tune.cells == kUnset && tune.xcd == kUnset &&
                 !(tune.cls != kUnset && tune.cls == 1) && env_ks < 1 && sms <= 0 && prob_k >= 1024 && cls_na == 0) {
@@ -1481,7 +1482,8 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                     }
                     return cut;
                 };
-                double best = 0.98 * m16_time(false, cut_of(false, cfg.wk, ks), a.m, g128, mbytes, cus);
+                us_wide = m16_time(false, cut_of(false, cfg.wk, ks), a.m, g128, mbytes, cus);
+                double best = (qc < prob_n ? kHalfMargin : kHalfMarginFp6) * us_wide;
                 int best_wk = 0;
                 long long best_ks = 0;
                 for (int wk = 4; wk <= 8; wk += 4)
@@ -1489,6 +1491,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                         // (what is not refused or cut back for want of scratch with 128 columns must not be with 64)
                         if (c > 1 && (size_t)(2 * a.tiles + 2 * a.tiles6) * c * (16 * 64 * sizeof(float)) > scratch_bytes) break;
                         const double us = m16_time(true, cut_of(true, wk, c), a.m, g128, mbytes, cus);
+                        if (us > 0.0 && (us_half == 0.0 || us < us_half)) us_half = us;
                         if (us > 0.0 && us < best) {
                             best = us;
                             best_wk = wk;
@@ -1597,8 +1600,8 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
             }
             dim3 grid((unsigned)wgs, 1);
             if (tune.verbose)
-                fprintf(stderr, "fp6m_mul m=%d n=%d k=%d: cfg %d%s (%dx%d waves) groups %d+%d ks4=%d ks6=%d (+ %d tiles in %d parts) gain %.1f grid=%u%s\n", a.m, prob_n,
-                        prob_k, cfg.id, half ? " half" : "", cfg.wn, cfg.wk, a.groups6, a.groups4, a.ks4, a.ks6, a.groups4b, a.ks4b, cls_gain, grid.x, a.xcd_local ? " (tiles placed per XCD)" : "");
+                fprintf(stderr, "fp6m_mul m=%d n=%d k=%d: cfg %d%s (%dx%d waves) groups %d+%d ks4=%d ks6=%d (+ %d tiles in %d parts) gain %.1f, 128 / 64 columns %.1f / %.1f us, grid=%u%s\n", a.m, prob_n,
+                        prob_k, cfg.id, half ? " half" : "", cfg.wn, cfg.wk, a.groups6, a.groups4, a.ks4, a.ks6, a.groups4b, a.ks4b, cls_gain, us_wide, us_half, grid.x, a.xcd_local ? " (tiles placed per XCD)" : "");
             if (half) {
                 const bool a8 = a.m <= 8;
                 if (cfg.wk == 8)

@@ -23,8 +23,12 @@ struct M16Cut {
 // 64-column tiles are taken on 55 % of those shapes; the choice is 1 % behind the best of all measured splits, 9.5 % faster than 128-column
 // tiles alone, and three of 650 lost (the worst 3 %).  us: 16 x 4096 x 4096 8.5 -> 7.1, 5 x 5120 x 15360 12.7 -> 10.6,
 // 8 x 11008 x 4096 11.2 -> 9.9, 16 x 2816 x 2304 9.3 -> 6.4; 16 x 8192 x 8192 keeps 128 columns (12.3, 13.1 with 64).
-// Fitted before either kernel stopped fetching past the end of a slice, which took 1 to 9 % off both; on fourteen shapes the choice is
-// still within 1.5 % of the best forced split.
+// Fitted before either kernel stopped fetching past the end of a slice, which took 1 to 9 % off both, and over INT4 tiles with up to
+// 1024 FP6 columns.  Hence the margins by which 64-column tiles have to be ahead: over 2013 calls at other random shapes they are
+// taken 1314 times and 16 % faster on average, twice more than 2 % slower (with 2 % instead of 4 eleven times, 9 x 18560 x 4352 14.6 us against
+// 13.5); over 2279 of FP6 columns alone, whose times the estimates miss by 4-10 %, 1539 times and 16 %, twice (with 2 % instead of 8
+// 35 times, 14 x 19328 x 4608 19.5 against 17.5).
+constexpr double kHalfMargin = 0.96, kHalfMarginFp6 = 0.92;
 struct M16Time {
     // us once; once with a split, per part, and per part and row; per step of the longest slice, of the mean one, of the mean one
     // at full occupation, per row that A is fetched in, and with group scales; per step by which 1.7 FP6 steps exceed an INT4

@@ -183,6 +183,29 @@ def test_where_the_narrow_tiles_are_taken(oracle, capfd):
 
 
 @pytest.mark.gpu
+def test_calls_near_the_line_keep_the_wide_tiles(oracle, capfd):
+    """Calls on which tiles of 64 columns were 5 to 12 % slower than tiles of 128, and two on which they are a quarter faster."""
+    import fp6_marlin
+
+    def takes(m, k, n, qc, gs):
+        B = torch.zeros(k * (n - qc) // 8 + k * qc * 3 // 16, dtype=torch.int32, device=dev())
+        s = torch.zeros((k // 128 if gs == 128 else 1) * (n - qc) + qc, dtype=torch.half, device=dev())
+        A, C = torch.zeros((m, k), dtype=torch.half, device=dev()), torch.empty((m, n), dtype=torch.half, device=dev())
+        ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+        capfd.readouterr()
+        with fp6_marlin.cabi.tuning(verbose=1):
+            fp6_marlin.mul(A, B, C, s, ws, qc if qc else -1, group_size=gs)
+            torch.cuda.synchronize()
+        return " half " in capfd.readouterr().err
+
+    for m, k, n, qc, gs in ((9, 18560, 4352, 256, 128), (7, 14464, 7040, 0, -1), (10, 17664, 4864, 256, 128), (15, 15616, 3968, 256, 128)):
+        assert not takes(m, k, n, qc, gs)
+    for m, k, n in ((14, 19328, 4608), (12, 12288, 7296), (10, 10752, 6912), (16, 17024, 5248), (15, 18560, 4608), (10, 11392, 7424)):
+        assert not takes(m, k, n, n, -1)
+    assert takes(6, 27776, 1536, 0, 128) and takes(7, 19968, 1024, 256, 128) and takes(5, 4096, 1024, 1024, -1)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [2, 7, 16])
 def test_gfx950_order_gives_the_same_bits(oracle, m):
     """Words in either order through tiles of 64 columns: the smallest tile, ragged units, all FP6, FP6 rows."""
