@@ -605,8 +605,8 @@ def sweep(args):
 def timeline(args):
     """Per-workgroup clock stamps of one GEMM (python fp6-marlin_amd/build.py --timeline builds the instrumented library):
     where the launch's time goes, and how far apart its workgroups end.  Stamps, microseconds after the first workgroup's
-    start: decode kernel (one wave per workgroup)  start, first weights landed, loop end, rows formed, atomics issued,
-    -, stored / cell cleared, end;  other kernels  start, first weights landed, loop end, slices summed through LDS,
+    start: one row  start, first weights landed, loop end, rows formed / slices summed through LDS, atomics
+    issued, -, stored / cell cleared, end;  other kernels  start, first weights landed, loop end, slices summed through LDS,
     partial tile published, counted, gathered and stored (last arrival only), end."""
     import ctypes
     import numpy as np
@@ -655,23 +655,26 @@ def timeline(args):
         torch.cuda.synchronize()
         t = stamps.cpu().numpy().reshape(-1, 8)
         used = t[:, 0] != 0
-        t = t[used].astype(np.float64)
-        raw = stamps.cpu().numpy().reshape(-1, 8)[used]
+        if not used.any():
+            sys.exit("bench.py --timeline: the kernel that this shape takes writes no stamps (rebuild the instrumented library)")
+        raw = t[used]
+        t = raw.astype(np.float64)
         reps.append(((t - t[:, 0].min()) / 100.0, np.nonzero(used)[0], (raw[:, 5] >> 32) & 15))   # the clock counts 100 MHz
+        waves = int(raw[0, 5] >> 40) or 1                  # (one row: waves per workgroup, where it is not a single one)
     names = ["start", "first weights", "loop end", "rows / slices summed", "atomics out / published", "counted",
              "stored (last arrival)", "end"]
     out = {"m": m, "k": k, "n": n, "quant_cols": qc, "group_size": gs, "knobs": args.knobs or "", "workgroups": int(len(reps[0][1])),
            "kernel_us": round(float(np.mean([r[0][:, 7].max() for r in reps])), 2), "percentiles": pct, "stamps_us": {}}
     for i, name in enumerate(names):
         if m == 1 and i == 5:
-            continue                                       # (the decode kernel keeps its hardware id there)
+            continue                                       # (the kernels for one row keep their hardware id there)
         rows = [np.percentile(r[0][:, i][r[0][:, i] > 0] if i else r[0][:, i], pct) for r in reps if (r[0][:, i] > 0).any() or i == 0]
         if rows:
             out["stamps_us"][name] = [round(float(v), 2) for v in np.mean(rows, axis=0)]
     # by generation: workgroup index / 8 is the index inside an XCD; the first 4 x CUs / 8 one-wave workgroups of an XCD
     # (CUs / 8 four-wave ones) start on SIMDs (CUs) of their own, the later ones share
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    per_gen = (4 if m == 1 else 1) * cus // 8
+    per_gen = (4 if m == 1 and waves == 1 else 1) * cus // 8
     gens = {}
     for r, idx, _ in reps:
         g = (idx >> 3) // per_gen
@@ -682,12 +685,12 @@ def timeline(args):
                                       "end_median_us": round(float(np.mean([x[2] for x in v])), 2),
                                       "end_max_us": round(float(np.mean([x[3] for x in v])), 2)} for gi, v in sorted(gens.items())}
     if m == 1:
-        # the decode kernel's waves also note the XCD they run on: the dies do not all stream at the same rate
+        # the kernels for one row also note the XCD they run on: the dies do not all stream at the same rate
         xcds = {}
         for r, _, xcc in reps:
             for x in np.unique(xcc):
                 xcds.setdefault(int(x), []).append([np.sum(xcc == x), np.median(r[xcc == x, 2]), r[xcc == x, 7].max()])
-        out["by_xcd"] = {str(x): {"waves": int(np.mean([v[0] for v in vs])), "loop_end_median_us": round(float(np.mean([v[1] for v in vs])), 2),
+        out["by_xcd"] = {str(x): {"workgroups": int(np.mean([v[0] for v in vs])), "loop_end_median_us": round(float(np.mean([v[1] for v in vs])), 2),
                                   "end_max_us": round(float(np.mean([v[2] for v in vs])), 2)} for x, vs in sorted(xcds.items())}
     print(json.dumps(out), flush=True)
 

@@ -977,6 +977,9 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                 d.lda = fu.lda;
                 d.tile4 = (size_t)(prob_k / 16) * 1024;
                 d.tile2 = (size_t)(prob_k / 16) * 512;
+#ifdef FP6M_TIMELINE
+                d.timeline = a.timeline;
+#endif
                 if (tune.verbose)
                     fprintf(stderr, "fp6m_mul m=1 n=%d k=%d: 64-column tiles, %d waves, ring of %d, ks4=%d ks6=%d grid=%lld (%.1f us, else %.1f)\n", prob_n, prob_k,
                             plan.wk, plan.depth, d.ks4, d.ks6, wgs, plan.us, sk_time(u, n4, qc, g128));

@@ -44,6 +44,9 @@ struct M1Args {
     const int32_t* a_cols;    // (a row of `lda` activations, of which the weight's rows take these)
     int lda;
     size_t tile4, tile2;      // bytes of a tile of 128 columns in that order, per k-block of 1024 (512)
+#ifdef FP6M_TIMELINE
+    unsigned long long* timeline;   // performance debugging builds only
+#endif
 };
 
 constexpr int kM1ABytes = kM1Steps * 128;
@@ -62,7 +65,7 @@ struct M1Gather {
     uint32_t row_lds;         // the staged row
 };
 template <bool FP6, bool GROUP, int DEPTH, bool STAGED>
-__device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t row4, const unsigned char* base2, uint32_t row2,
+__device__ __forceinline__ void stream_m1(const M1Args& p, const unsigned char* base4, uint32_t row4, const unsigned char* base2, uint32_t row2,
                                           const unsigned char* base_a, const unsigned char* base_gs, uint32_t gs_row,
                                           unsigned char* ring, unsigned char* a_lds, unsigned char* gs_lds, int steps, bool native, const M1Gather& gather, f4 (&acc)[4])
 {
@@ -201,6 +204,7 @@ __device__ __forceinline__ void stream_m1(const unsigned char* base4, uint32_t r
 
     Regs regs[2];
     wait_steps<kOps, false, false, DEPTH - 2>(issued - 1);
+    FP6M_MARK(p, 1);
     fetch(regs[0]);
     f4 grp[4];
 #pragma unroll 1
@@ -256,6 +260,14 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_m1_kernel(const M1Args p)
                         "s"(p.n4), "s"(p.qc), "s"(p.groups6), "s"(p.groups4), "s"(p.ks6), "s"(p.ks4), "s"(gridDim.x));
     asm volatile("" : : "s"(p.rule6.lo), "s"(p.rule6.ly), "s"(p.rule6.eo), "s"(p.rule6.ey), "s"(p.rule4.lo), "s"(p.rule4.ly),
                         "s"(p.rule4.eo), "s"(p.rule4.ey), "s"(p.div6.d), "s"(p.div6.magic), "s"(p.div4.d), "s"(p.div4.magic));
+    FP6M_MARK(p, 0);
+#ifdef FP6M_TIMELINE
+    if (p.timeline && threadIdx.x < 64) {                         // waves per workgroup, and where this one runs: XCC_ID and HW_ID
+        const uint32_t hw = __builtin_amdgcn_s_getreg((4 << 0) | (0 << 6) | (31 << 11));
+        const uint32_t xcc = __builtin_amdgcn_s_getreg((20 << 0) | (0 << 6) | (3 << 11));
+        p.timeline[(size_t)blockIdx.x * 8 + 5] = ((unsigned long long)WK << 40) | ((unsigned long long)xcc << 32) | hw;
+    }
+#endif
     const int lane = threadIdx.x & 63;
     const int wk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int logical = xcd_contiguous_id(blockIdx.x, gridDim.x);
@@ -295,12 +307,12 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_m1_kernel(const M1Args p)
         const size_t at2 = native ? (group >> 1) * p.tile2 + 64 * (group & 1) : 256 * (size_t)group;
         if (fp6) {
             const uint32_t row4 = native ? 1024 : 8 * (uint32_t)p.qc, row2 = native ? 512 : 4 * (uint32_t)p.qc;
-            stream_m1<true, false, D6, STAGED>(reinterpret_cast<const unsigned char*>(p.b_fp6_4) + at4 + 8 * (size_t)unit * row4, row4,
+            stream_m1<true, false, D6, STAGED>(p, reinterpret_cast<const unsigned char*>(p.b_fp6_4) + at4 + 8 * (size_t)unit * row4, row4,
                                        reinterpret_cast<const unsigned char*>(p.b_fp6_2) + at2 + 8 * (size_t)unit * row2, row2,
                                        base_a, nullptr, 0, ring, a_lds, gs_lds, steps, native, gather, acc);
         } else {
             const uint32_t row4 = native ? 1024 : 8 * (uint32_t)p.n4, gs_row = 2 * (uint32_t)p.n4;
-            stream_m1<false, G128, D4, STAGED>(reinterpret_cast<const unsigned char*>(p.b_int4) + at4 + 8 * (size_t)unit * row4, row4,
+            stream_m1<false, G128, D4, STAGED>(p, reinterpret_cast<const unsigned char*>(p.b_int4) + at4 + 8 * (size_t)unit * row4, row4,
                                        nullptr, 0, base_a,
                                        reinterpret_cast<const unsigned char*>(p.s_int4) + 128 * (size_t)group + (size_t)unit * gs_row, gs_row,
                                        ring, a_lds, gs_lds, steps, native, gather, acc);
@@ -309,6 +321,7 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_m1_kernel(const M1Args p)
         __builtin_amdgcn_s_waitcnt(vmcnt_only(0));                // (its piece of the row, for the others)
         __builtin_amdgcn_s_barrier();
     }
+    FP6M_MARK(p, 2);
     // Every lane column c holds the one row; the slab of a wave's 64 sums lies in its drained ring.
     const int q = lane >> 4;
     if ((lane & 15) == 0) {
@@ -322,13 +335,18 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_m1_kernel(const M1Args p)
     float v = 0.f;
 #pragma unroll
     for (int j = 0; j < WK; j++) v += *reinterpret_cast<const float*>(smem + j * kWaveLds + 4 * lane);
+    FP6M_MARK(p, 3);
     if (column_scales) v *= (float)reinterpret_cast<const _Float16*>(gs_lds)[(lane & 32) + scale_slot(lane & 31)];
     int col = (fp6 ? p.n4 : 0) + 64 * group + lane;
     if (ks > 1) {                                                 // (the protocol, and why it holds: gemm_sk.h)
         unsigned long long* cell = p.cells + 64 * (size_t)(fp6 ? group : p.groups6 + group) + lane;
         const unsigned long long mine = cell_contribution(v);
         const unsigned long long old = __hip_atomic_fetch_add(cell, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if ((int)(old >> 56) != ks - 1) return;
+        FP6M_MARK(p, 4);
+        if ((int)(old >> 56) != ks - 1) {
+            FP6M_MARK(p, 7);
+            return;
+        }
         v = cell_total(old, mine, ks);
         __hip_atomic_store(cell, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -341,6 +359,8 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_m1_kernel(const M1Args p)
         if (p.residual) v += (float)__builtin_bit_cast(_Float16, p.residual[col]);
     }
     p.C[col] = __builtin_bit_cast(uint16_t, (_Float16)v);
+    FP6M_MARK(p, 6);
+    FP6M_MARK(p, 7);
 }
 
 }  // namespace fp6m

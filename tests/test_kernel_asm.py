@@ -138,6 +138,15 @@ def test_kernel_arguments_are_loaded_in_one_batch(asm):
     assert seen == 82            # (the m <= 16 kernel's builds with the partial tiles exchanged inside one XCD are 8 of them)
 
 
+def test_every_kernel_with_a_ring_per_wave_writes_its_stamps():
+    """Start, first weights, loop end and end of a workgroup, in the build that bench.py --timeline loads: without them it finds no
+    workgroup at all.  (The kernel whose waves share a ring has none.)"""
+    for name in ("gemm_sk.h", "gemm_m1.h", "gemm_m16.h", "gemm_m16h.h", "gemm_mb.h"):
+        with open(os.path.join(os.path.dirname(SRC), name)) as f:
+            text = f.read()
+        assert "__global__" in text and all(f"FP6M_MARK(p, {i});" in text for i in (0, 1, 2, 3, 7)), name
+
+
 def test_the_packer_tells_the_host_one_word_and_releases_it(tmp_path_factory):
     """A host that does not wait for the stream learns from pack_kernel that the range of the FP6 cast is known and what it is.
     That has to be one store: a system-scope load of the earlier kernel's flag, a wait for it, then the verdict, released
