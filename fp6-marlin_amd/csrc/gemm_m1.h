@@ -260,6 +260,9 @@ __global__ __launch_bounds__(64 * WK, 2) void gemm_m1_kernel(const M1Args p)
                         "s"(p.n4), "s"(p.qc), "s"(p.groups6), "s"(p.groups4), "s"(p.ks6), "s"(p.ks4), "s"(gridDim.x));
     asm volatile("" : : "s"(p.rule6.lo), "s"(p.rule6.ly), "s"(p.rule6.eo), "s"(p.rule6.ey), "s"(p.rule4.lo), "s"(p.rule4.ly),
                         "s"(p.rule4.eo), "s"(p.rule4.ey), "s"(p.div6.d), "s"(p.div6.magic), "s"(p.div4.d), "s"(p.div4.magic));
+    if constexpr (EXTRAS)
+        asm volatile("" : : "s"(p.native), "s"(p.tile4), "s"(p.tile2), "s"(p.n), "s"(p.c_cols), "s"(p.bias), "s"(p.residual));
+    if constexpr (STAGED) asm volatile("" : : "s"(p.a_cols), "s"(p.lda));
     FP6M_MARK(p, 0);
 #ifdef FP6M_TIMELINE
     if (p.timeline && threadIdx.x < 64) {                         // waves per workgroup, and where this one runs: XCC_ID and HW_ID

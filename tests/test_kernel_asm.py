@@ -123,7 +123,7 @@ def test_kernel_arguments_are_loaded_in_one_batch(asm):
     argument block itself: four loads, one wait, and no other argument load anywhere."""
     seen = 0
     for name, ins in kernels(asm):
-        if not any(k in name for k in ("gemm_m16_kernel", "gemm_sk_kernel", "gemm_mb_kernel")):
+        if not any(k in name for k in ("gemm_m16_kernel", "gemm_m16h_kernel", "gemm_sk_kernel", "gemm_m1_kernel", "gemm_mb_kernel")):
             continue
         seen += 1
         if "gemm_sk_kernel" in name:
@@ -135,7 +135,8 @@ def test_kernel_arguments_are_loaded_in_one_batch(asm):
         # the code of the epilogue may be laid out ahead of the loops: its loads (fused-epilogue pointers) do not count
         late = [(n, l) for n, l in late if not re.search(r"0x(c8|d0|d8)$", l)]
         assert not late, f"{name}: kernel-argument loads after the prologue: {late[:4]}"
-    assert seen == 82            # (the m <= 16 kernel's builds with the partial tiles exchanged inside one XCD are 8 of them)
+    # (the m <= 16 kernel's builds with the partial tiles exchanged inside one XCD are 8 of the 82; then 32 and 24 on 64-column tiles)
+    assert seen == 82 + 32 + 24
 
 
 def test_every_kernel_with_a_ring_per_wave_writes_its_stamps():
