@@ -613,6 +613,8 @@ int fp6m_tuning_set(const char* knob, int value)
         return FP6M_OK;
     }
     if (!strcmp(knob, "wide") && (value < 0 || value > fp6m::kWidePlanCount)) return FP6M_ERR_ARG;
+    if (!strcmp(knob, "m1") && value != 0 && value != 3 && value != 4) return FP6M_ERR_ARG;
+    if (!strcmp(knob, "half") && value != 0 && value != 1) return FP6M_ERR_ARG;
     const struct { const char* name; int* field; } knobs[] = {
         {"mb", &g_tuning.mb}, {"ksplit", &g_tuning.ksplit},
         {"wk16", &g_tuning.wk16}, {"half", &g_tuning.half}, {"m1", &g_tuning.m1}, {"wk", &g_tuning.wk}, {"pair", &g_tuning.pair}, {"wgs", &g_tuning.wgs}, {"share", &g_tuning.share}, {"share6", &g_tuning.share6}, {"cap", &g_tuning.cap}, {"sk", &g_tuning.sk}, {"gather", &g_tuning.gather}, {"cells", &g_tuning.cells}, {"xcd", &g_tuning.xcd}, {"gen", &g_tuning.gen}, {"gen2", &g_tuning.gen2}, {"gen3", &g_tuning.gen3}, {"young", &g_tuning.young}, {"cls", &g_tuning.cls}, {"cus", &g_tuning.cus}, {"cap2", &g_tuning.cap2}, {"wide", &g_tuning.wide},

@@ -43,5 +43,7 @@ def test_the_many_rows_tile_is_refused_outside_its_table():
     try:
         assert [L.fp6m_tuning_set(b"wide", v) for v in (0, 1, 9)] == [0, 0, 0]
         assert [L.fp6m_tuning_set(b"wide", v) for v in (10, 100, -1)] == [fp6_marlin.cabi.ERR_ARG] * 3
+        assert [L.fp6m_tuning_set(b"m1", v) for v in (0, 3, 4, 1, 7, -1)] == [0] * 3 + [fp6_marlin.cabi.ERR_ARG] * 3
+        assert [L.fp6m_tuning_set(b"half", v) for v in (0, 1, 2, -1)] == [0] * 2 + [fp6_marlin.cabi.ERR_ARG] * 2
     finally:
         L.fp6m_tuning_set(None, 0)
