@@ -14,7 +14,7 @@ fp16, activations N(0,1) fp16 (the reference's own bench does the same, bench.py
 
 value        packed-weight GB/s over the timed steps: algorithmic weight bytes / wall time, where
              weight bytes = K(N-qc)/2 + K*qc*3/4 + scale bytes.
-roofline     the GEMM kernel against the 8 TB/s HBM peak: algorithmic bytes per launch / mean time per
+roofline     the GEMM kernels against the 8 TB/s HBM peak: algorithmic bytes per launch / mean time per
              launch, measured with HIP events on the launch stream over the same timed region.
 cpu_baseline the oracle's CPU path (quantise + prepack + dequantise-then-matmul) on config 0 (16 x 4096 x 4096), stage
              by stage, single-threaded like the reference (`value`) and on all cores, on this box's host cores.
@@ -34,9 +34,9 @@ for _p in (ROOT, os.path.join(ROOT, "fp6-marlin_amd")):
 HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch of the headline workload (mean of its four GEMMs): FETCH_SIZE + WRITE_SIZE from two
 # `rocprofv3 --pmc` runs of `bench.py --traffic-probe`, each scaled by what the same counter reads for a
-# 256 MiB device copy (x2.000 and x1.000); figures in profiles/gemm_sk_kernel_decode7b_hbm_traffic.txt.
-MEASURED_TRAFFIC_BYTES_PER_LAUNCH = 28742537
-TRAFFIC_PROFILE = "profiles/gemm_sk_kernel_decode7b_hbm_traffic.txt"
+# 256 MiB device copy (x2.000 and x1.000); figures in profiles/gemm_m1_kernel_decode7b_hbm_traffic.txt.
+MEASURED_TRAFFIC_BYTES_PER_LAUNCH = 27430040
+TRAFFIC_PROFILE = "profiles/gemm_m1_kernel_decode7b_hbm_traffic.txt"
 MFMA_F16_PEAK_TFLOPS = 2500.0
 LLAMA7B = [(4096, 12288), (4096, 4096), (4096, 22016), (11008, 4096)]
 LLAMA70B = [(8192, 10240), (8192, 8192), (8192, 57344), (28672, 8192)]
@@ -341,7 +341,9 @@ def headline(args):
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": MEASURED_TRAFFIC_BYTES_PER_LAUNCH,
                      "traffic_source": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs recorded in " + TRAFFIC_PROFILE +
                                        ", not measured in this run",
-                     "kernel": "fp6m::gemm_sk_kernel<true, 0, false, false>", "us_per_launch": round(per_launch * 1e6, 3),
+                     "kernel": "fp6m::gemm_m1_kernel<true, 8, 4, 3, false, false> (4096x12288, 11008x4096), "
+                               "<true, 4, 3, 3, false, false> (4096x4096); fp6m::gemm_sk_kernel<true, 0, false, false> (4096x22016)",
+                     "us_per_launch": round(per_launch * 1e6, 3),
                      "bytes_per_launch": step_bytes // launches_per_step},
         "cpu_baseline": cpu_baseline(torch),
         "fp16_hipblaslt": {"ms_per_step": round(wall16 / args.steps * 1e3, 5),
