@@ -56,8 +56,9 @@ def newer_step_ops(word_ops, a_ops, first, n):
     return word_ops * n + sum(a_ops for t in range(n) if (first + t) % 2 == 0)
 
 
-def run_m16(steps, depth, arows, fp6, group):
-    """gemm_m16.h stream_tile: one wave, `steps` k steps (even; a multiple of four with group scales)."""
+def run_m16(steps, depth, arows, fp6, group, lenient_tail=0):
+    """gemm_m16.h stream_tile: one wave, `steps` k steps (even; a multiple of four with group scales).  With four rows of A, and
+    three steps at least where it fetches so many ahead, it is gemm_sk.h sk_wave too, for a wave with one chunk and no gather."""
     group = group and not fp6
     word_ops, a_ops = (3 if fp6 else 2), (2 if arows == 16 else 1)
     pair_slots = (depth + 2) // 2
@@ -115,7 +116,7 @@ def run_m16(steps, depth, arows, fp6, group):
             if more:
                 mem.wait((wait_odd if u % 2 else wait_even) + (1 if one_more else 0))
             else:
-                mem.wait(word_ops if depth == 4 and steps - (s + u) == 3 else 0)
+                mem.wait((word_ops if depth == 4 and steps - (s + u) == 3 else 0) + lenient_tail)
             if u % 2:
                 pair_rd = (pair_rd + 1) % pair_slots
             if s + u + 1 <= last:
@@ -145,6 +146,12 @@ def test_decode_loop_notices_a_lenient_wait(monkeypatch):
     monkeypatch.setattr(me, "newer_step_ops", lambda *a: real(*a) + 1)
     with pytest.raises(AssertionError, match="before its load completed"):
         run_m16(16, 4, 16, fp6=False, group=True)
+
+
+@pytest.mark.parametrize("fp6,group", [(False, True), (False, False), (True, False)])
+def test_decode_loop_notices_a_lenient_wait_past_the_last_fetch(fp6, group):
+    with pytest.raises(AssertionError, match="before its load completed"):
+        run_m16(16, 3 if fp6 else 4, 4, fp6, group, lenient_tail=1)
 
 
 def run_mb_ring(steps, depth, mb, fp6, group):

@@ -95,10 +95,12 @@ def test_fused_epilogue_with_int4_tiles_in_two_classes(oracle, m):
     assert oracle.rel_err(want.cpu().numpy(), oracle.matmul_ref(A.cpu().numpy(), ref)) <= TOL
 
 
+@pytest.mark.parametrize("m1", [None, 0])
 @pytest.mark.parametrize("k,n,qc,gs", [(4096, 4096, 256, 128), (4096, 4096, 256, -1), (1024, 768, 256, 128), (2048, 512, -1, 128),
                                        (2048, 512, -1, -1), (1024, 384, 384, -1), (11008, 1024, 128, 128), (8192, 2048, 256, -1)])
-def test_one_row_gather_inside_the_decode_kernel(oracle, k, n, qc, gs):
-    """One row: the decode kernel gathers A itself (no pass of its own).  Bit for bit the result of `mul` on the
+def test_one_row_gather_inside_the_decode_kernel(oracle, capfd, k, n, qc, gs, m1):
+    """One row: the decode kernels gather A themselves (no pass of its own): the one on 64-column tiles, which all of these shapes take
+    except the one with a short k and many FP6 columns, and with m1 = 0 the one of one-wave workgroups.  Bit for bit the result of `mul` on the
     materialised row, and of the same call with the gather forced into the separate pass; map entries outside the row
     are clamped to it, as the pass does."""
     import fp6_marlin
@@ -111,13 +113,19 @@ def test_one_row_gather_inside_the_decode_kernel(oracle, k, n, qc, gs):
     a_cols[5], a_cols[k - 3] = -7, lda + 11                        # clamped to columns 0 and lda - 1
     clamped = a_cols.clamp(0, lda - 1).long().to(dev())
     a_cols = a_cols.to(dev())
-    want = plain(fp6_marlin, A_wide[:, clamped].contiguous(), B, s, n, qc, gs)
+    knobs = {} if m1 is None else {"m1": m1}
+    capfd.readouterr()
+    with fp6_marlin.cabi.tuning(verbose=1, **knobs):
+        want = plain(fp6_marlin, A_wide[:, clamped].contiguous(), B, s, n, qc, gs)
+    kernel = "64-column tiles" if m1 is None and (k, n) != (1024, 768) else "one-wave workgroups"
+    assert kernel in capfd.readouterr().err
     ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
     for inside in (1, 0, 1):
         C = torch.full((1, n), float("nan"), dtype=torch.half, device=dev())
-        with fp6_marlin.cabi.tuning(gather=inside):
+        with fp6_marlin.cabi.tuning(gather=inside, verbose=1, **knobs):
             fp6_marlin.mul_fused(A_wide, B, C, s, ws, qc, gs, a_cols=a_cols)
         torch.cuda.synchronize()
+        assert kernel in capfd.readouterr().err
         assert torch.equal(C, want), inside
         assert int(ws.abs().sum()) == 0
     err = oracle.rel_err(want.cpu().numpy(), oracle.matmul_ref(A_wide[:, clamped].cpu().numpy(), ref))

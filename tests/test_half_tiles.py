@@ -1,11 +1,12 @@
 """The m <= 16 kernel on tiles of 64 columns (gemm_m16h.h): its fetch schedule replayed on the CPU, and on the GPU every ring width,
 wave count and protocol forced on the smallest and on ragged problems, against the oracle and, where only the split of the
 columns differs, bit for bit against tiles of 128."""
+import numpy as np
 import pytest
 import torch
 
 from test_fetch_schedule import Memory
-from test_gemm_gpu import dev, one_hot_case, run
+from test_gemm_gpu import dev, one_hot_case, problem, run
 from test_rows_gpu import run as run_rows
 
 
@@ -89,6 +90,55 @@ def test_against_oracle(oracle, m, wk):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 2, 4, 5, 8, 9, 16])
+def test_tiles_of_128_columns_give_the_same_bits(oracle, m):
+    """Whole numbers and scales of one: every order of the sums is exact, whatever the tile, its parts and how they meet."""
+    import fp6_marlin
+    for k, n, qc, gs in ((1152, 640, 256, 128), (1152, 640, 256, -1), (640, 256, 256, -1), (2048, 384, -1, 128)):
+        rng, n6 = np.random.default_rng(k + m), max(qc, 0)
+        w = rng.integers(-4, 5, (k, n)).astype(np.float16)
+        w[::128, :n - n6] = 7.5                                     # the largest of every group of rows: INT4 scale 1
+        w[0, n - n6:] = 28.0                                        # and of every column: FP6 scale 1
+        ref, b, s = oracle.gen_mixed_weight(w, qc, gs, strict=False)
+        assert (s == 1).all()
+        B, sd = torch.from_numpy(b).to(dev()), torch.from_numpy(s).to(dev())
+        a = rng.integers(-1, 2, (m, k)).astype(np.float16)
+        A, ws = torch.from_numpy(a).to(dev()), torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+        want = (a.astype(np.float64) @ ref.astype(np.float64)).astype(np.float16)
+        plans = [{"m1": 0}, {"m1": 3, "wk16": 4, "ksplit": 2}, {"m1": 4, "wk16": 8, "ksplit": 1}] if m == 1 else [{"half": 0}]
+        plans += [{"half": 1, "wk16": wk, "ksplit": ks} for wk in (4, 8) for ks in (1, 3)] if m > 1 else []
+        for plan in plans:
+            C = torch.full((m, n), float("nan"), dtype=torch.half, device=dev())
+            with fp6_marlin.cabi.tuning(**plan):
+                fp6_marlin.mul(A, B, C, sd, ws, qc, group_size=gs)
+                torch.cuda.synchronize()
+            assert np.array_equal(C.cpu().numpy(), want), plan
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [2, 7, 16])
+def test_rows_that_are_not_finite_stay_their_own(oracle, m):
+    """One row with an infinity and one with a NaN: none of their outputs is finite, and the other rows are what they are without."""
+    import fp6_marlin
+    n, k, qc = 384, 1152, 128
+    _, B, s = problem(oracle, n, k, qc, 128)
+    clean = torch.randn((m, k), generator=torch.Generator().manual_seed(m)).half()
+    bad = clean.clone()
+    bad[0, 700], bad[m - 1, 3] = float("-inf"), float("nan")
+    ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+    for wk in (4, 8):
+        for ks in (1, 3):
+            out = []
+            for A in (clean, bad):
+                out.append(torch.zeros((m, n), dtype=torch.half, device=dev()))
+                with fp6_marlin.cabi.tuning(half=1, wk16=wk, ksplit=ks):
+                    fp6_marlin.mul(A.to(dev()), B, out[-1], s, ws, qc, group_size=128)
+                    torch.cuda.synchronize()
+            assert torch.isfinite(out[0]).all() and torch.equal(out[0][1:m - 1], out[1][1:m - 1])
+            assert not torch.isfinite(out[1][0]).any() and not torch.isfinite(out[1][m - 1]).any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", [5, 8, 16])
 def test_placement_per_xcd_only_where_it_is_built(oracle, capfd, m):
     """Ten tiles of 64 columns in two parts are 20 workgroups; placed per XCD the grid is padded to 32.  Workgroups of eight waves
@@ -133,7 +183,6 @@ def test_additions_are_an_exact_reorder_of_the_plain_call(oracle, m):
     import fp6_marlin
     n, k, qc = 640, 1152, 128
     g = torch.Generator().manual_seed(m)
-    from test_gemm_gpu import problem
     _, B, s = problem(oracle, n, k, qc, 128)
     A = torch.randn((m, k), generator=g).half().to(dev())
     c_cols = torch.randperm(n, generator=g).to(torch.int32).to(dev())
@@ -217,7 +266,6 @@ def test_gfx950_order_gives_the_same_bits(oracle, m):
             gpu_case(oracle, m, 128, 256, 128, 128, env)
             gpu_case(oracle, m, 1152, 640, 256, -1, env)
             gpu_case(oracle, m, 640, 256, 256, -1, env)
-    import numpy as np
     k, n, qr = 1024 + 384, 384, 384
     ref, b, s = oracle.gen_row_mix_weight(np.random.default_rng(m).normal(0, 0.02, (k, n)).astype(np.float16), qr)
     B, sd = torch.from_numpy(b).to(dev()), torch.from_numpy(s).to(dev())

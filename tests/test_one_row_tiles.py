@@ -1,12 +1,15 @@
 """One row on tiles of 64 columns (gemm_m1.h): every ring, wave count and number of k parts forced on the smallest and on ragged problems,
-against the oracle; both word orders, the additions, and which calls take it (the estimate, m1_plan.h, also by itself on the CPU)."""
+against the oracle; both word orders, the additions, and which calls take it.  On the CPU: its fetch schedule replayed, and the
+estimate (m1_plan.h) by itself."""
 import ctypes
 import os
+import re
 import subprocess
 
 import pytest
 import torch
 
+from test_fetch_schedule import Memory
 from test_gemm_gpu import dev, one_hot_case, problem, run
 from test_repack_layout import gpu_case
 
@@ -14,6 +17,96 @@ from test_repack_layout import gpu_case
 SHAPES = [(128, 128, -1), (256, 128, 256), (384, 640, 128), (512, 1152, 256), (640, 2048, -1), (256, 1408, 256), (256, 4096, 128)]
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def replay(steps, depth, fp6, group, staged, pieces=2, lenient=0):
+    """stream_m1 and what the kernel issues in front of it: `steps` steps of 64 rows of k (even, 2 .. 16)."""
+    group, ops = group and not fp6, 3 if fp6 else 2
+    mem, issued, slot_in = Memory(), 0, 0
+
+    def issue():
+        nonlocal issued, slot_in
+        for o in range(ops):
+            mem.load(("step", slot_in, o), issued)
+        mem.expect(("step", slot_in, 0), issued)
+        issued, slot_in = issued + 1, (slot_in + 1) % depth
+
+    def wait(newer, most):                                      # wait_steps
+        newer = max(0, min(newer, most))
+        mem.wait(ops * newer + (lenient if newer else 0))
+
+    def fetch(step, slot):
+        for o in range(ops):
+            mem.read(("step", slot, o), step)
+        if not staged:                                          # (staged: the wave wrote them itself)
+            mem.read(("A", 0 if step < 8 else 1), "A")
+
+    if not group:
+        mem.load(("column scales", 0), "S")
+    for o in range(pieces if staged else 0):
+        mem.load(("row", o), "row")
+    if staged:
+        for t in range(-(-steps // 4) * 4):
+            mem.load(("entry", t), t)
+    else:
+        for o in range(1 + (steps > 8)):
+            mem.load(("A", o), "A")
+    if group:
+        mem.load(("group scales", 0), "S")
+    for _ in range(depth - 1):
+        if issued < steps:
+            issue()
+    if staged:
+        wait(issued, depth - 1)
+        for o in range(pieces):                                 # (for the others too, behind the barrier)
+            mem.read(("row", o), "row")
+        for t in range(-(-steps // 4) * 4):
+            mem.read(("entry", t), t)
+    wait(issued - 1, depth - 2)
+    fetch(0, 0)
+    slot_rd = 1 % depth
+    for s in range(0, steps, 2):
+        for u in range(2):
+            if issued < steps:
+                issue()
+            wait(issued - (s + u + 2), depth - 2)
+            if s + u + 1 < steps:
+                fetch(s + u + 1, slot_rd)
+            else:                                               # the look-ahead past the end reads what nobody uses
+                mem.pending_reads.clear()
+            slot_rd = (slot_rd + 1) % depth
+        if group:
+            mem.read(("group scales", 0), "S")
+    mem.wait(0)
+
+
+@pytest.mark.parametrize("staged", [False, True])
+def test_fetch_schedule(staged):
+    for steps in range(2, 17, 2):
+        for depth in (3, 4):
+            for group in (False, True):
+                replay(steps, depth, False, group, staged)
+        replay(steps, 3, True, False, staged)
+
+
+@pytest.mark.parametrize("staged", [False, True])
+def test_fetch_schedule_notices_a_lenient_wait(staged):
+    for fp6, group in ((False, True), (False, False), (True, False)):
+        with pytest.raises(AssertionError, match="before its load completed"):
+            replay(16, 3, fp6, group, staged, lenient=1)
+
+
+def test_every_wave_of_a_staged_row_meets_one_barrier():
+    """The row's pieces are for the whole workgroup: a wave with a slice meets the barrier inside stream_m1, one without meets its own,
+    each behind a wait for its pieces."""
+    with open(os.path.join(ROOT, "fp6-marlin_amd", "csrc", "gemm_m1.h")) as f:
+        text = f.read()
+    inside, kernel = text.split("__global__")
+    assert inside.count("__builtin_amdgcn_s_barrier") == 1 and kernel.count("__builtin_amdgcn_s_barrier") == 1
+    assert re.search(r"if constexpr \(STAGED\) \{\s+wait_steps<[^;]*;[^\n]*\n\s+__builtin_amdgcn_s_barrier", inside)
+    assert re.search(r"else if constexpr \(STAGED\) \{\s+__builtin_amdgcn_s_waitcnt\(vmcnt_only\(0\)\);[^\n]*\n\s+__builtin_amdgcn_s_barrier", kernel)
+
+
 WRAPPER = """
 #include "m1_plan.h"
 extern "C" int takes(int units, long long n4, long long qc, int group) { return fp6m::m1_choice(units, n4, qc, group != 0, 256, 72).us > 0.0; }
@@ -74,9 +167,10 @@ def test_gfx950_order_gives_the_same_bits(oracle, gs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m1", [4, 0])
 @pytest.mark.parametrize("ks", [1, 3])
-def test_additions(oracle, ks):
-    """Column map, bias and residual (in place too) are added in float32 and rounded once."""
+def test_additions(oracle, ks, m1):
+    """Column map, bias and residual (in place too) are added in float32 and rounded once, here and by one-wave workgroups."""
     import fp6_marlin
     n, k, qc = 640, 1152, 128
     g = torch.Generator().manual_seed(ks)
@@ -86,7 +180,7 @@ def test_additions(oracle, ks):
     bias, res = torch.randn(n, generator=g).half().to(dev()), torch.randn((1, n), generator=g).half().to(dev())
     ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
     plain, mapped, full = (torch.empty((1, n), dtype=torch.half, device=dev()) for _ in range(3))
-    with fp6_marlin.cabi.tuning(m1=4, ksplit=ks):
+    with fp6_marlin.cabi.tuning(m1=m1, ksplit=ks):
         fp6_marlin.mul(A, B, plain, s, ws, qc, group_size=128)
         fp6_marlin.mul_fused(A, B, mapped, s, ws, qc, 128, c_cols=c_cols)
         fp6_marlin.mul_fused(A, B, full, s, ws, qc, 128, c_cols=c_cols, bias=bias, residual=res)
@@ -171,3 +265,44 @@ def test_a_gather_that_no_staged_row_serves_stays_with_the_one_wave_kernel(oracl
     assert takes(4096, 11008, 11008) and takes(12288, 4096, 4104) and takes(8192, 8192, 14336)
     assert not takes(4096, 11008, 11009) and not takes(8192, 8192, 14344) and not takes(24192, 2048, 18432)
     assert not takes(4096, 28672, 28672) and not takes(40960, 2048, 2048)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wk", [4, 8])
+def test_gather_on_gfx950_order_gives_the_same_bits(oracle, wk):
+    import fp6_marlin
+    for n, k, qc, gs in ((512, 640, 256, 128), (256, 2048, 256, -1), (384, 1152, 128, -1)):
+        _, B, s = problem(oracle, n, k, qc, gs)
+        Bn = fp6_marlin.repack_gfx950(B, k, n, qc)
+        g, lda = torch.Generator().manual_seed(k), k + 72
+        A = torch.randn((1, lda), generator=g).half().to(dev())
+        cols = torch.randperm(lda, generator=g)[:k].to(torch.int32).to(dev())
+        ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+        for ks in (1, 3):
+            out = [torch.full((1, n), float("nan"), dtype=torch.half, device=dev()) for _ in range(3)]
+            with fp6_marlin.cabi.tuning(m1=3, wk16=wk, ksplit=ks):
+                fp6_marlin.mul(A[:, cols.long()].contiguous(), B, out[0], s, ws, qc, group_size=gs)
+                fp6_marlin.mul_fused(A, B, out[1], s, ws, qc, gs, a_cols=cols)
+                fp6_marlin.mul_fused(A, Bn, out[2], s, ws, qc, gs, a_cols=cols, layout="gfx950")
+                torch.cuda.synchronize()
+            assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_an_activation_that_is_not_finite_leaves_no_finite_output(oracle, value):
+    """Times a weight of zero it is a NaN too; a tile in parts saturates beyond the range of half."""
+    import fp6_marlin
+    n, k, qc = 384, 1152, 128
+    for gs in (-1, 128):
+        _, B, s = problem(oracle, n, k, qc, gs)
+        A = torch.randn((1, k), generator=torch.Generator().manual_seed(1)).half()
+        A[0, 700] = value
+        ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
+        for wk in (4, 8):
+            for ks in (1, 3):
+                C = torch.zeros((1, n), dtype=torch.half, device=dev())
+                with fp6_marlin.cabi.tuning(m1=4, wk16=wk, ksplit=ks):
+                    fp6_marlin.mul(A.to(dev()), B, C, s, ws, qc, group_size=gs)
+                    torch.cuda.synchronize()
+                assert not torch.isfinite(C).any()
