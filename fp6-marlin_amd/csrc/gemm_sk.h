@@ -505,29 +505,26 @@ __device__ __forceinline__ void sk_wave(const SkArgs& p, int j, FP6M_AS3 unsigne
         for (int s = 0; s < seg_steps; s += kUnroll) {
 #pragma unroll
             for (int uu = 0; uu < kUnroll; uu++) {
-                const bool fetches = DRAW || GR > 0 || i_left > 0;        // (past the end of its one chunk a wave fetches nothing)
-                bool scales = false;
-                if (fetches) {
-                    scales = issue(slot_in, ((uu + DEPTH - 1) & 1) == 0);
+                if (DRAW || GR > 0 || i_left > 0) {                       // (uniform)
+                    const bool scales = issue(slot_in, ((uu + DEPTH - 1) & 1) == 0);
                     slot_in = slot_in + 1 == DEPTH ? 0 : slot_in + 1;
-                }
-                if (kGroup && uu == 1) scales_in_flight = scales;         // the fetch of the step four on: a multiple of four
-                const bool one_more = kGroup && (uu == 1 || uu == 2) && scales_in_flight;
-                if (!fetches) {                                           // (one step newer than the next at most: the chunk's last)
-                    if (DEPTH == 4 && seg_steps - (s + uu) == 3)
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(kWordOps));
-                    else
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-                } else if (uu & 1) {                                      // the next step has landed
-                    if (one_more)
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(kWaitOdd + 1));
-                    else
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(kWaitOdd));
+                    if (kGroup && uu == 1) scales_in_flight = scales;     // the fetch of the step four on: a multiple of four
+                    const bool one_more = kGroup && (uu == 1 || uu == 2) && scales_in_flight;
+                    if (uu & 1) {                                         // the next step has landed
+                        if (one_more)
+                            __builtin_amdgcn_s_waitcnt(vmcnt_only(kWaitOdd + 1));
+                        else
+                            __builtin_amdgcn_s_waitcnt(vmcnt_only(kWaitOdd));
+                    } else {
+                        if (one_more)
+                            __builtin_amdgcn_s_waitcnt(vmcnt_only(kWaitEven + 1));
+                        else
+                            __builtin_amdgcn_s_waitcnt(vmcnt_only(kWaitEven));
+                    }
+                } else if (DEPTH == 4 && seg_steps - (s + uu) == 3) {     // past the end of its one chunk a wave fetches nothing
+                    __builtin_amdgcn_s_waitcnt(vmcnt_only(kWordOps));     // (the only newer step: the chunk's last)
                 } else {
-                    if (one_more)
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(kWaitEven + 1));
-                    else
-                        __builtin_amdgcn_s_waitcnt(vmcnt_only(kWaitEven));
+                    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
                 }
                 if (uu & 1) pair_rd = pair_rd + 1 == kPairSlots ? 0 : pair_rd + 1;   // the next step opens a pair
                 if constexpr (GR > 0) {
