@@ -1488,7 +1488,7 @@ int mul_common(const void* A, const void* B, void* C, const void* s, int prob_m,
                     return cut;
                 };
                 us_wide = m16_time(false, cut_of(false, cfg.wk, ks), a.m, g128, mbytes, cus);
-                double best = (qc < prob_n ? kHalfMargin : kHalfMarginFp6) * us_wide;
+                double best = half_margin(qc == prob_n, row_mix) * us_wide;
                 int best_wk = 0;
                 long long best_ks = 0;
                 for (int wk = 4; wk <= 8; wk += 4)

@@ -27,8 +27,10 @@ struct M16Cut {
 // 1024 FP6 columns.  Hence the margins by which 64-column tiles have to be ahead: over 2013 calls at other random shapes they are
 // taken 1314 times and 16 % faster on average, twice more than 2 % slower (with 2 % instead of 4 eleven times, 9 x 18560 x 4352 14.6 us against
 // 13.5); over 2279 of FP6 columns alone, whose times the estimates miss by 4-10 %, 1539 times and 16 %, twice (with 2 % instead of 8
-// 35 times, 14 x 19328 x 4608 19.5 against 17.5).
-constexpr double kHalfMargin = 0.96, kHalfMarginFp6 = 0.92;
+// 35 times, 14 x 19328 x 4608 19.5 against 17.5).  Row mixes: with 4 % five of 2342 calls were 5 to 12 % slower (1 x 1792 x 20224 with 512
+// FP6 rows 9.2 against 8.2), with 8 % one of 2150, by 3 %.  (Words in gfx950 order gain less -- of 714 such calls six are 4 to 8 % slower
+// -- but take what the reference's order takes, for the same bits.)
+inline double half_margin(bool all_fp6, bool row_mix) { return all_fp6 || row_mix ? 0.92 : 0.96; }
 struct M16Time {
     // us once; once with a split, per part, and per part and row; per step of the longest slice, of the mean one, of the mean one
     // at full occupation, per row that A is fetched in, and with group scales; per step by which 1.7 FP6 steps exceed an INT4

@@ -100,6 +100,8 @@ inline double sk_time(int units, long long n4, long long qc, bool g128)
 // by it, 14 % faster on average; 25 of those are more than 2 % slower, the worst 8 %.  With 6 % instead of 5 it would be fewer, but square
 // shapes in whole parts, 8192 x 8192 9.4 us against 10.3, would go back.  Fewer than twelve units with a fifth or more of the columns in FP6,
 // whose few waves then end last, were 2 % slower on average (1280 x 3968, 1024 of them FP6, 4.9 us against 4.5).
+// Words in gfx950 order, of which a 64-column tile reads half of every tile's lines, gain 4 % less: 15 of 1096 such calls are more than
+// 4 % slower than one-wave workgroups (20224 x 6272 17.5 us against 15.7).  They take what the reference's order takes, for the same bits.
 inline M1Plan m1_choice(int units, long long n4, long long qc, bool g128, int cus, int young_pct)
 {
     M1Plan plan = m1_plan(units, n4, qc, g128, cus, young_pct);

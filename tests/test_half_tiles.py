@@ -233,20 +233,26 @@ def test_where_the_narrow_tiles_are_taken(oracle, capfd):
 
 @pytest.mark.gpu
 def test_calls_near_the_line_keep_the_wide_tiles(oracle, capfd):
-    """Calls on which tiles of 64 columns were 5 to 12 % slower than tiles of 128, and two on which they are a quarter faster."""
+    """Calls on which tiles of 64 columns were 5 to 12 % slower than tiles of 128, and some on which they are far faster."""
     import fp6_marlin
 
-    def takes(m, k, n, qc, gs):
-        B = torch.zeros(k * (n - qc) // 8 + k * qc * 3 // 16, dtype=torch.int32, device=dev())
-        s = torch.zeros((k // 128 if gs == 128 else 1) * (n - qc) + qc, dtype=torch.half, device=dev())
+    def takes(m, k, n, qc, gs, qr=0):
+        B = torch.zeros((k - qr) * (n - qc) // 8 + (k * qc + qr * n) * 3 // 16, dtype=torch.int32, device=dev())
+        s = torch.zeros(((k - qr) // 128 if gs == 128 else 1) * (n - qc) + (n if qr else qc), dtype=torch.half, device=dev())
         A, C = torch.zeros((m, k), dtype=torch.half, device=dev()), torch.empty((m, n), dtype=torch.half, device=dev())
         ws = torch.zeros(n // 128 * 16, dtype=torch.int32, device=dev())
         capfd.readouterr()
         with fp6_marlin.cabi.tuning(verbose=1):
-            fp6_marlin.mul(A, B, C, s, ws, qc if qc else -1, group_size=gs)
+            if qr:
+                fp6_marlin.mul_rows(A, B, C, s, ws, qr)
+            else:
+                fp6_marlin.mul(A, B, C, s, ws, qc if qc else -1, group_size=gs)
             torch.cuda.synchronize()
         return " half " in capfd.readouterr().err
 
+    for m, k, n, qr in ((1, 1792, 20224, 512), (1, 1792, 17664, 512), (3, 1664, 21248, 512), (12, 1664, 17024, 512)):
+        assert not takes(m, k, n, 0, 128, qr=qr)
+    assert takes(16, 4096, 4096, 0, 128, qr=256)
     for m, k, n, qc, gs in ((9, 18560, 4352, 256, 128), (7, 14464, 7040, 0, -1), (10, 17664, 4864, 256, 128), (15, 15616, 3968, 256, 128)):
         assert not takes(m, k, n, qc, gs)
     for m, k, n in ((14, 19328, 4608), (12, 12288, 7296), (10, 10752, 6912), (16, 17024, 5248), (15, 18560, 4608), (10, 11392, 7424)):
